@@ -59,6 +59,43 @@ __device__ __forceinline__ double recip_refined(double b) {
   return r;
 }
 
+// Reciprocals of two, three or four denominators from one hardware reciprocal
+// of their product: R = 1/(b1 b2 ..) takes the first refinement, R times the
+// other denominators approximates each 1/b_k to 2^-48 (as one refined rcp
+// does: its seed is good to 2^-24.4), and the last refinement is the one of
+// recip_refined.  v_rcp_f64 takes the issue time of 3.4 multiplications
+// (7.2 against 2.1 ns per wave and SIMD), so three reciprocals cost 17 slots
+// instead of 22 and four 22 instead of 29.  Callers keep the product inside
+// the exponent range (kWenoLo, kWenoHi).
+__device__ __forceinline__ double newton(double b, double r) { return fma(r, fma(-b, r, 1.0), r); }
+
+__device__ __forceinline__ void recip2(double b1, double b2, double& r1, double& r2) {
+  const double P = b1 * b2;
+  const double R = newton(P, __builtin_amdgcn_rcp(P));
+  r1 = newton(b1, R * b2);
+  r2 = newton(b2, R * b1);
+}
+
+__device__ __forceinline__ void recip3(double b1, double b2, double b3, double& r1, double& r2,
+                                       double& r3) {
+  const double p = b1 * b2, P = p * b3;
+  const double R = newton(P, __builtin_amdgcn_rcp(P));
+  const double t = R * b3;
+  r1 = newton(b1, t * b2);
+  r2 = newton(b2, t * b1);
+  r3 = newton(b3, R * p);
+}
+
+__device__ __forceinline__ void recip4(const double b[4], double r[4]) {
+  const double p = b[0] * b[1], q = b[2] * b[3], P = p * q;
+  const double R = newton(P, __builtin_amdgcn_rcp(P));
+  const double tp = R * q, tq = R * p;
+  r[0] = newton(b[0], tp * b[1]);
+  r[1] = newton(b[1], tp * b[0]);
+  r[2] = newton(b[2], tq * b[3]);
+  r[3] = newton(b[3], tq * b[2]);
+}
+
 __device__ __forceinline__ double div_by(double a, double b, double rb) {
   double q = a * rb;
   double e = fma(-b, q, a);
@@ -87,7 +124,8 @@ __device__ __forceinline__ void cons_to_prim(double h, double hu, double hv, dou
 }
 
 // Smoothness indicators shared by both WENO5 sweeps,
-// src/reconstruction.f90:699-704 and :1024-1029, and (eps + beta)^2.
+// src/reconstruction.f90:699-704 and :1024-1029, and (eps + beta)^2, with the
+// reference's operations one by one.
 __device__ __forceinline__ void weno5_den(double qm2, double qm1, double q0, double qp1,
                                           double qp2, double& d1, double& d2, double& d3) {
   double b1 = (1.0 / 3.0) * (4.0 * qm2 * qm2 - 19.0 * qm2 * qm1 + 25.0 * qm1 * qm1 +
@@ -101,44 +139,78 @@ __device__ __forceinline__ void weno5_den(double qm2, double qm1, double q0, dou
   d3 = (kWenoEps + b3) * (kWenoEps + b3);
 }
 
+// The same d1..d3 bit for bit wherever weno5_regular accepts them, with the
+// factors 4 folded into exact FMAs: 4*q*q = 4*(q*q) and fma(4, q*q, y) rounds
+// 4*q*q + y once, as the separate addition does.  Scaling by 4 commutes with
+// rounding unless q*q is subnormal; an error there is at most 2^-1074 and can
+// pass through a rounded sum only where the sum is below 2^-960 (a later sum
+// of this chain: below 2^-690), so it never reaches eps + beta with
+// eps = 10^-24 = 2^-79.7.
+__device__ __forceinline__ void weno5_den_exact(double qm2, double qm1, double q0, double qp1,
+                                                double qp2, double& d1, double& d2, double& d3) {
+  const double s1 = qm1 * qm1, sp1 = qp1 * qp1;
+  const double x0 = 13.0 * q0, c0 = 10.0 * q0 * q0;
+  const double b1 = (1.0 / 3.0) * (fma(4.0, qm2 * qm2, -(19.0 * qm2 * qm1)) + 25.0 * qm1 * qm1 +
+                                   11.0 * qm2 * q0 - 31.0 * qm1 * q0 + c0);
+  const double b2 = (1.0 / 3.0) * fma(4.0, sp1, fma(4.0, s1, -(13.0 * qm1 * q0)) + x0 * q0 +
+                                                    5.0 * qm1 * qp1 - x0 * qp1);
+  const double b3 = (1.0 / 3.0) * fma(4.0, qp2 * qp2, c0 - 31.0 * q0 * qp1 + 25.0 * qp1 * qp1 +
+                                                          11.0 * q0 * qp2 - 19.0 * qp1 * qp2);
+  d1 = (kWenoEps + b1) * (kWenoEps + b1);
+  d2 = (kWenoEps + b2) * (kWenoEps + b2);
+  d3 = (kWenoEps + b3) * (kWenoEps + b3);
+}
+
+// The range in which a reconstruction takes the shared reciprocals: the three
+// (eps + beta)^2 in [2^-240, 2^240).  Then the products of recip3 and recip4
+// lie in 2^+-976, the alphas in [2^-244, 2^240], their sums in
+// [2^-244, 2^242] and the weights above 2^-486; and every q is finite and
+// below 2^100, since an Inf or NaN q would make one of the three Inf or NaN.
+// They are squares, so their high words compare as unsigned integers (a NaN
+// of either sign is above the range): two three-operand min/max and two
+// compares instead of six FP64 compares.
+constexpr unsigned kWenoLo = (1023u - 240u) << 20;
+constexpr unsigned kWenoHi = (1023u + 240u) << 20;
+__device__ __forceinline__ bool weno5_regular(double d1, double d2, double d3) {
+  const unsigned h1 = __double2hiint(d1), h2 = __double2hiint(d2), h3 = __double2hiint(d3);
+  return (int)(min(min(h1, h2), h3) >= kWenoLo) & (int)(max(max(h1, h2), h3) < kWenoHi);
+}
+
 // WENO5_FirstSweep, src/reconstruction.f90:673-755: cell average line values
 // at the left (wm) and right (wp) faces.
 __device__ __forceinline__ void weno5_first(double qm2, double qm1, double q0, double qp1,
                                             double qp2, double& wm, double& wp) {
   double d1, d2, d3;
-  weno5_den(qm2, qm1, q0, qp1, qp2, d1, d2, d3);
 #if SWM_SHARED_RECIP
-  // With the (eps+beta)^2 in [2^-400, 2^400] the alphas lie in
-  // [2^-404, 2^400], their sum in [2^-404, 2^402] and the weights above 2^-806.
-  if (recip_range(d1) & recip_range(d2) & recip_range(d3)) {
-    const double r1 = recip_refined(d1), r2 = recip_refined(d2), r3 = recip_refined(d3);
+  weno5_den_exact(qm2, qm1, q0, qp1, qp2, d1, d2, d3);
+  if (weno5_regular(d1, d2, d3)) {
+    double r1, r2, r3;
+    recip3(d1, d2, d3, r1, r2, r3);
+    const double am1 = div_by(3.0 / 10.0, d1, r1), ap1 = div_by(1.0 / 10.0, d1, r1);
+    const double a2 = div_by(3.0 / 5.0, d2, r2);
+    const double am3 = div_by(1.0 / 10.0, d3, r3), ap3 = div_by(3.0 / 10.0, d3, r3);
+    const double sm = am1 + a2 + am3, sp = ap1 + a2 + ap3;
+    double rm, rp;
+    recip2(sm, sp, rm, rp);
+    // doubling is exact, so 2*q + y is one FMA
     {
-      double a1 = div_by(3.0 / 10.0, d1, r1);
-      double a2 = div_by(3.0 / 5.0, d2, r2);
-      double a3 = div_by(1.0 / 10.0, d3, r3);
-      double s = a1 + a2 + a3;
-      double rs = recip_refined(s);
-      double o1 = div_by(a1, s, rs), o2 = div_by(a2, s, rs), o3 = div_by(a3, s, rs);
-      double w1 = (1.0 / 6.0) * (-qm2 + 5.0 * qm1 + 2.0 * q0);
-      double w2 = (1.0 / 6.0) * (2.0 * qm1 + 5.0 * q0 - qp1);
-      double w3 = (1.0 / 6.0) * (11.0 * q0 - 7.0 * qp1 + 2.0 * qp2);
+      const double o1 = div_by(am1, sm, rm), o2 = div_by(a2, sm, rm), o3 = div_by(am3, sm, rm);
+      const double w1 = (1.0 / 6.0) * fma(2.0, q0, -qm2 + 5.0 * qm1);
+      const double w2 = (1.0 / 6.0) * (fma(2.0, qm1, 5.0 * q0) - qp1);
+      const double w3 = (1.0 / 6.0) * fma(2.0, qp2, 11.0 * q0 - 7.0 * qp1);
       wm = o1 * w1 + o2 * w2 + o3 * w3;
     }
     {
-      double a1 = div_by(1.0 / 10.0, d1, r1);
-      double a2 = div_by(3.0 / 5.0, d2, r2);
-      double a3 = div_by(3.0 / 10.0, d3, r3);
-      double s = a1 + a2 + a3;
-      double rs = recip_refined(s);
-      double o1 = div_by(a1, s, rs), o2 = div_by(a2, s, rs), o3 = div_by(a3, s, rs);
-      double w1 = (1.0 / 6.0) * (2.0 * qm2 - 7.0 * qm1 + 11.0 * q0);
-      double w2 = (1.0 / 6.0) * (-qm1 + 5.0 * q0 + 2.0 * qp1);
-      double w3 = (1.0 / 6.0) * (2.0 * q0 + 5.0 * qp1 - qp2);
+      const double o1 = div_by(ap1, sp, rp), o2 = div_by(a2, sp, rp), o3 = div_by(ap3, sp, rp);
+      const double w1 = (1.0 / 6.0) * (fma(2.0, qm2, -(7.0 * qm1)) + 11.0 * q0);
+      const double w2 = (1.0 / 6.0) * fma(2.0, qp1, -qm1 + 5.0 * q0);
+      const double w3 = (1.0 / 6.0) * (fma(2.0, q0, 5.0 * qp1) - qp2);
       wp = o1 * w1 + o2 * w2 + o3 * w3;
     }
     return;
   }
 #endif
+  weno5_den(qm2, qm1, q0, qp1, qp2, d1, d2, d3);
   {
     double a1 = (3.0 / 10.0) / d1;
     double a2 = (3.0 / 5.0) / d2;
@@ -209,39 +281,57 @@ __device__ __forceinline__ void weno2_cand(double qm2, double qm1, double q0, do
   w3 = C.c30 * qm2 + C.c31 * qm1 + C.c32 * q0 + C.c33 * qp1 + C.c34 * qp2;
 }
 
-// omega_k = alpha_k / sum(alpha), alpha_k = gamma_k / (eps + beta_k)^2
-// (src/reconstruction.f90:1030-1035), through shared reciprocals (SHARED) or '/'.
-template <int G, bool SHARED>
-__device__ __forceinline__ void weno2_weights(double d1, double d2, double d3, double r1,
-                                              double r2, double r3, double& o1, double& o2,
-                                              double& o3) {
+// The same candidates without the 0.0*Q terms, for finite q: they can change
+// only the sign of a zero sum, and every sum has a positive coefficient
+// (at least 0.4) on q0, so no sum is -0 unless q0 is -0 or a negative
+// subnormal that the product rounds to -0 (weno5_second sends those to the
+// full form).
+template <int G>
+__device__ __forceinline__ void weno2_cand_nz(double qm2, double qm1, double q0, double qp1,
+                                              double qp2, double& w1, double& w2, double& w3) {
   constexpr Weno2Coef C = weno2_coef<G>();
-  if constexpr (SHARED) {
-    double a1 = div_by(C.g1, d1, r1);
-    double a2 = div_by(C.g2, d2, r2);
-    double a3 = div_by(C.g3, d3, r3);
-    double s = a1 + a2 + a3;
-    double rs = recip_refined(s);
-    o1 = div_by(a1, s, rs);
-    o2 = div_by(a2, s, rs);
-    o3 = div_by(a3, s, rs);
-  } else {
-    double a1 = C.g1 / d1;
-    double a2 = C.g2 / d2;
-    double a3 = C.g3 / d3;
-    double s = a1 + a2 + a3;
-    o1 = a1 / s;
-    o2 = a2 / s;
-    o3 = a3 / s;
-  }
+  static_assert(C.c13 == 0. && C.c14 == 0. && C.c20 == 0. && C.c24 == 0. && C.c30 == 0. &&
+                    C.c31 == 0. && C.c12 > 0.4 && C.c22 > 0.4 && C.c32 > 0.4,
+                "the terms left out are zeros");
+  w1 = C.c10 * qm2 + C.c11 * qm1 + C.c12 * q0;
+  w2 = C.c21 * qm1 + C.c22 * q0 + C.c23 * qp1;
+  w3 = C.c32 * q0 + C.c33 * qp1 + C.c34 * qp2;
 }
 
-template <int G, bool SHARED>
+// alpha_k = gamma_k / (eps + beta_k)^2 (src/reconstruction.f90:1030-1032)
+// through the shared reciprocals, and their sum.
+template <int G>
+__device__ __forceinline__ double weno2_alpha(double d1, double d2, double d3, double r1,
+                                              double r2, double r3, double a[3]) {
+  constexpr Weno2Coef C = weno2_coef<G>();
+  a[0] = div_by(C.g1, d1, r1);
+  a[1] = div_by(C.g2, d2, r2);
+  a[2] = div_by(C.g3, d3, r3);
+  return a[0] + a[1] + a[2];
+}
+
+// omega_k = alpha_k / sum(alpha) (src/reconstruction.f90:1033-1035) and the
+// weighted candidates.
+template <int G>
+__device__ __forceinline__ double weno2_blend(double qm2, double qm1, double q0, double qp1,
+                                              double qp2, const double a[3], double s, double rs) {
+  const double o1 = div_by(a[0], s, rs), o2 = div_by(a[1], s, rs), o3 = div_by(a[2], s, rs);
+  double w1, w2, w3;
+  weno2_cand_nz<G>(qm2, qm1, q0, qp1, qp2, w1, w2, w3);
+  return (o1 * w1 + o2 * w2 + o3 * w3);
+}
+
+// One Gauss point with '/' and every term.
+template <int G>
 __device__ __forceinline__ double weno5_second_gp(double qm2, double qm1, double q0, double qp1,
-                                                  double qp2, double d1, double d2, double d3,
-                                                  double r1, double r2, double r3) {
-  double o1, o2, o3, w1, w2, w3;
-  weno2_weights<G, SHARED>(d1, d2, d3, r1, r2, r3, o1, o2, o3);
+                                                  double qp2, double d1, double d2, double d3) {
+  constexpr Weno2Coef C = weno2_coef<G>();
+  double a1 = C.g1 / d1;
+  double a2 = C.g2 / d2;
+  double a3 = C.g3 / d3;
+  double s = a1 + a2 + a3;
+  double o1 = a1 / s, o2 = a2 / s, o3 = a3 / s;
+  double w1, w2, w3;
   weno2_cand<G>(qm2, qm1, q0, qp1, qp2, w1, w2, w3);
   return (o1 * w1 + o2 * w2 + o3 * w3);
 }
@@ -251,22 +341,30 @@ __device__ __forceinline__ double weno5_second_gp(double qm2, double qm1, double
 __device__ __forceinline__ void weno5_second(double qm2, double qm1, double q0, double qp1,
                                              double qp2, double w[4]) {
   double d1, d2, d3;
-  weno5_den(qm2, qm1, q0, qp1, qp2, d1, d2, d3);
 #if SWM_SHARED_RECIP
-  // the gammas lie in [0.12, 0.62]: same ranges as in weno5_first
-  if (recip_range(d1) & recip_range(d2) & recip_range(d3)) {
-    const double r1 = recip_refined(d1), r2 = recip_refined(d2), r3 = recip_refined(d3);
-    w[0] = weno5_second_gp<0, true>(qm2, qm1, q0, qp1, qp2, d1, d2, d3, r1, r2, r3);
-    w[1] = weno5_second_gp<1, true>(qm2, qm1, q0, qp1, qp2, d1, d2, d3, r1, r2, r3);
-    w[2] = weno5_second_gp<2, true>(qm2, qm1, q0, qp1, qp2, d1, d2, d3, r1, r2, r3);
-    w[3] = weno5_second_gp<3, true>(qm2, qm1, q0, qp1, qp2, d1, d2, d3, r1, r2, r3);
+  weno5_den_exact(qm2, qm1, q0, qp1, qp2, d1, d2, d3);
+  // the gammas lie in [0.12, 0.62]: the ranges of weno5_regular hold
+  if ((int)weno5_regular(d1, d2, d3) &
+      (int)((unsigned)__double2hiint(q0) != 0x80000000u)) {
+    double r1, r2, r3, a[4][3], s[4], rs[4];
+    recip3(d1, d2, d3, r1, r2, r3);
+    s[0] = weno2_alpha<0>(d1, d2, d3, r1, r2, r3, a[0]);
+    s[1] = weno2_alpha<1>(d1, d2, d3, r1, r2, r3, a[1]);
+    s[2] = weno2_alpha<2>(d1, d2, d3, r1, r2, r3, a[2]);
+    s[3] = weno2_alpha<3>(d1, d2, d3, r1, r2, r3, a[3]);
+    recip4(s, rs);
+    w[0] = weno2_blend<0>(qm2, qm1, q0, qp1, qp2, a[0], s[0], rs[0]);
+    w[1] = weno2_blend<1>(qm2, qm1, q0, qp1, qp2, a[1], s[1], rs[1]);
+    w[2] = weno2_blend<2>(qm2, qm1, q0, qp1, qp2, a[2], s[2], rs[2]);
+    w[3] = weno2_blend<3>(qm2, qm1, q0, qp1, qp2, a[3], s[3], rs[3]);
     return;
   }
 #endif
-  w[0] = weno5_second_gp<0, false>(qm2, qm1, q0, qp1, qp2, d1, d2, d3, 0., 0., 0.);
-  w[1] = weno5_second_gp<1, false>(qm2, qm1, q0, qp1, qp2, d1, d2, d3, 0., 0., 0.);
-  w[2] = weno5_second_gp<2, false>(qm2, qm1, q0, qp1, qp2, d1, d2, d3, 0., 0., 0.);
-  w[3] = weno5_second_gp<3, false>(qm2, qm1, q0, qp1, qp2, d1, d2, d3, 0., 0., 0.);
+  weno5_den(qm2, qm1, q0, qp1, qp2, d1, d2, d3);
+  w[0] = weno5_second_gp<0>(qm2, qm1, q0, qp1, qp2, d1, d2, d3);
+  w[1] = weno5_second_gp<1>(qm2, qm1, q0, qp1, qp2, d1, d2, d3);
+  w[2] = weno5_second_gp<2>(qm2, qm1, q0, qp1, qp2, d1, d2, d3);
+  w[3] = weno5_second_gp<3>(qm2, qm1, q0, qp1, qp2, d1, d2, d3);
 }
 
 #ifndef SWM_LIMITER_SKIP
