@@ -129,6 +129,51 @@ struct FaceTile {
   static constexpr int LDS = (3 * NV + 6 * NQ > 12 * NT) ? 3 * NV + 6 * NQ : 12 * NT;
 };
 
+// Gauss sum of the Rusanov fluxes of one face (src/finitevolume.f90:546-640)
+// between WP of the cell below the face and wm of the one above it (value a
+// of 12 at wm[a * stride]).  The regular form holds for finite states with
+// depths in range (irregular = 0); a state that is not finite shows in one of
+// its sums, and the face is then taken again with the reference's operations
+// one by one.
+template <bool X>
+__device__ __forceinline__ void face_flux(const JobDev& J, const double WP[3][4],
+                                          const double* wm, int stride, int irregular,
+                                          double& acc1, double& acc2, double& acc3) {
+  constexpr int N = X ? 1 : 2, T = X ? 2 : 1;  // normal and tangential velocity
+  if (!irregular) {
+    double a1 = 0.0, an = 0.0, at = 0.0;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      double F1, Fn, Ft;
+      rusanov_regular(WP[0][g], WP[N][g], WP[T][g], wm[g * stride], wm[(4 * N + g) * stride],
+                      wm[(4 * T + g) * stride], J.g, F1, Fn, Ft);
+      a1 = a1 + J.wbnd[g] * F1;
+      an = an + J.wbnd[g] * Fn;
+      at = at + J.wbnd[g] * Ft;
+    }
+    acc1 = a1;
+    acc2 = X ? an : at;
+    acc3 = X ? at : an;
+    if ((int)is_finite(a1) & (int)is_finite(an) & (int)is_finite(at)) return;
+  }
+  acc1 = acc2 = acc3 = 0.0;
+#pragma unroll 1
+  for (int g = 0; g < 4; ++g) {
+    double F1, F2, F3;
+    // the Gauss point's values by selects: WP stays in registers
+    double wp[3];
+#pragma unroll
+    for (int v = 0; v < 3; ++v)
+      wp[v] = g == 0 ? WP[v][0] : g == 1 ? WP[v][1] : g == 2 ? WP[v][2] : WP[v][3];
+    rusanov<X ? 1 : 0, X ? 0 : 1, X ? 0 : -1, X ? 1 : 0>(wp[0], wp[1], wp[2], wm[g * stride],
+                                                         wm[(4 + g) * stride],
+                                                         wm[(8 + g) * stride], J.g, F1, F2, F3);
+    acc1 = acc1 + J.wbnd[g] * F1;
+    acc2 = acc2 + J.wbnd[g] * F2;
+    acc3 = acc3 + J.wbnd[g] * F3;
+  }
+}
+
 template <int TW, int TH>
 __global__ __launch_bounds__(TW * TH) void k_fvtd_x(EngineArgs E, const TileRef* tiles,
                                                     NodeList L) {
@@ -139,6 +184,7 @@ __global__ __launch_bounds__(TW * TH) void k_fvtd_x(EngineArgs E, const TileRef*
   double* sV = smem;            // [3][VH rows][VW cols]
   double* sQM = smem + 3 * NV;  // [3][VH rows][TW cols]
   double* sQP = sQM + 3 * NQ;
+  __shared__ int irregular;  // a cell whose depths sqrt_regular may not take
   const TileRef T = tiles[blockIdx.x];
   const JobDev& J = E.jobs[T.job];
   if (skipped(E, J)) return;
@@ -150,6 +196,8 @@ __global__ __launch_bounds__(TW * TH) void k_fvtd_x(EngineArgs E, const TileRef*
   const int j0 = (T.tile / ntx) * TH + 1;
   const gdouble *h, *hu, *hv;
   node_state(J, m, h, hu, hv);
+  // g h stays in the range of sqrt_regular for the depths of depths_regular
+  if (tid == 0) irregular = !(J.g >= 0x1p-60 && J.g <= 0x1p60);
 
   for (int t = tid; t < NV; t += NT) {
     int lx = t % VW, ly = t / VW;
@@ -196,7 +244,14 @@ __global__ __launch_bounds__(TW * TH) void k_fvtd_x(EngineArgs E, const TileRef*
     }
   }
   const double vh = sV[(ty + 2) * VW + tx + 2];
-  if (c <= nx) positivity_limit(vh, J.wbnd, WM[0], WP[0]);
+  double mn = vh;
+  if (c <= nx) {
+    mn = positivity_limit(vh, J.wbnd, WM[0], WP[0]);
+  } else {  // the unlimited ghost: only its WM is used
+#pragma unroll
+    for (int g = 0; g < 4; ++g) mn = min_n(mn, WM[0][g]);
+  }
+  if (!depths_regular(vh, mn)) irregular = 1;
   __syncthreads();
   double* sWM = smem;  // [12][NT]
 #pragma unroll
@@ -204,17 +259,8 @@ __global__ __launch_bounds__(TW * TH) void k_fvtd_x(EngineArgs E, const TileRef*
   __syncthreads();
   const int j = j0 + ty;
   if (tx < TW - 1 && c <= nx && j <= ny) {
-    double acc1 = 0.0, acc2 = 0.0, acc3 = 0.0;
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      double F1, F2, F3;
-      rusanov<1, 0, 0, 1>(WP[0][g], WP[1][g], WP[2][g], sWM[(0 + g) * NT + tid + 1],
-                          sWM[(4 + g) * NT + tid + 1], sWM[(8 + g) * NT + tid + 1], J.g, F1,
-                          F2, F3);
-      acc1 = acc1 + J.wbnd[g] * F1;
-      acc2 = acc2 + J.wbnd[g] * F2;
-      acc3 = acc3 + J.wbnd[g] * F3;
-    }
+    double acc1, acc2, acc3;
+    face_flux<true>(J, WP, sWM + tid + 1, NT, irregular, acc1, acc2, acc3);
     size_t o = (size_t)(j - 1) * (nx + 1) + c;
     if (J.wb && !L.wb_init) {  // FX = FX - FXWB (src/finitevolume.f90:485-486)
       acc1 = acc1 - G(J.FXWB[0])[o];
@@ -241,6 +287,7 @@ __global__ __launch_bounds__(TW * TH) void k_fvtd_y(EngineArgs E, const TileRef*
   double* sV = smem;            // [3][VH rows][VW cols]
   double* sQM = smem + 3 * NV;  // [3][TH rows][VW cols]
   double* sQP = sQM + 3 * NQ;
+  __shared__ int irregular;  // a cell whose depths sqrt_regular may not take
   const TileRef T = tiles[blockIdx.x];
   const JobDev& J = E.jobs[T.job];
   if (skipped(E, J)) return;
@@ -252,6 +299,8 @@ __global__ __launch_bounds__(TW * TH) void k_fvtd_y(EngineArgs E, const TileRef*
   const int r0 = (T.tile / ntx) * (TH - 1);
   const gdouble *h, *hu, *hv;
   node_state(J, m, h, hu, hv);
+  // g h stays in the range of sqrt_regular for the depths of depths_regular
+  if (tid == 0) irregular = !(J.g >= 0x1p-60 && J.g <= 0x1p60);
 
   for (int t = tid; t < NV; t += NT) {
     int lx = t % VW, ly = t / VW;
@@ -295,7 +344,14 @@ __global__ __launch_bounds__(TW * TH) void k_fvtd_y(EngineArgs E, const TileRef*
     }
   }
   const double vh = sV[(ty + 2) * VW + tx + 2];
-  if (r <= ny) positivity_limit(vh, J.wbnd, WM[0], WP[0]);
+  double mn = vh;
+  if (r <= ny) {
+    mn = positivity_limit(vh, J.wbnd, WM[0], WP[0]);
+  } else {  // the unlimited ghost: only its WM is used
+#pragma unroll
+    for (int g = 0; g < 4; ++g) mn = min_n(mn, WM[0][g]);
+  }
+  if (!depths_regular(vh, mn)) irregular = 1;
   __syncthreads();
   double* sWM = smem;  // [12][NT]
 #pragma unroll
@@ -303,17 +359,8 @@ __global__ __launch_bounds__(TW * TH) void k_fvtd_y(EngineArgs E, const TileRef*
   __syncthreads();
   const int i = i0 + tx;
   if (ty < TH - 1 && r <= ny && i <= nx) {
-    double acc1 = 0.0, acc2 = 0.0, acc3 = 0.0;
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      double F1, F2, F3;
-      rusanov<0, 1, -1, 0>(WP[0][g], WP[1][g], WP[2][g], sWM[(0 + g) * NT + tid + TW],
-                           sWM[(4 + g) * NT + tid + TW], sWM[(8 + g) * NT + tid + TW], J.g,
-                           F1, F2, F3);
-      acc1 = acc1 + J.wbnd[g] * F1;
-      acc2 = acc2 + J.wbnd[g] * F2;
-      acc3 = acc3 + J.wbnd[g] * F3;
-    }
+    double acc1, acc2, acc3;
+    face_flux<false>(J, WP, sWM + tid + TW, NT, irregular, acc1, acc2, acc3);
     size_t o = (size_t)r * nx + (i - 1);
     if (J.wb && !L.wb_init) {  // FY = FY - FYWB (src/finitevolume.f90:487-488)
       acc1 = acc1 - G(J.FYWB[0])[o];

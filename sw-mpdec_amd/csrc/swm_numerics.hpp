@@ -115,6 +115,14 @@ __device__ __forceinline__ double div_pos(double a, double b, double rb) {
   return a / b;
 }
 
+// The smaller of two values, the other one where one is NaN, in one
+// instruction (fmin() first quiets each operand with one of its own).
+__device__ __forceinline__ double min_n(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
 // ConsToPrim, src/equation.f90:912-945:  ht = h + MIN_DEPTH/h; u = hu/ht.
 __device__ __forceinline__ void cons_to_prim(double h, double hu, double hv, double& u,
                                              double& v) {
@@ -367,40 +375,79 @@ __device__ __forceinline__ void weno5_second(double qm2, double qm1, double q0, 
   w[3] = weno5_second_gp<3>(qm2, qm1, q0, qp1, qp2, d1, d2, d3);
 }
 
-#ifndef SWM_LIMITER_SKIP
-#define SWM_LIMITER_SKIP 1
-#endif
-
 // PositivityLimiterX/Y body, src/finitevolume.f90:671-691: theta-scaling of
 // the h values at the Gauss points of one cell towards the cell mean vh.
-__device__ __forceinline__ void positivity_limit(double vh, const double wbnd[4], double wm[4],
-                                                 double wp[4]) {
-  double alpha = 0., beta = 0.;
+// Returns the smallest of the unlimited values and csi (a NaN among them may
+// hide behind the others; then csi is NaN too).
+//
+// A theta is 1 without a division where |num| >= |den| with num finite (the
+// rounded |num/den| is then at least 1).  Every den_g = vh - mmin_g has mmin_g
+// between the smallest of all nine values and csi, and rounding is monotonic,
+// so comparing num with those two ends settles the four thetas at once -- the
+// usual case, the Gauss values lying close to the mean: 30 instructions
+// instead of 80.  A NaN or Inf among the values makes csi one, which fails
+// the comparison.
+__device__ __forceinline__ double positivity_limit(double vh, const double wbnd[4], double wm[4],
+                                                   double wp[4]) {
+  double alpha = wbnd[0] * wm[0], beta = wbnd[0] * wp[0];
+  double mn = min_n(wm[0], wp[0]);
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
+  for (int g = 1; g < 4; ++g) {
     alpha = alpha + wbnd[g] * wm[g];
     beta = beta + wbnd[g] * wp[g];
+    mn = min_n(mn, min_n(wm[g], wp[g]));
   }
-  double csi = (vh - kWLobatto * alpha - kWLobatto * beta) / (1. - 2. * kWLobatto);
+  constexpr double c = 1. - 2. * kWLobatto;
+  const double csi = div_pos(vh - kWLobatto * alpha - kWLobatto * beta, c, 1. / c);
+  mn = min_n(mn, csi);
+  const double num = vh - kMinDepth;
+  if ((int)(fabs(num) >= fabs(vh - csi)) & (int)(fabs(num) >= fabs(vh - mn))) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      wp[g] = vh + (wp[g] - vh);
+      wm[g] = vh + (wm[g] - vh);
+    }
+    return mn;
+  }
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     double mmin = min_r(min_r(csi, wm[g]), wp[g]);
-    const double num = vh - kMinDepth, den = vh - mmin;
+    const double den = vh - mmin;
     double theta;
     if (vh == mmin)
       theta = 1.;
-#if SWM_LIMITER_SKIP
-    // |num| >= |den| with num finite makes the rounded |num/den| >= 1, so
-    // MIN(1, |num/den|) is 1 without the division (the usual case: the
-    // Gauss values lie close to the mean)
     else if ((int)(fabs(num) >= fabs(den)) & (int)(fabs(num) <= kHuge))
       theta = 1.;
-#endif
     else
       theta = min_r(1., fabs(num / den));
     wp[g] = vh + theta * (wp[g] - vh);
     wm[g] = vh + theta * (wm[g] - vh);
   }
+  return mn;
+}
+
+// 1 when every limited depth of a cell is certain to lie in the range of
+// sqrt_regular: with the unlimited ones at least 2^-40 vh (mn is their
+// minimum), the limited ones, between them and vh but for two roundings of
+// vh, are at least 2^-41 vh.
+__device__ __forceinline__ bool depths_regular(double vh, double mn) {
+  return (int)(mn >= vh * 0x1p-40) & (int)(vh >= 0x1p-600);
+}
+
+// sqrt(x) for finite x in [2^-767, 2^1023): y ~ 1/sqrt(x) to 2^-24, one
+// Goldschmidt step for s ~ sqrt(x) and h ~ 1/(2 sqrt(x)), then two residual
+// corrections s + (x - s*s)*h with the residual exact in one FMA; the last
+// rounds a value accurate to 2^-99, the bits of sqrt().  sqrt() adds the
+// scaling of subnormal operands and the cases of 0 and Inf: 8 instructions
+// of 18.
+__device__ __forceinline__ double sqrt_regular(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double s = x * y, h = 0.5 * y;
+  const double e = fma(-h, s, 0.5);
+  s = fma(s, e, s);
+  h = fma(h, e, h);
+  s = fma(fma(-s, s, x), h, s);
+  return fma(fma(-s, s, x), h, s);
 }
 
 // EvaluateFlux1D, src/equation.f90:1014-1016
@@ -435,6 +482,28 @@ __device__ __forceinline__ void rusanov(double hl, double ul, double vl, double 
   F1 = f1;
   F2 = n1 * f2 + t1 * f3;
   F3 = n2 * f2 + t2 * f3;
+}
+
+// The same flux by normal velocity n* and tangential velocity t*, for finite
+// states with depths in the range of sqrt_regular: mass, normal and tangential
+// momentum.  The rotation's products with 0 only fix signs of zeros here, and
+// those die in the Gauss sum, which starts at +0; so they are left out, and
+// hl*nl serves as conserved momentum and as mass flux.
+__device__ __forceinline__ void rusanov_regular(double hl, double nl, double tl, double hr,
+                                                double nr, double tr, double g, double& F1,
+                                                double& Fn, double& Ft) {
+  const double ml = hl * nl, mr = hr * nr;
+  const double lmax =
+      max_r(fabs(nl + sqrt_regular(g * hl)), fabs(nr + sqrt_regular(g * hr)));
+  const double hg = 0.5 * g;
+  F1 = 0.5 * ((ml + mr) - lmax * (hr - hl));
+  Fn = 0.5 * (((hl * (nl * nl) + hg * (hl * hl)) + (hr * (nr * nr) + hg * (hr * hr))) -
+              lmax * (mr - ml));
+  Ft = 0.5 * ((ml * tl + mr * tr) - lmax * (hr * tr - hl * tl));
+}
+
+__device__ __forceinline__ bool is_finite(double a) {
+  return __builtin_amdgcn_class(a, 0x1F8);  // zero, subnormal or normal
 }
 
 // JamesonIndicator, src/shocksindicator.f90:93-129, on the depths of three
