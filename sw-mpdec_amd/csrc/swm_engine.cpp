@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -83,6 +84,7 @@ JobLayout job_layout(int nx, int ny, int wb, int bathy) {
   }
   add((size_t)(kMaxSys + 1) * L.nblk);                   // Jacobi partial sums
   add(3 * (size_t)L.nblk);                               // TimeStep partials
+  add(solve_slot((int)L.n, kSolveForms, 0, 0, 0));       // k_solve's slots
   L.bytes = b;
   (void)bathy;  // the bathymetry tables are a separate allocation (bathy_bytes)
   return L;
@@ -133,6 +135,18 @@ struct Tables {
   DevVec<TileRef> dxt[kNumShapes], dyt[kNumShapes], dct, dcb;
   DevVec<int> djl;
   int nxt[kNumShapes] = {}, nyt[kNumShapes] = {}, nct = 0, ncb = 0, njobs = 0;
+  // The Patankar solves: k_solve's blocks for launches of one and of kMaxSys
+  // systems, cut into launches (first block, blocks); and the cell blocks and
+  // jobs of the grids k_solve does not take, swept by a launch per sweep.
+  std::vector<SolveRef> sv[2];
+  std::vector<std::pair<int, int>> svl[2];
+  bool solve_waits = false;  // some systems have several blocks
+  std::vector<TileRef> cbw;
+  std::vector<int> jlw;
+  DevVec<SolveRef> dsv[2];
+  DevVec<TileRef> dcbw;
+  DevVec<int> djlw;
+  int ncbw = 0, njobsw = 0;
 };
 
 enum JobState { JOB_RUNNING = 0, JOB_DONE = 1, JOB_FAILED = 2, JOB_FREE = 3 };
@@ -199,6 +213,9 @@ struct swm_engine {
   double tol = 1.e-16;
   long long ambiguous = 0;
   bool track_min = false;        // fold every stage depth into JobStatus::hmin
+  int device = -1;
+  int solve_blocks_max = 0;      // blocks of k_solve the device holds at once
+  bool solve_lost = false;       // a wait inside k_solve ran out: not used any more
   // Step execution (results are identical either way; only speed differs):
   // speculative steps launch each correction's predicted sweeps without host
   // reads and check once at the end; they may be replayed from a captured
@@ -217,13 +234,14 @@ struct swm_engine {
   struct Captured {
     long long epoch = -1;
     int device_dt = 0, track = 0;
-    int sweeps[5] = {0, 0, 0, 0, 0};
+    int sweeps[5] = {0, 0, 0, 0, 0}, limit[5] = {0, 0, 0, 0, 0};
+    int solve = 0;
     const void* tables = nullptr;
     int group = -1, shape = -1;
     long long used = 0;
     hipGraphExec_t exec = nullptr;
   };
-  Captured caps[kGroups];        // one captured step per table set in use
+  Captured caps[2 * kGroups];    // captured steps by table set in use, with and without k_solve
   long long cap_clock = 0;
   Profiler prof;
   std::string err;
@@ -295,7 +313,112 @@ void add_tiles(Tables& T, int id, const JobDev& d) {
   T.jl.push_back(id);
 }
 
+// The right to launch k_solve blocks that wait for each other, one engine per
+// device at a time: two such launches side by side, from the streams of two
+// threads, could each hold part of the device and wait for the rest.  A batch
+// holds it until its status read has shown the kernels done; a batch that does
+// not get it runs a launch per sweep.
+class SolveRight {
+ public:
+  bool take(int device) {
+    if (device < 0 || device >= kDevices) return false;
+    int free = 0;
+    if (held().at[device].compare_exchange_strong(free, 1)) device_ = device;
+    return device_ >= 0;
+  }
+  ~SolveRight() {
+    if (device_ >= 0) held().at[device_].store(0);
+  }
+
+ private:
+  static constexpr int kDevices = 64;
+  struct Held {
+    std::atomic<int> at[kDevices] = {};
+  };
+  static Held& held() {
+    static Held h;
+    return h;
+  }
+  int device_ = -1;
+};
+
+// Rows of the largest system that one k_solve block takes alone.  At 2048 rows
+// (4 per thread) its assembly is issue-bound at about 10 us and a sweep costs
+// 1.2 us; four blocks of one row per thread assemble in 3 us and pay 2.3 us a
+// sweep, and at the 10 to 15 sweeps a solve needs the two break even.
+constexpr int kSolveAlone = 2048;
+
+// k_solve's blocks for the jobs of T.  A grid is taken when the blocks of one
+// system fit the device at once (blocks of a system wait for each other); the
+// blocks of several systems share a launch as long as all of them fit.  The
+// systems with several blocks take the form with the fewest rows per thread
+// that needs one launch, else the one with the most: a sweep's cost hardly
+// depends on the rows (2.4 to 6 us), a further launch repeats all of it.
+// Blocks without others to wait for come last and are not counted.
+void solve_tables(swm_engine* e, Tables& T) {
+  const int cap = std::min(e->solve_blocks_max, 256);
+  T.cbw.clear();
+  T.jlw.clear();
+  std::vector<int> alone, shared;
+  for (int id : T.jl) {
+    const int n = e->jobs[id]->dev.n;
+    if (n <= kSolveAlone && cap > 0) {
+      alone.push_back(id);
+    } else if (cap > 0 && solve_blocks(n, kSolveForms - 1) <= cap) {
+      shared.push_back(id);
+    } else {
+      for (int t = 0; t < e->jobs[id]->dev.nblk; ++t) T.cbw.push_back({id, t});
+      T.jlw.push_back(id);
+    }
+  }
+  T.solve_waits = !shared.empty();
+  for (int c = 0; c < 2; ++c) {
+    const int nsys = c == 0 ? 1 : kMaxSys;
+    std::vector<SolveRef>& v = T.sv[c];
+    v.clear();
+    T.svl[c].clear();
+    int form = 0;
+    for (; form < kSolveForms - 1; ++form) {
+      long total = 0;
+      for (int id : shared) total += (long)nsys * solve_blocks(e->jobs[id]->dev.n, form);
+      if (total <= cap) break;
+    }
+    int first = 0;
+    for (int id : shared) {
+      const int nb = solve_blocks(e->jobs[id]->dev.n, form);
+      for (int s = 0; s < nsys; ++s) {
+        if ((int)v.size() - first + nb > cap) {
+          T.svl[c].push_back({first, (int)v.size() - first});
+          first = (int)v.size();
+        }
+        for (int b = 0; b < nb; ++b) v.push_back({id, b, nb, (short)s, (short)form});
+      }
+    }
+    for (int id : alone) {
+      int f = 0;
+      while (solve_blocks(e->jobs[id]->dev.n, f) > 1) ++f;
+      for (int s = 0; s < nsys; ++s) v.push_back({id, 0, 1, (short)s, (short)f});
+    }
+    if ((int)v.size() > first) T.svl[c].push_back({first, (int)v.size() - first});
+  }
+}
+
 int upload_tables(swm_engine* e, Tables& T) {
+  solve_tables(e, T);
+  for (int c = 0; c < 2; ++c) {
+    HIPCK(e, T.dsv[c].reserve(T.sv[c].size()));
+    if (!T.sv[c].empty())
+      HIPCK(e, hipMemcpy(T.dsv[c].p, T.sv[c].data(), T.sv[c].size() * sizeof(SolveRef),
+                         hipMemcpyHostToDevice));
+  }
+  T.ncbw = (int)T.cbw.size();
+  T.njobsw = (int)T.jlw.size();
+  HIPCK(e, T.dcbw.reserve(T.cbw.size()));
+  HIPCK(e, T.djlw.reserve(T.jlw.size()));
+  if (T.ncbw)
+    HIPCK(e, hipMemcpy(T.dcbw.p, T.cbw.data(), T.ncbw * sizeof(TileRef), hipMemcpyHostToDevice));
+  if (T.njobsw)
+    HIPCK(e, hipMemcpy(T.djlw.p, T.jlw.data(), T.njobsw * sizeof(int), hipMemcpyHostToDevice));
   for (int sh = 0; sh < kNumShapes; ++sh) {
     T.nxt[sh] = (int)T.xt[sh].size();
     T.nyt[sh] = (int)T.yt[sh].size();
@@ -405,7 +528,9 @@ struct StepPlan {
   int hp_view;    // the reference's depth view of the two-node schemes
   bool device_dt;
   bool speculative;
+  bool solve;     // the grids k_solve takes go through it (speculative only)
   int sweeps[5];  // speculative: sweeps per correction, counting the fused one
+  int limit[5];   // speculative: the most sweeps k_solve does
 };
 
 // Systems solved in correction kk (1-based): nodes 1..MSteps-1, or only the
@@ -605,12 +730,23 @@ int step_body(swm_engine* e, Tables& T, const StepPlan& P) {
     else
       for (int m = 1; m < D.msteps; ++m) S.m[S.count++] = m;
     if (S.hp_view) timed(e, 4, [&] { launch_hp_view(a, T.dcb.p, T.ncb, kk == 1, s); });
-    // the DeC momentum update runs inside the assembly kernel
-    timed(e, 4, [&] { launch_assemble(a, T.dcb.p, T.ncb, T.djl.p, T.njobs, S, s); });
+    // the DeC momentum update runs inside the assembly and the solve kernels
+    if (P.solve) {
+      const int c = S.count == 1 ? 0 : 1;
+      for (const auto& l : T.svl[c])
+        timed(e, 5, [&] {
+          launch_solve(a, T.dsv[c].p + l.first, l.second, S, P.limit[kk - 1], solve, s);
+        });
+    }
+    // the grids swept by a launch per sweep: all of them without k_solve
+    const TileRef* cb = P.solve ? T.dcbw.p : T.dcb.p;
+    const int* jl = P.solve ? T.djlw.p : T.djl.p;
+    const int ncb = P.solve ? T.ncbw : T.ncb, njobs = P.solve ? T.njobsw : T.njobs;
+    if (ncb) timed(e, 4, [&] { launch_assemble(a, cb, ncb, jl, njobs, S, s); });
     LAUNCHCK(e);
     if (P.speculative) {
-      for (int b = 1; b < P.sweeps[kk - 1]; ++b)
-        timed(e, 5, [&] { launch_sweep(a, T.dcb.p, T.ncb, T.djl.p, T.njobs, S, s); });
+      for (int b = 1; ncb && b < P.sweeps[kk - 1]; ++b)
+        timed(e, 5, [&] { launch_sweep(a, cb, ncb, jl, njobs, S, s); });
       LAUNCHCK(e);
     } else {
       int pred = 1;
@@ -621,7 +757,7 @@ int step_body(swm_engine* e, Tables& T, const StepPlan& P) {
       long launched = 1;
       for (;;) {
         for (int b = 0; b < batch; ++b)
-          timed(e, 5, [&] { launch_sweep(a, T.dcb.p, T.ncb, T.djl.p, T.njobs, S, s); });
+          timed(e, 5, [&] { launch_sweep(a, cb, ncb, jl, njobs, S, s); });
         LAUNCHCK(e);
         launched += batch;
         rc = read_status(e);
@@ -643,8 +779,10 @@ int step_body(swm_engine* e, Tables& T, const StepPlan& P) {
         batch = std::max(2, kmin / 4);
       }
     }
-    timed(e, 7, [&] { launch_solve_done(a, T.djl.p, T.njobs, S, solve, s); });
-    timed(e, 7, [&] { launch_finalize(a, T.dcb.p, T.ncb, T.djl.p, T.njobs, S, s); });
+    if (ncb) {
+      timed(e, 7, [&] { launch_solve_done(a, jl, njobs, S, solve, s); });
+      timed(e, 7, [&] { launch_finalize(a, cb, ncb, jl, njobs, S, s); });
+    }
     LAUNCHCK(e);
     solve += S.count;
     if (kk != D.kcorr) {
@@ -689,12 +827,12 @@ void drop_graphs(swm_engine* e) {
 
 // Speculative step (body, gate, commit) through a captured graph (capturing it when the job set,
 // the scheme or the sweep counts changed).  Each table set keeps its own
-// graph, so groups of jobs stepped one after another do not recapture.
+// graphs, so groups of jobs stepped one after another do not recapture.
 int step_body_graph(swm_engine* e, Tables& T, const StepPlan& P) {
   const int group = group_of(P.sc, P.hp_view ? SWM_HP_AS_REFERENCE : SWM_HP_BY_NODE);
   swm_engine::Captured* cp = nullptr;
   for (auto& c : e->caps)
-    if (c.exec && c.tables == (const void*)&T) cp = &c;
+    if (c.exec && c.tables == (const void*)&T && c.solve == (int)P.solve) cp = &c;
   if (!cp) {  // a free entry, else the least recently used
     cp = &e->caps[0];
     for (auto& c : e->caps)
@@ -703,8 +841,9 @@ int step_body_graph(swm_engine* e, Tables& T, const StepPlan& P) {
   auto& c = *cp;
   bool same = c.exec && c.epoch == e->graph_epoch && c.device_dt == (int)P.device_dt &&
               c.track == (int)e->track_min && c.tables == (const void*)&T && c.group == group &&
-              c.shape == e->cur_shape;
-  for (int i = 0; same && i < 5; ++i) same = c.sweeps[i] == P.sweeps[i];
+              c.shape == e->cur_shape && c.solve == (int)P.solve;
+  for (int i = 0; same && i < 5; ++i)
+    same = c.sweeps[i] == P.sweeps[i] && c.limit[i] == P.limit[i];
   c.used = ++e->cap_clock;
   if (!same) {
     drop_graph(c);
@@ -729,7 +868,11 @@ int step_body_graph(swm_engine* e, Tables& T, const StepPlan& P) {
     c.tables = &T;
     c.group = group;
     c.shape = e->cur_shape;
-    for (int i = 0; i < 5; ++i) c.sweeps[i] = P.sweeps[i];
+    c.solve = P.solve;
+    for (int i = 0; i < 5; ++i) {
+      c.sweeps[i] = P.sweeps[i];
+      c.limit[i] = P.limit[i];
+    }
     ++e->graph_captures;
   }
   HIPCK(e, hipGraphLaunch(c.exec, e->stream));
@@ -851,13 +994,23 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
   P.sc = sc;
   P.hp_view = (!is_explicit(*sc) && sc->msteps < 4 && hp_assoc == SWM_HP_AS_REFERENCE) ? 1 : 0;
   P.device_dt = host_dt == nullptr;
+  // Steps run speculatively where nothing has to be predicted (k_solve takes
+  // every grid and no sweep limit is set) or every job swept by a launch per
+  // sweep has a prediction for the scheme.
   bool spec = e->margin != -2 && !is_explicit(*sc);  // nothing to predict without solves
-  for (int q = 0; q < T.njobs; ++q) {
-    const Job& J = *e->jobs[T.jl[q]];
+  P.solve = spec && !e->solve_lost && !e->track_min && !T.sv[0].empty();
+  SolveRight right;
+  if (P.solve && T.solve_waits) P.solve = right.take(e->device);
+  const bool open_limit = P.solve && e->margin < 0;  // k_solve runs to the stop rule
+  const bool all_solved = open_limit && T.njobsw == 0;
+  for (int id : open_limit ? T.jlw : T.jl) {
+    const Job& J = *e->jobs[id];
     spec = spec && J.have_pred && J.pred_sc == sc;
   }
+  P.solve = P.solve && spec;
   steps = std::max(1, std::min(steps, kMaxBatch));
-  if (host_dt || (!spec && !is_explicit(*sc)) || (spec && tuning(e))) steps = 1;
+  const bool tune = spec && !all_solved && tuning(e);
+  if (host_dt || (!spec && !is_explicit(*sc)) || tune) steps = 1;
   BatchArgs B{};
   B.max_steps = steps;
   if (loop) {
@@ -883,15 +1036,21 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
   }
   if (spec) {
     int graph, margin;
-    tune_choice(e, graph, margin);
+    if (all_solved) {
+      graph = e->use_graph != 0;
+      margin = 0;
+    } else {
+      tune_choice(e, graph, margin);
+    }
     P.speculative = true;
     int first = 0;
     for (int kk = 0; kk < sc->kcorr; ++kk) {
       int mx = 1;
       const int ns = systems_in(*sc, kk + 1);
-      for (int q = 0; q < T.njobs; ++q)
-        for (int k = 0; k < ns; ++k) mx = std::max(mx, e->jobs[T.jl[q]]->pred[first + k]);
+      for (int id : open_limit ? T.jlw : T.jl)
+        for (int k = 0; k < ns; ++k) mx = std::max(mx, e->jobs[id]->pred[first + k]);
       P.sweeps[kk] = std::min(mx + margin, e->max_iter);
+      P.limit[kk] = open_limit ? e->max_iter : P.sweeps[kk];
       first += ns;
     }
     // a tile-shape candidate is timed by HIP events around the face kernels
@@ -899,7 +1058,7 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
     // events itself or has set graph replay on (events keep it off); the
     // other candidates by the step's wall time
     const bool face_events =
-        tuning(e) && tune_id(e->tune_phase) < kNumShapes && !e->prof.mask && !graph;
+        tune && tune_id(e->tune_phase) < kNumShapes && !e->prof.mask && !graph;
     const size_t rec0 = e->prof.cats.size();  // records a caller has not read yet stay
     if (face_events) e->prof.mask = 0x3u;     // fvtd_x, fvtd_y
     const auto t0 = std::chrono::steady_clock::now();
@@ -932,8 +1091,11 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
     if (rc) return rc;
     e->spec_steps += steps;
     bool overrun = false;
-    for (int q = 0; q < T.njobs; ++q) overrun = overrun || e->hstatus[T.jl[q]].halt == kHaltOverrun;
-    if (!overrun) {
+    for (int q = 0; q < T.njobs; ++q) {
+      overrun = overrun || e->hstatus[T.jl[q]].halt == kHaltOverrun;
+      e->solve_lost = e->solve_lost || e->hstatus[T.jl[q]].solve_lost;
+    }
+    if (tune && !overrun) {
       const bool captured = e->graph_captures != captures0;
       if (captured && e->tune_skips < 2) {
         ++e->tune_skips;
@@ -945,7 +1107,6 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
       }
     }
   } else {
-    P.speculative = false;
     for (int b = 0; b < steps; ++b) {
       int rc = step_full(e, T, P);
       if (rc) return rc;
@@ -969,6 +1130,7 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
     LAUNCHCK(e);
     for (int q = 0; q < T.njobs; ++q) e->redone_steps += redo[q];
     P.speculative = false;
+    P.solve = false;
     int rc = step_full(e, T, P);
     if (rc) return rc;
     rc = read_status(e);
@@ -1172,6 +1334,8 @@ int alloc_job(swm_engine* e, int nx, int ny, double dx, double dy, double g, dou
   }
   D.part = take((size_t)(kMaxSys + 1) * lay.nblk);
   D.tspart = take(3 * (size_t)lay.nblk);
+  const size_t nslots = solve_slot(D.n, kSolveForms, 0, 0, 0);
+  D.slots = reinterpret_cast<unsigned long long*>(take(nslots));
   if (off > lay.bytes) FAIL(e, SWM_E_STATE, "internal: job slab overflow");
   e->in_use += (long long)lay.bytes;
   J.state = JOB_RUNNING;
@@ -1193,6 +1357,8 @@ int alloc_job(swm_engine* e, int nx, int ny, double dx, double dy, double g, dou
   int rc = upload_tables(e, J.own);
   if (rc) return rc;
   HIPCK(e, hipMemsetAsync(e->dstatus.p + id, 0, sizeof(JobStatus), e->stream));
+  // no slot holds the tag a first round expects
+  HIPCK(e, hipMemsetAsync(D.slots, 0, nslots * sizeof(*D.slots), e->stream));
   // the step-count stop of the device time loop (-1: none)
   launch_set_steps_left(e->dstatus.p + id, nsteps > 0 ? nsteps : -1, e->stream);
   LAUNCHCK(e);
@@ -1487,6 +1653,10 @@ int swm_engine_create(long long budget_bytes, swm_engine_t** out) {
     return SWM_E_HIP;
   }
   int rc = status_capacity(e, 8);
+  int cus = 0;
+  if (hipGetDevice(&e->device) == hipSuccess &&
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, e->device) == hipSuccess)
+    e->solve_blocks_max = cus;  // a k_solve block's registers fill at most one CU
   if (rc == SWM_OK && hipHostMalloc((void**)&e->hdt, sizeof(double), hipHostMallocDefault) != hipSuccess) {
     e->hdt = nullptr;
     g_error = "hipHostMalloc failed";

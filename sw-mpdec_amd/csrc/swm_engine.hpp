@@ -37,6 +37,8 @@ struct FaceShape {
 constexpr int kNumShapes = 2;
 constexpr FaceShape kShapes[kNumShapes] = {{16, 16, 16, 16}, {32, 16, 16, 32}};
 constexpr int kCellBlock = 256;       // cells per block of the pointwise kernels
+constexpr int kSolveThreads = 512;    // threads of a k_solve block
+constexpr int kSolveForms = 4;        // k_solve forms: 1 << form rows per thread
 constexpr int kMaxSys = 3;            // Patankar systems solved together (nodes 2..4)
 constexpr int kSlots = 3;             // concurrent FVTD evaluations per job
 constexpr int kStates = 6;            // state / derivative slots of the explicit schemes
@@ -57,6 +59,15 @@ struct JacState {
 // loop (k_batch_begin, k_gate) runs up to kMaxBatch steps between reads of
 // the status, recording each committed step.
 constexpr int kMaxBatch = 16;
+
+// How a solve of a step ended.
+enum SolveEnd {
+  kSolveConverged = 0,
+  kSolveLimit = 1,  // stopped at max_iter with the residual above tolerance
+  kSolveOpen = 2,   // still running when its phase ended (the step ran with too
+                    // few sweeps launched, or k_solve left a decision open) and
+                    // the step must be redone
+};
 
 // Why a job's batch stopped (JobStatus::halt); while halt != 0 every gated
 // kernel of the job returns at once and k_commit commits nothing.
@@ -92,10 +103,8 @@ struct JobStatus {
   double hmin_step;   // gate: a redone attempt's stages never reach hmin
   // the current step's solves, recorded after each correction's Jacobi phase
   int iters[13];  // sweeps of each solve, in execution order
-  int nonconv;    // solves stopped at the iteration limit
-  int ambiguous;  // stop decisions settled by the exact sequential sum
-  int overrun;    // a solve was still running when its phase ended (the
-                  // step ran with too few sweeps launched and must be redone)
+  int ambiguous[13];      // its stop decisions settled by the exact sequential sum
+  signed char ended[13];  // SolveEnd
   double dt_min;  // TimeStep's value before the time loop's clipping
   // the device time loop (k_batch_begin sets, k_gate advances)
   int halt;        // HaltCode
@@ -108,6 +117,10 @@ struct JobStatus {
                    // 0 all run (k_batch_begin keeps the job halted), < 0 none
   double t, t_an, t_end;
   StepRec rec[kMaxBatch];
+  // k_solve: rounds done so far by form and system, the base of the tags its
+  // blocks exchange; and 1 once a wait on another block ran out
+  unsigned rounds[kSolveForms][kMaxSys];
+  int solve_lost;
 };
 
 struct JobDev {
@@ -149,6 +162,7 @@ struct JobDev {
   // reductions
   double* part;     // [kMaxSys + 1][nblk] Jacobi partial sums
   double* tspart;   // [nblk][3] TimeStep partial maxima
+  unsigned long long* slots;  // k_solve's tagged sums (solve_slot)
   JobStatus* status;  // this job's status record
 };
 
@@ -156,6 +170,28 @@ struct TileRef {
   int job;
   int tile;
 };
+
+// One block of k_solve: block blk of the nb blocks of one system of a job, in
+// the form with 1 << form rows per thread.
+struct SolveRef {
+  int job, blk, nb;
+  short sys, form;
+};
+
+// Blocks of one system of n rows in a form.
+inline __host__ __device__ int solve_blocks(int n, int form) {
+  const int rows = kSolveThreads << form;
+  return (n + rows - 1) / rows;
+}
+
+// JobDev::slots: per form, system, kind (0: residual, 1: right-hand side) and
+// parity of the round, one slot per block.  The forms have slots of their own,
+// so that each slot is written in every second round of its form.
+inline __host__ __device__ size_t solve_slot(int n, int form, int sys, int kind, int parity) {
+  size_t o = 0;
+  for (int f = 0; f < form; ++f) o += (size_t)kMaxSys * 4 * solve_blocks(n, f);
+  return o + (size_t)((sys * 2 + kind) * 2 + parity) * solve_blocks(n, form);
+}
 
 // Arguments shared by every launch of one engine step.  gated = 1 in the
 // steps of a batch: a job whose JobStatus::halt is set is skipped.
@@ -285,6 +321,10 @@ void launch_sweep(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl
                   const SysList& S, hipStream_t s);
 void launch_finalize(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl, int njobs,
                      const SysList& S, hipStream_t s);
+// k_solve over nblk blocks: assembly, momentum update and the whole Jacobi
+// iteration of each block's system, up to `limit` sweeps
+void launch_solve(const EngineArgs& E, const SolveRef* refs, int nblk, const SysList& S, int limit,
+                  int first_solve, hipStream_t s);
 void launch_timestep(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl, int njobs,
                      hipStream_t s);
 void launch_commit(const EngineArgs& E, const TileRef* cb, int ncb, int final_node,

@@ -503,12 +503,12 @@ __global__ __launch_bounds__(256) void k_fvtd_update(EngineArgs E, const TileRef
 // :717-721): Ua(m,2:3) = Ua(1,2:3); DO r=1,R: Ua(m) = Ua(m) + (dt*theta(m,r))*FUp(r)
 // with R = MSteps.
 // ------------------------------------------------------------------------
-// One cell, every system's node m.  It runs inside the assembly kernel (the
+// One cell, the nodes m of systems s0..s1-1.  It runs inside the assembly kernel (the
 // two read and write disjoint arrays), so that its loads overlap the
 // assembly's latency-bound work.
 template <int R>
-__device__ __forceinline__ void momentum_cell(const JobDev& J, const SysList& S, int k,
-                                              double dt) {
+__device__ __forceinline__ void momentum_cell(const JobDev& J, const SysList& S, int s0, int s1,
+                                              int k, double dt) {
   double fu2[R], fu3[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -516,7 +516,7 @@ __device__ __forceinline__ void momentum_cell(const JobDev& J, const SysList& S,
     fu3[r] = G(J.FU3[S.src[r]])[k];
   }
   const double u0 = G(J.hu)[k], v0 = G(J.hv)[k];
-  for (int s = 0; s < S.count; ++s) {
+  for (int s = s0; s < s1; ++s) {
     const int m = S.m[s];
     double u = u0, v = v0;
 #pragma unroll
@@ -572,11 +572,13 @@ __device__ double block_sum_array(const double* part, int nb, double* red) {
 // (n-1)u*sum(d), so whenever tol lies outside [S - B, S + B]/n with
 // B = 8nuS the decision is that of the sequential sum; inside the window the
 // caller recomputes the sequential sum exactly.  1 continue, 0 stop, -1 open.
-__device__ __forceinline__ int certified_continue(double S, int n, double tol) {
+// extra: a further relative error of S.
+__device__ __forceinline__ int certified_continue(double S, int n, double tol,
+                                                  double extra = 0.) {
   if (isnan(S)) return 0;
   if (isinf(S)) return 1;
   const double u = 1.1102230246251565e-16;  // 2^-53
-  double B = 8.0 * (double)n * u * S;
+  double B = (8.0 * (double)n * u + extra) * S;
   double lo = (S - B) / (double)n, hi = (S + B) / (double)n;
   if (tol < lo) return 1;
   if (!(tol < hi)) return 0;
@@ -670,7 +672,8 @@ __device__ __forceinline__ void patankar_slot(int pos, const double c[R], const 
 // The four stencil slots of one row-system (sparse_matmul in CSR order S, W,
 // self (value 0), E, N): writes the slots' matrix entries, accumulates the
 // diagonal into D and returns the product with the neighbours' rhs values.
-template <int R, bool WET>
+// sq: the row's column of the staged fluxes, NT apart.
+template <int R, bool WET, int NT>
 __device__ __forceinline__ double patankar_row(const JobDev& J, int s, size_t k, const double* sq,
                                                int pos, const double c[R], const PdDepth& pK,
                                                double hS, double hW, double hE, double hN,
@@ -684,7 +687,7 @@ __device__ __forceinline__ double patankar_row(const JobDev& J, int s, size_t k,
     const double bL = sl == 0 ? bS : sl == 1 ? bW : sl == 2 ? bE : bN;
     double q[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) q[r] = sq[(sl * R + r) * 256];
+    for (int r = 0; r < R; ++r) q[r] = sq[(sl * R + r) * NT];
     double M;
     patankar_slot<R, WET>(pos, c, q, pd_depth(hL), pK, M, D);
     G(J.M[s][sl])[k] = M;
@@ -742,7 +745,7 @@ __global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* b
     bW = rhs[kW];
     bE = rhs[kE];
     bN = rhs[kN];
-    momentum_cell<R>(J, S, k, dt);
+    momentum_cell<R>(J, S, 0, S.count, k, dt);
   }
   // One system at a time, and within it one stencil slot at a time (S, W, E,
   // N: the CSR order), so that only one slot's divisions are live.  Each
@@ -765,10 +768,10 @@ __global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* b
       const bool dry = pK.dry | (hS < kMinDepth) | (hW < kMinDepth) | (hE < kMinDepth) |
                        (hN < kMinDepth);
       const double p =
-          __any(dry) ? patankar_row<R, false>(J, s, k, sq + tid, pos, c, pK, hS, hW, hE, hN, bS,
-                                              bW, bE, bN, b, D)
-                     : patankar_row<R, true>(J, s, k, sq + tid, pos, c, pK, hS, hW, hE, hN, bS,
-                                             bW, bE, bN, b, D);
+          __any(dry) ? patankar_row<R, false, 256>(J, s, k, sq + tid, pos, c, pK, hS, hW, hE, hN,
+                                                   bS, bW, bE, bN, b, D)
+                     : patankar_row<R, true, 256>(J, s, k, sq + tid, pos, c, pK, hS, hW, hE, hN,
+                                                  bS, bW, bE, bN, b, D);
       G(J.M[s][4])[k] = D;
       double x1 = (b - p) / D;
       G(J.xj[m][1])[k] = x1;
@@ -904,6 +907,309 @@ __global__ __launch_bounds__(256) void k_decide(EngineArgs E, const int* jobs, S
   }
 }
 
+// ------------------------------------------------------------------------
+// The whole Patankar solve of a correction in one launch, for grids whose
+// systems fit the register files.
+//
+// A system of n rows belongs to nb blocks of 512 threads, 1 << FORM rows per
+// thread.  A block assembles its rows as k_assemble does, keeps the matrix
+// rows in registers and the iterate in LDS, and sweeps until the stop rule
+// ends the solve: no sweep reads the matrix from memory, and no launch, host
+// prediction or empty sweep is paid per sweep.  A sweep of a launch of its own
+// with its stop decision took 13 us at any size up to 257^2 (5.2 + 3.9 us and
+// two launch gaps at 32^2), and 34 us at 1024^2.  mPDeC5 passes with the
+// state's transfer, before and after: 32^2, 20 steps 17.8 -> 6.3 ms; 257^2, 10
+// steps 9.5 -> 6.0 ms; 1024^2 dam break, 4 steps 25.1 -> 22.0 ms.
+//
+// Several blocks of a system (nb > 1) exchange, per sweep, the rows that other
+// blocks' stencils reach (all within nx rows of the block's ends) and their
+// part of the residual sum.  All of that goes through agent-scope atomic
+// stores and loads, which bypass the XCDs' separate L2s, so no cache is
+// written back: a block drains its row stores (s_waitcnt vmcnt(0)), then
+// publishes its sum in a slot whose low 8 bits carry the round's tag, and
+// polls the other blocks' slots for that tag.  Measured per round: 2.4 us for
+// 8 blocks, 3.3 us for 64, 4.3 us for 240; with a counter instead of tags 3.0,
+// 3.7, 6.7 us; with agent-scope fences 5.1 us for 64.  The rows of round t go
+// to buffer t & 1: a block overwrites it in round t + 2, after every block has
+// published round t + 1 and so finished reading round t.
+//
+// The tag takes the sum's low 8 bits, a relative change below 2^-44, which
+// certified_continue is told of.  Tags count on over the launches
+// (JobStatus::rounds), and a slot is rewritten in every second round of its
+// form, so the tag it held before is the expected one less 2.
+//
+// The host launches no more blocks at once than the device holds
+// concurrently, and no two such launches side by side.  A wait is bounded all
+// the same: when it runs out (another process on the device, say), or a stop decision lies inside the certified
+// window, the solve ends as kSolveOpen, the step is not committed and the host
+// runs it again with the launches of one sweep each.
+// ------------------------------------------------------------------------
+constexpr int kSolvePolls = 1 << 15;  // about 25 ms
+
+__device__ __forceinline__ double agent_load(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void agent_store(double* p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Sum of v over the block in LDS buffer red (one double per wave); every thread calls,
+// and the sum is ready after the barrier inside.
+__device__ __forceinline__ double solve_block_sum(double v, double* red) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double t = red[0];
+#pragma unroll
+  for (int w = 1; w < kSolveThreads / 64; ++w) t += red[w];
+  return t;
+}
+
+template <int R>
+struct SolveShared {
+  static constexpr int kDoubles = 4 * R * kSolveThreads > 2 * (kSolveThreads << (kSolveForms - 1))
+                                      ? 4 * R * kSolveThreads
+                                      : 2 * (kSolveThreads << (kSolveForms - 1));
+  // assembly: [slot*R + node][thread] face mass fluxes; then the iterate [2][rows]
+  double sm[kDoubles];
+  double red[2][2][kSolveThreads / 64];  // [parity][kind]
+  double tot[2][2][4];                   // the blocks' sums, by wave
+  int lost;
+};
+
+template <int FORM, int R>
+__device__ __forceinline__ void solve_block(SolveShared<R>& L, const EngineArgs& E,
+                                            const SolveRef W, const SysList& S, int limit,
+                                            int first_solve) {
+  constexpr int NT = kSolveThreads, RPT = 1 << FORM, ROWS = NT * RPT;
+  double* sm = L.sm;
+  auto& red = L.red;
+  auto& tot = L.tot;
+  int& lost = L.lost;
+  const JobDev& J = E.jobs[W.job];
+  const int tid = threadIdx.x, s = W.sys, nb = W.nb, m = S.m[s];
+  const int nx = J.nx, ny = J.ny, n = J.n;
+  const int base = W.blk * ROWS, len = min(n - base, ROWS);
+  JobStatus* st = J.status;
+  const double dt = st->dt;
+  const unsigned round0 = st->rounds[FORM][s];
+  const gdouble* rhs = system_rhs(J, S);
+  if (tid == 0) lost = 0;
+
+  // assembly and momentum, one row at a time; the matrix rows go through
+  // memory (their own thread reads them back) so that the loop stays rolled
+  double dsum = 0., bsum = 0.;
+#pragma unroll 1
+  for (int i = 0; i < RPT; ++i) {
+    const int l = i * NT + tid;
+    if (l >= len) break;
+    const int k = base + l, cj = k / nx, ci = k - cj * nx;
+    const int kS = (cj == 0 ? ny - 1 : cj - 1) * nx + ci;
+    const int kW = cj * nx + (ci == 0 ? nx - 1 : ci - 1);
+    const int kE = cj * nx + (ci == nx - 1 ? 0 : ci + 1);
+    const int kN = (cj == ny - 1 ? 0 : cj + 1) * nx + ci;
+    const size_t fW = (size_t)cj * (nx + 1) + ci, fE = fW + 1;
+    const size_t gS = (size_t)cj * nx + ci, gN = gS + nx;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      sm[(0 * R + r) * NT + tid] = G(J.qy[S.src[r]])[gS];
+      sm[(1 * R + r) * NT + tid] = G(J.qx[S.src[r]])[fW];
+      sm[(2 * R + r) * NT + tid] = -G(J.qx[S.src[r]])[fE];
+      sm[(3 * R + r) * NT + tid] = -G(J.qy[S.src[r]])[gN];
+    }
+    const double b = rhs[k], bS = rhs[kS], bW = rhs[kW], bE = rhs[kE], bN = rhs[kN];
+    const gdouble* hp = system_hp(J, S, m);
+    const double hK = hp[k], hS = hp[kS], hW = hp[kW], hE = hp[kE], hN = hp[kN];
+    momentum_cell<R>(J, S, s, s + 1, k, dt);
+    const PdDepth pK = pd_depth(hK);
+    const int pos = THETA_POS[S.theta][m];
+    double c[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) c[r] = dt * THETA[S.theta][m][r];
+    double D = 1.;
+    const bool dry = pK.dry | (hS < kMinDepth) | (hW < kMinDepth) | (hE < kMinDepth) |
+                     (hN < kMinDepth);
+    const double p =
+        __any(dry) ? patankar_row<R, false, NT>(J, s, k, sm + tid, pos, c, pK, hS, hW, hE, hN, bS,
+                                                bW, bE, bN, b, D)
+                   : patankar_row<R, true, NT>(J, s, k, sm + tid, pos, c, pK, hS, hW, hE, hN, bS,
+                                               bW, bE, bN, b, D);
+    const double x1 = (b - p) / D;
+    G(J.M[s][4])[k] = D;
+    G(J.xj[m][1])[k] = x1;
+    dsum += fabs(x1 - b);
+    bsum += fabs(0.0 - b);
+  }
+  __syncthreads();  // the fluxes have been read: sm takes the iterate
+
+  double M[RPT][4], D[RPT], b[RPT], x[RPT];
+  int at[RPT][4];  // neighbours' row numbers less base
+#pragma unroll
+  for (int i = 0; i < RPT; ++i) {
+    const int l = i * NT + tid, k = base + l;
+    if (l < len) {
+      const int cj = k / nx, ci = k - cj * nx;
+      at[i][0] = (cj == 0 ? ny - 1 : cj - 1) * nx + ci - base;
+      at[i][1] = cj * nx + (ci == 0 ? nx - 1 : ci - 1) - base;
+      at[i][2] = cj * nx + (ci == nx - 1 ? 0 : ci + 1) - base;
+      at[i][3] = (cj == ny - 1 ? 0 : cj + 1) * nx + ci - base;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) M[i][q] = G(J.M[s][q])[k];
+      D[i] = G(J.M[s][4])[k];
+      x[i] = G(J.xj[m][1])[k];
+      b[i] = rhs[k];
+    }
+  }
+
+  int k_sweeps = 1, zero = 0, end = kSolveConverged;
+  unsigned t = 0;
+  for (;; ++t) {
+    // publish round t: the iterate in LDS, its outer rows and the block's sums
+    const int par = t & 1;
+    double* sx = sm + par * ROWS;
+    double* buf = J.FX[s][par];  // free between an FVTD's update and the next one's face kernels
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {
+      const int l = i * NT + tid;
+      if (l < len) {
+        sx[l] = x[i];
+        if (nb > 1 && (l < nx || l >= len - nx)) agent_store(buf + base + l, x[i]);
+      }
+    }
+    if (t == 0) bsum = wave_sum(bsum);
+    if (t == 0 && (tid & 63) == 0) red[par][1][tid >> 6] = bsum;
+    if (nb > 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    double S1 = solve_block_sum(dsum, red[par][0]), S0 = 0.;
+    if (t == 0)
+      for (int w = 0; w < NT / 64; ++w) S0 += red[par][1][w];
+    if (nb > 1) {
+      const unsigned tag = (round0 + t + 1u) & 0xffu, tp = (round0 + t) & 1u;
+      unsigned long long* slot[2];
+      for (int q = 0; q < 2; ++q) slot[q] = J.slots + solve_slot(n, FORM, s, q, tp);
+      if (tid == 0)
+        for (int q = (t == 0 ? 1 : 0); q >= 0; --q)
+          __hip_atomic_store(slot[q] + W.blk,
+                             ((unsigned long long)__double_as_longlong(q ? S0 : S1) & ~0xffull) |
+                                 tag,
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (tid < 256) {  // nb <= 256: the first four waves poll
+        for (int q = (t == 0 ? 1 : 0); q >= 0; --q) {
+          unsigned long long v = tag;
+          if (tid < nb) {
+            int polls = 0;
+            do {
+              v = __hip_atomic_load(slot[q] + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            } while ((unsigned)(v & 0xffu) != tag && ++polls < kSolvePolls);
+            if ((unsigned)(v & 0xffu) != tag) lost = 1;
+          }
+          const double w = wave_sum(__longlong_as_double((long long)(v & ~0xffull)));
+          if ((tid & 63) == 0) tot[par][q][tid >> 6] = w;
+        }
+      }
+      __syncthreads();
+      S1 = ((tot[par][0][0] + tot[par][0][1]) + tot[par][0][2]) + tot[par][0][3];
+      if (t == 0) S0 = ((tot[par][1][0] + tot[par][1][1]) + tot[par][1][2]) + tot[par][1][3];
+      if (lost) {  // set before the barrier: every thread of the block sees it
+        end = kSolveOpen;
+        break;
+      }
+    }
+    // the stop rule (src/jacobi_iteration.f90:63-84): the same numbers, and so
+    // the same decision, in every block of the system
+    const double extra = nb > 1 ? 0x1p-43 : 0.;
+    if (t == 0) {
+      const int c0 = certified_continue(S0, n, E.tol, extra);
+      if (c0 < 0) {
+        end = kSolveOpen;
+        break;
+      }
+      if (!c0 || E.max_iter <= 0) {
+        k_sweeps = 0;
+        zero = 1;
+        end = c0 ? kSolveLimit : kSolveConverged;
+        break;
+      }
+    }
+    const int c1 = certified_continue(S1, n, E.tol, extra);
+    if (c1 <= 0) {
+      end = c1 < 0 ? kSolveOpen : kSolveConverged;
+      break;
+    }
+    if (k_sweeps >= E.max_iter) {
+      end = kSolveLimit;
+      break;
+    }
+    if (k_sweeps >= limit) {
+      end = kSolveOpen;
+      break;
+    }
+    ++k_sweeps;
+    // one sweep (src/jacobi_iteration.f90:72-80)
+    dsum = 0.;
+    constexpr int GR = RPT < 4 ? RPT : 2;  // rows with their loads in flight together
+#pragma unroll
+    for (int i0 = 0; i0 < RPT; i0 += GR) {
+      double y[GR][4];
+#pragma unroll
+      for (int i = i0; i < i0 + GR; ++i)
+        if (i * NT + tid < len) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int a = at[i][q];
+            if ((unsigned)a < (unsigned)ROWS)
+              y[i - i0][q] = sx[a];
+            else
+              y[i - i0][q] = agent_load(buf + base + a);
+          }
+        }
+#pragma unroll
+      for (int i = i0; i < i0 + GR; ++i)
+        if (i * NT + tid < len) {
+          double p = 0.;
+          p = p + M[i][0] * y[i - i0][0];
+          p = p + M[i][1] * y[i - i0][1];
+          p = p + 0. * x[i];
+          p = p + M[i][2] * y[i - i0][2];
+          p = p + M[i][3] * y[i - i0][3];
+          const double xv = (b[i] - p) / D[i];
+          dsum += fabs(xv - x[i]);
+          x[i] = xv;
+        }
+    }
+  }
+  if (end != kSolveOpen) {
+#pragma unroll
+    for (int i = 0; i < RPT; ++i)
+      if (i * NT + tid < len) G(J.hres[m])[base + i * NT + tid] = zero ? 0. : x[i];
+  }
+  if (tid == 0) {
+    if (lost) st->solve_lost = 1;  // k_gate keeps the step from being committed
+    if (W.blk == 0) {
+      st->ended[first_solve + s] = end;
+      st->iters[first_solve + s] = k_sweeps;
+      st->ambiguous[first_solve + s] = 0;
+      st->rounds[FORM][s] = round0 + t + 1u;
+    }
+  }
+}
+
+template <int R>
+__global__ __launch_bounds__(kSolveThreads) void k_solve(EngineArgs E, const SolveRef* refs,
+                                                         SysList S, int limit, int first_solve) {
+  __shared__ SolveShared<R> L;
+  const SolveRef W = refs[blockIdx.x];
+  if (skipped(E, E.jobs[W.job])) return;
+  static_assert(kSolveForms == 4, "the forms below");
+  if (W.form == 0)
+    solve_block<0, R>(L, E, W, S, limit, first_solve);
+  else if (W.form == 1)
+    solve_block<1, R>(L, E, W, S, limit, first_solve);
+  else if (W.form == 2)
+    solve_block<2, R>(L, E, W, S, limit, first_solve);
+  else
+    solve_block<3, R>(L, E, W, S, limit, first_solve);
+}
+
 // min that propagates NaN (the stage check must see a NaN depth)
 __device__ __forceinline__ double nan_min(double a, double b) {
   return (a != a || b != b) ? __builtin_nan("") : (a < b ? a : b);
@@ -964,25 +1270,20 @@ __global__ __launch_bounds__(256) void k_stage_min(EngineArgs E, const int* jobs
   }
 }
 
-// After a correction's Jacobi phase, one thread per job records the solves
-// (sweep counts, non-converged and ambiguous stops) and whether any system was
-// still running, i.e. needed more sweeps than were launched.
+// After a correction's Jacobi phase, one thread per job records the solves:
+// sweep counts, ambiguous stops and how each ended (a system still running
+// needed more sweeps than were launched).
 __global__ void k_solve_done(EngineArgs E, const int* jobs, SysList S, int first_solve) {
   if (threadIdx.x != 0) return;
   JobStatus* st = E.jobs[jobs[blockIdx.x]].status;
   if (E.gated && st->halt) return;
-  if (first_solve == 0) {
-    st->nonconv = 0;
-    st->ambiguous = 0;
-    st->overrun = 0;
-    st->hmin_step_set = 0;  // this attempt's stages start a new minimum
-  }
   for (int s = 0; s < S.count; ++s) {
     const JacState& q = st->st[s];
     st->iters[first_solve + s] = q.k;
-    st->nonconv += q.nonconv;
-    st->ambiguous += q.ambiguous;
-    st->overrun |= q.active;
+    st->ambiguous[first_solve + s] = q.ambiguous;
+    st->ended[first_solve + s] = q.active    ? kSolveOpen
+                                 : q.nonconv ? kSolveLimit
+                                             : kSolveConverged;
   }
 }
 
@@ -1025,7 +1326,7 @@ __global__ void k_batch_begin(EngineArgs E, const int* jobs, BatchArgs B) {
   }
   st->halt = kHaltNone;
   st->commit = 0;
-  st->overrun = 0;
+  st->solve_lost = 0;
   st->batch_done = 0;
   st->batch_max = B.max_steps;
   if (B.redo) return;  // the redone step keeps the loop's t
@@ -1042,11 +1343,19 @@ __global__ void k_gate(EngineArgs E, const int* jobs, int nsolve) {
   JobStatus* st = E.jobs[jobs[blockIdx.x]].status;
   st->commit = 0;
   if (st->halt) return;
-  if (st->overrun) {
+  int open = st->solve_lost, nonconv = 0, ambiguous = 0;
+  for (int i = 0; i < nsolve; ++i) {
+    open |= st->ended[i] == kSolveOpen;
+    nonconv += st->ended[i] == kSolveLimit;
+    ambiguous += st->ambiguous[i];
+  }
+  if (open) {
     st->halt = kHaltOverrun;
+    st->hmin_step_set = 0;  // the redone attempt's stages start a new minimum
     return;
   }
   if (st->dt_bad) {
+    st->hmin_step_set = 0;
     st->halt = kHaltDtBad;
     return;
   }
@@ -1054,8 +1363,8 @@ __global__ void k_gate(EngineArgs E, const int* jobs, int nsolve) {
   StepRec& r = st->rec[st->batch_done];
   r.dt = st->dt;
   for (int i = 0; i < 13; ++i) r.iters[i] = i < nsolve ? st->iters[i] : 0;
-  r.nonconv = nsolve > 0 ? st->nonconv : 0;
-  r.ambiguous = nsolve > 0 ? st->ambiguous : 0;
+  r.nonconv = nonconv;
+  r.ambiguous = ambiguous;
   st->batch_done += 1;
   if (st->hmin_step_set) {  // the accepted step's stage minimum joins the record
     st->hmin = st->hmin_set ? nan_min(st->hmin, st->hmin_step) : st->hmin_step;
@@ -1349,6 +1658,17 @@ void launch_sweep(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl
   if (!ncb) return;
   hipLaunchKernelGGL(k_sweep, dim3(ncb), dim3(256), 0, s, E, cb, S);
   hipLaunchKernelGGL(k_decide<false>, dim3(njobs), dim3(256), 0, s, E, jl, S);
+}
+
+void launch_solve(const EngineArgs& E, const SolveRef* refs, int nblk, const SysList& S, int limit,
+                  int first_solve, hipStream_t s) {
+  if (!nblk) return;
+  if (S.nr == 2)
+    hipLaunchKernelGGL(k_solve<2>, dim3(nblk), dim3(kSolveThreads), 0, s, E, refs, S, limit,
+                       first_solve);
+  else
+    hipLaunchKernelGGL(k_solve<4>, dim3(nblk), dim3(kSolveThreads), 0, s, E, refs, S, limit,
+                       first_solve);
 }
 
 void launch_finalize(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl, int njobs,
