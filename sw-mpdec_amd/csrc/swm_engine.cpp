@@ -84,7 +84,7 @@ JobLayout job_layout(int nx, int ny, int wb, int bathy) {
   }
   add((size_t)(kMaxSys + 1) * L.nblk);                   // Jacobi partial sums
   add(3 * (size_t)L.nblk);                               // TimeStep partials
-  add(solve_slot((int)L.n, kSolveForms, 0, 0, 0));       // k_solve's slots
+  add(solve_slot(nx, ny, kSolveForms, 0, 0, 0));         // k_solve's slots
   L.bytes = b;
   (void)bathy;  // the bathymetry tables are a separate allocation (bathy_bytes)
   return L;
@@ -141,12 +141,12 @@ struct Tables {
   std::vector<SolveRef> sv[2];
   std::vector<std::pair<int, int>> svl[2];
   bool solve_waits = false;  // some systems have several blocks
-  std::vector<TileRef> cbw;
+  std::vector<TileRef> cbs, cbw;  // of the grids k_solve takes, and of the others
   std::vector<int> jlw;
   DevVec<SolveRef> dsv[2];
-  DevVec<TileRef> dcbw;
+  DevVec<TileRef> dcbs, dcbw;
   DevVec<int> djlw;
-  int ncbw = 0, njobsw = 0;
+  int ncbs = 0, ncbw = 0, njobsw = 0;
 };
 
 enum JobState { JOB_RUNNING = 0, JOB_DONE = 1, JOB_FAILED = 2, JOB_FREE = 3 };
@@ -344,32 +344,35 @@ class SolveRight {
 
 // Rows of the largest system that one k_solve block takes alone.  At 2048 rows
 // (4 per thread) its assembly is issue-bound at about 10 us and a sweep costs
-// 1.2 us; four blocks of one row per thread assemble in 3 us and pay 2.3 us a
-// sweep, and at the 10 to 15 sweeps a solve needs the two break even.
+// about 1 us; tiles of 24x24 assemble in 5 us and pay 1.2 us a sweep with
+// their exchange, and at the 10 to 15 sweeps a solve needs the two break even.
 constexpr int kSolveAlone = 2048;
 
 // k_solve's blocks for the jobs of T.  A grid is taken when the blocks of one
 // system fit the device at once (blocks of a system wait for each other); the
 // blocks of several systems share a launch as long as all of them fit.  The
-// systems with several blocks take the form with the fewest rows per thread
-// that needs one launch, else the one with the most: a sweep's cost hardly
-// depends on the rows (2.4 to 6 us), a further launch repeats all of it.
-// Blocks without others to wait for come last and are not counted.
+// systems with several blocks take the smallest tiles that need one launch,
+// else the largest: a larger tile makes a sweep and the assembly longer, a
+// further launch repeats all of it.  Blocks without others to wait for come
+// last and are not counted.
 void solve_tables(swm_engine* e, Tables& T) {
   const int cap = std::min(e->solve_blocks_max, 256);
+  T.cbs.clear();
   T.cbw.clear();
   T.jlw.clear();
   std::vector<int> alone, shared;
+  auto blocks = [&](int id, int form) {
+    return solve_blocks(e->jobs[id]->dev.nx, e->jobs[id]->dev.ny, form);
+  };
   for (int id : T.jl) {
-    const int n = e->jobs[id]->dev.n;
-    if (n <= kSolveAlone && cap > 0) {
-      alone.push_back(id);
-    } else if (cap > 0 && solve_blocks(n, kSolveForms - 1) <= cap) {
-      shared.push_back(id);
-    } else {
-      for (int t = 0; t < e->jobs[id]->dev.nblk; ++t) T.cbw.push_back({id, t});
+    const JobDev& d = e->jobs[id]->dev;
+    const bool single = d.n <= kSolveAlone && cap > 0;
+    const bool solved = single || (cap > 0 && blocks(id, kSolveForms - 1) <= cap);
+    if (solved)
+      (single ? alone : shared).push_back(id);
+    else
       T.jlw.push_back(id);
-    }
+    for (int t = 0; t < d.nblk; ++t) (solved ? T.cbs : T.cbw).push_back({id, t});
   }
   T.solve_waits = !shared.empty();
   for (int c = 0; c < 2; ++c) {
@@ -380,24 +383,24 @@ void solve_tables(swm_engine* e, Tables& T) {
     int form = 0;
     for (; form < kSolveForms - 1; ++form) {
       long total = 0;
-      for (int id : shared) total += (long)nsys * solve_blocks(e->jobs[id]->dev.n, form);
+      for (int id : shared) total += (long)nsys * blocks(id, form);
       if (total <= cap) break;
     }
     int first = 0;
     for (int id : shared) {
-      const int nb = solve_blocks(e->jobs[id]->dev.n, form);
+      const int nb = blocks(id, form);
       for (int s = 0; s < nsys; ++s) {
         if ((int)v.size() - first + nb > cap) {
           T.svl[c].push_back({first, (int)v.size() - first});
           first = (int)v.size();
         }
-        for (int b = 0; b < nb; ++b) v.push_back({id, b, nb, (short)s, (short)form});
+        for (int b = 0; b < nb; ++b) v.push_back({id, b, (short)s, (short)form});
       }
     }
     for (int id : alone) {
-      int f = 0;
-      while (solve_blocks(e->jobs[id]->dev.n, f) > 1) ++f;
-      for (int s = 0; s < nsys; ++s) v.push_back({id, 0, 1, (short)s, (short)f});
+      int f = 0;  // 1 << f rows per thread
+      while (e->jobs[id]->dev.n > kSolveThreads << f) ++f;
+      for (int s = 0; s < nsys; ++s) v.push_back({id, 0, (short)s, (short)(kSolveForms + f)});
     }
     if ((int)v.size() > first) T.svl[c].push_back({first, (int)v.size() - first});
   }
@@ -411,10 +414,14 @@ int upload_tables(swm_engine* e, Tables& T) {
       HIPCK(e, hipMemcpy(T.dsv[c].p, T.sv[c].data(), T.sv[c].size() * sizeof(SolveRef),
                          hipMemcpyHostToDevice));
   }
+  T.ncbs = (int)T.cbs.size();
   T.ncbw = (int)T.cbw.size();
   T.njobsw = (int)T.jlw.size();
+  HIPCK(e, T.dcbs.reserve(T.cbs.size()));
   HIPCK(e, T.dcbw.reserve(T.cbw.size()));
   HIPCK(e, T.djlw.reserve(T.jlw.size()));
+  if (T.ncbs)
+    HIPCK(e, hipMemcpy(T.dcbs.p, T.cbs.data(), T.ncbs * sizeof(TileRef), hipMemcpyHostToDevice));
   if (T.ncbw)
     HIPCK(e, hipMemcpy(T.dcbw.p, T.cbw.data(), T.ncbw * sizeof(TileRef), hipMemcpyHostToDevice));
   if (T.njobsw)
@@ -730,8 +737,9 @@ int step_body(swm_engine* e, Tables& T, const StepPlan& P) {
     else
       for (int m = 1; m < D.msteps; ++m) S.m[S.count++] = m;
     if (S.hp_view) timed(e, 4, [&] { launch_hp_view(a, T.dcb.p, T.ncb, kk == 1, s); });
-    // the DeC momentum update runs inside the assembly and the solve kernels
+    // the DeC momentum update runs inside the assembly kernel
     if (P.solve) {
+      timed(e, 4, [&] { launch_assemble_matrix(a, T.dcbs.p, T.ncbs, S, s); });
       const int c = S.count == 1 ? 0 : 1;
       for (const auto& l : T.svl[c])
         timed(e, 5, [&] {
@@ -1334,7 +1342,7 @@ int alloc_job(swm_engine* e, int nx, int ny, double dx, double dy, double g, dou
   }
   D.part = take((size_t)(kMaxSys + 1) * lay.nblk);
   D.tspart = take(3 * (size_t)lay.nblk);
-  const size_t nslots = solve_slot(D.n, kSolveForms, 0, 0, 0);
+  const size_t nslots = solve_slot(nx, ny, kSolveForms, 0, 0, 0);
   D.slots = reinterpret_cast<unsigned long long*>(take(nslots));
   if (off > lay.bytes) FAIL(e, SWM_E_STATE, "internal: job slab overflow");
   e->in_use += (long long)lay.bytes;

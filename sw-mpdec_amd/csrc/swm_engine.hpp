@@ -38,7 +38,8 @@ constexpr int kNumShapes = 2;
 constexpr FaceShape kShapes[kNumShapes] = {{16, 16, 16, 16}, {32, 16, 16, 32}};
 constexpr int kCellBlock = 256;       // cells per block of the pointwise kernels
 constexpr int kSolveThreads = 512;    // threads of a k_solve block
-constexpr int kSolveForms = 4;        // k_solve forms: 1 << form rows per thread
+constexpr int kSolveWindow = 4;       // Jacobi sweeps between two exchanges of k_solve's blocks
+constexpr int kSolveForms = 4;        // k_solve's tile sizes (solve_tiles)
 constexpr int kMaxSys = 3;            // Patankar systems solved together (nodes 2..4)
 constexpr int kSlots = 3;             // concurrent FVTD evaluations per job
 constexpr int kStates = 6;            // state / derivative slots of the explicit schemes
@@ -171,26 +172,49 @@ struct TileRef {
   int tile;
 };
 
-// One block of k_solve: block blk of the nb blocks of one system of a job, in
-// the form with 1 << form rows per thread.
+// One block of k_solve: tile `tile` of one system of a job, in tile size
+// `form`; form >= kSolveForms: the whole grid in one block, with
+// 1 << (form - kSolveForms) rows per thread.
 struct SolveRef {
-  int job, blk, nb;
+  int job, tile;
   short sys, form;
 };
 
-// Blocks of one system of n rows in a form.
-inline __host__ __device__ int solve_blocks(int n, int form) {
-  const int rows = kSolveThreads << form;
-  return (n + rows - 1) / rows;
+// The tiles of a system in a form: ntx x nty tiles of at most tw x th cells,
+// the grid dealt out evenly.  With the window's halo the largest tile has
+// (tw + 8)(th + 8) = 1024, 2016, 4032 and 5184 rows: 2, 4, 8 and 11 per thread.
+struct SolveTiles {
+  int tw, th, ntx, nty;
+};
+inline __host__ __device__ SolveTiles solve_tiles(int nx, int ny, int form) {
+  const int mw = form == 0 ? 24 : form == 1 ? 40 : 64;
+  const int mh = form == 0 ? 24 : form == 1 ? 34 : form == 2 ? 48 : 64;
+  SolveTiles t;
+  t.ntx = (nx + mw - 1) / mw;
+  t.nty = (ny + mh - 1) / mh;
+  t.tw = (nx + t.ntx - 1) / t.ntx;
+  t.th = (ny + t.nty - 1) / t.nty;
+  t.ntx = (nx + t.tw - 1) / t.tw;  // rounding may leave the last ones empty
+  t.nty = (ny + t.th - 1) / t.th;
+  return t;
+}
+inline __host__ __device__ int solve_blocks(int nx, int ny, int form) {
+  const SolveTiles t = solve_tiles(nx, ny, form);
+  return t.ntx * t.nty;
 }
 
-// JobDev::slots: per form, system, kind (0: residual, 1: right-hand side) and
-// parity of the round, one slot per block.  The forms have slots of their own,
-// so that each slot is written in every second round of its form.
-inline __host__ __device__ size_t solve_slot(int n, int form, int sys, int kind, int parity) {
+// JobDev::slots: per form, system, parity of the round and kind (a sweep of
+// the window, or kSolveWindow: the right-hand side), one slot per block.  The
+// forms have slots of their own, so that each slot is written in every second
+// round of its form.
+constexpr int kSolveKinds = kSolveWindow + 1;
+inline __host__ __device__ size_t solve_slot(int nx, int ny, int form, int sys, int parity,
+                                             int kind) {
   size_t o = 0;
-  for (int f = 0; f < form; ++f) o += (size_t)kMaxSys * 4 * solve_blocks(n, f);
-  return o + (size_t)((sys * 2 + kind) * 2 + parity) * solve_blocks(n, form);
+  for (int f = 0; f < form; ++f)
+    o += (size_t)kMaxSys * 2 * kSolveKinds * solve_blocks(nx, ny, f);
+  if (form == kSolveForms) return o;
+  return o + (size_t)((sys * 2 + parity) * kSolveKinds + kind) * solve_blocks(nx, ny, form);
 }
 
 // Arguments shared by every launch of one engine step.  gated = 1 in the
@@ -321,8 +345,11 @@ void launch_sweep(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl
                   const SysList& S, hipStream_t s);
 void launch_finalize(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl, int njobs,
                      const SysList& S, hipStream_t s);
-// k_solve over nblk blocks: assembly, momentum update and the whole Jacobi
-// iteration of each block's system, up to `limit` sweeps
+// the matrix rows and the momentum update alone, for the grids k_solve takes
+void launch_assemble_matrix(const EngineArgs& E, const TileRef* cb, int ncb, const SysList& S,
+                            hipStream_t s);
+// k_solve over nblk blocks: the Jacobi iteration of each block's system, up to
+// `limit` sweeps
 void launch_solve(const EngineArgs& E, const SolveRef* refs, int nblk, const SysList& S, int limit,
                   int first_solve, hipStream_t s);
 void launch_timestep(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl, int njobs,

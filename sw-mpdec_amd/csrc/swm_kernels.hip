@@ -572,13 +572,11 @@ __device__ double block_sum_array(const double* part, int nb, double* red) {
 // (n-1)u*sum(d), so whenever tol lies outside [S - B, S + B]/n with
 // B = 8nuS the decision is that of the sequential sum; inside the window the
 // caller recomputes the sequential sum exactly.  1 continue, 0 stop, -1 open.
-// extra: a further relative error of S.
-__device__ __forceinline__ int certified_continue(double S, int n, double tol,
-                                                  double extra = 0.) {
+__device__ __forceinline__ int certified_continue(double S, int n, double tol) {
   if (isnan(S)) return 0;
   if (isinf(S)) return 1;
   const double u = 1.1102230246251565e-16;  // 2^-53
-  double B = (8.0 * (double)n * u + extra) * S;
+  double B = 8.0 * (double)n * u * S;
   double lo = (S - B) / (double)n, hi = (S + B) / (double)n;
   if (tol < lo) return 1;
   if (!(tol < hi)) return 0;
@@ -670,15 +668,15 @@ __device__ __forceinline__ void patankar_slot(int pos, const double c[R], const 
 }
 
 // The four stencil slots of one row-system (sparse_matmul in CSR order S, W,
-// self (value 0), E, N): writes the slots' matrix entries, accumulates the
+// self (value 0), E, N): hands the slots' matrix entries to put, accumulates the
 // diagonal into D and returns the product with the neighbours' rhs values.
 // sq: the row's column of the staged fluxes, NT apart.
-template <int R, bool WET, int NT>
-__device__ __forceinline__ double patankar_row(const JobDev& J, int s, size_t k, const double* sq,
-                                               int pos, const double c[R], const PdDepth& pK,
-                                               double hS, double hW, double hE, double hN,
-                                               double bS, double bW, double bE, double bN,
-                                               double b, double& D) {
+template <int R, bool WET, int NT, class Put>
+__device__ __forceinline__ double patankar_row(Put put, const double* sq, int pos,
+                                               const double c[R], const PdDepth& pK, double hS,
+                                               double hW, double hE, double hN, double bS,
+                                               double bW, double bE, double bN, double b,
+                                               double& D) {
   double p = 0.;
 #pragma unroll 1
   for (int sl = 0; sl < 4; ++sl) {
@@ -690,7 +688,7 @@ __device__ __forceinline__ double patankar_row(const JobDev& J, int s, size_t k,
     for (int r = 0; r < R; ++r) q[r] = sq[(sl * R + r) * NT];
     double M;
     patankar_slot<R, WET>(pos, c, q, pd_depth(hL), pK, M, D);
-    G(J.M[s][sl])[k] = M;
+    put(sl, M);
     p = p + M * bL;
     if (sl == 1) p = p + 0. * b;
   }
@@ -707,7 +705,10 @@ __device__ __forceinline__ const gdouble* system_rhs(const JobDev& J, const SysL
   return G(S.hp_view ? J.hres[2] : J.h);
 }
 
-template <int R>
+// FIRST: the first sweep and its residual sums, for a launch per sweep; without
+// it only the matrix, for k_solve.  blockIdx.y picks the system where the grid
+// has that dimension (launch_assemble_matrix), else the block does them all.
+template <int R, bool FIRST>
 __global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* blocks,
                                                   SysList S) {
   __shared__ double red[4];
@@ -720,6 +721,7 @@ __global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* b
   const int k = T.tile * kCellBlock + tid;
   const bool in = k < n;
   const double dt = J.status->dt;
+  const int s0 = gridDim.y > 1 ? blockIdx.y : 0, s1 = gridDim.y > 1 ? s0 + 1 : S.count;
   int kS = 0, kW = 0, kE = 0, kN = 0;  // neighbours
   double b = 0., bS = 0., bW = 0., bE = 0., bN = 0.;
   if (in) {
@@ -740,18 +742,20 @@ __global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* b
       sq[(3 * R + r) * 256 + tid] = -G(J.qy[S.src[r]])[gN];  // the flux oriented into the cell
     }
     const gdouble* rhs = system_rhs(J, S);
-    b = rhs[k];
-    bS = rhs[kS];
-    bW = rhs[kW];
-    bE = rhs[kE];
-    bN = rhs[kN];
-    momentum_cell<R>(J, S, 0, S.count, k, dt);
+    if (FIRST) {
+      b = rhs[k];
+      bS = rhs[kS];
+      bW = rhs[kW];
+      bE = rhs[kE];
+      bN = rhs[kN];
+    }
+    momentum_cell<R>(J, S, s0, s1, k, dt);
   }
   // One system at a time, and within it one stencil slot at a time (S, W, E,
   // N: the CSR order), so that only one slot's divisions are live.  Each
   // thread reads back only its own column of sq, so no barrier is needed.
 #pragma unroll 1
-  for (int s = 0; s < S.count; ++s) {
+  for (int s = s0; s < s1; ++s) {
     double d = 0.;
     if (in) {
       const int m = S.m[s];
@@ -767,19 +771,24 @@ __global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* b
       double D = 1.;
       const bool dry = pK.dry | (hS < kMinDepth) | (hW < kMinDepth) | (hE < kMinDepth) |
                        (hN < kMinDepth);
-      const double p =
-          __any(dry) ? patankar_row<R, false, 256>(J, s, k, sq + tid, pos, c, pK, hS, hW, hE, hN,
-                                                   bS, bW, bE, bN, b, D)
-                     : patankar_row<R, true, 256>(J, s, k, sq + tid, pos, c, pK, hS, hW, hE, hN,
-                                                  bS, bW, bE, bN, b, D);
+      auto put = [&](int sl, double v) { G(J.M[s][sl])[k] = v; };
+      const double p = __any(dry)
+                           ? patankar_row<R, false, 256>(put, sq + tid, pos, c, pK, hS, hW, hE, hN,
+                                                         bS, bW, bE, bN, b, D)
+                           : patankar_row<R, true, 256>(put, sq + tid, pos, c, pK, hS, hW, hE, hN,
+                                                        bS, bW, bE, bN, b, D);
       G(J.M[s][4])[k] = D;
-      double x1 = (b - p) / D;
-      G(J.xj[m][1])[k] = x1;
-      d = fabs(x1 - b);
+      if (FIRST) {
+        double x1 = (b - p) / D;
+        G(J.xj[m][1])[k] = x1;
+        d = fabs(x1 - b);
+      }
     }
+    if (!FIRST) continue;
     double t = block_sum_all(d, red);
     if (tid == 0) J.part[(size_t)s * J.nblk + T.tile] = t;
   }
+  if (!FIRST) return;
   double t = block_sum_all(in ? fabs(0.0 - b) : 0., red);
   if (tid == 0) J.part[(size_t)kMaxSys * J.nblk + T.tile] = t;
 }
@@ -908,41 +917,48 @@ __global__ __launch_bounds__(256) void k_decide(EngineArgs E, const int* jobs, S
 }
 
 // ------------------------------------------------------------------------
-// The whole Patankar solve of a correction in one launch, for grids whose
+// The Jacobi iteration of a correction's solves in one launch, for grids whose
 // systems fit the register files.
 //
-// A system of n rows belongs to nb blocks of 512 threads, 1 << FORM rows per
-// thread.  A block assembles its rows as k_assemble does, keeps the matrix
-// rows in registers and the iterate in LDS, and sweeps until the stop rule
-// ends the solve: no sweep reads the matrix from memory, and no launch, host
-// prediction or empty sweep is paid per sweep.  A sweep of a launch of its own
-// with its stop decision took 13 us at any size up to 257^2 (5.2 + 3.9 us and
-// two launch gaps at 32^2), and 34 us at 1024^2.  mPDeC5 passes with the
-// state's transfer, before and after: 32^2, 20 steps 17.8 -> 6.3 ms; 257^2, 10
-// steps 9.5 -> 6.0 ms; 1024^2 dam break, 4 steps 25.1 -> 22.0 ms.
+// A block of 512 threads owns a tile of a system and holds it with a halo of
+// kSolveWindow = 4 cells: the matrix rows in registers (up to 11 per thread),
+// the iterate in LDS.  It sweeps 4 times
+// without looking at the other blocks -- each sweep spoils one more ring of
+// the halo -- then the blocks exchange their outer 4 rings and the residual
+// sums of the 4 sweeps, and the stop rule is applied to the sums in order.  A
+// solve that stopped inside the window takes the iterate of that sweep, which
+// is in LDS or at most two sweeps from the window's start.  The first window
+// needs no exchange before it: it starts from the right-hand side, known
+// everywhere.  So no sweep reads the matrix from memory, and no launch, host
+// prediction or empty sweep is paid per sweep.
 //
-// Several blocks of a system (nb > 1) exchange, per sweep, the rows that other
-// blocks' stencils reach (all within nx rows of the block's ends) and their
-// part of the residual sum.  All of that goes through agent-scope atomic
-// stores and loads, which bypass the XCDs' separate L2s, so no cache is
-// written back: a block drains its row stores (s_waitcnt vmcnt(0)), then
-// publishes its sum in a slot whose low 8 bits carry the round's tag, and
-// polls the other blocks' slots for that tag.  Measured per round: 2.4 us for
-// 8 blocks, 3.3 us for 64, 4.3 us for 240; with a counter instead of tags 3.0,
-// 3.7, 6.7 us; with agent-scope fences 5.1 us for 64.  The rows of round t go
-// to buffer t & 1: a block overwrites it in round t + 2, after every block has
-// published round t + 1 and so finished reading round t.
+// Measured per correction (three systems): 32^2 190 -> 33 -> SOLVE32 us,
+// 257^2 135 -> 61 -> SOLVE257 us; the first figure with a launch per sweep and
+// one per stop decision, the second with row strips exchanged after every
+// sweep.  The exchange dominates there: 3.3 us for 64 blocks, against 0.6 us
+// for the sweep of a 40x40 tile.
 //
-// The tag takes the sum's low 8 bits, a relative change below 2^-44, which
-// certified_continue is told of.  Tags count on over the launches
+// The exchange goes through agent-scope atomic stores and loads, which bypass
+// the XCDs' separate L2s, so no cache is written back: a block drains its
+// stores (s_waitcnt vmcnt(0)), then publishes its sums in slots whose low 8
+// bits carry the round's tag, and polls the other blocks' slots for that tag.
+// Measured per round: 2.4 us for 8 blocks, 3.3 us for 64, 4.3 us for 240; with
+// a counter instead of tags 3.0, 3.7, 6.7 us; with agent-scope fences 5.1 us
+// for 64.  The cells of round t go to buffer t & 1: a block overwrites it in
+// round t + 2, after every block has published round t + 1 and so finished
+// reading round t.
+//
+// The tag takes the sum's low 8 bits, a relative change below 2^-44, which the
+// stop rule allows for.  Tags count on over the launches
 // (JobStatus::rounds), and a slot is rewritten in every second round of its
 // form, so the tag it held before is the expected one less 2.
 //
 // The host launches no more blocks at once than the device holds
 // concurrently, and no two such launches side by side.  A wait is bounded all
-// the same: when it runs out (another process on the device, say), or a stop decision lies inside the certified
-// window, the solve ends as kSolveOpen, the step is not committed and the host
-// runs it again with the launches of one sweep each.
+// the same: when it runs out (another process on the device, say), or a stop
+// decision lies inside the certified window, the solve ends as kSolveOpen, the
+// step is not committed and the host runs it again with the launches of one
+// sweep each.
 // ------------------------------------------------------------------------
 constexpr int kSolvePolls = 1 << 15;  // about 25 ms
 
@@ -953,261 +969,329 @@ __device__ __forceinline__ void agent_store(double* p, double v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Sum of v over the block in LDS buffer red (one double per wave); every thread calls,
-// and the sum is ready after the barrier inside.
-__device__ __forceinline__ double solve_block_sum(double v, double* red) {
-  v = wave_sum(v);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  double t = red[0];
-#pragma unroll
-  for (int w = 1; w < kSolveThreads / 64; ++w) t += red[w];
-  return t;
+// v of lane (this - n) within rows of 16 lanes, or of the previous rows' last
+// lane (CTRL of the DPP encoding); 0 where there is none.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
+  return __hiloint2double(hi, lo);
 }
 
-template <int R>
+// Sum over the wave in a fixed order, in every lane; six dependent steps
+// without LDS (the shuffles of wave_sum are LDS instructions of 130 cycles).
+__device__ __forceinline__ double wave_sum_dpp(double v) {
+  v += dpp<0x111, 0xf>(v);  // row_shr:1
+  v += dpp<0x112, 0xf>(v);
+  v += dpp<0x114, 0xf>(v);
+  v += dpp<0x118, 0xf>(v);
+  v += dpp<0x142, 0xa>(v);  // row_bcast:15
+  v += dpp<0x143, 0xc>(v);  // row_bcast:31
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                          __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
+constexpr int kSolveRows = 11 * kSolveThreads;  // rows of the largest tile with its halo
+constexpr int kSolveWaves = kSolveThreads / 64;
+
 struct SolveShared {
-  static constexpr int kDoubles = 4 * R * kSolveThreads > 2 * (kSolveThreads << (kSolveForms - 1))
-                                      ? 4 * R * kSolveThreads
-                                      : 2 * (kSolveThreads << (kSolveForms - 1));
-  // assembly: [slot*R + node][thread] face mass fluxes; then the iterate [2][rows]
-  double sm[kDoubles];
-  double red[2][2][kSolveThreads / 64];  // [parity][kind]
-  double tot[2][2][4];                   // the blocks' sums, by wave
+  double x[3][kSolveRows];  // the iterate: the window's start and two buffers
+
+  double red[kSolveKinds][kSolveWaves];
+  double tot[kSolveKinds][4];
   int lost;
 };
-
-template <int FORM, int R>
-__device__ __forceinline__ void solve_block(SolveShared<R>& L, const EngineArgs& E,
-                                            const SolveRef W, const SysList& S, int limit,
-                                            int first_solve) {
-  constexpr int NT = kSolveThreads, RPT = 1 << FORM, ROWS = NT * RPT;
-  double* sm = L.sm;
-  auto& red = L.red;
-  auto& tot = L.tot;
-  int& lost = L.lost;
+// ALONE: the whole grid in the block, no halo and no exchange.
+template <int RPT, bool ALONE>
+__device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E, const SolveRef W,
+                                            const SysList& S, int limit, int first_solve) {
+  constexpr int NT = kSolveThreads, HALO = ALONE ? 0 : kSolveWindow;
   const JobDev& J = E.jobs[W.job];
-  const int tid = threadIdx.x, s = W.sys, nb = W.nb, m = S.m[s];
+  const int tid = threadIdx.x, s = W.sys, m = S.m[s];
   const int nx = J.nx, ny = J.ny, n = J.n;
-  const int base = W.blk * ROWS, len = min(n - base, ROWS);
   JobStatus* st = J.status;
-  const double dt = st->dt;
-  const unsigned round0 = st->rounds[FORM][s];
   const gdouble* rhs = system_rhs(J, S);
-  if (tid == 0) lost = 0;
+  // own cells [ox, ox + ow) x [oy, oy + oh); EW x EH with the halo
+  int nb = 1, ox = 0, oy = 0, ow = nx, oh = ny, EW = nx, EH = ny;
+  unsigned round0 = 0;
+  if (!ALONE) {
+    const SolveTiles T = solve_tiles(nx, ny, W.form);
+    nb = T.ntx * T.nty;
+    ox = (W.tile % T.ntx) * T.tw;
+    oy = (W.tile / T.ntx) * T.th;
+    ow = min(T.tw, nx - ox);
+    oh = min(T.th, ny - oy);
+    EW = T.tw + 2 * HALO;
+    EH = T.th + 2 * HALO;
+    round0 = st->rounds[W.form][s];
+  }
+  const int rows = EW * EH;
+  if (tid == 0) L.lost = 0;
 
-  // assembly and momentum, one row at a time; the matrix rows go through
-  // memory (their own thread reads them back) so that the loop stays rolled
-  double dsum = 0., bsum = 0.;
-#pragma unroll 1
+  // The thread's matrix rows, as k_assemble left them, and the start x = b.
+  // act: rows with all four neighbours in the tile; own: the block's own
+  // cells; outer: those that other blocks read.
+  double M[RPT][4], D[RPT], b[RPT];
+  int at[ALONE ? RPT : 1][4], gk[RPT];
+  unsigned act = 0, own = 0, outer = 0;
+  double bsum = 0.;
+#pragma unroll
   for (int i = 0; i < RPT; ++i) {
     const int l = i * NT + tid;
-    if (l >= len) break;
-    const int k = base + l, cj = k / nx, ci = k - cj * nx;
-    const int kS = (cj == 0 ? ny - 1 : cj - 1) * nx + ci;
-    const int kW = cj * nx + (ci == 0 ? nx - 1 : ci - 1);
-    const int kE = cj * nx + (ci == nx - 1 ? 0 : ci + 1);
-    const int kN = (cj == ny - 1 ? 0 : cj + 1) * nx + ci;
-    const size_t fW = (size_t)cj * (nx + 1) + ci, fE = fW + 1;
-    const size_t gS = (size_t)cj * nx + ci, gN = gS + nx;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      sm[(0 * R + r) * NT + tid] = G(J.qy[S.src[r]])[gS];
-      sm[(1 * R + r) * NT + tid] = G(J.qx[S.src[r]])[fW];
-      sm[(2 * R + r) * NT + tid] = -G(J.qx[S.src[r]])[fE];
-      sm[(3 * R + r) * NT + tid] = -G(J.qy[S.src[r]])[gN];
-    }
-    const double b = rhs[k], bS = rhs[kS], bW = rhs[kW], bE = rhs[kE], bN = rhs[kN];
-    const gdouble* hp = system_hp(J, S, m);
-    const double hK = hp[k], hS = hp[kS], hW = hp[kW], hE = hp[kE], hN = hp[kN];
-    momentum_cell<R>(J, S, s, s + 1, k, dt);
-    const PdDepth pK = pd_depth(hK);
-    const int pos = THETA_POS[S.theta][m];
-    double c[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) c[r] = dt * THETA[S.theta][m][r];
-    double D = 1.;
-    const bool dry = pK.dry | (hS < kMinDepth) | (hW < kMinDepth) | (hE < kMinDepth) |
-                     (hN < kMinDepth);
-    const double p =
-        __any(dry) ? patankar_row<R, false, NT>(J, s, k, sm + tid, pos, c, pK, hS, hW, hE, hN, bS,
-                                                bW, bE, bN, b, D)
-                   : patankar_row<R, true, NT>(J, s, k, sm + tid, pos, c, pK, hS, hW, hE, hN, bS,
-                                               bW, bE, bN, b, D);
-    const double x1 = (b - p) / D;
-    G(J.M[s][4])[k] = D;
-    G(J.xj[m][1])[k] = x1;
-    dsum += fabs(x1 - b);
-    bsum += fabs(0.0 - b);
-  }
-  __syncthreads();  // the fluxes have been read: sm takes the iterate
-
-  double M[RPT][4], D[RPT], b[RPT], x[RPT];
-  int at[RPT][4];  // neighbours' row numbers less base
-#pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-    const int l = i * NT + tid, k = base + l;
-    if (l < len) {
-      const int cj = k / nx, ci = k - cj * nx;
-      at[i][0] = (cj == 0 ? ny - 1 : cj - 1) * nx + ci - base;
-      at[i][1] = cj * nx + (ci == 0 ? nx - 1 : ci - 1) - base;
-      at[i][2] = cj * nx + (ci == nx - 1 ? 0 : ci + 1) - base;
-      at[i][3] = (cj == ny - 1 ? 0 : cj + 1) * nx + ci - base;
+    if (l < rows) {
+      const int ly = l / EW, lx = l - ly * EW;
+      int ci = lx, cj = ly;
+      if (ALONE) {
+        act |= 1u << i;
+        own |= 1u << i;
+        at[i][0] = (cj == 0 ? ny - 1 : cj - 1) * nx + ci;
+        at[i][1] = cj * nx + (ci == 0 ? nx - 1 : ci - 1);
+        at[i][2] = cj * nx + (ci == nx - 1 ? 0 : ci + 1);
+        at[i][3] = (cj == ny - 1 ? 0 : cj + 1) * nx + ci;
+      } else {
+        const int tx = lx - HALO, ty = ly - HALO;  // within the own cells
+        ci = (ox + tx) % nx;
+        cj = (oy + ty) % ny;
+        if (ci < 0) ci += nx;
+        if (cj < 0) cj += ny;
+        if (lx >= 1 && lx < EW - 1 && ly >= 1 && ly < EH - 1) act |= 1u << i;
+        if (tx >= 0 && tx < ow && ty >= 0 && ty < oh) {
+          own |= 1u << i;
+          if (tx < HALO || tx >= ow - HALO || ty < HALO || ty >= oh - HALO) outer |= 1u << i;
+        }
+      }
+      const int k = cj * nx + ci;
+      gk[i] = k;
 #pragma unroll
       for (int q = 0; q < 4; ++q) M[i][q] = G(J.M[s][q])[k];
       D[i] = G(J.M[s][4])[k];
-      x[i] = G(J.xj[m][1])[k];
       b[i] = rhs[k];
     }
   }
-
-  int k_sweeps = 1, zero = 0, end = kSolveConverged;
-  unsigned t = 0;
-  for (;; ++t) {
-    // publish round t: the iterate in LDS, its outer rows and the block's sums
-    const int par = t & 1;
-    double* sx = sm + par * ROWS;
-    double* buf = J.FX[s][par];  // free between an FVTD's update and the next one's face kernels
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-      const int l = i * NT + tid;
-      if (l < len) {
-        sx[l] = x[i];
-        if (nb > 1 && (l < nx || l >= len - nx)) agent_store(buf + base + l, x[i]);
-      }
-    }
-    if (t == 0) bsum = wave_sum(bsum);
-    if (t == 0 && (tid & 63) == 0) red[par][1][tid >> 6] = bsum;
-    if (nb > 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    double S1 = solve_block_sum(dsum, red[par][0]), S0 = 0.;
-    if (t == 0)
-      for (int w = 0; w < NT / 64; ++w) S0 += red[par][1][w];
-    if (nb > 1) {
-      const unsigned tag = (round0 + t + 1u) & 0xffu, tp = (round0 + t) & 1u;
-      unsigned long long* slot[2];
-      for (int q = 0; q < 2; ++q) slot[q] = J.slots + solve_slot(n, FORM, s, q, tp);
-      if (tid == 0)
-        for (int q = (t == 0 ? 1 : 0); q >= 0; --q)
-          __hip_atomic_store(slot[q] + W.blk,
-                             ((unsigned long long)__double_as_longlong(q ? S0 : S1) & ~0xffull) |
-                                 tag,
-                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (tid < 256) {  // nb <= 256: the first four waves poll
-        for (int q = (t == 0 ? 1 : 0); q >= 0; --q) {
-          unsigned long long v = tag;
-          if (tid < nb) {
-            int polls = 0;
-            do {
-              v = __hip_atomic_load(slot[q] + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } while ((unsigned)(v & 0xffu) != tag && ++polls < kSolvePolls);
-            if ((unsigned)(v & 0xffu) != tag) lost = 1;
-          }
-          const double w = wave_sum(__longlong_as_double((long long)(v & ~0xffull)));
-          if ((tid & 63) == 0) tot[par][q][tid >> 6] = w;
-        }
-      }
-      __syncthreads();
-      S1 = ((tot[par][0][0] + tot[par][0][1]) + tot[par][0][2]) + tot[par][0][3];
-      if (t == 0) S0 = ((tot[par][1][0] + tot[par][1][1]) + tot[par][1][2]) + tot[par][1][3];
-      if (lost) {  // set before the barrier: every thread of the block sees it
-        end = kSolveOpen;
-        break;
-      }
-    }
-    // the stop rule (src/jacobi_iteration.f90:63-84): the same numbers, and so
-    // the same decision, in every block of the system
-    const double extra = nb > 1 ? 0x1p-43 : 0.;
-    if (t == 0) {
-      const int c0 = certified_continue(S0, n, E.tol, extra);
-      if (c0 < 0) {
-        end = kSolveOpen;
-        break;
-      }
-      if (!c0 || E.max_iter <= 0) {
-        k_sweeps = 0;
-        zero = 1;
-        end = c0 ? kSolveLimit : kSolveConverged;
-        break;
-      }
-    }
-    const int c1 = certified_continue(S1, n, E.tol, extra);
-    if (c1 <= 0) {
-      end = c1 < 0 ? kSolveOpen : kSolveConverged;
-      break;
-    }
-    if (k_sweeps >= E.max_iter) {
-      end = kSolveLimit;
-      break;
-    }
-    if (k_sweeps >= limit) {
-      end = kSolveOpen;
-      break;
-    }
-    ++k_sweeps;
-    // one sweep (src/jacobi_iteration.f90:72-80)
-    dsum = 0.;
-    constexpr int GR = RPT < 4 ? RPT : 2;  // rows with their loads in flight together
+  for (int i = 0; i < RPT; ++i) {
+    const int l = i * NT + tid;
+    if (l < rows) L.x[0][l] = b[i];
+    if ((own >> i) & 1u) bsum += fabs(0.0 - b[i]);
+  }
+
+  // One sweep (src/jacobi_iteration.f90:72-80) of every row with its
+  // neighbours in the tile; returns the thread's part of the own cells'
+  // SUM(ABS(x_new - x_old)).
+  auto sweep = [&](const double* from, double* to) {
+    double dsum = 0.;
+    constexpr int GR = RPT < 4 ? RPT : 4;  // rows with their loads in flight together
 #pragma unroll
     for (int i0 = 0; i0 < RPT; i0 += GR) {
-      double y[GR][4];
 #pragma unroll
-      for (int i = i0; i < i0 + GR; ++i)
-        if (i * NT + tid < len) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int a = at[i][q];
-            if ((unsigned)a < (unsigned)ROWS)
-              y[i - i0][q] = sx[a];
-            else
-              y[i - i0][q] = agent_load(buf + base + a);
-          }
-        }
-#pragma unroll
-      for (int i = i0; i < i0 + GR; ++i)
-        if (i * NT + tid < len) {
+      for (int i = i0; i < i0 + GR && i < RPT; ++i)
+        if ((act >> i) & 1u) {
+          const int l = i * NT + tid;
+          const int* a = at[ALONE ? i : 0];
+          const double yS = from[ALONE ? a[0] : l - EW], yW = from[ALONE ? a[1] : l - 1];
+          const double yE = from[ALONE ? a[2] : l + 1], yN = from[ALONE ? a[3] : l + EW];
+          const double x = from[l];
           double p = 0.;
-          p = p + M[i][0] * y[i - i0][0];
-          p = p + M[i][1] * y[i - i0][1];
-          p = p + 0. * x[i];
-          p = p + M[i][2] * y[i - i0][2];
-          p = p + M[i][3] * y[i - i0][3];
+          p = p + M[i][0] * yS;
+          p = p + M[i][1] * yW;
+          p = p + 0. * x;
+          p = p + M[i][2] * yE;
+          p = p + M[i][3] * yN;
           const double xv = (b[i] - p) / D[i];
-          dsum += fabs(xv - x[i]);
-          x[i] = xv;
+          to[l] = xv;
+          if ((own >> i) & 1u) dsum += fabs(xv - x);
         }
     }
+    __syncthreads();
+    return dsum;
+  };
+
+  // certified_continue with the division by n taken to the other side: n tol
+  // widened by 2^-50 covers the roundings of both forms, 2^-43 the tags.
+  const double tn = E.tol * (double)n, width = fabs(tn) * 0x1p-50;
+  const double tn_lo = tn - width, tn_hi = tn + width;
+  const double relS = 8.0 * (double)n * 0x1p-53 + (ALONE ? 0. : 0x1p-43);
+  auto certified = [&](double sum) {
+    const double B = relS * sum;
+    if (isnan(sum)) return 0;
+    if (isinf(sum) || sum - B > tn_hi) return 1;
+    return sum + B <= tn_lo ? 0 : -1;
+  };
+
+  __syncthreads();
+  double *p0 = L.x[0], *q0 = L.x[1], *q1 = L.x[2];
+  const double* result = nullptr;
+  int k_sweeps = 0, end = kSolveConverged;
+  bool zero = false;
+  unsigned t = 0;
+  for (;; ++t) {
+    double sum[kSolveKinds];
+    sum[0] = sweep(p0, q0);
+    sum[1] = sweep(q0, q1);
+    sum[2] = sweep(q1, q0);
+    sum[3] = sweep(q0, q1);
+    static_assert(kSolveWindow == 4, "the sweeps above");
+    sum[kSolveWindow] = bsum;  // used in the first round only
+    double* buf = J.FX[s][t & 1];  // free between an FVTD's update and the next one's face kernels
+    if (!ALONE) {
+#pragma unroll
+      for (int i = 0; i < RPT; ++i)
+        if ((outer >> i) & 1u) agent_store(buf + gk[i], q1[i * NT + tid]);
+    }
+#pragma unroll
+    for (int q = 0; q < kSolveKinds; ++q) {
+      const double w = wave_sum_dpp(sum[q]);
+      if ((tid & 63) == 0) L.red[q][tid >> 6] = w;
+    }
+    if (!ALONE) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    const unsigned tag = (round0 + t + 1u) & 0xffu;
+    if (!ALONE) {
+      const size_t slot = solve_slot(nx, ny, W.form, s, (round0 + t) & 1u, 0);
+      if (tid < kSolveKinds) {
+        double v = L.red[tid][0];
+        for (int w = 1; w < kSolveWaves; ++w) v += L.red[tid][w];
+        __hip_atomic_store(J.slots + slot + (size_t)tid * nb + W.tile,
+                           ((unsigned long long)__double_as_longlong(v) & ~0xffull) | tag,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      // waves 0-3 poll kinds 0, 1 and 4 of block tid (nb <= 256), waves 4-7
+      // kinds 2 and 3
+      const int half = tid >> 8, blk = tid & 255;
+      const int nk = half == 0 && t == 0 ? 3 : 2;
+      unsigned long long v[3] = {tag, tag, tag};
+      if (blk < nb) {
+        int polls = 0;
+        bool missing;
+        do {
+          missing = false;
+          for (int q = 0; q < nk; ++q) {
+            const int kind = q == 2 ? kSolveWindow : 2 * half + q;
+            v[q] = __hip_atomic_load(J.slots + slot + (size_t)kind * nb + blk, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
+            missing |= (unsigned)(v[q] & 0xffu) != tag;
+          }
+        } while (missing && ++polls < kSolvePolls);
+        if (missing) L.lost = 1;
+      }
+      for (int q = 0; q < nk; ++q) {
+        const double w = wave_sum_dpp(__longlong_as_double((long long)(v[q] & ~0xffull)));
+        if ((tid & 63) == 0) L.tot[q == 2 ? kSolveWindow : 2 * half + q][(tid >> 6) & 3] = w;
+      }
+      __syncthreads();
+      if (L.lost) {  // set before the barrier: every thread of the block sees it
+        end = kSolveOpen;
+        break;
+      }
+    }
+    auto total = [&](int q) {
+      double v;
+      if (ALONE) {
+        v = L.red[q][0];
+        for (int w = 1; w < kSolveWaves; ++w) v += L.red[q][w];
+      } else {
+        v = ((L.tot[q][0] + L.tot[q][1]) + L.tot[q][2]) + L.tot[q][3];
+      }
+      return v;
+    };
+    // the stop rule (src/jacobi_iteration.f90:63-84), sweep by sweep: the same
+    // numbers, and so the same decisions, in every block of the system
+    bool stop = false;
+    if (t == 0) {
+      const int c0 = certified(total(kSolveWindow));
+      if (c0 < 0) {
+        stop = true;
+        end = kSolveOpen;
+      } else if (!c0 || E.max_iter <= 0) {
+        stop = true;
+        zero = true;
+        end = c0 ? kSolveLimit : kSolveConverged;
+      }
+    }
+    int j = 0;
+    for (; j < kSolveWindow && !stop; ++j) {
+      ++k_sweeps;
+      const int c1 = certified(total(j));
+      stop = true;
+      if (c1 < 0)
+        end = kSolveOpen;
+      else if (c1 == 0)
+        end = kSolveConverged;
+      else if (k_sweeps >= E.max_iter)
+        end = kSolveLimit;
+      else if (k_sweeps >= limit)
+        end = kSolveOpen;
+      else
+        stop = false;
+    }
+    if (stop) {
+      // the iterate of the window's sweep j (counted from 1)
+      if (end == kSolveOpen || zero) break;
+      if (j == 4) {
+        result = q1;
+      } else if (j == 3) {
+        result = q0;
+      } else {
+        sweep(p0, q0);
+        result = q0;
+        if (j == 2) {
+          sweep(q0, q1);
+          result = q1;
+        }
+      }
+      break;
+    }
+    if (!ALONE) {
+      // the halo of the next window
+#pragma unroll
+      for (int i = 0; i < RPT; ++i) {
+        const int l = i * NT + tid;
+        if (l < rows && !((own >> i) & 1u)) q1[l] = agent_load(buf + gk[i]);
+      }
+    }
+    __syncthreads();  // also: the sums have been read
+    double* w = p0;
+    p0 = q1;
+    q1 = q0;
+    q0 = w;
   }
   if (end != kSolveOpen) {
 #pragma unroll
     for (int i = 0; i < RPT; ++i)
-      if (i * NT + tid < len) G(J.hres[m])[base + i * NT + tid] = zero ? 0. : x[i];
+      if ((own >> i) & 1u) G(J.hres[m])[gk[i]] = zero ? 0. : result[i * NT + tid];
   }
   if (tid == 0) {
-    if (lost) st->solve_lost = 1;  // k_gate keeps the step from being committed
-    if (W.blk == 0) {
+    if (!ALONE && L.lost) st->solve_lost = 1;  // k_gate keeps the step from being committed
+    if (W.tile == 0) {
       st->ended[first_solve + s] = end;
       st->iters[first_solve + s] = k_sweeps;
       st->ambiguous[first_solve + s] = 0;
-      st->rounds[FORM][s] = round0 + t + 1u;
+      if (!ALONE) st->rounds[W.form][s] = round0 + t + 1u;
     }
   }
 }
 
-template <int R>
 __global__ __launch_bounds__(kSolveThreads) void k_solve(EngineArgs E, const SolveRef* refs,
                                                          SysList S, int limit, int first_solve) {
-  __shared__ SolveShared<R> L;
+  __shared__ SolveShared L;
   const SolveRef W = refs[blockIdx.x];
   if (skipped(E, E.jobs[W.job])) return;
-  static_assert(kSolveForms == 4, "the forms below");
-  if (W.form == 0)
-    solve_block<0, R>(L, E, W, S, limit, first_solve);
-  else if (W.form == 1)
-    solve_block<1, R>(L, E, W, S, limit, first_solve);
-  else if (W.form == 2)
-    solve_block<2, R>(L, E, W, S, limit, first_solve);
-  else
-    solve_block<3, R>(L, E, W, S, limit, first_solve);
+  switch (W.form) {
+    case 0:
+      return solve_block<2, false>(L, E, W, S, limit, first_solve);
+    case 1:
+      return solve_block<4, false>(L, E, W, S, limit, first_solve);
+    case 2:
+      return solve_block<8, false>(L, E, W, S, limit, first_solve);
+    case 3:
+      return solve_block<11, false>(L, E, W, S, limit, first_solve);
+    case kSolveForms:
+      return solve_block<1, true>(L, E, W, S, limit, first_solve);
+    case kSolveForms + 1:
+      return solve_block<2, true>(L, E, W, S, limit, first_solve);
+    default:
+      return solve_block<4, true>(L, E, W, S, limit, first_solve);
+  }
 }
 
 // min that propagates NaN (the stage check must see a NaN depth)
@@ -1638,9 +1722,9 @@ void launch_assemble(const EngineArgs& E, const TileRef* cb, int ncb, const int*
                      const SysList& S, hipStream_t s) {
   if (!ncb) return;
   if (S.nr == 2)
-    hipLaunchKernelGGL(k_assemble<2>, dim3(ncb), dim3(256), 0, s, E, cb, S);
+    hipLaunchKernelGGL((k_assemble<2, true>), dim3(ncb), dim3(256), 0, s, E, cb, S);
   else
-    hipLaunchKernelGGL(k_assemble<4>, dim3(ncb), dim3(256), 0, s, E, cb, S);
+    hipLaunchKernelGGL((k_assemble<4, true>), dim3(ncb), dim3(256), 0, s, E, cb, S);
   hipLaunchKernelGGL(k_decide<true>, dim3(njobs), dim3(256), 0, s, E, jl, S);
 }
 
@@ -1660,14 +1744,23 @@ void launch_sweep(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl
   hipLaunchKernelGGL(k_decide<false>, dim3(njobs), dim3(256), 0, s, E, jl, S);
 }
 
+// A block of k_assemble holds 33 KB of LDS, so 1024 run at once; below that
+// the systems of a cell get blocks of their own (32^2: 12 -> ASM32 us), from
+// there on one block shares the face fluxes between them.
+void launch_assemble_matrix(const EngineArgs& E, const TileRef* cb, int ncb, const SysList& S,
+                            hipStream_t s) {
+  if (!ncb) return;
+  const dim3 grid(ncb, ncb < 1024 ? S.count : 1);
+  if (S.nr == 2)
+    hipLaunchKernelGGL((k_assemble<2, false>), grid, dim3(256), 0, s, E, cb, S);
+  else
+    hipLaunchKernelGGL((k_assemble<4, false>), grid, dim3(256), 0, s, E, cb, S);
+}
+
 void launch_solve(const EngineArgs& E, const SolveRef* refs, int nblk, const SysList& S, int limit,
                   int first_solve, hipStream_t s) {
-  if (!nblk) return;
-  if (S.nr == 2)
-    hipLaunchKernelGGL(k_solve<2>, dim3(nblk), dim3(kSolveThreads), 0, s, E, refs, S, limit,
-                       first_solve);
-  else
-    hipLaunchKernelGGL(k_solve<4>, dim3(nblk), dim3(kSolveThreads), 0, s, E, refs, S, limit,
+  if (nblk)
+    hipLaunchKernelGGL(k_solve, dim3(nblk), dim3(kSolveThreads), 0, s, E, refs, S, limit,
                        first_solve);
 }
 

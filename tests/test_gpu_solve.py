@@ -25,12 +25,14 @@ def random_state(n, ny, seed, amp=0.3):
     return P.Problem(n, U, kind="random", ny=ny)
 
 
-# nx, ny, steps: 512, 1024 and 2048 rows are the most that one block takes at
-# 1, 2 and 4 rows per thread; from 2049 on the blocks of a system share a
-# solve, from 43691 on with 2 rows per thread, from 87382 with 4, from 174763
-# with 8
+# nx, ny, steps: 512, 1024 and 2048 cells are the most that one block takes at
+# 1, 2 and 4 rows per thread; from 2049 on the tiles of a system share a
+# solve: tiles of at most 24x24 cells (one of 24x24 and its neighbours one
+# wider; thinner than the 4 cells of halo; a grid thinner than its halo), of
+# 40x34 (both its edges), of 64x48 and of 64x64
 SIZES = [(3, 3, 3), (32, 16, 3), (27, 19, 3), (32, 32, 2), (41, 25, 2), (64, 32, 2), (3, 683, 2),
-         (683, 3, 2), (1500, 4, 2), (101, 67, 2), (211, 208, 1), (293, 299, 1), (419, 418, 1)]
+         (683, 3, 2), (1500, 4, 2), (48, 48, 2), (49, 73, 2), (101, 67, 2), (192, 193, 1),
+         (240, 238, 1), (241, 239, 1), (419, 418, 1), (517, 513, 1)]
 
 
 @pytest.mark.parametrize("size", SIZES, ids=lambda s: f"{s[0]}x{s[1]}")
