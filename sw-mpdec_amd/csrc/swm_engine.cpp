@@ -130,11 +130,14 @@ struct DevVec {
 };
 
 struct Tables {
-  std::vector<TileRef> xt[kNumShapes], yt[kNumShapes], ct, cb;  // face tiles per shape
+  // k_fvtd's tiles per shape: x faces, y faces, sources; k_fvtd_source_update's
+  // tiles; cell blocks; jobs
+  std::vector<TileRef> xt[kNumShapes], yt[kNumShapes], st[kNumShapes], ct, cb;
   std::vector<int> jl;
-  DevVec<TileRef> dxt[kNumShapes], dyt[kNumShapes], dct, dcb;
+  DevVec<TileRef> dxt[kNumShapes], dyt[kNumShapes], dst[kNumShapes], dct, dcb;
   DevVec<int> djl;
-  int nxt[kNumShapes] = {}, nyt[kNumShapes] = {}, nct = 0, ncb = 0, njobs = 0;
+  int nxt[kNumShapes] = {}, nyt[kNumShapes] = {}, nst[kNumShapes] = {};
+  int nct = 0, ncb = 0, njobs = 0;
   // The Patankar solves: k_solve's blocks for launches of one and of kMaxSys
   // systems, cut into launches (first block, blocks); and the cell blocks and
   // jobs of the grids k_solve does not take, swept by a launch per sweep.
@@ -171,6 +174,7 @@ struct Job {
   const SchemeDef* scheme = &kSchemes[0];  // time scheme of engine / multi-step runs
   int hp_assoc = SWM_HP_AS_REFERENCE;     // depth view of the two-node schemes
   Tables own;          // tables covering this job alone
+  int own_bathy = 0;   // dev.bathy as the tables have it
   double* vout_buf = nullptr;  // the writer's state (dev.vout), when kept
   bool vout_valid = false;     // vout holds the state of the last step
 };
@@ -299,6 +303,14 @@ void timed(swm_engine* e, int cat, F&& launch) {
     e->prof.used = 2 * e->prof.cats.size();
 }
 
+void add_sources(Tables& T, int id, const JobDev& d) {
+  if (!d.bathy) return;
+  for (int sh = 0; sh < kNumShapes; ++sh) {
+    const int nst = cdiv(d.nx, kShapes[sh].sw) * cdiv(d.ny, kShapes[sh].sh);
+    for (int t = 0; t < nst; ++t) T.st[sh].push_back({id, t});
+  }
+}
+
 void add_tiles(Tables& T, int id, const JobDev& d) {
   for (int sh = 0; sh < kNumShapes; ++sh) {
     const FaceShape& F = kShapes[sh];
@@ -307,6 +319,7 @@ void add_tiles(Tables& T, int id, const JobDev& d) {
     for (int t = 0; t < nxt; ++t) T.xt[sh].push_back({id, t});
     for (int t = 0; t < nyt; ++t) T.yt[sh].push_back({id, t});
   }
+  add_sources(T, id, d);
   const int nct = cdiv(d.nx, kTile) * cdiv(d.ny, kTile);
   for (int t = 0; t < nct; ++t) T.ct.push_back({id, t});
   for (int t = 0; t < d.nblk; ++t) T.cb.push_back({id, t});
@@ -427,24 +440,24 @@ int upload_tables(swm_engine* e, Tables& T) {
   if (T.njobsw)
     HIPCK(e, hipMemcpy(T.djlw.p, T.jlw.data(), T.njobsw * sizeof(int), hipMemcpyHostToDevice));
   for (int sh = 0; sh < kNumShapes; ++sh) {
-    T.nxt[sh] = (int)T.xt[sh].size();
-    T.nyt[sh] = (int)T.yt[sh].size();
-    HIPCK(e, T.dxt[sh].reserve(T.xt[sh].size()));
-    HIPCK(e, T.dyt[sh].reserve(T.yt[sh].size()));
-    if (T.nxt[sh])
-      HIPCK(e, hipMemcpy(T.dxt[sh].p, T.xt[sh].data(), T.nxt[sh] * sizeof(TileRef),
-                         hipMemcpyHostToDevice));
-    if (T.nyt[sh])
-      HIPCK(e, hipMemcpy(T.dyt[sh].p, T.yt[sh].data(), T.nyt[sh] * sizeof(TileRef),
-                         hipMemcpyHostToDevice));
+    auto put = [&](DevVec<TileRef>& d, const std::vector<TileRef>& v, int& count) {
+      count = (int)v.size();
+      hipError_t er = d.reserve(v.size());
+      if (er == hipSuccess && count)
+        er = hipMemcpy(d.p, v.data(), v.size() * sizeof(TileRef), hipMemcpyHostToDevice);
+      return er;
+    };
+    HIPCK(e, put(T.dxt[sh], T.xt[sh], T.nxt[sh]));
+    HIPCK(e, put(T.dyt[sh], T.yt[sh], T.nyt[sh]));
+    HIPCK(e, put(T.dst[sh], T.st[sh], T.nst[sh]));
   }
   T.nct = (int)T.ct.size();
   T.ncb = (int)T.cb.size();
   T.njobs = (int)T.jl.size();
   HIPCK(e, T.dct.reserve(T.ct.size()));
+  if (T.nct) HIPCK(e, hipMemcpy(T.dct.p, T.ct.data(), T.nct * sizeof(TileRef), hipMemcpyHostToDevice));
   HIPCK(e, T.dcb.reserve(T.cb.size()));
   HIPCK(e, T.djl.reserve(T.jl.size()));
-  if (T.nct) HIPCK(e, hipMemcpy(T.dct.p, T.ct.data(), T.nct * sizeof(TileRef), hipMemcpyHostToDevice));
   if (T.ncb) HIPCK(e, hipMemcpy(T.dcb.p, T.cb.data(), T.ncb * sizeof(TileRef), hipMemcpyHostToDevice));
   if (T.njobs) HIPCK(e, hipMemcpy(T.djl.p, T.jl.data(), T.njobs * sizeof(int), hipMemcpyHostToDevice));
   return SWM_OK;
@@ -463,13 +476,21 @@ int refresh(swm_engine* e) {
     for (int sh = 0; sh < kNumShapes; ++sh) {
       T.xt[sh].clear();
       T.yt[sh].clear();
+      T.st[sh].clear();
     }
     T.ct.clear();
     T.cb.clear();
     T.jl.clear();
   }
   for (size_t i = 0; i < nj; ++i) {
-    const Job& J = *e->jobs[i];
+    Job& J = *e->jobs[i];
+    if (J.state != JOB_FREE && J.own_bathy != J.dev.bathy) {  // its source tiles came or went
+      for (auto& st : J.own.st) st.clear();
+      add_sources(J.own, (int)i, J.dev);
+      J.own_bathy = J.dev.bathy;
+      int rc = upload_tables(e, J.own);
+      if (rc) return rc;
+    }
     if (J.state == JOB_RUNNING) add_tiles(e->groups[group_of(J.scheme, J.hp_assoc)], (int)i, J.dev);
   }
   for (Tables& T : e->groups) {
@@ -490,13 +511,26 @@ EngineArgs eargs(swm_engine* e) {
   return a;
 }
 
+// Threads of face tiles up to which the three kinds of k_fvtd's tiles share a
+// launch.  The device holds 262,144 at 4 waves per SIMD.
+constexpr long kFvtdTogether = 8L * 262144;
+
 int fvtd_launch(swm_engine* e, Tables& T, const NodeList& L) {
   EngineArgs a = eargs(e);
   hipStream_t s = e->stream;
   const int sh = e->cur_shape;
-  timed(e, 0, [&] { launch_fvtd(a, sh, T.dxt[sh].p, T.nxt[sh], nullptr, 0, nullptr, 0, L, s); });
-  timed(e, 1, [&] { launch_fvtd(a, sh, nullptr, 0, T.dyt[sh].p, T.nyt[sh], nullptr, 0, L, s); });
-  timed(e, 2, [&] { launch_fvtd(a, sh, nullptr, 0, nullptr, 0, T.dct.p, T.nct, L, s); });
+  const TileRef *xt = T.dxt[sh].p, *yt = T.dyt[sh].p, *st = T.dst[sh].p;
+  const int nxt = T.nxt[sh], nyt = T.nyt[sh], nst = T.nst[sh];
+  const FaceShape& F = kShapes[sh];
+  const bool small = (long)(nxt + nyt) * L.count * F.xw * F.xh <= kFvtdTogether;
+  if (small && !(e->prof.mask & 7u)) {
+    launch_fvtd(a, sh, xt, nxt, yt, nyt, st, nst, L, s);
+    launch_fvtd_update(a, T.dcb.p, T.ncb, L, s);
+  } else {  // also while events tell the kinds apart
+    timed(e, 0, [&] { launch_fvtd(a, sh, xt, nxt, nullptr, 0, nullptr, 0, L, s); });
+    timed(e, 1, [&] { launch_fvtd(a, sh, nullptr, 0, yt, nyt, nullptr, 0, L, s); });
+    timed(e, 2, [&] { launch_fvtd_source_update(a, T.dct.p, T.nct, L, s); });
+  }
   LAUNCHCK(e);
   return SWM_OK;
 }
@@ -1361,6 +1395,7 @@ int alloc_job(swm_engine* e, int nx, int ny, double dx, double dy, double g, dou
   J.hp_assoc = SWM_HP_AS_REFERENCE;
   e->dirty = true;
   add_tiles(J.own, id, D);
+  J.own_bathy = D.bathy;
   ++e->graph_epoch;
   int rc = upload_tables(e, J.own);
   if (rc) return rc;

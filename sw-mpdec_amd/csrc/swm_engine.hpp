@@ -25,17 +25,18 @@ namespace swm {
 // Sets the message swm_last_error(NULL) returns on the calling thread.
 void set_thread_error(const std::string& msg);
 
-constexpr int kTile = 16;             // k_fvtd_update tiles: 16x16 cells, 256 threads
+constexpr int kTile = 16;             // k_fvtd_source_update tiles: 16x16 cells, 256 threads
 
-// Tile shapes of the face kernels: k_fvtd_x runs xw x xh threads per tile and
-// produces xw-1 faces per row; k_fvtd_y runs yw x yh threads and yh-1 faces
-// per column.  Wider tiles recompute fewer halo sweeps; narrower ones waste
+// Tile shapes of k_fvtd: an x-face tile takes xw x xh threads and produces
+// xw-1 faces per row; a y-face tile yw x yh threads and yh-1 faces per column;
+// a source tile sw x sh threads and cells.  Wider tiles recompute fewer halo sweeps; narrower ones waste
 // fewer threads on small grids.  The engine's autotuner picks one.
 struct FaceShape {
-  int xw, xh, yw, yh;
+  int xw, xh, yw, yh, sw, sh;
 };
 constexpr int kNumShapes = 2;
-constexpr FaceShape kShapes[kNumShapes] = {{16, 16, 16, 16}, {32, 16, 16, 32}};
+constexpr FaceShape kShapes[kNumShapes] = {{16, 16, 16, 16, 16, 16},
+                                            {32, 16, 16, 32, 32, 16}};
 constexpr int kCellBlock = 256;       // cells per block of the pointwise kernels
 constexpr int kSolveThreads = 512;    // threads of a k_solve block
 constexpr int kSolveWindow = 4;       // Jacobi sweeps between two exchanges of k_solve's blocks
@@ -336,9 +337,14 @@ void launch_primitives(size_t n, const double* h, const double* hu, const double
                        hipStream_t s);
 
 // ---- launches (swm_kernels.hip) -------------------------------------------
-// xt / yt: face tiles of shape kShapes[shape]; ct: k_fvtd_update tiles.
+// xt / yt / st: x-face, y-face and source tiles of shape kShapes[shape]
 void launch_fvtd(const EngineArgs& E, int shape, const TileRef* xt, int nxt, const TileRef* yt,
-                 int nyt, const TileRef* ct, int nct, const NodeList& L, hipStream_t s);
+                 int nyt, const TileRef* st, int nst, const NodeList& L, hipStream_t s);
+// ct: tiles of kTile x kTile cells
+void launch_fvtd_source_update(const EngineArgs& E, const TileRef* ct, int nct, const NodeList& L,
+                               hipStream_t s);
+void launch_fvtd_update(const EngineArgs& E, const TileRef* cb, int ncb, const NodeList& L,
+                        hipStream_t s);
 void launch_assemble(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl, int njobs,
                      const SysList& S, hipStream_t s);
 void launch_sweep(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl, int njobs,

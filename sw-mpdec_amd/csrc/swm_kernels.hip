@@ -3,15 +3,14 @@
 // build, and the explicit schemes of the build without it -- over all active
 // jobs of an engine.
 //
-// One FVTimeDerivative (src/finitevolume.f90:402-440) is three launches, each
-// covering every job and up to three DeC nodes (blockIdx.y in the face
-// kernels, XCD-grouped block numbers in k_fvtd_update):
-//   k_fvtd_x       x faces: halo tile -> ConsToPrim -> WENO5 first sweep along
+// One FVTimeDerivative (src/finitevolume.f90:402-440) is two launches, each
+// covering every job and up to three DeC nodes:
+//   k_fvtd         x faces: halo tile -> ConsToPrim -> WENO5 first sweep along
 //                  x (shared through LDS) -> second sweep along y at the 4 Gauss
-//                  points -> positivity limiter on h -> Rusanov -> Gauss sum
-//   k_fvtd_y       the same for y faces
-//   k_fvtd_update  source term (h-only WENO5 point values times -g db) and
-//                  UpdateTimeDerivative: Ut(2:3) and face mass fluxes / dx
+//                  points -> positivity limiter on h -> Rusanov -> Gauss sum;
+//                  y faces: the same; source term (h-only WENO5 point values
+//                  times -g db)
+//   k_fvtd_update  UpdateTimeDerivative: Ut(2:3) and face mass fluxes / dx
 // The Patankar assembly fuses the first Jacobi sweep and carries the DeC
 // momentum update of the same nodes (disjoint arrays).  Every Jacobi sweep
 // writes per-block sums of |x_new - x_old|; a one-block-per-job kernel takes
@@ -175,25 +174,19 @@ __device__ __forceinline__ void face_flux(const JobDev& J, const double WP[3][4]
 }
 
 template <int TW, int TH>
-__global__ __launch_bounds__(TW * TH) void k_fvtd_x(EngineArgs E, const TileRef* tiles,
-                                                    NodeList L) {
+__device__ __forceinline__ void x_faces(double* smem, int& irregular, const JobDev& J, int tile,
+                                        int m, int slot, const NodeList& L) {
   using FT = FaceTile<TW, TH>;
   constexpr int NT = FT::NT, VW = FT::VW, VH = FT::VH, NV = FT::NV;
   constexpr int NQ = VH * TW;  // first sweeps per variable: VH rows x TW cells
-  __shared__ double smem[FT::LDS];
   double* sV = smem;            // [3][VH rows][VW cols]
   double* sQM = smem + 3 * NV;  // [3][VH rows][TW cols]
   double* sQP = sQM + 3 * NQ;
-  __shared__ int irregular;  // a cell whose depths sqrt_regular may not take
-  const TileRef T = tiles[blockIdx.x];
-  const JobDev& J = E.jobs[T.job];
-  if (skipped(E, J)) return;
-  const int m = L.m[blockIdx.y], slot = L.slot[blockIdx.y];
   const int nx = J.nx, ny = J.ny;
   const int ntx = cdiv_d(nx + 1, TW - 1);
   const int tid = threadIdx.x, tx = tid % TW, ty = tid / TW;
-  const int c0 = (T.tile % ntx) * (TW - 1);
-  const int j0 = (T.tile / ntx) * TH + 1;
+  const int c0 = (tile % ntx) * (TW - 1);
+  const int j0 = (tile / ntx) * TH + 1;
   const gdouble *h, *hu, *hv;
   node_state(J, m, h, hu, hv);
   // g h stays in the range of sqrt_regular for the depths of depths_regular
@@ -274,29 +267,23 @@ __global__ __launch_bounds__(TW * TH) void k_fvtd_x(EngineArgs E, const TileRef*
 }
 
 // ------------------------------------------------------------------------
-// y faces: the transpose of k_fvtd_x.  Tile (bx, by): columns
+// y faces: the transpose of x_faces.  Tile (bx, by): columns
 // i = TW*bx + 1 + tx, Fortran rows r = (TH-1)*by + ty (0..ny+1); face g = r.
 // ------------------------------------------------------------------------
 template <int TW, int TH>
-__global__ __launch_bounds__(TW * TH) void k_fvtd_y(EngineArgs E, const TileRef* tiles,
-                                                    NodeList L) {
+__device__ __forceinline__ void y_faces(double* smem, int& irregular, const JobDev& J, int tile,
+                                        int m, int slot, const NodeList& L) {
   using FT = FaceTile<TW, TH>;
   constexpr int NT = FT::NT, VW = FT::VW, NV = FT::NV;
   constexpr int NQ = TH * VW;  // first sweeps per variable: TH rows x VW columns
-  __shared__ double smem[FT::LDS];
   double* sV = smem;            // [3][VH rows][VW cols]
   double* sQM = smem + 3 * NV;  // [3][TH rows][VW cols]
   double* sQP = sQM + 3 * NQ;
-  __shared__ int irregular;  // a cell whose depths sqrt_regular may not take
-  const TileRef T = tiles[blockIdx.x];
-  const JobDev& J = E.jobs[T.job];
-  if (skipped(E, J)) return;
-  const int m = L.m[blockIdx.y], slot = L.slot[blockIdx.y];
   const int nx = J.nx, ny = J.ny;
   const int ntx = cdiv_d(nx, TW);
   const int tid = threadIdx.x, tx = tid % TW, ty = tid / TW;
-  const int i0 = (T.tile % ntx) * TW + 1;
-  const int r0 = (T.tile / ntx) * (TH - 1);
+  const int i0 = (tile % ntx) * TW + 1;
+  const int r0 = (tile / ntx) * (TH - 1);
   const gdouble *h, *hu, *hv;
   node_state(J, m, h, hu, hv);
   // g h stays in the range of sqrt_regular for the depths of depths_regular
@@ -332,7 +319,7 @@ __global__ __launch_bounds__(TW * TH) void k_fvtd_y(EngineArgs E, const TileRef*
   const int r = r0 + ty;
   if (J.recfix) {
     // Ind(2, i, r) = Shock(i, min(r + 1, ny)) (src/shocksindicator.f90:84-89),
-    // as in k_fvtd_x
+    // as in x_faces
     const int lr = min(r + 1, ny) - r0 + 2;
     const double* hcol = sV + tx + 2;
     if (jameson_shock(hcol[(lr - 1) * VW], hcol[lr * VW], hcol[(lr + 1) * VW])) {
@@ -374,128 +361,235 @@ __global__ __launch_bounds__(TW * TH) void k_fvtd_y(EngineArgs E, const TileRef*
 }
 
 // ------------------------------------------------------------------------
-// Source term + UpdateTimeDerivative.  Tile: 16x16 cells (1-based
-// i = 16*bx + 1 + tx, j = 16*by + 1 + ty).  SourceTerms
-// (src/equation.f90:352-388): h point values at the 4x4 Gauss points from a
-// WENO5 second sweep along y (columns i-2..i+2) followed by one along x per
-// y Gauss point; SW = -g*h*db; S = sum over x-GP (outer), y-GP (inner) of W*SW.
+// Source term of a tile of TW x TH cells (1-based i = TW*bx + 1 + tx, j =
+// TH*by + 1 + ty).  SourceTerms (src/equation.f90:352-388): h point values at
+// the 4x4 Gauss points from a WENO5 second sweep along y (columns i-2..i+2)
+// followed by one along x per y Gauss point; SW = -g*h*db; S = sum over x-GP
+// (outer), y-GP (inner) of W*SW.
 // ------------------------------------------------------------------------
-// Blocks are numbered so that the L.count nodes of one tile share an XCD:
-// workgroups are dealt round-robin to the 8 XCDs, so block
-// ((t / 8) * count + node) * 8 + t % 8 runs tile t on XCD t % 8 for every
-// node, close together in time, and the tile's bathymetry and well-balanced
-// tables are read from HBM once and from that XCD's L2 for the other nodes.
-__global__ __launch_bounds__(256) void k_fvtd_update(EngineArgs E, const TileRef* tiles,
-                                                     int ntiles, NodeList L) {
-  __shared__ double sH[400];           // [20 rows][20 cols]
-  __shared__ double sVt[4 * 16 * 20];  // [yg][16 rows][20 cols]
-  const int grp = blockIdx.x / (8 * L.count), rem = blockIdx.x % (8 * L.count);
-  const int node = rem / 8, tile = grp * 8 + (rem % 8);
-  if (tile >= ntiles) return;
-  const TileRef T = tiles[tile];
-  const JobDev& J = E.jobs[T.job];
-  if (skipped(E, J)) return;
+template <int TW, int TH>
+__device__ __forceinline__ void source_tile(double* smem, const JobDev& J, int tile, int m,
+                                            double& S2, double& S3) {
+  constexpr int NT = TW * TH, VW = TW + 4, VH = TH + 4, NV = VW * VH, NQ = VW * TH;
+  double* sH = smem;        // [VH rows][VW cols]
+  double* sVt = smem + NV;  // [yg][TH rows][VW cols]
   const int nx = J.nx, ny = J.ny;
-  const int ntx = cdiv_d(nx, kTile);
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int i0 = (T.tile % ntx) * kTile + 1, j0 = (T.tile / ntx) * kTile + 1;
+  const int ntx = cdiv_d(nx, TW);
+  const int tid = threadIdx.x, tx = tid % TW, ty = tid / TW;
+  const int i0 = (tile % ntx) * TW + 1, j0 = (tile / ntx) * TH + 1;
   const int i = i0 + tx, j = j0 + ty;
-  const bool in = i <= nx && j <= ny;
   const size_t n = (size_t)J.n;
-  const size_t k = in ? (size_t)(j - 1) * nx + (i - 1) : 0;
-  {
-    const int m = L.m[node], slot = L.slot[node];
-    const gdouble *h, *hu, *hv;
-    node_state(J, m, h, hu, hv);
-    double S2 = 0.0, S3 = 0.0;
-    if (J.bathy) {  // uniform per block
-      for (int t = tid; t < 400; t += 256) {
-        int lx = t % 20, ly = t / 20;
-        sH[t] = h[(size_t)wrap1(j0 - 2 + ly, ny) * nx + wrap1(i0 - 2 + lx, nx)];
-      }
-      __syncthreads();
-      for (int t = tid; t < 320; t += 256) {
-        int ly = t / 20, lx = t % 20;
-        const double* qh = sH + ly * 20 + lx;
-        double w[4];
-        weno5_second(qh[0], qh[20], qh[40], qh[60], qh[80], w);
+  const gdouble *h, *hu, *hv;
+  node_state(J, m, h, hu, hv);
+  for (int t = tid; t < NV; t += NT) {
+    int lx = t % VW, ly = t / VW;
+    sH[t] = h[(size_t)wrap1(j0 - 2 + ly, ny) * nx + wrap1(i0 - 2 + lx, nx)];
+  }
+  __syncthreads();
+  for (int t = tid; t < NQ; t += NT) {
+    const double* qh = sH + t;  // row ly, column lx of the halo tile
+    double w[4];
+    weno5_second(qh[0], qh[VW], qh[2 * VW], qh[3 * VW], qh[4 * VW], w);
 #pragma unroll
-        for (int yg = 0; yg < 4; ++yg) sVt[yg * 320 + t] = w[yg];
-      }
-      __syncthreads();
-      if (in) {
-        double hgp[4][4];  // [yg][xg]
+    for (int yg = 0; yg < 4; ++yg) sVt[yg * NQ + t] = w[yg];
+  }
+  __syncthreads();
+  if (i > nx || j > ny) return;
+  const size_t k = (size_t)(j - 1) * nx + (i - 1);
+  double hgp[4][4];  // [yg][xg]
 #pragma unroll
-        for (int yg = 0; yg < 4; ++yg) {
-          const double* qv = sVt + yg * 320 + ty * 20 + tx;
-          weno5_second(qv[0], qv[1], qv[2], qv[3], qv[4], hgp[yg]);
-        }
+  for (int yg = 0; yg < 4; ++yg) {
+    const double* qv = sVt + yg * NQ + ty * VW + tx;
+    weno5_second(qv[0], qv[1], qv[2], qv[3], qv[4], hgp[yg]);
+  }
+  S2 = 0.0;
+  S3 = 0.0;
 #pragma unroll
-        for (int xg = 0; xg < 4; ++xg)
+  for (int xg = 0; xg < 4; ++xg)
 #pragma unroll
-          for (int yg = 0; yg < 4; ++yg) {
-            double hh = hgp[yg][xg];
-            double bx = G(J.bx)[(size_t)(yg * 4 + xg) * n + k];
-            double by = G(J.by)[(size_t)(yg * 4 + xg) * n + k];
-            double sw2 = -J.g * hh * bx;
-            double sw3 = -J.g * hh * by;
-            S2 = S2 + J.wgp[xg][yg] * sw2;
-            S3 = S3 + J.wgp[xg][yg] * sw3;
-          }
-      }
+    for (int yg = 0; yg < 4; ++yg) {
+      double hh = hgp[yg][xg];
+      double bx = G(J.bx)[(size_t)(yg * 4 + xg) * n + k];
+      double by = G(J.by)[(size_t)(yg * 4 + xg) * n + k];
+      double sw2 = -J.g * hh * bx;
+      double sw3 = -J.g * hh * by;
+      S2 = S2 + J.wgp[xg][yg] * sw2;
+      S3 = S3 + J.wgp[xg][yg] * sw3;
     }
-    if (!in) return;
-    if (L.wb_init) {  // building the well-balanced reference: keep S as SWB
-      G(J.SWB2)[k] = S2;
-      G(J.SWB3)[k] = S3;
-      return;
-    }
-    const size_t fe = (size_t)(j - 1) * (nx + 1) + i, fw = fe - 1;  // x faces i, i-1
-    const size_t gn = (size_t)j * nx + (i - 1), gs = gn - nx;        // y faces j, j-1
-    if (J.wb) {
+}
+
+// ------------------------------------------------------------------------
+// The face fluxes of one FVTimeDerivative for up to three nodes and, in small
+// launches, the sources: x-face, y-face and source tiles of every job in one
+// launch, the three kinds being independent of each other.  On grids that do
+// not fill the device they then run side by side (32^2: 11.8 us for 11.3 + 10.6
+// one after the other; 128^2 lake: 20.9 us with the sources).  Launches that
+// fill it several times over gain nothing from that, and their sources run
+// better with the update (k_fvtd_source_update).
+//
+// Blocks come in groups of 8, one per XCD (workgroups are dealt round-robin to
+// the 8 XCDs).  The sources' groups are spread evenly between the faces', and
+// the L.count nodes of a source tile are 8 blocks apart: on one XCD and close
+// together in time, so that the tile's bathymetry and well-balanced tables
+// come from HBM once and from that XCD's L2 for the other nodes.
+// ------------------------------------------------------------------------
+struct FvtdTiles {
+  const TileRef *xt, *yt, *st;
+  int nxt, nyt, nst;
+};
+
+template <int XW, int XH, int YW, int YH, int SW, int SH>
+__global__ __launch_bounds__(XW * XH, 4) void k_fvtd(EngineArgs E, FvtdTiles T, NodeList L) {
+  static_assert(XW * XH == YW * YH && XW * XH == SW * SH, "one block size");
+  constexpr int LX = FaceTile<XW, XH>::LDS, LY = FaceTile<YW, YH>::LDS;
+  constexpr int LS = (SW + 4) * (SH + 4) + 4 * (SW + 4) * SH;
+  __shared__ double smem[LX > LY ? (LX > LS ? LX : LS) : (LY > LS ? LY : LS)];
+  __shared__ int irregular;  // a cell whose depths sqrt_regular may not take
+  const int faces = (T.nxt + T.nyt) * L.count;
+  const int gf = (faces + 7) / 8, gs = (T.nst + 7) / 8 * L.count;
+  const int g = blockIdx.x / 8, r = blockIdx.x % 8;
+  const int s0 = (int)((long long)g * gs / (gf + gs));  // source groups before this one
+  const bool src = (int)((long long)(g + 1) * gs / (gf + gs)) > s0;
+  if (src) {
+    const int t = s0 / L.count * 8 + r, node = s0 % L.count;
+    if (t >= T.nst) return;
+    const TileRef R = T.st[t];
+    const JobDev& J = E.jobs[R.job];
+    if (skipped(E, J)) return;
+    double S2, S3;
+    source_tile<SW, SH>(smem, J, R.tile, L.m[node], S2, S3);
+    const int ntx = cdiv_d(J.nx, SW);
+    const int ci = (R.tile % ntx) * SW + threadIdx.x % SW;
+    const int cj = (R.tile / ntx) * SH + threadIdx.x / SW;
+    if (ci >= J.nx || cj >= J.ny) return;
+    const int k = cj * J.nx + ci, out = L.out[node];
+    if (J.wb && !L.wb_init) {
       S2 = S2 - G(J.SWB2)[k];
       S3 = S3 - G(J.SWB3)[k];
     }
-    if (L.debug_S) {  // parity tests read S(2:3) from the first matrix scratch
-      G(J.M[0][0])[k] = S2;
-      G(J.M[0][1])[k] = S3;
-    }
-    // the face fluxes, with FXWB / FYWB already subtracted by the face kernels
-    double fxe[3], fxw[3], fyn[3], fys[3];
-#pragma unroll
-    for (int v = 0; v < 3; ++v) {
-      fxe[v] = G(J.FX[slot][v])[fe];
-      fxw[v] = G(J.FX[slot][v])[fw];
-      fyn[v] = G(J.FY[slot][v])[gn];
-      fys[v] = G(J.FY[slot][v])[gs];
-    }
-    // the divisions by dx and dy share one reciprocal each (uniform per job)
-    const double dx = J.dx, dy = J.dy;
-    const bool shared = recip_range(dx) & recip_range(dy);
-    const double rdx = recip_refined(dx), rdy = recip_refined(dy);
-    auto over_dx = [&](double a) { return shared ? div_pos(a, dx, rdx) : a / dx; };
-    auto over_dy = [&](double a) { return shared ? div_pos(a, dy, rdy) : a / dy; };
-    // Ut(2:3) = S - (FX(i)-FX(i-1))/dx - (FY(j)-FY(j-1))/dy  (:525-527)
-    const int o = L.out[node];
-    const double ut2 = S2 - over_dx(fxe[1] - fxw[1]) - over_dy(fyn[1] - fys[1]);
-    const double ut3 = S3 - over_dx(fxe[2] - fxw[2]) - over_dy(fyn[2] - fys[2]);
-    if (L.ut1) {
-      // the build without PATANKAR: Ut(1:3) (:529-533), with S(1) = 0 exactly
-      // (SourceFunc's first component is 0., src/equation.f90:408)
-      G(J.d1[o])[k] = 0.0 - over_dx(fxe[0] - fxw[0]) - over_dy(fyn[0] - fys[0]);
-      G(J.d2[o])[k] = ut2;
-      G(J.d3[o])[k] = ut3;
-      return;
-    }
-    G(J.FU2[o])[k] = ut2;
-    G(J.FU3[o])[k] = ut3;
-    // mass flux per face / dx: the production/destruction entries of
-    // src/finitevolume.f90:496-523 are max(+-q, 0) and -min(+-q, 0) of these.
-    G(J.qx[o])[fe] = over_dx(fxe[0]);
-    G(J.qy[o])[gn] = over_dy(fyn[0]);
-    if (i == 1) G(J.qx[o])[fw] = over_dx(fxw[0]);
-    if (j == 1) G(J.qy[o])[gs] = over_dy(fys[0]);
+    G(J.d2[out])[k] = S2;  // k_fvtd_update takes it from there
+    G(J.d3[out])[k] = S3;
+    return;
   }
+  const int f = (g - s0) * 8 + r;
+  if (f >= faces) return;
+  const bool x = f < T.nxt * L.count;
+  const int q = x ? f : f - T.nxt * L.count, nt = x ? T.nxt : T.nyt;
+  const int node = q / nt;
+  const TileRef R = (x ? T.xt : T.yt)[q - node * nt];
+  const JobDev& J = E.jobs[R.job];
+  if (skipped(E, J)) return;
+  if (x)
+    x_faces<XW, XH>(smem, irregular, J, R.tile, L.m[node], L.slot[node], L);
+  else
+    y_faces<YW, YH>(smem, irregular, J, R.tile, L.m[node], L.slot[node], L);
+}
+
+// ------------------------------------------------------------------------
+// UpdateTimeDerivative (src/finitevolume.f90:446-540) of cell k = (ci, cj) from
+// the fluxes in `slot` and its source S, into derivative slot o.
+// ------------------------------------------------------------------------
+__device__ __forceinline__ void update_cell(const JobDev& J, const NodeList& L, int o, int slot,
+                                            int k, int ci, int cj, double S2, double S3) {
+  const int nx = J.nx;
+  if (L.wb_init) {  // building the well-balanced reference: keep S as SWB
+    G(J.SWB2)[k] = S2;
+    G(J.SWB3)[k] = S3;
+    return;
+  }
+  const size_t fw = (size_t)cj * (nx + 1) + ci, fe = fw + 1;  // x faces
+  const size_t gs = (size_t)cj * nx + ci, gn = gs + nx;       // y faces
+  if (L.debug_S) {  // parity tests read S(2:3) from the first matrix scratch
+    G(J.M[0][0])[k] = S2;
+    G(J.M[0][1])[k] = S3;
+  }
+  // the face fluxes, with FXWB / FYWB already subtracted by the face kernels
+  double fxe[3], fxw[3], fyn[3], fys[3];
+#pragma unroll
+  for (int v = 0; v < 3; ++v) {
+    fxe[v] = G(J.FX[slot][v])[fe];
+    fxw[v] = G(J.FX[slot][v])[fw];
+    fyn[v] = G(J.FY[slot][v])[gn];
+    fys[v] = G(J.FY[slot][v])[gs];
+  }
+  // the divisions by dx and dy share one reciprocal each (uniform per job)
+  const double dx = J.dx, dy = J.dy;
+  const bool shared = recip_range(dx) & recip_range(dy);
+  const double rdx = recip_refined(dx), rdy = recip_refined(dy);
+  auto over_dx = [&](double a) { return shared ? div_pos(a, dx, rdx) : a / dx; };
+  auto over_dy = [&](double a) { return shared ? div_pos(a, dy, rdy) : a / dy; };
+  // Ut(2:3) = S - (FX(i)-FX(i-1))/dx - (FY(j)-FY(j-1))/dy  (:525-527)
+  const double ut2 = S2 - over_dx(fxe[1] - fxw[1]) - over_dy(fyn[1] - fys[1]);
+  const double ut3 = S3 - over_dx(fxe[2] - fxw[2]) - over_dy(fyn[2] - fys[2]);
+  if (L.ut1) {
+    // the build without PATANKAR: Ut(1:3) (:529-533), with S(1) = 0 exactly
+    // (SourceFunc's first component is 0., src/equation.f90:408)
+    G(J.d1[o])[k] = 0.0 - over_dx(fxe[0] - fxw[0]) - over_dy(fyn[0] - fys[0]);
+    G(J.d2[o])[k] = ut2;
+    G(J.d3[o])[k] = ut3;
+    return;
+  }
+  G(J.d2[o])[k] = ut2;  // FU2, FU3
+  G(J.d3[o])[k] = ut3;
+  // mass flux per face / dx: the production/destruction entries of
+  // src/finitevolume.f90:496-523 are max(+-q, 0) and -min(+-q, 0) of these.
+  G(J.qx[o])[fe] = over_dx(fxe[0]);
+  G(J.qy[o])[gn] = over_dy(fyn[0]);
+  if (ci == 0) G(J.qx[o])[fw] = over_dx(fxw[0]);
+  if (cj == 0) G(J.qy[o])[gs] = over_dy(fys[0]);
+}
+
+// The update alone, one cell per thread, blockIdx.y = node; the sources of
+// jobs with bathymetry are in the derivative slots already, less the
+// well-balanced state's.  Bound by memory.
+__global__ __launch_bounds__(256) void k_fvtd_update(EngineArgs E, const TileRef* blocks,
+                                                     NodeList L) {
+  const TileRef T = blocks[blockIdx.x];
+  const JobDev& J = E.jobs[T.job];
+  if (skipped(E, J)) return;
+  const int o = L.out[blockIdx.y], nx = J.nx, k0 = T.tile * kCellBlock, k = k0 + threadIdx.x;
+  if (k >= J.n) return;
+  int ci, cj;
+  cell_ij(k0 % nx, k0 / nx, threadIdx.x, nx, ci, cj);
+  double S2 = 0.0, S3 = 0.0;
+  if (J.bathy) {
+    S2 = G(J.d2[o])[k];
+    S3 = G(J.d3[o])[k];
+  } else if (J.wb && !L.wb_init) {
+    S2 = S2 - G(J.SWB2)[k];
+    S3 = S3 - G(J.SWB3)[k];
+  }
+  update_cell(J, L, o, L.slot[blockIdx.y], k, ci, cj, S2, S3);
+}
+
+// Source and update in one pass over tiles of 16x16 cells, for launches large
+// enough to fill the device without the sources beside the faces: the table
+// loads of some blocks then overlap the WENO work of others at 5 waves per
+// SIMD, and S needs no trip through memory (2048^2, 2.6 nodes on average: 700
+// us, against 740 + 190 us for source tiles at the face kernels' 4 waves and
+// the update alone).
+__global__ __launch_bounds__(256) void k_fvtd_source_update(EngineArgs E, const TileRef* tiles,
+                                                            int ntiles, NodeList L) {
+  constexpr int TW = kTile, TH = kTile;
+  __shared__ double smem[(TW + 4) * (TH + 4) + 4 * (TW + 4) * TH];
+  const int grp = blockIdx.x / (8 * L.count), rem = blockIdx.x % (8 * L.count);
+  const int node = rem / 8, t = grp * 8 + (rem % 8);
+  if (t >= ntiles) return;
+  const TileRef T = tiles[t];
+  const JobDev& J = E.jobs[T.job];
+  if (skipped(E, J)) return;
+  const int ntx = cdiv_d(J.nx, TW);
+  const int ci = (T.tile % ntx) * TW + threadIdx.x % TW;
+  const int cj = (T.tile / ntx) * TH + threadIdx.x / TW;
+  double S2 = 0.0, S3 = 0.0;
+  if (J.bathy) source_tile<TW, TH>(smem, J, T.tile, L.m[node], S2, S3);
+  if (ci >= J.nx || cj >= J.ny) return;
+  const int k = cj * J.nx + ci;
+  if (J.wb && !L.wb_init) {
+    S2 = S2 - G(J.SWB2)[k];
+    S3 = S3 - G(J.SWB3)[k];
+  }
+  update_cell(J, L, L.out[node], L.slot[node], k, ci, cj, S2, S3);
 }
 
 // ------------------------------------------------------------------------
@@ -1690,28 +1784,36 @@ __global__ __launch_bounds__(256) void k_keep_state(EngineArgs E, const TileRef*
 // ------------------------------------------------------------------------
 static inline unsigned cdiv(long a, long b) { return (unsigned)((a + b - 1) / b); }
 
-template <int XW, int XH, int YW, int YH>
-static void launch_faces(const EngineArgs& E, const TileRef* xt, int nxt, const TileRef* yt,
-                         int nyt, const NodeList& L, hipStream_t s) {
-  if (nxt)
-    hipLaunchKernelGGL((k_fvtd_x<XW, XH>), dim3(nxt, L.count), dim3(XW * XH), 0, s, E, xt, L);
-  if (nyt)
-    hipLaunchKernelGGL((k_fvtd_y<YW, YH>), dim3(nyt, L.count), dim3(YW * YH), 0, s, E, yt, L);
+void launch_fvtd(const EngineArgs& E, int shape, const TileRef* xt, int nxt, const TileRef* yt,
+                 int nyt, const TileRef* st, int nst, const NodeList& L, hipStream_t s) {
+  static_assert(kNumShapes == 2 && kShapes[0].xw == 16 && kShapes[0].xh == 16 &&
+                    kShapes[0].yw == 16 && kShapes[0].yh == 16 && kShapes[0].sw == 16 &&
+                    kShapes[0].sh == 16 && kShapes[1].xw == 32 && kShapes[1].xh == 16 &&
+                    kShapes[1].yw == 16 && kShapes[1].yh == 32 && kShapes[1].sw == 32 &&
+                    kShapes[1].sh == 16,
+                "the instantiations below follow kShapes");
+  const FvtdTiles T = {xt, yt, st, nxt, nyt, nst};
+  const unsigned groups = cdiv((long)(nxt + nyt) * L.count, 8) + cdiv(nst, 8) * L.count;
+  if (!groups) return;
+  if (shape == 1)
+    hipLaunchKernelGGL((k_fvtd<32, 16, 16, 32, 32, 16>), dim3(groups * 8), dim3(512), 0, s, E, T,
+                       L);
+  else
+    hipLaunchKernelGGL((k_fvtd<16, 16, 16, 16, 16, 16>), dim3(groups * 8), dim3(256), 0, s, E, T,
+                       L);
 }
 
-void launch_fvtd(const EngineArgs& E, int shape, const TileRef* xt, int nxt, const TileRef* yt,
-                 int nyt, const TileRef* ct, int nct, const NodeList& L, hipStream_t s) {
-  static_assert(kNumShapes == 2 && kShapes[0].xw == 16 && kShapes[0].xh == 16 &&
-                    kShapes[0].yw == 16 && kShapes[0].yh == 16 && kShapes[1].xw == 32 &&
-                    kShapes[1].xh == 16 && kShapes[1].yw == 16 && kShapes[1].yh == 32,
-                "the instantiations below follow kShapes");
-  if (shape == 1)
-    launch_faces<32, 16, 16, 32>(E, xt, nxt, yt, nyt, L, s);
-  else
-    launch_faces<16, 16, 16, 16>(E, xt, nxt, yt, nyt, L, s);
+void launch_fvtd_source_update(const EngineArgs& E, const TileRef* ct, int nct, const NodeList& L,
+                               hipStream_t s) {
   if (nct)
-    hipLaunchKernelGGL(k_fvtd_update, dim3(cdiv(nct, 8) * 8 * L.count), dim3(256), 0, s, E, ct,
-                       nct, L);
+    hipLaunchKernelGGL(k_fvtd_source_update, dim3(cdiv(nct, 8) * 8 * L.count), dim3(256), 0, s, E,
+                       ct, nct, L);
+}
+
+void launch_fvtd_update(const EngineArgs& E, const TileRef* cb, int ncb, const NodeList& L,
+                        hipStream_t s) {
+  if (ncb)
+    hipLaunchKernelGGL(k_fvtd_update, dim3(ncb, L.count), dim3(256), 0, s, E, cb, L);
 }
 
 void launch_keep_state(const EngineArgs& E, const TileRef* cb, int ncb, int m, hipStream_t s) {
