@@ -17,6 +17,7 @@
 
 #include "swm.h"
 #include "swm_engine.hpp"
+#include "swm_transfer.hpp"
 
 using namespace swm;
 
@@ -134,8 +135,9 @@ struct Tables {
   // tiles; cell blocks; jobs
   std::vector<TileRef> xt[kNumShapes], yt[kNumShapes], st[kNumShapes], ct, cb;
   std::vector<int> jl;
-  DevVec<TileRef> dxt[kNumShapes], dyt[kNumShapes], dst[kNumShapes], dct, dcb;
-  DevVec<int> djl;
+  TileRef *dxt[kNumShapes] = {}, *dyt[kNumShapes] = {}, *dst[kNumShapes] = {};
+  TileRef *dct = nullptr, *dcb = nullptr;
+  int* djl = nullptr;
   int nxt[kNumShapes] = {}, nyt[kNumShapes] = {}, nst[kNumShapes] = {};
   int nct = 0, ncb = 0, njobs = 0;
   // The Patankar solves: k_solve's blocks for launches of one and of kMaxSys
@@ -146,10 +148,11 @@ struct Tables {
   bool solve_waits = false;  // some systems have several blocks
   std::vector<TileRef> cbs, cbw;  // of the grids k_solve takes, and of the others
   std::vector<int> jlw;
-  DevVec<SolveRef> dsv[2];
-  DevVec<TileRef> dcbs, dcbw;
-  DevVec<int> djlw;
+  SolveRef* dsv[2] = {};
+  TileRef *dcbs = nullptr, *dcbw = nullptr;
+  int* djlw = nullptr;
   int ncbs = 0, ncbw = 0, njobsw = 0;
+  DevVec<char> dev;  // all of them, in one allocation and one copy
 };
 
 enum JobState { JOB_RUNNING = 0, JOB_DONE = 1, JOB_FAILED = 2, JOB_FREE = 3 };
@@ -248,6 +251,7 @@ struct swm_engine {
   Captured caps[2 * kGroups];    // captured steps by table set in use, with and without k_solve
   long long cap_clock = 0;
   Profiler prof;
+  std::shared_ptr<HostRing> ring;  // transfers of states
   std::string err;
 };
 
@@ -419,47 +423,35 @@ void solve_tables(swm_engine* e, Tables& T) {
   }
 }
 
+// The tables of T to the device.  They go in one copy: each costs about 35 us
+// whatever its size, and a job has a dozen tables of its own.
 int upload_tables(swm_engine* e, Tables& T) {
   solve_tables(e, T);
-  for (int c = 0; c < 2; ++c) {
-    HIPCK(e, T.dsv[c].reserve(T.sv[c].size()));
-    if (!T.sv[c].empty())
-      HIPCK(e, hipMemcpy(T.dsv[c].p, T.sv[c].data(), T.sv[c].size() * sizeof(SolveRef),
-                         hipMemcpyHostToDevice));
-  }
-  T.ncbs = (int)T.cbs.size();
-  T.ncbw = (int)T.cbw.size();
-  T.njobsw = (int)T.jlw.size();
-  HIPCK(e, T.dcbs.reserve(T.cbs.size()));
-  HIPCK(e, T.dcbw.reserve(T.cbw.size()));
-  HIPCK(e, T.djlw.reserve(T.jlw.size()));
-  if (T.ncbs)
-    HIPCK(e, hipMemcpy(T.dcbs.p, T.cbs.data(), T.ncbs * sizeof(TileRef), hipMemcpyHostToDevice));
-  if (T.ncbw)
-    HIPCK(e, hipMemcpy(T.dcbw.p, T.cbw.data(), T.ncbw * sizeof(TileRef), hipMemcpyHostToDevice));
-  if (T.njobsw)
-    HIPCK(e, hipMemcpy(T.djlw.p, T.jlw.data(), T.njobsw * sizeof(int), hipMemcpyHostToDevice));
+  std::vector<char> host;
+  std::vector<std::pair<void**, size_t>> where;  // device pointer, offset
+  auto put = [&](auto*& dev, const auto& v) {
+    const size_t off = (host.size() + 15) & ~size_t(15), bytes = v.size() * sizeof(v[0]);
+    host.resize(off + bytes);
+    if (bytes) std::memcpy(host.data() + off, v.data(), bytes);
+    where.push_back({(void**)&dev, off});
+    return (int)v.size();
+  };
   for (int sh = 0; sh < kNumShapes; ++sh) {
-    auto put = [&](DevVec<TileRef>& d, const std::vector<TileRef>& v, int& count) {
-      count = (int)v.size();
-      hipError_t er = d.reserve(v.size());
-      if (er == hipSuccess && count)
-        er = hipMemcpy(d.p, v.data(), v.size() * sizeof(TileRef), hipMemcpyHostToDevice);
-      return er;
-    };
-    HIPCK(e, put(T.dxt[sh], T.xt[sh], T.nxt[sh]));
-    HIPCK(e, put(T.dyt[sh], T.yt[sh], T.nyt[sh]));
-    HIPCK(e, put(T.dst[sh], T.st[sh], T.nst[sh]));
+    T.nxt[sh] = put(T.dxt[sh], T.xt[sh]);
+    T.nyt[sh] = put(T.dyt[sh], T.yt[sh]);
+    T.nst[sh] = put(T.dst[sh], T.st[sh]);
   }
-  T.nct = (int)T.ct.size();
-  T.ncb = (int)T.cb.size();
-  T.njobs = (int)T.jl.size();
-  HIPCK(e, T.dct.reserve(T.ct.size()));
-  if (T.nct) HIPCK(e, hipMemcpy(T.dct.p, T.ct.data(), T.nct * sizeof(TileRef), hipMemcpyHostToDevice));
-  HIPCK(e, T.dcb.reserve(T.cb.size()));
-  HIPCK(e, T.djl.reserve(T.jl.size()));
-  if (T.ncb) HIPCK(e, hipMemcpy(T.dcb.p, T.cb.data(), T.ncb * sizeof(TileRef), hipMemcpyHostToDevice));
-  if (T.njobs) HIPCK(e, hipMemcpy(T.djl.p, T.jl.data(), T.njobs * sizeof(int), hipMemcpyHostToDevice));
+  T.nct = put(T.dct, T.ct);
+  T.ncb = put(T.dcb, T.cb);
+  T.njobs = put(T.djl, T.jl);
+  T.ncbs = put(T.dcbs, T.cbs);
+  T.ncbw = put(T.dcbw, T.cbw);
+  T.njobsw = put(T.djlw, T.jlw);
+  for (int c = 0; c < 2; ++c) put(T.dsv[c], T.sv[c]);
+  if (host.empty()) return SWM_OK;
+  HIPCK(e, T.dev.reserve(host.size()));
+  HIPCK(e, hipMemcpy(T.dev.p, host.data(), host.size(), hipMemcpyHostToDevice));
+  for (const auto& w : where) *w.first = T.dev.p + w.second;
   return SWM_OK;
 }
 
@@ -519,17 +511,17 @@ int fvtd_launch(swm_engine* e, Tables& T, const NodeList& L) {
   EngineArgs a = eargs(e);
   hipStream_t s = e->stream;
   const int sh = e->cur_shape;
-  const TileRef *xt = T.dxt[sh].p, *yt = T.dyt[sh].p, *st = T.dst[sh].p;
+  const TileRef *xt = T.dxt[sh], *yt = T.dyt[sh], *st = T.dst[sh];
   const int nxt = T.nxt[sh], nyt = T.nyt[sh], nst = T.nst[sh];
   const FaceShape& F = kShapes[sh];
   const bool small = (long)(nxt + nyt) * L.count * F.xw * F.xh <= kFvtdTogether;
   if (small && !(e->prof.mask & 7u)) {
     launch_fvtd(a, sh, xt, nxt, yt, nyt, st, nst, L, s);
-    launch_fvtd_update(a, T.dcb.p, T.ncb, L, s);
+    launch_fvtd_update(a, T.dcb, T.ncb, L, s);
   } else {  // also while events tell the kinds apart
     timed(e, 0, [&] { launch_fvtd(a, sh, xt, nxt, nullptr, 0, nullptr, 0, L, s); });
     timed(e, 1, [&] { launch_fvtd(a, sh, nullptr, 0, yt, nyt, nullptr, 0, L, s); });
-    timed(e, 2, [&] { launch_fvtd_source_update(a, T.dct.p, T.nct, L, s); });
+    timed(e, 2, [&] { launch_fvtd_source_update(a, T.dct, T.nct, L, s); });
   }
   LAUNCHCK(e);
   return SWM_OK;
@@ -643,12 +635,12 @@ int explicit_body(swm_engine* e, Tables& T, const SchemeDef& D) {
     return fvtd_launch(e, T, L);
   };
   auto comb = [&](const CombOp& op) {
-    timed(e, 3, [&] { launch_combine(a, T.dcb.p, T.ncb, op, s); });
+    timed(e, 3, [&] { launch_combine(a, T.dcb, T.ncb, op, s); });
   };
   // the writer's state: the input of the step's last FVTD, before a stage
   // combination overwrites its slot
   auto keep = [&](int m) {
-    if (e->keep_count) launch_keep_state(a, T.dcb.p, T.ncb, m, s);
+    if (e->keep_count) launch_keep_state(a, T.dcb, T.ncb, m, s);
   };
   constexpr int X = 0, F = 1;
   int rc = SWM_OK;
@@ -740,7 +732,7 @@ int step_body(swm_engine* e, Tables& T, const StepPlan& P) {
   EngineArgs a = eargs(e);
   hipStream_t s = e->stream;
   if (P.device_dt) {
-    timed(e, 6, [&] { launch_timestep(a, T.dcb.p, T.ncb, T.djl.p, T.njobs, s); });
+    timed(e, 6, [&] { launch_timestep(a, T.dcb, T.ncb, T.djl, T.njobs, s); });
     LAUNCHCK(e);
   }
   const SchemeDef& D = *P.sc;
@@ -755,7 +747,7 @@ int step_body(swm_engine* e, Tables& T, const StepPlan& P) {
   if (rc) return rc;
   // the writer's state: the input of the step's last FVTD (U^n when the
   // scheme has a single correction)
-  if (e->keep_count && D.kcorr == 1) launch_keep_state(a, T.dcb.p, T.ncb, 0, s);
+  if (e->keep_count && D.kcorr == 1) launch_keep_state(a, T.dcb, T.ncb, 0, s);
   SysList S{};
   for (int r = 0; r < 4; ++r) S.src[r] = 0;
   S.hp_is_un = 1;
@@ -770,19 +762,19 @@ int step_body(swm_engine* e, Tables& T, const StepPlan& P) {
       S.m[S.count++] = D.msteps - 1;
     else
       for (int m = 1; m < D.msteps; ++m) S.m[S.count++] = m;
-    if (S.hp_view) timed(e, 4, [&] { launch_hp_view(a, T.dcb.p, T.ncb, kk == 1, s); });
+    if (S.hp_view) timed(e, 4, [&] { launch_hp_view(a, T.dcb, T.ncb, kk == 1, s); });
     // the DeC momentum update runs inside the assembly kernel
     if (P.solve) {
-      timed(e, 4, [&] { launch_assemble_matrix(a, T.dcbs.p, T.ncbs, S, s); });
+      timed(e, 4, [&] { launch_assemble_matrix(a, T.dcbs, T.ncbs, S, s); });
       const int c = S.count == 1 ? 0 : 1;
       for (const auto& l : T.svl[c])
         timed(e, 5, [&] {
-          launch_solve(a, T.dsv[c].p + l.first, l.second, S, P.limit[kk - 1], solve, s);
+          launch_solve(a, T.dsv[c] + l.first, l.second, S, P.limit[kk - 1], solve, s);
         });
     }
     // the grids swept by a launch per sweep: all of them without k_solve
-    const TileRef* cb = P.solve ? T.dcbw.p : T.dcb.p;
-    const int* jl = P.solve ? T.djlw.p : T.djl.p;
+    const TileRef* cb = P.solve ? T.dcbw : T.dcb;
+    const int* jl = P.solve ? T.djlw : T.djl;
     const int ncb = P.solve ? T.ncbw : T.ncb, njobs = P.solve ? T.njobsw : T.njobs;
     if (ncb) timed(e, 4, [&] { launch_assemble(a, cb, ncb, jl, njobs, S, s); });
     LAUNCHCK(e);
@@ -838,7 +830,7 @@ int step_body(swm_engine* e, Tables& T, const StepPlan& P) {
       rc = fvtd_launch(e, T, L);
       if (rc) return rc;
       if (e->keep_count && kk == D.kcorr - 1)
-        launch_keep_state(a, T.dcb.p, T.ncb, D.msteps - 1, s);
+        launch_keep_state(a, T.dcb, T.ncb, D.msteps - 1, s);
       for (int r = 0; r < 4; ++r) S.src[r] = r;
       S.hp_is_un = 0;
     }
@@ -852,8 +844,8 @@ int step_full(swm_engine* e, Tables& T, const StepPlan& P) {
   if (rc) return rc;
   EngineArgs a = eargs(e);
   hipStream_t s = e->stream;
-  timed(e, 7, [&] { launch_gate(a, T.djl.p, T.njobs, P.sc->nsolve, s); });
-  timed(e, 7, [&] { launch_commit(a, T.dcb.p, T.ncb, P.sc->final_state, s); });
+  timed(e, 7, [&] { launch_gate(a, T.djl, T.njobs, P.sc->nsolve, s); });
+  timed(e, 7, [&] { launch_commit(a, T.dcb, T.ncb, P.sc->final_state, s); });
   LAUNCHCK(e);
   return SWM_OK;
 }
@@ -1066,7 +1058,7 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
     swm_engine* e;
     ~Ungate() { e->gated = 0; }
   } ungate{e};
-  launch_batch_begin(eargs(e), T.djl.p, T.njobs, B, s);
+  launch_batch_begin(eargs(e), T.djl, T.njobs, B, s);
   LAUNCHCK(e);
   if (host_dt) {
     *e->hdt = *host_dt;
@@ -1168,7 +1160,7 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
     // that step in polling mode; every other job keeps its stop and is skipped
     B.redo = 1;
     B.max_steps = 1;
-    launch_batch_begin(eargs(e), T.djl.p, T.njobs, B, s);
+    launch_batch_begin(eargs(e), T.djl, T.njobs, B, s);
     LAUNCHCK(e);
     for (int q = 0; q < T.njobs; ++q) e->redone_steps += redo[q];
     P.speculative = false;
@@ -1189,20 +1181,55 @@ int job_from_id(swm_engine* e, int id, Job** out) {
   return SWM_OK;
 }
 
+// Device memory for the layout conversion of a transfer: the job's face fluxes
+// and matrices, which hold nothing between two calls (they are adjacent in the
+// slab, 33 doubles a cell), else an allocation of its own.
+struct Staging {
+  double* p = nullptr;
+  bool owned = false;
+  hipError_t get(Job& J, size_t doubles) {
+    double* first = J.dev.FX[0][0];
+    const double* end = J.dev.M[kMaxSys - 1][4] + J.lay.n;
+    if (first + doubles <= end) {
+      p = first;
+      return hipSuccess;
+    }
+    const hipError_t er = hipMalloc((void**)&p, doubles * sizeof(double));
+    if (er != hipSuccess) p = nullptr;
+    owned = p != nullptr;
+    return er;
+  }
+  ~Staging() {
+    if (owned) (void)hipFree(p);
+  }
+};
+
 int upload_state(swm_engine* e, Job& J, const double* U, int ghosts, double* h, double* hu,
                  double* hv) {
   const int nx = J.dev.nx, ny = J.dev.ny;
   size_t cnt = 3 * (size_t)(nx + 2 * ghosts) * (ny + 2 * ghosts);
-  double* tmp = nullptr;
-  HIPCK(e, hipMalloc((void**)&tmp, cnt * sizeof(double)));
-  hipError_t er = hipMemcpyAsync(tmp, U, cnt * sizeof(double), hipMemcpyHostToDevice, e->stream);
+  Staging tmp;
+  HIPCK(e, tmp.get(J, cnt));
+  hipError_t er = e->ring->to_device(tmp.p, U, cnt * sizeof(double), e->stream);
   if (er == hipSuccess) {
-    launch_aos_to_soa(nx, ny, ghosts, tmp, h, hu, hv, e->stream);
+    launch_aos_to_soa(nx, ny, ghosts, tmp.p, h, hu, hv, e->stream);
     er = hipGetLastError();
   }
   if (er == hipSuccess) er = hipStreamSynchronize(e->stream);
-  (void)hipFree(tmp);
   if (er != hipSuccess) FAIL(e, SWM_E_HIP, "upload failed: %s", hipGetErrorString(er));
+  return SWM_OK;
+}
+
+// What `launch` leaves in the staging memory (3 doubles a cell) to the host.
+template <class Launch>
+int download_state(swm_engine* e, Job& J, double* out, const char* what, Launch launch) {
+  const size_t cnt = 3 * J.lay.n;
+  Staging tmp;
+  HIPCK(e, tmp.get(J, cnt));
+  launch(tmp.p);
+  hipError_t er = hipGetLastError();
+  if (er == hipSuccess) er = e->ring->to_host(out, tmp.p, cnt * sizeof(double), e->stream);
+  if (er != hipSuccess) FAIL(e, SWM_E_HIP, "%s failed: %s", what, hipGetErrorString(er));
   return SWM_OK;
 }
 
@@ -1220,7 +1247,7 @@ int build_wb(swm_engine* e, int id) {
   L.wb_init = 1;
   rc = fvtd_launch(e, J.own, L);
   if (rc) return rc;
-  launch_copy_wb(eargs(e), J.own.dcb.p, J.own.ncb, 0, e->stream);
+  launch_copy_wb(eargs(e), J.own.dcb, J.own.ncb, 0, e->stream);
   LAUNCHCK(e);
   HIPCK(e, hipStreamSynchronize(e->stream));
   J.wb_ready = true;
@@ -1697,7 +1724,12 @@ int swm_engine_create(long long budget_bytes, swm_engine_t** out) {
   }
   int rc = status_capacity(e, 8);
   int cus = 0;
-  if (hipGetDevice(&e->device) == hipSuccess &&
+  if (rc == SWM_OK && (hipGetDevice(&e->device) != hipSuccess || e->device < 0)) {
+    g_error = "hipGetDevice failed";
+    rc = SWM_E_HIP;
+  }
+  if (rc == SWM_OK) e->ring = HostRing::of_device(e->device);
+  if (rc == SWM_OK &&
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, e->device) == hipSuccess)
     e->solve_blocks_max = cus;  // a k_solve block's registers fill at most one CU
   if (rc == SWM_OK && hipHostMalloc((void**)&e->hdt, sizeof(double), hipHostMallocDefault) != hipSuccess) {
@@ -1862,17 +1894,9 @@ int swm_engine_fetch(swm_engine_t* e, int job_id, double* U) {
   Job* J;
   int rc = job_from_id(e, job_id, &J);
   if (rc) return rc;
-  const size_t n = J->lay.n;
-  double* tmp = nullptr;
-  HIPCK(e, hipMalloc((void**)&tmp, 3 * n * sizeof(double)));
-  launch_soa_to_aos(J->dev.nx, J->dev.ny, J->dev.h, J->dev.hu, J->dev.hv, tmp, e->stream);
-  hipError_t er = hipGetLastError();
-  if (er == hipSuccess)
-    er = hipMemcpyAsync(U, tmp, 3 * n * sizeof(double), hipMemcpyDeviceToHost, e->stream);
-  if (er == hipSuccess) er = hipStreamSynchronize(e->stream);
-  (void)hipFree(tmp);
-  if (er != hipSuccess) FAIL(e, SWM_E_HIP, "fetch failed: %s", hipGetErrorString(er));
-  return SWM_OK;
+  return download_state(e, *J, U, "fetch", [&](double* tmp) {
+    launch_soa_to_aos(J->dev.nx, J->dev.ny, J->dev.h, J->dev.hu, J->dev.hv, tmp, e->stream);
+  });
 }
 
 int swm_engine_release(swm_engine_t* e, int job_id) {
@@ -2065,17 +2089,9 @@ int swm_download_primitive(swm_solver_t* s, double* V) {
   swm_engine* e = s->e;
   if (!V) FAIL(e, SWM_E_ARG, "V is NULL");
   Job& J = *plain_job(s);
-  const size_t n = J.lay.n;
-  double* tmp = nullptr;
-  HIPCK(e, hipMalloc((void**)&tmp, 3 * n * sizeof(double)));
-  launch_primitives(n, J.dev.h, J.dev.hu, J.dev.hv, tmp, e->stream);
-  hipError_t er = hipGetLastError();
-  if (er == hipSuccess)
-    er = hipMemcpyAsync(V, tmp, 3 * n * sizeof(double), hipMemcpyDeviceToHost, e->stream);
-  if (er == hipSuccess) er = hipStreamSynchronize(e->stream);
-  (void)hipFree(tmp);
-  if (er != hipSuccess) FAIL(e, SWM_E_HIP, "primitive download failed: %s", hipGetErrorString(er));
-  return SWM_OK;
+  return download_state(e, J, V, "primitive download", [&](double* tmp) {
+    launch_primitives(J.lay.n, J.dev.h, J.dev.hu, J.dev.hv, tmp, e->stream);
+  });
 }
 
 // Keeping (or not) the writer's state of job J (swm_keep_output_state).
@@ -2108,16 +2124,9 @@ static int job_output_primitive(swm_engine* e, Job& J, double* V) {
     FAIL(e, SWM_E_STATE,
          "no kept output state: swm_keep_output_state before a step of a Patankar scheme");
   const size_t n = J.lay.n;
-  double* tmp = nullptr;
-  HIPCK(e, hipMalloc((void**)&tmp, 3 * n * sizeof(double)));
-  launch_primitives(n, J.vout_buf, J.vout_buf + n, J.vout_buf + 2 * n, tmp, e->stream);
-  hipError_t er = hipGetLastError();
-  if (er == hipSuccess)
-    er = hipMemcpyAsync(V, tmp, 3 * n * sizeof(double), hipMemcpyDeviceToHost, e->stream);
-  if (er == hipSuccess) er = hipStreamSynchronize(e->stream);
-  (void)hipFree(tmp);
-  if (er != hipSuccess) FAIL(e, SWM_E_HIP, "output download failed: %s", hipGetErrorString(er));
-  return SWM_OK;
+  return download_state(e, J, V, "output download", [&](double* tmp) {
+    launch_primitives(n, J.vout_buf, J.vout_buf + n, J.vout_buf + 2 * n, tmp, e->stream);
+  });
 }
 
 int swm_keep_output_state(swm_solver_t* s, int on) {
@@ -2200,7 +2209,7 @@ int swm_timestep(swm_solver_t* s, double* dt_min, double* lmx, double* lmy) {
   int rc = refresh(e);
   if (rc) return rc;
   Tables& T = plain_job(s)->own;
-  timed(e, 6, [&] { launch_timestep(eargs(e), T.dcb.p, T.ncb, T.djl.p, T.njobs, e->stream); });
+  timed(e, 6, [&] { launch_timestep(eargs(e), T.dcb, T.ncb, T.djl, T.njobs, e->stream); });
   LAUNCHCK(e);
   rc = read_status(e);
   if (rc) return rc;
