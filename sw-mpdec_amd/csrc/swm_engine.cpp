@@ -64,6 +64,12 @@ struct JobLayout {
   size_t bytes;
 };
 
+// TimeStep's partial maxima: three per cell block, or per wave where
+// k_step_end commits.
+size_t timestep_parts(size_t n) {
+  return 3 * (n <= (size_t)kStepEndCells ? (n + 63) / 64 + 15 : (n + kCellBlock - 1) / kCellBlock);
+}
+
 JobLayout job_layout(int nx, int ny, int wb, int bathy) {
   JobLayout L;
   L.n = (size_t)nx * ny;
@@ -84,7 +90,7 @@ JobLayout job_layout(int nx, int ny, int wb, int bathy) {
     add(L.n);
   }
   add((size_t)(kMaxSys + 1) * L.nblk);                   // Jacobi partial sums
-  add(3 * (size_t)L.nblk);                               // TimeStep partials
+  add(timestep_parts(L.n));                              // TimeStep partials
   add(solve_slot(nx, ny, kSolveForms, 0, 0, 0));         // k_solve's slots
   L.bytes = b;
   (void)bathy;  // the bathymetry tables are a separate allocation (bathy_bytes)
@@ -494,11 +500,19 @@ int refresh(swm_engine* e) {
   return SWM_OK;
 }
 
-EngineArgs eargs(swm_engine* e) {
+// Cells up to which a grid's stage kernels do not look at halt: its batch runs
+// on after a stop only when a solve was left open, dt was not finite or the
+// output time came a step earlier than expected, for 15 steps at most.
+constexpr int kEagerCells = 1 << 17;
+
+EngineArgs eargs(swm_engine* e, const Tables& T) {
   EngineArgs a;
   a.jobs = e->djobs.p;
+  a.status = e->dstatus.p;
+  a.single = T.njobs == 1 ? T.jl[0] : -1;
   a.max_iter = e->max_iter;
   a.gated = e->gated;
+  a.eager = a.single >= 0 && T.njobsw == 0 && e->jobs[a.single]->dev.n <= kEagerCells;
   a.tol = e->tol;
   return a;
 }
@@ -508,7 +522,7 @@ EngineArgs eargs(swm_engine* e) {
 constexpr long kFvtdTogether = 8L * 262144;
 
 int fvtd_launch(swm_engine* e, Tables& T, const NodeList& L) {
-  EngineArgs a = eargs(e);
+  EngineArgs a = eargs(e, T);
   hipStream_t s = e->stream;
   const int sh = e->cur_shape;
   const TileRef *xt = T.dxt[sh], *yt = T.dyt[sh], *st = T.dst[sh];
@@ -541,7 +555,7 @@ int read_status(swm_engine* e) {
 // (src/timediscretization.f90:458-566), mPEuler (:671-764) or mPDeC2
 // (:571-664), which differ only in MSteps, KCorr and thetaDeC.
 //
-// The launch sequence: [TimeStep] -> FVTD(U^n) -> KCorr corrections, each
+// The launch sequence: FVTD(U^n) -> KCorr corrections, each
 // [depth view] -> momentum -> assembly (+ first sweep) -> Jacobi sweeps ->
 // record -> finalize -> FVTD of the new nodes (all corrections but the last)
 // -> (after the host check) commit.  Each sweep is followed by the
@@ -620,7 +634,7 @@ constexpr double kBRK65[6] = {0.077777777777777778, 0., 0.35555555555555556,
                               0.13333333333333333, 0.35555555555555556, 0.077777777777777778};
 
 int explicit_body(swm_engine* e, Tables& T, const SchemeDef& D) {
-  EngineArgs a = eargs(e);
+  EngineArgs a = eargs(e, T);
   hipStream_t s = e->stream;
   // FVTimeDerivative of state slots into derivative slots, Ut(1:3)
   auto fvtd = [&](std::initializer_list<std::pair<int, int>> in_out) {
@@ -729,12 +743,8 @@ int explicit_body(swm_engine* e, Tables& T, const SchemeDef& D) {
 
 // The step's launches; returns after the last finalize / FVTD (no commit).
 int step_body(swm_engine* e, Tables& T, const StepPlan& P) {
-  EngineArgs a = eargs(e);
+  EngineArgs a = eargs(e, T);
   hipStream_t s = e->stream;
-  if (P.device_dt) {
-    timed(e, 6, [&] { launch_timestep(a, T.dcb, T.ncb, T.djl, T.njobs, s); });
-    LAUNCHCK(e);
-  }
   const SchemeDef& D = *P.sc;
   if (is_explicit(D)) return explicit_body(e, T, D);
   // FVTimeDerivative(U^n): node 0, shared by all nodes at kk = 1
@@ -767,9 +777,12 @@ int step_body(swm_engine* e, Tables& T, const StepPlan& P) {
     if (P.solve) {
       timed(e, 4, [&] { launch_assemble_matrix(a, T.dcbs, T.ncbs, S, s); });
       const int c = S.count == 1 ? 0 : 1;
+      // one job: its blocks system by system, all in one form
+      const int nb = a.single >= 0 ? (int)T.sv[c].size() / (c == 0 ? 1 : kMaxSys) : 0;
       for (const auto& l : T.svl[c])
         timed(e, 5, [&] {
-          launch_solve(a, T.dsv[c] + l.first, l.second, S, P.limit[kk - 1], solve, s);
+          launch_solve(a, T.dsv[c], l.first, l.second, T.sv[c][l.first].form, nb, S,
+                       P.limit[kk - 1], solve, s);
         });
     }
     // the grids swept by a launch per sweep: all of them without k_solve
@@ -838,14 +851,30 @@ int step_body(swm_engine* e, Tables& T, const StepPlan& P) {
   return SWM_OK;
 }
 
-// The step's launches, then the commit decision (k_gate) and the commit.
+// TimeStep of every job's state, before the first step of a batch (the
+// following ones take theirs from the end of the step before).
+int first_dt(swm_engine* e, Tables& T) {
+  EngineArgs a = eargs(e, T);
+  timed(e, 6, [&] { launch_timestep(a, T.dcb, T.ncb, T.djl, T.njobs, e->stream); });
+  LAUNCHCK(e);
+  return SWM_OK;
+}
+
+// The step's launches, the commit, the step's record and the next dt.
 int step_full(swm_engine* e, Tables& T, const StepPlan& P) {
   int rc = step_body(e, T, P);
   if (rc) return rc;
-  EngineArgs a = eargs(e);
+  EngineArgs a = eargs(e, T);
   hipStream_t s = e->stream;
-  timed(e, 7, [&] { launch_gate(a, T.djl, T.njobs, P.sc->nsolve, s); });
-  timed(e, 7, [&] { launch_commit(a, T.dcb, T.ncb, P.sc->final_state, s); });
+  const int ns = P.sc->nsolve, dt = P.device_dt;
+  int most = 0;  // cells of the largest grid
+  for (int id : T.jl) most = std::max(most, e->jobs[id]->dev.n);
+  if (most <= kStepEndCells) {
+    timed(e, 7, [&] { launch_step_end(a, T.djl, T.njobs, P.sc->final_state, ns, dt, s); });
+  } else {
+    timed(e, 7, [&] { launch_commit(a, T.dcb, T.ncb, P.sc->final_state, ns, dt, s); });
+    timed(e, 7, [&] { launch_step_end(a, T.djl, T.njobs, -1, ns, dt, s); });
+  }
   LAUNCHCK(e);
   return SWM_OK;
 }
@@ -1013,7 +1042,7 @@ struct LoopArgs {
 
 // A batch: up to `steps` steps of every job of T with one read of the status
 // at the end (the device decides, step by step, which jobs go on; see
-// k_gate).  host_dt: one step with this dt for every job (steps = 1).
+// k_step_end).  host_dt: one step with this dt for every job (steps = 1).
 // Steps run speculatively when every job has a sweep-count prediction for the
 // scheme, else one step in polling mode (the explicit schemes, which solve
 // nothing, run every step of the batch without host reads).  A job whose
@@ -1058,7 +1087,7 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
     swm_engine* e;
     ~Ungate() { e->gated = 0; }
   } ungate{e};
-  launch_batch_begin(eargs(e), T.djl, T.njobs, B, s);
+  launch_batch_begin(eargs(e, T), T.djl, T.njobs, B, s);
   LAUNCHCK(e);
   if (host_dt) {
     *e->hdt = *host_dt;
@@ -1067,6 +1096,10 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
       HIPCK(e, hipMemcpyAsync(&st->dt, e->hdt, sizeof(double), hipMemcpyHostToDevice, s));
       HIPCK(e, hipMemcpyAsync(&st->dt_bad, e->hzero, sizeof(int), hipMemcpyHostToDevice, s));
     }
+  }
+  if (P.device_dt) {
+    int rc = first_dt(e, T);
+    if (rc) return rc;
   }
   if (spec) {
     int graph, margin;
@@ -1160,7 +1193,7 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
     // that step in polling mode; every other job keeps its stop and is skipped
     B.redo = 1;
     B.max_steps = 1;
-    launch_batch_begin(eargs(e), T.djl, T.njobs, B, s);
+    launch_batch_begin(eargs(e, T), T.djl, T.njobs, B, s);
     LAUNCHCK(e);
     for (int q = 0; q < T.njobs; ++q) e->redone_steps += redo[q];
     P.speculative = false;
@@ -1247,7 +1280,7 @@ int build_wb(swm_engine* e, int id) {
   L.wb_init = 1;
   rc = fvtd_launch(e, J.own, L);
   if (rc) return rc;
-  launch_copy_wb(eargs(e), J.own.dcb, J.own.ncb, 0, e->stream);
+  launch_copy_wb(eargs(e, J.own), J.own.dcb, J.own.ncb, 0, e->stream);
   LAUNCHCK(e);
   HIPCK(e, hipStreamSynchronize(e->stream));
   J.wb_ready = true;
@@ -1402,7 +1435,7 @@ int alloc_job(swm_engine* e, int nx, int ny, double dx, double dy, double g, dou
     D.SWB3 = take(lay.n);
   }
   D.part = take((size_t)(kMaxSys + 1) * lay.nblk);
-  D.tspart = take(3 * (size_t)lay.nblk);
+  D.tspart = take(timestep_parts(lay.n));
   const size_t nslots = solve_slot(nx, ny, kSolveForms, 0, 0, 0);
   D.slots = reinterpret_cast<unsigned long long*>(take(nslots));
   if (off > lay.bytes) FAIL(e, SWM_E_STATE, "internal: job slab overflow");
@@ -2209,7 +2242,7 @@ int swm_timestep(swm_solver_t* s, double* dt_min, double* lmx, double* lmy) {
   int rc = refresh(e);
   if (rc) return rc;
   Tables& T = plain_job(s)->own;
-  timed(e, 6, [&] { launch_timestep(eargs(e), T.dcb, T.ncb, T.djl, T.njobs, e->stream); });
+  timed(e, 6, [&] { launch_timestep(eargs(e, T), T.dcb, T.ncb, T.djl, T.njobs, e->stream); });
   LAUNCHCK(e);
   rc = read_status(e);
   if (rc) return rc;
@@ -2372,7 +2405,7 @@ int swm_advance(swm_solver_t* s, double* t, double t_analyze, double t_end, int 
   double dt_prev = 0.0;
   while (k < max_steps) {
     // src/timediscretization.f90:58-59 and :83-94 on the device; a batch
-    // covers about the steps left to the next stop (k_gate ends it there)
+    // covers about the steps left to the next stop (k_step_end ends it there)
     int batch = 1;
     if (dt_prev > 0.0) {
       const double left = std::min(t_analyze, t_end) - *t;
@@ -2385,7 +2418,7 @@ int swm_advance(swm_solver_t* s, double* t, double t_analyze, double t_end, int 
     if (rc) return rc;
     for (const StepRec& r : L.log) {
       if (dts) dts[k] = r.dt;
-      *t = *t + r.dt;  // as k_gate: the loop's t = t + dt
+      *t = *t + r.dt;  // as k_step_end: the loop's t = t + dt
       dt_prev = r.dt;
       ++k;
     }

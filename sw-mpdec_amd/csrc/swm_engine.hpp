@@ -58,7 +58,7 @@ struct JacState {
 };
 
 // Steps of one job that one host synchronisation can cover: the device time
-// loop (k_batch_begin, k_gate) runs up to kMaxBatch steps between reads of
+// loop (k_batch_begin, k_step_end) runs up to kMaxBatch steps between reads of
 // the status, recording each committed step.
 constexpr int kMaxBatch = 16;
 
@@ -72,7 +72,7 @@ enum SolveEnd {
 };
 
 // Why a job's batch stopped (JobStatus::halt); while halt != 0 every gated
-// kernel of the job returns at once and k_commit commits nothing.
+// kernel of the job returns at once, k_commit among them.
 enum HaltCode {
   kHaltNone = 0,
   kHaltBatch = 1,    // the batch's step count was reached
@@ -108,14 +108,13 @@ struct JobStatus {
   int ambiguous[13];      // its stop decisions settled by the exact sequential sum
   signed char ended[13];  // SolveEnd
   double dt_min;  // TimeStep's value before the time loop's clipping
-  // the device time loop (k_batch_begin sets, k_gate advances)
+  // the device time loop (k_batch_begin sets, k_step_end advances)
   int halt;        // HaltCode
-  int commit;      // 1: k_commit commits the step just run
   int batch_done;  // steps committed in this batch (records rec[0..batch_done))
   int batch_max;   // steps this batch may commit
   int loop;        // 1: dt = MIN(MIN(dt_min, t_an - t), MIN(dt_min, t_end - t))
                    // (src/timediscretization.f90:58-59) and t advances here
-  int steps_left;  // step-count stop, counted down by k_gate: > 0 steps to go,
+  int steps_left;  // step-count stop, counted down by k_step_end: > 0 steps to go,
                    // 0 all run (k_batch_begin keeps the job halted), < 0 none
   double t, t_an, t_end;
   StepRec rec[kMaxBatch];
@@ -222,8 +221,13 @@ inline __host__ __device__ size_t solve_slot(int nx, int ny, int form, int sys, 
 // steps of a batch: a job whose JobStatus::halt is set is skipped.
 struct EngineArgs {
   const JobDev* jobs;
+  JobStatus* status;  // by job, as JobDev::status
+  int single;         // >= 0: the launch covers this job alone, block or tile t
+                      // its t-th one, so that no kernel has to look it up
   int max_iter;
   int gated;
+  int eager;  // with gated: the kernels that write only what a step recomputes
+              // do not look at halt (one small grid)
   double tol;
 };
 
@@ -354,16 +358,22 @@ void launch_finalize(const EngineArgs& E, const TileRef* cb, int ncb, const int*
 // the matrix rows and the momentum update alone, for the grids k_solve takes
 void launch_assemble_matrix(const EngineArgs& E, const TileRef* cb, int ncb, const SysList& S,
                             hipStream_t s);
-// k_solve over nblk blocks: the Jacobi iteration of each block's system, up to
-// `limit` sweeps
-void launch_solve(const EngineArgs& E, const SolveRef* refs, int nblk, const SysList& S, int limit,
-                  int first_solve, hipStream_t s);
+// k_solve over the blocks refs[first .. first + nblk): the Jacobi iteration of
+// each block's system, up to `limit` sweeps.  nb > 0 (E.single): block b is
+// tile b % nb of system b / nb in this form.
+void launch_solve(const EngineArgs& E, const SolveRef* refs, int first, int nblk, int form, int nb,
+                  const SysList& S, int limit, int first_solve, hipStream_t s);
 void launch_timestep(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl, int njobs,
                      hipStream_t s);
-void launch_commit(const EngineArgs& E, const TileRef* cb, int ncb, int final_node,
-                   hipStream_t s);
-// k_gate: the commit decision and record of each job's step
-void launch_gate(const EngineArgs& E, const int* jl, int njobs, int nsolve, hipStream_t s);
+// commits the accepted steps and, with next_dt, leaves TimeStep's partial
+// maxima of the committed states
+void launch_commit(const EngineArgs& E, const TileRef* cb, int ncb, int final_node, int nsolve,
+                   int next_dt, hipStream_t s);
+// k_step_end: the record of each job's step and, with next_dt, the next step's
+// dt; final_node >= 0: also the commit, for grids of at most kStepEndCells
+constexpr int kStepEndCells = 4096;
+void launch_step_end(const EngineArgs& E, const int* jl, int njobs, int final_node, int nsolve,
+                     int next_dt, hipStream_t s);
 void launch_batch_begin(const EngineArgs& E, const int* jl, int njobs, const BatchArgs& B,
                         hipStream_t s);
 // sets JobStatus::steps_left of one job (its step-count stop)

@@ -92,8 +92,29 @@ __device__ __forceinline__ int cdiv_d(int a, int b) { return (a + b - 1) / b; }
 
 // In the steps of a batch (E.gated) a job whose batch has stopped
 // (JobStatus::halt) is skipped by every kernel; the test is uniform per block.
-__device__ __forceinline__ bool skipped(const EngineArgs& E, const JobDev& J) {
-  return E.gated && J.status->halt != 0;
+// The status is reached from the launch's arguments, not through the job's
+// descriptor: a small kernel is a chain of dependent loads of 0.5 to 1 us each
+// (arguments, block's tile, job's descriptor, its data), and the look-ups saved
+// here and in tile_of and job_of are most of what its latency can lose.
+__device__ __forceinline__ bool skipped(const EngineArgs& E, int job) {
+  return E.gated && E.status[job].halt != 0;
+}
+
+// The same for kernels that write only stage buffers, which the next step
+// computes anew: one small grid is not worth the load (halt was written by
+// another XCD, so it comes from memory before anything else may start; 1 us of
+// a kernel of 4 to 5), its steps after a stop run in vain, uncommitted.
+__device__ __forceinline__ bool skipped_stage(const EngineArgs& E, int job) {
+  return E.gated && !E.eager && E.status[job].halt != 0;
+}
+
+// Entry b of a table of tiles or of jobs.
+__device__ __forceinline__ TileRef tile_of(const EngineArgs& E, const TileRef* tiles, int b) {
+  if (E.single >= 0) return {E.single, b};
+  return tiles[b];
+}
+__device__ __forceinline__ int job_of(const EngineArgs& E, const int* jobs, int b) {
+  return E.single >= 0 ? E.single : jobs[b];
 }
 
 // State slot m of a job: m = 0 is U^n, 1..3 the DeC nodes.
@@ -453,9 +474,9 @@ __global__ __launch_bounds__(XW * XH, 4) void k_fvtd(EngineArgs E, FvtdTiles T, 
   if (src) {
     const int t = s0 / L.count * 8 + r, node = s0 % L.count;
     if (t >= T.nst) return;
-    const TileRef R = T.st[t];
+    const TileRef R = tile_of(E, T.st, t);
     const JobDev& J = E.jobs[R.job];
-    if (skipped(E, J)) return;
+    if (skipped_stage(E, R.job)) return;
     double S2, S3;
     source_tile<SW, SH>(smem, J, R.tile, L.m[node], S2, S3);
     const int ntx = cdiv_d(J.nx, SW);
@@ -476,9 +497,9 @@ __global__ __launch_bounds__(XW * XH, 4) void k_fvtd(EngineArgs E, FvtdTiles T, 
   const bool x = f < T.nxt * L.count;
   const int q = x ? f : f - T.nxt * L.count, nt = x ? T.nxt : T.nyt;
   const int node = q / nt;
-  const TileRef R = (x ? T.xt : T.yt)[q - node * nt];
+  const TileRef R = tile_of(E, x ? T.xt : T.yt, q - node * nt);
   const JobDev& J = E.jobs[R.job];
-  if (skipped(E, J)) return;
+  if (skipped_stage(E, R.job)) return;
   if (x)
     x_faces<XW, XH>(smem, irregular, J, R.tile, L.m[node], L.slot[node], L);
   else
@@ -544,9 +565,9 @@ __device__ __forceinline__ void update_cell(const JobDev& J, const NodeList& L, 
 // well-balanced state's.  Bound by memory.
 __global__ __launch_bounds__(256) void k_fvtd_update(EngineArgs E, const TileRef* blocks,
                                                      NodeList L) {
-  const TileRef T = blocks[blockIdx.x];
+  const TileRef T = tile_of(E, blocks, blockIdx.x);
   const JobDev& J = E.jobs[T.job];
-  if (skipped(E, J)) return;
+  if (skipped_stage(E, T.job)) return;
   const int o = L.out[blockIdx.y], nx = J.nx, k0 = T.tile * kCellBlock, k = k0 + threadIdx.x;
   if (k >= J.n) return;
   int ci, cj;
@@ -575,9 +596,9 @@ __global__ __launch_bounds__(256) void k_fvtd_source_update(EngineArgs E, const 
   const int grp = blockIdx.x / (8 * L.count), rem = blockIdx.x % (8 * L.count);
   const int node = rem / 8, t = grp * 8 + (rem % 8);
   if (t >= ntiles) return;
-  const TileRef T = tiles[t];
+  const TileRef T = tile_of(E, tiles, t);
   const JobDev& J = E.jobs[T.job];
-  if (skipped(E, J)) return;
+  if (skipped_stage(E, T.job)) return;
   const int ntx = cdiv_d(J.nx, TW);
   const int ci = (T.tile % ntx) * TW + threadIdx.x % TW;
   const int cj = (T.tile / ntx) * TH + threadIdx.x / TW;
@@ -807,14 +828,14 @@ __global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* b
                                                   SysList S) {
   __shared__ double red[4];
   __shared__ double sq[4 * R * 256];  // [slot*R + node][thread]: face mass fluxes
-  const TileRef T = blocks[blockIdx.x];
+  const TileRef T = tile_of(E, blocks, blockIdx.x);
   const JobDev& J = E.jobs[T.job];
-  if (skipped(E, J)) return;
+  if (skipped_stage(E, T.job)) return;
   const int nx = J.nx, ny = J.ny, n = J.n;
   const int tid = threadIdx.x;
   const int k = T.tile * kCellBlock + tid;
   const bool in = k < n;
-  const double dt = J.status->dt;
+  const double dt = E.status[T.job].dt;
   const int s0 = gridDim.y > 1 ? blockIdx.y : 0, s1 = gridDim.y > 1 ? s0 + 1 : S.count;
   int kS = 0, kW = 0, kE = 0, kN = 0;  // neighbours
   double b = 0., bS = 0., bW = 0., bE = 0., bN = 0.;
@@ -890,14 +911,14 @@ __global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* b
 // One Jacobi sweep of every still-active system (src/jacobi_iteration.f90:72-80).
 __global__ __launch_bounds__(256) void k_sweep(EngineArgs E, const TileRef* blocks, SysList S) {
   __shared__ double red[4];
-  const TileRef T = blocks[blockIdx.x];
+  const TileRef T = tile_of(E, blocks, blockIdx.x);
   const JobDev& J = E.jobs[T.job];
-  if (skipped(E, J)) return;
+  if (skipped(E, T.job)) return;
   int act[kMaxSys] = {0, 0, 0}, cur[kMaxSys] = {0, 0, 0};
   bool any = false;
   for (int s = 0; s < S.count; ++s) {
-    act[s] = J.status->st[s].active;
-    cur[s] = J.status->st[s].cur;
+    act[s] = E.status[T.job].st[s].active;
+    cur[s] = E.status[T.job].st[s].cur;
     any = any || act[s];
   }
   if (!any) return;  // every system of this job has stopped
@@ -940,9 +961,10 @@ __global__ __launch_bounds__(256) void k_sweep(EngineArgs E, const TileRef* bloc
 template <bool FIRST>
 __global__ __launch_bounds__(256) void k_decide(EngineArgs E, const int* jobs, SysList S) {
   __shared__ double red[4];
-  const JobDev& J = E.jobs[jobs[blockIdx.x]];
-  JobStatus* st = J.status;
-  if (skipped(E, J)) return;
+  const int job = job_of(E, jobs, blockIdx.x);
+  const JobDev& J = E.jobs[job];
+  JobStatus* st = E.status + job;
+  if (skipped(E, job)) return;
   const int n = J.n, nb = J.nblk;
   double tot[kMaxSys + 1] = {0., 0., 0., 0.};
   int act[kMaxSys] = {0, 0, 0}, cur[kMaxSys] = {0, 0, 0};
@@ -1103,7 +1125,7 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
   const JobDev& J = E.jobs[W.job];
   const int tid = threadIdx.x, s = W.sys, m = S.m[s];
   const int nx = J.nx, ny = J.ny, n = J.n;
-  JobStatus* st = J.status;
+  JobStatus* st = E.status + W.job;
   const gdouble* rhs = system_rhs(J, S);
   // own cells [ox, ox + ow) x [oy, oy + oh); EW x EH with the halo
   int nb = 1, ox = 0, oy = 0, ow = nx, oh = ny, EW = nx, EH = ny;
@@ -1355,7 +1377,7 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
       if ((own >> i) & 1u) G(J.hres[m])[gk[i]] = zero ? 0. : result[i * NT + tid];
   }
   if (tid == 0) {
-    if (!ALONE && L.lost) st->solve_lost = 1;  // k_gate keeps the step from being committed
+    if (!ALONE && L.lost) st->solve_lost = 1;  // keeps the step from being committed
     if (W.tile == 0) {
       st->ended[first_solve + s] = end;
       st->iters[first_solve + s] = k_sweeps;
@@ -1366,10 +1388,17 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
 }
 
 __global__ __launch_bounds__(kSolveThreads) void k_solve(EngineArgs E, const SolveRef* refs,
-                                                         SysList S, int limit, int first_solve) {
+                                                         int first, int form, int nb, SysList S,
+                                                         int limit, int first_solve) {
   __shared__ SolveShared L;
-  const SolveRef W = refs[blockIdx.x];
-  if (skipped(E, E.jobs[W.job])) return;
+  SolveRef W;
+  if (nb > 0) {
+    const int b = first + blockIdx.x;
+    W = {E.single, b % nb, (short)(b / nb), (short)form};
+  } else {
+    W = refs[first + blockIdx.x];
+  }
+  if (skipped_stage(E, W.job)) return;
   switch (W.form) {
     case 0:
       return solve_block<2, false>(L, E, W, S, limit, first_solve);
@@ -1412,15 +1441,15 @@ __device__ __forceinline__ double block_min_all(double v, double* red) {
 __global__ __launch_bounds__(256) void k_finalize(EngineArgs E, const TileRef* blocks,
                                                   SysList S) {
   __shared__ double red[4];
-  const TileRef T = blocks[blockIdx.x];
+  const TileRef T = tile_of(E, blocks, blockIdx.x);
   const JobDev& J = E.jobs[T.job];
-  if (skipped(E, J)) return;
+  if (skipped(E, T.job)) return;
   const int k = T.tile * kCellBlock + threadIdx.x;
   double mn = __builtin_inf();
   if (k < J.n) {
     for (int s = 0; s < S.count; ++s) {
       const int m = S.m[s];
-      const JacState& q = J.status->st[s];
+      const JacState& q = E.status[T.job].st[s];
       const double v = q.zero ? 0. : G(J.xj[m][q.cur])[k];
       G(J.hres[m])[k] = v;
       mn = nan_min(mn, v);
@@ -1436,13 +1465,14 @@ __global__ __launch_bounds__(256) void k_finalize(EngineArgs E, const TileRef* b
 // accepted).
 __global__ __launch_bounds__(256) void k_stage_min(EngineArgs E, const int* jobs) {
   __shared__ double red[4];
-  const JobDev& J = E.jobs[jobs[blockIdx.x]];
-  if (skipped(E, J)) return;
+  const int job = job_of(E, jobs, blockIdx.x);
+  const JobDev& J = E.jobs[job];
+  if (skipped(E, job)) return;
   double mn = __builtin_inf();
   for (int t = threadIdx.x; t < J.nblk; t += blockDim.x) mn = nan_min(mn, J.part[t]);
   mn = block_min_all(mn, red);
   if (threadIdx.x == 0) {
-    JobStatus* st = J.status;
+    JobStatus* st = E.status + job;
     st->hmin_step = st->hmin_step_set ? nan_min(st->hmin_step, mn) : mn;
     st->hmin_step_set = 1;
   }
@@ -1453,7 +1483,7 @@ __global__ __launch_bounds__(256) void k_stage_min(EngineArgs E, const int* jobs
 // needed more sweeps than were launched).
 __global__ void k_solve_done(EngineArgs E, const int* jobs, SysList S, int first_solve) {
   if (threadIdx.x != 0) return;
-  JobStatus* st = E.jobs[jobs[blockIdx.x]].status;
+  JobStatus* st = E.status + job_of(E, jobs, blockIdx.x);
   if (E.gated && st->halt) return;
   for (int s = 0; s < S.count; ++s) {
     const JacState& q = st->st[s];
@@ -1465,45 +1495,60 @@ __global__ void k_solve_done(EngineArgs E, const int* jobs, SysList S, int first
   }
 }
 
+// Whether the step just run is committed: not when the job's batch has already
+// stopped, when a solve was left open (U^n is intact and the host redoes the
+// step), or when dt is not finite.
+__device__ __forceinline__ bool solves_open(const JobStatus* st, int nsolve) {
+  int open = st->solve_lost;
+  for (int i = 0; i < nsolve; ++i) open |= st->ended[i] == kSolveOpen;
+  return open != 0;
+}
+
 // U^{n+1} = Ua(MSteps) (src/timediscretization.f90:564,662,762), node
-// mf = MSteps - 1 here, for the jobs whose step k_gate accepted.
-__global__ __launch_bounds__(256) void k_commit(EngineArgs E, const TileRef* blocks, int mf) {
-  const TileRef T = blocks[blockIdx.x];
+// mf = MSteps - 1 here, of the accepted steps.  TimeStep's partial maxima of
+// the next step (next_dt) come from the values on their way, for a pass over
+// the state less (2048^2: 35 + 35 -> COMMIT2048 us).
+__global__ __launch_bounds__(256) void k_commit(EngineArgs E, const TileRef* blocks, int mf,
+                                                int nsolve, int next_dt) {
+  const TileRef T = tile_of(E, blocks, blockIdx.x);
   const JobDev& J = E.jobs[T.job];
+  const JobStatus* st = E.status + T.job;
+  if (st->halt || st->dt_bad || solves_open(st, nsolve)) return;
   const int k = T.tile * kCellBlock + threadIdx.x;
-  if (!J.status->commit || k >= J.n) return;
-  G(J.h)[k] = G(J.hres[mf])[k];
-  G(J.hu)[k] = G(J.hun[mf])[k];
-  G(J.hv)[k] = G(J.hvn[mf])[k];
+  const bool in = k < J.n;
+  double h = 0., hu = 0., hv = 0.;
+  if (in) {
+    h = G(J.hres[mf])[k];
+    hu = G(J.hun[mf])[k];
+    hv = G(J.hvn[mf])[k];
+    G(J.h)[k] = h;
+    G(J.hu)[k] = hu;
+    G(J.hv)[k] = hv;
+  }
+  if (next_dt) timestep_partial(in, J.g, h, hu, hv, J.tspart + 3 * (size_t)T.tile);
 }
 
 // ------------------------------------------------------------------------
 // The device time loop: up to kMaxBatch steps between host reads.
 //
-// k_batch_begin starts a batch (one thread per job).  After each step k_gate
-// (one thread per job) decides whether the step is committed: not when the
-// job's batch has already stopped, when a speculative step overran its
-// launched Jacobi sweeps (U^n is intact and the host redoes the step), or when
-// dt is not finite.  A committed step is recorded and advances the loop: t =
-// t + dt and the output/end test of src/timediscretization.f90:83-94, the
-// job's step count and the batch's.  Whatever stops the batch sets halt, and
-// every later kernel of the batch skips the job.
+// k_batch_begin starts a batch (one thread per job).  After each step's commit
+// k_step_end (one block per job) records a committed step and advances the
+// loop: t = t + dt and the output/end test of src/timediscretization.f90:83-94,
+// the job's step count and the batch's.  Whatever stops the batch sets halt,
+// and every later kernel of the batch skips the job.
 // ------------------------------------------------------------------------
 __global__ void k_batch_begin(EngineArgs E, const int* jobs, BatchArgs B) {
   if (threadIdx.x != 0) return;
-  JobStatus* st = E.jobs[jobs[blockIdx.x]].status;
+  JobStatus* st = E.status + job_of(E, jobs, blockIdx.x);
   if (B.redo && st->halt != kHaltOverrun) {  // keeps its own stop
     if (!st->halt) st->halt = kHaltMasked;
-    st->commit = 0;
     return;
   }
   if (st->steps_left == 0) {  // the job has run all its steps
     st->halt = kHaltCount;
-    st->commit = 0;
     return;
   }
   st->halt = kHaltNone;
-  st->commit = 0;
   st->solve_lost = 0;
   st->batch_done = 0;
   st->batch_max = B.max_steps;
@@ -1516,46 +1561,111 @@ __global__ void k_batch_begin(EngineArgs E, const int* jobs, BatchArgs B) {
   }
 }
 
-__global__ void k_gate(EngineArgs E, const int* jobs, int nsolve) {
-  if (threadIdx.x != 0) return;
-  JobStatus* st = E.jobs[jobs[blockIdx.x]].status;
-  st->commit = 0;
-  if (st->halt) return;
-  int open = st->solve_lost, nonconv = 0, ambiguous = 0;
-  for (int i = 0; i < nsolve; ++i) {
-    open |= st->ended[i] == kSolveOpen;
-    nonconv += st->ended[i] == kSolveLimit;
-    ambiguous += st->ambiguous[i];
-  }
-  if (open) {
-    st->halt = kHaltOverrun;
-    st->hmin_step_set = 0;  // the redone attempt's stages start a new minimum
+__device__ __forceinline__ void record_step(JobStatus* st, int nsolve) {
+  // lanes 0..12 take a solve each
+  const int i = threadIdx.x;
+  const bool mine = i < nsolve;
+  const int end = mine ? st->ended[i] : kSolveConverged;
+  const int amb = mine ? st->ambiguous[i] : 0, sweeps = mine ? st->iters[i] : 0;
+  const int done = st->batch_done, bad = st->dt_bad, lost = st->solve_lost;
+  const bool open = __any(end == kSolveOpen) || lost;
+  const int nonconv = __popcll(__ballot(end == kSolveLimit));
+  if (!open && !bad && i < 13) st->rec[done].iters[i] = sweeps;
+  int ambiguous = 0;
+  if (__any(amb != 0))
+    for (int q = 0; q < 13; ++q) ambiguous += __shfl(amb, q, 64);
+  if (i != 0) return;
+  if (open || bad) {
+    st->halt = open ? kHaltOverrun : kHaltDtBad;
+    st->hmin_step_set = 0;  // a redone attempt's stages start a new minimum
     return;
   }
-  if (st->dt_bad) {
-    st->hmin_step_set = 0;
-    st->halt = kHaltDtBad;
-    return;
-  }
-  st->commit = 1;
-  StepRec& r = st->rec[st->batch_done];
+  StepRec& r = st->rec[done];
   r.dt = st->dt;
-  for (int i = 0; i < 13; ++i) r.iters[i] = i < nsolve ? st->iters[i] : 0;
   r.nonconv = nonconv;
   r.ambiguous = ambiguous;
-  st->batch_done += 1;
+  st->batch_done = done + 1;
   if (st->hmin_step_set) {  // the accepted step's stage minimum joins the record
     st->hmin = st->hmin_set ? nan_min(st->hmin, st->hmin_step) : st->hmin_step;
     st->hmin_set = 1;
     st->hmin_step_set = 0;
   }
+  int halt = kHaltNone;
   if (st->loop) {
-    st->t = st->t + st->dt;
-    if (fabs(st->t_an - st->t) < 1.0E-10 || fabs(st->t - st->t_end) < 1.0E-10)
-      st->halt = kHaltReached;
+    const double t = st->t + st->dt;
+    st->t = t;
+    if (fabs(st->t_an - t) < 1.0E-10 || fabs(t - st->t_end) < 1.0E-10) halt = kHaltReached;
   }
-  if (st->steps_left > 0 && --st->steps_left == 0 && !st->halt) st->halt = kHaltCount;  // < 0: none
-  if (!st->halt && st->batch_done >= st->batch_max) st->halt = kHaltBatch;
+  const int left = st->steps_left;  // < 0: none
+  if (left > 0) {
+    st->steps_left = left - 1;
+    if (left == 1 && !halt) halt = kHaltCount;
+  }
+  if (!halt && done + 1 >= st->batch_max) halt = kHaltBatch;
+  if (halt) st->halt = halt;
+}
+
+// TimeStep of the job's state from the partial maxima, and the time loop's
+// dt = MIN(MIN(dt_min, tAnalyze-t), MIN(dt_min, tEnd-t))
+// (src/timediscretization.f90:58-59) when the device runs the loop.
+template <int NT>
+__device__ __forceinline__ void next_step_dt(const JobDev& J, JobStatus* st, int nparts) {
+  const gdouble *h = G(J.h), *hu = G(J.hu), *hv = G(J.hv);
+  double ts, LX, LY;
+  timestep_final<NT>(
+      J.tspart, nparts, J.n,
+      [&](int k, double& a, double& b, double& c) {
+        a = h[k];
+        b = hu[k];
+        c = hv[k];
+      },
+      J.g, J.dx, J.dy, J.cfl, ts, LX, LY);
+  if (threadIdx.x != 0) return;
+  st->dt_min = ts;
+  const double dt =
+      st->loop ? min_r(min_r(ts, st->t_an - st->t), min_r(ts, st->t_end - st->t)) : ts;
+  st->dt = dt;
+  st->lmx = LX;
+  st->lmy = LY;
+  st->dt_bad = isfinite(dt) ? 0 : 1;
+}
+
+// The step's record and, when the batch goes on, the next step's dt: one launch
+// where the record, TimeStep's maxima and their fold were three (of 4.4 us each
+// at 32^2).  mf >= 0: the commit of node mf too, by the job's one block.
+__global__ __launch_bounds__(1024) void k_step_end(EngineArgs E, const int* jobs, int mf,
+                                                   int nsolve, int next_dt) {
+  constexpr int NT = 1024;
+  const int job = job_of(E, jobs, blockIdx.x);
+  const JobDev& J = E.jobs[job];
+  JobStatus* st = E.status + job;
+  if (st->halt) return;
+  const bool committed = mf < 0 || (!st->dt_bad && !solves_open(st, nsolve));
+  if (mf >= 0 && committed) {
+    // each 256-thread quarter stands for a block of k_commit
+    for (int k0 = 0; k0 < J.n; k0 += NT) {
+      const int k = k0 + threadIdx.x;
+      const bool in = k < J.n;
+      double h = 0., hu = 0., hv = 0.;
+      if (in) {
+        h = G(J.hres[mf])[k];
+        hu = G(J.hun[mf])[k];
+        hv = G(J.hvn[mf])[k];
+        G(J.h)[k] = h;
+        G(J.hu)[k] = hu;
+        G(J.hv)[k] = hv;
+      }
+      if (next_dt) timestep_wave(in, J.g, h, hu, hv, J.tspart + 3 * (k >> 6));
+    }
+  }
+  __shared__ int go_on;
+  __syncthreads();  // the maxima are written, and every thread has read the status
+  if (threadIdx.x < 64) {
+    record_step(st, nsolve);
+    if (threadIdx.x == 0) go_on = !st->halt;
+  }
+  __syncthreads();
+  if (next_dt && go_on) next_step_dt<NT>(J, st, mf >= 0 ? (J.n + 63) / 64 : J.nblk);
 }
 
 __global__ void k_set_steps_left(JobStatus* st, int steps_left) {
@@ -1576,9 +1686,9 @@ __global__ void k_set_steps_left(JobStatus* st, int steps_left) {
 // after it.  hres[2] and hres[3] are free: only node 1 is solved.
 __global__ __launch_bounds__(256) void k_hp_view(EngineArgs E, const TileRef* blocks,
                                                  int from_un) {
-  const TileRef T = blocks[blockIdx.x];
+  const TileRef T = tile_of(E, blocks, blockIdx.x);
   const JobDev& J = E.jobs[T.job];
-  if (skipped(E, J)) return;
+  if (skipped_stage(E, T.job)) return;
   const int k = T.tile * kCellBlock + threadIdx.x;
   if (k >= J.n) return;
   const gdouble* up2 = G(from_un ? J.h : J.hres[1]);
@@ -1601,12 +1711,12 @@ __device__ __forceinline__ const gdouble* deriv_var(const JobDev& J, int v, int 
 // kMaxTerms, guarded by nterm, so the values stay in registers) and serves
 // each of the op.nout outputs, which differ only in their weights.
 __global__ __launch_bounds__(256) void k_combine(EngineArgs E, const TileRef* blocks, CombOp op) {
-  const TileRef T = blocks[blockIdx.x];
+  const TileRef T = tile_of(E, blocks, blockIdx.x);
   const JobDev& J = E.jobs[T.job];
-  if (skipped(E, J)) return;
+  if (skipped_stage(E, T.job)) return;
   const int k = T.tile * kCellBlock + threadIdx.x;
   if (k >= J.n) return;
-  const double dt = J.status->dt;
+  const double dt = E.status[T.job].dt;
 #pragma unroll
   for (int v = 0; v < 3; ++v) {
     double x[kMaxTerms];
@@ -1651,7 +1761,7 @@ __global__ __launch_bounds__(256) void k_combine(EngineArgs E, const TileRef* bl
 // FXWB/FYWB from the slot scratch after the well-balanced FVTD.  The job's
 // cell blocks cover n indices; the loop also covers the nx (ny) extra faces.
 __global__ __launch_bounds__(256) void k_copy_wb(EngineArgs E, const TileRef* blocks, int slot) {
-  const TileRef T = blocks[blockIdx.x];
+  const TileRef T = tile_of(E, blocks, blockIdx.x);
   const JobDev& J = E.jobs[T.job];
   const int nfx = (J.nx + 1) * J.ny, nfy = J.nx * (J.ny + 1);
   for (int k = T.tile * kCellBlock + threadIdx.x; k < nfx || k < nfy;
@@ -1669,39 +1779,19 @@ __global__ __launch_bounds__(256) void k_copy_wb(EngineArgs E, const TileRef* bl
 // loop's clipping.
 // ------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_timestep(EngineArgs E, const TileRef* blocks) {
-  const TileRef T = blocks[blockIdx.x];
+  const TileRef T = tile_of(E, blocks, blockIdx.x);
   const JobDev& J = E.jobs[T.job];
-  if (skipped(E, J)) return;
+  if (skipped(E, T.job)) return;
   const int k = T.tile * kCellBlock + threadIdx.x;
   const bool in = k < J.n;
   timestep_partial(in, J.g, in ? G(J.h)[k] : 0., in ? G(J.hu)[k] : 0., in ? G(J.hv)[k] : 0.,
                    J.tspart + 3 * (size_t)T.tile);
 }
 
-__global__ __launch_bounds__(256) void k_timestep_final(EngineArgs E, const int* jobs) {
-  const JobDev& J = E.jobs[jobs[blockIdx.x]];
-  if (skipped(E, J)) return;
-  const gdouble *h = G(J.h), *hu = G(J.hu), *hv = G(J.hv);
-  double ts, LX, LY;
-  timestep_final(
-      J.tspart, J.nblk, J.n,
-      [&](int k, double& a, double& b, double& c) {
-        a = h[k];
-        b = hu[k];
-        c = hv[k];
-      },
-      J.g, J.dx, J.dy, J.cfl, ts, LX, LY);
-  if (threadIdx.x != 0) return;
-  JobStatus* st = J.status;
-  st->dt_min = ts;
-  // the time loop's dt = MIN(MIN(dt_min, tAnalyze-t), MIN(dt_min, tEnd-t))
-  // (src/timediscretization.f90:58-59) when the device runs the loop
-  const double dt =
-      st->loop ? min_r(min_r(ts, st->t_an - st->t), min_r(ts, st->t_end - st->t)) : ts;
-  st->dt = dt;
-  st->lmx = LX;
-  st->lmy = LY;
-  st->dt_bad = isfinite(dt) ? 0 : 1;
+__global__ __launch_bounds__(1024) void k_timestep_final(EngineArgs E, const int* jobs) {
+  const int job = job_of(E, jobs, blockIdx.x);
+  if (skipped(E, job)) return;
+  next_step_dt<1024>(E.jobs[job], E.status + job, E.jobs[job].nblk);
 }
 
 // ------------------------------------------------------------------------
@@ -1765,9 +1855,9 @@ __global__ void k_weno5(int n, const double* q, double* first, double* second) {
 // of that node's state for the jobs that asked for it (vout != null).
 // ------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_keep_state(EngineArgs E, const TileRef* blocks, int m) {
-  const TileRef T = blocks[blockIdx.x];
+  const TileRef T = tile_of(E, blocks, blockIdx.x);
   const JobDev& J = E.jobs[T.job];
-  if (skipped(E, J)) return;
+  if (skipped(E, T.job)) return;
   if (!J.vout) return;
   const int k = T.tile * kCellBlock + threadIdx.x;
   if (k >= J.n) return;
@@ -1859,11 +1949,11 @@ void launch_assemble_matrix(const EngineArgs& E, const TileRef* cb, int ncb, con
     hipLaunchKernelGGL((k_assemble<4, false>), grid, dim3(256), 0, s, E, cb, S);
 }
 
-void launch_solve(const EngineArgs& E, const SolveRef* refs, int nblk, const SysList& S, int limit,
-                  int first_solve, hipStream_t s) {
+void launch_solve(const EngineArgs& E, const SolveRef* refs, int first, int nblk, int form, int nb,
+                  const SysList& S, int limit, int first_solve, hipStream_t s) {
   if (nblk)
-    hipLaunchKernelGGL(k_solve, dim3(nblk), dim3(kSolveThreads), 0, s, E, refs, S, limit,
-                       first_solve);
+    hipLaunchKernelGGL(k_solve, dim3(nblk), dim3(kSolveThreads), 0, s, E, refs, first, form, nb, S,
+                       limit, first_solve);
 }
 
 void launch_finalize(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl, int njobs,
@@ -1877,16 +1967,20 @@ void launch_timestep(const EngineArgs& E, const TileRef* cb, int ncb, const int*
                      hipStream_t s) {
   if (!ncb) return;
   hipLaunchKernelGGL(k_timestep, dim3(ncb), dim3(256), 0, s, E, cb);
-  hipLaunchKernelGGL(k_timestep_final, dim3(njobs), dim3(256), 0, s, E, jl);
+  hipLaunchKernelGGL(k_timestep_final, dim3(njobs), dim3(1024), 0, s, E, jl);
 }
 
-void launch_commit(const EngineArgs& E, const TileRef* cb, int ncb, int final_node,
-                   hipStream_t s) {
-  if (ncb) hipLaunchKernelGGL(k_commit, dim3(ncb), dim3(256), 0, s, E, cb, final_node);
+void launch_commit(const EngineArgs& E, const TileRef* cb, int ncb, int final_node, int nsolve,
+                   int next_dt, hipStream_t s) {
+  if (ncb)
+    hipLaunchKernelGGL(k_commit, dim3(ncb), dim3(256), 0, s, E, cb, final_node, nsolve, next_dt);
 }
 
-void launch_gate(const EngineArgs& E, const int* jl, int njobs, int nsolve, hipStream_t s) {
-  if (njobs) hipLaunchKernelGGL(k_gate, dim3(njobs), dim3(64), 0, s, E, jl, nsolve);
+void launch_step_end(const EngineArgs& E, const int* jl, int njobs, int final_node, int nsolve,
+                     int next_dt, hipStream_t s) {
+  if (njobs)
+    hipLaunchKernelGGL(k_step_end, dim3(njobs), dim3(1024), 0, s, E, jl, final_node, nsolve,
+                       next_dt);
 }
 
 void launch_batch_begin(const EngineArgs& E, const int* jl, int njobs, const BatchArgs& B,

@@ -34,6 +34,29 @@ __device__ __forceinline__ double wave_max(double v) {
   return v;
 }
 
+// One cell (or none: in = false) per lane: lane 0 writes the wave's
+// (max a, max b, NaN seen) to p[0..2].
+__device__ __forceinline__ void timestep_wave(bool in, double g, double h, double hu, double hv,
+                                              double* p) {
+  double a = 0.0, b = 0.0, nan = 0.0;
+  if (in) {
+    wave_speeds(g, h, hu, hv, a, b);
+    if (isnan(a) || isnan(b)) {
+      nan = 1.0;
+      a = 0.0;
+      b = 0.0;
+    }
+  }
+  a = wave_max(a);
+  b = wave_max(b);
+  nan = wave_max(nan);
+  if ((threadIdx.x & 63) == 0) {
+    p[0] = a;
+    p[1] = b;
+    p[2] = nan;
+  }
+}
+
 // Block of 256 threads, one cell (or none: in = false) per thread: thread 0
 // writes the block's (max a, max b, NaN seen) to p[0..2].
 __device__ __forceinline__ void timestep_partial(bool in, double g, double h, double hu, double hv,
@@ -65,15 +88,16 @@ __device__ __forceinline__ void timestep_partial(bool in, double g, double h, do
   }
 }
 
-// One block of 256 threads over the nb partial triples part[3*t..3*t+2];
+// One block of NT threads over the nb partial triples part[3*t..3*t+2];
 // returns TimeStep's value (after the CFL factor and the MIN_TIMESTEP floor)
 // and the maxima LambdaMaxX/Y in thread 0.  cell(k, h, hu, hv) loads cell k
 // (0-based, x fastest) for the sequential replay when a speed was NaN.
-template <class Cell>
+template <int NT = 256, class Cell>
 __device__ __forceinline__ void timestep_final(const double* part, int nb, int n, Cell cell,
                                                double g, double dx, double dy, double cfl,
                                                double& ts_out, double& lx_out, double& ly_out) {
-  __shared__ double sa[4], sb[4], sn[4];
+  constexpr int NW = NT / 64;
+  __shared__ double sa[NW], sb[NW], sn[NW];
   double a = 0.0, b = 0.0, nan = 0.0;
   for (int t = threadIdx.x; t < nb; t += blockDim.x) {
     a = max_r(a, part[3 * (size_t)t]);
@@ -92,11 +116,12 @@ __device__ __forceinline__ void timestep_final(const double* part, int nb, int n
   __syncthreads();
   if (threadIdx.x != 0) return;
   double LX = 0.0, LY = 0.0;
-  for (int q = 0; q < 4; ++q) {
+  bool anynan = false;
+  for (int q = 0; q < NW; ++q) {
     LX = max_r(LX, sa[q]);
     LY = max_r(LY, sb[q]);
+    anynan = anynan || sn[q] != 0.0;
   }
-  const bool anynan = (sn[0] + sn[1] + sn[2] + sn[3]) != 0.0;
   double ts;
   if (!anynan) {
     ts = min_r(min_r(kHuge, dx / LX), dy / LY);
