@@ -374,10 +374,12 @@ constexpr int kSolveAlone = 2048;
 // k_solve's blocks for the jobs of T.  A grid is taken when the blocks of one
 // system fit the device at once (blocks of a system wait for each other); the
 // blocks of several systems share a launch as long as all of them fit.  The
-// systems with several blocks take the smallest tiles that need one launch,
-// else the largest: a larger tile makes a sweep and the assembly longer, a
-// further launch repeats all of it.  Blocks without others to wait for come
-// last and are not counted.
+// systems with several blocks take the tile size with the least launches times
+// launch time, kSolveUs (nine sweeps; 200 to 256 blocks): a larger tile makes
+// a sweep longer, a further launch repeats all of it.  Blocks without others
+// to wait for come last and are not counted.
+constexpr double kSolveUs[kSolveForms] = {24., 30., 50., 70.};
+
 void solve_tables(swm_engine* e, Tables& T) {
   const int cap = std::min(e->solve_blocks_max, 256);
   T.cbs.clear();
@@ -403,11 +405,24 @@ void solve_tables(swm_engine* e, Tables& T) {
     std::vector<SolveRef>& v = T.sv[c];
     v.clear();
     T.svl[c].clear();
-    int form = 0;
-    for (; form < kSolveForms - 1; ++form) {
-      long total = 0;
-      for (int id : shared) total += (long)nsys * blocks(id, form);
-      if (total <= cap) break;
+    int form = kSolveForms - 1;
+    double least = HUGE_VAL;
+    for (int f = 0; f < kSolveForms; ++f) {
+      int launches = 1, used = 0;
+      bool fits = true;
+      for (int id : shared)
+        for (int s = 0, nb = blocks(id, f); s < nsys; ++s) {
+          fits = fits && nb <= cap;
+          if (used + nb > cap) {
+            ++launches;
+            used = 0;
+          }
+          used += nb;
+        }
+      if (fits && launches * kSolveUs[f] < least) {
+        least = launches * kSolveUs[f];
+        form = f;
+      }
     }
     int first = 0;
     for (int id : shared) {

@@ -506,6 +506,21 @@ __global__ __launch_bounds__(XW * XH, 4) void k_fvtd(EngineArgs E, FvtdTiles T, 
     y_faces<YW, YH>(smem, irregular, J, R.tile, L.m[node], L.slot[node], L);
 }
 
+// Divisions by a job's dx and dy through one reciprocal each.
+struct OverDx {
+  double dx, dy, rdx, rdy;
+  bool shared;
+  __device__ __forceinline__ explicit OverDx(const JobDev& J)
+      : dx(J.dx), dy(J.dy), rdx(recip_refined(J.dx)), rdy(recip_refined(J.dy)),
+        shared(recip_range(J.dx) & recip_range(J.dy)) {}
+  __device__ __forceinline__ double x(double a) const {
+    return shared ? div_pos(a, dx, rdx) : a / dx;
+  }
+  __device__ __forceinline__ double y(double a) const {
+    return shared ? div_pos(a, dy, rdy) : a / dy;
+  }
+};
+
 // ------------------------------------------------------------------------
 // UpdateTimeDerivative (src/finitevolume.f90:446-540) of cell k = (ci, cj) from
 // the fluxes in `slot` and its source S, into derivative slot o.
@@ -533,19 +548,14 @@ __device__ __forceinline__ void update_cell(const JobDev& J, const NodeList& L, 
     fyn[v] = G(J.FY[slot][v])[gn];
     fys[v] = G(J.FY[slot][v])[gs];
   }
-  // the divisions by dx and dy share one reciprocal each (uniform per job)
-  const double dx = J.dx, dy = J.dy;
-  const bool shared = recip_range(dx) & recip_range(dy);
-  const double rdx = recip_refined(dx), rdy = recip_refined(dy);
-  auto over_dx = [&](double a) { return shared ? div_pos(a, dx, rdx) : a / dx; };
-  auto over_dy = [&](double a) { return shared ? div_pos(a, dy, rdy) : a / dy; };
+  const OverDx over(J);
   // Ut(2:3) = S - (FX(i)-FX(i-1))/dx - (FY(j)-FY(j-1))/dy  (:525-527)
-  const double ut2 = S2 - over_dx(fxe[1] - fxw[1]) - over_dy(fyn[1] - fys[1]);
-  const double ut3 = S3 - over_dx(fxe[2] - fxw[2]) - over_dy(fyn[2] - fys[2]);
+  const double ut2 = S2 - over.x(fxe[1] - fxw[1]) - over.y(fyn[1] - fys[1]);
+  const double ut3 = S3 - over.x(fxe[2] - fxw[2]) - over.y(fyn[2] - fys[2]);
   if (L.ut1) {
     // the build without PATANKAR: Ut(1:3) (:529-533), with S(1) = 0 exactly
     // (SourceFunc's first component is 0., src/equation.f90:408)
-    G(J.d1[o])[k] = 0.0 - over_dx(fxe[0] - fxw[0]) - over_dy(fyn[0] - fys[0]);
+    G(J.d1[o])[k] = 0.0 - over.x(fxe[0] - fxw[0]) - over.y(fyn[0] - fys[0]);
     G(J.d2[o])[k] = ut2;
     G(J.d3[o])[k] = ut3;
     return;
@@ -554,10 +564,10 @@ __device__ __forceinline__ void update_cell(const JobDev& J, const NodeList& L, 
   G(J.d3[o])[k] = ut3;
   // mass flux per face / dx: the production/destruction entries of
   // src/finitevolume.f90:496-523 are max(+-q, 0) and -min(+-q, 0) of these.
-  G(J.qx[o])[fe] = over_dx(fxe[0]);
-  G(J.qy[o])[gn] = over_dy(fyn[0]);
-  if (ci == 0) G(J.qx[o])[fw] = over_dx(fxw[0]);
-  if (cj == 0) G(J.qy[o])[gs] = over_dy(fys[0]);
+  G(J.qx[o])[fe] = over.x(fxe[0]);
+  G(J.qy[o])[gn] = over.y(fyn[0]);
+  if (ci == 0) G(J.qx[o])[fw] = over.x(fxw[0]);
+  if (cj == 0) G(J.qy[o])[gs] = over.y(fys[0]);
 }
 
 // The update alone, one cell per thread, blockIdx.y = node; the sources of
@@ -1109,6 +1119,7 @@ __device__ __forceinline__ double wave_sum_dpp(double v) {
 
 constexpr int kSolveRows = 11 * kSolveThreads;  // rows of the largest tile with its halo
 constexpr int kSolveWaves = kSolveThreads / 64;
+static_assert(kSolveWaves == 8 && kSolveKinds <= 8, "the stop rule's lanes");
 
 struct SolveShared {
   double x[3][kSolveRows];  // the iterate: the window's start and two buffers
@@ -1300,21 +1311,36 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
         break;
       }
     }
-    auto total = [&](int q) {
-      double v;
-      if (ALONE) {
-        v = L.red[q][0];
-        for (int w = 1; w < kSolveWaves; ++w) v += L.red[q][w];
-      } else {
-        v = ((L.tot[q][0] + L.tot[q][1]) + L.tot[q][2]) + L.tot[q][3];
-      }
-      return v;
+    // the halo of the next window, on its way while the stop rule is applied
+    double halo[ALONE ? 1 : RPT];
+    if (!ALONE) {
+#pragma unroll
+      for (int i = 0; i < RPT; ++i)
+        if (i * NT + tid < rows && !((own >> i) & 1u))
+          halo[ALONE ? 0 : i] = agent_load(buf + gk[i]);
+    }
+    // The stop rule (src/jacobi_iteration.f90:63-84), sweep by sweep: the same
+    // numbers, and so the same decisions, in every block of the system.  Lane
+    // 8q + w of each wave takes part w of sum q; its group of 8 lanes adds
+    // them up, and the decisions of all sums come as bits of two ballots.
+    double part = 0.;
+    if (ALONE) {
+      if ((tid & 63) < 8 * kSolveKinds) part = L.red[(tid & 63) >> 3][tid & 7];
+    } else {
+      if ((tid & 63) < 8 * kSolveKinds && (tid & 7) < 4) part = L.tot[(tid & 63) >> 3][tid & 3];
+    }
+    part += dpp<0x111, 0xf>(part);
+    part += dpp<0x112, 0xf>(part);
+    part += dpp<0x114, 0xf>(part);  // lane 8q + 7 (and 8q + 15 of a row) holds its eight
+    const int c = certified(part);
+    const unsigned long long go = __ballot(c > 0), open = __ballot(c < 0);
+    auto decision = [&](int q) {
+      const int bit = 8 * q + 7;
+      return (int)((go >> bit) & 1u) - (int)((open >> bit) & 1u);
     };
-    // the stop rule (src/jacobi_iteration.f90:63-84), sweep by sweep: the same
-    // numbers, and so the same decisions, in every block of the system
     bool stop = false;
     if (t == 0) {
-      const int c0 = certified(total(kSolveWindow));
+      const int c0 = decision(kSolveWindow);
       if (c0 < 0) {
         stop = true;
         end = kSolveOpen;
@@ -1327,7 +1353,7 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
     int j = 0;
     for (; j < kSolveWindow && !stop; ++j) {
       ++k_sweeps;
-      const int c1 = certified(total(j));
+      const int c1 = decision(j);
       stop = true;
       if (c1 < 0)
         end = kSolveOpen;
@@ -1358,12 +1384,9 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
       break;
     }
     if (!ALONE) {
-      // the halo of the next window
 #pragma unroll
-      for (int i = 0; i < RPT; ++i) {
-        const int l = i * NT + tid;
-        if (l < rows && !((own >> i) & 1u)) q1[l] = agent_load(buf + gk[i]);
-      }
+      for (int i = 0; i < RPT; ++i)
+        if (i * NT + tid < rows && !((own >> i) & 1u)) q1[i * NT + tid] = halo[ALONE ? 0 : i];
     }
     __syncthreads();  // also: the sums have been read
     double* w = p0;
