@@ -536,7 +536,9 @@ EngineArgs eargs(swm_engine* e, const Tables& T) {
 // launch.  The device holds 262,144 at 4 waves per SIMD.
 constexpr long kFvtdTogether = 8L * 262144;
 
-int fvtd_launch(swm_engine* e, Tables& T, const NodeList& L) {
+// fluxes_left, where an assembly for k_solve follows: set when the update is
+// left to it (SysList::fresh).
+int fvtd_launch(swm_engine* e, Tables& T, const NodeList& L, int* fluxes_left = nullptr) {
   EngineArgs a = eargs(e, T);
   hipStream_t s = e->stream;
   const int sh = e->cur_shape;
@@ -546,7 +548,10 @@ int fvtd_launch(swm_engine* e, Tables& T, const NodeList& L) {
   const bool small = (long)(nxt + nyt) * L.count * F.xw * F.xh <= kFvtdTogether;
   if (small && !(e->prof.mask & 7u)) {
     launch_fvtd(a, sh, xt, nxt, yt, nyt, st, nst, L, s);
-    launch_fvtd_update(a, T.dcb, T.ncb, L, s);
+    if (fluxes_left)
+      *fluxes_left = 1;
+    else
+      launch_fvtd_update(a, T.dcb, T.ncb, L, s);
   } else {  // also while events tell the kinds apart
     timed(e, 0, [&] { launch_fvtd(a, sh, xt, nxt, nullptr, 0, nullptr, 0, L, s); });
     timed(e, 1, [&] { launch_fvtd(a, sh, nullptr, 0, yt, nyt, nullptr, 0, L, s); });
@@ -855,7 +860,8 @@ int step_body(swm_engine* e, Tables& T, const StepPlan& P) {
         L.out[k] = S.m[k];
         L.slot[k] = k;
       }
-      rc = fvtd_launch(e, T, L);
+      S.fresh = 0;
+      rc = fvtd_launch(e, T, L, P.solve && T.ncbw == 0 ? &S.fresh : nullptr);
       if (rc) return rc;
       if (e->keep_count && kk == D.kcorr - 1)
         launch_keep_state(a, T.dcb, T.ncb, D.msteps - 1, s);

@@ -278,6 +278,8 @@ struct SysList {
   int nr;               // thetaDeC columns summed (MSteps): 4 or 2
   int theta;            // THETA block: 0 mPDeC5, 1 the two-node schemes
   int hp_view;          // 1: denominators from hres[3], rhs from hres[2] (k_hp_view)
+  int fresh;            // 1: nodes 1.. have their fluxes in slots 0.. and their sources in
+                        // d2, d3, and the assembly takes Ut and the mass fluxes from those
 };
 
 // The time schemes, by the reference's timescheme number: the modified-

@@ -521,6 +521,17 @@ struct OverDx {
   }
 };
 
+// Whether div_by may take every numerator seen: 0 or in [2^-400, 2^400]; the
+// sign of a zero quotient is not kept.
+struct Numerators {
+  bool ok;
+  __device__ __forceinline__ double operator()(double a) {
+    const double m = fabs(a);
+    ok = ok & (((int)(m >= kRecipLo) & (int)(m <= kRecipHi)) | (int)(a == 0.));
+    return a;
+  }
+};
+
 // ------------------------------------------------------------------------
 // UpdateTimeDerivative (src/finitevolume.f90:446-540) of cell k = (ci, cj) from
 // the fluxes in `slot` and its source S, into derivative slot o.
@@ -633,13 +644,8 @@ __global__ __launch_bounds__(256) void k_fvtd_source_update(EngineArgs E, const 
 // assembly's latency-bound work.
 template <int R>
 __device__ __forceinline__ void momentum_cell(const JobDev& J, const SysList& S, int s0, int s1,
-                                              int k, double dt) {
-  double fu2[R], fu3[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    fu2[r] = G(J.FU2[S.src[r]])[k];
-    fu3[r] = G(J.FU3[S.src[r]])[k];
-  }
+                                              int k, double dt, const double fu2[R],
+                                              const double fu3[R]) {
   const double u0 = G(J.hu)[k], v0 = G(J.hv)[k];
   for (int s = s0; s < s1; ++s) {
     const int m = S.m[s];
@@ -654,6 +660,84 @@ __device__ __forceinline__ void momentum_cell(const JobDev& J, const SysList& S,
     G(J.hvn[m])[k] = v;
   }
 }
+
+// What the assembly and the momentum update of a cell take from the FVTDs: the
+// mass fluxes / dx of its south, west, east and north faces at the R DeC nodes
+// and Ut(2:3).  Node 0's are kept by k_fvtd_update for all corrections.  With
+// FRESH the other nodes' are formed here from the face fluxes and the source
+// (as update_cell does), for a launch less per correction; all loads go out
+// before the first quotient.
+template <int R, bool FRESH>
+struct CellFluxes {
+  double q[4][R], fu2[R], fu3[R];
+  __device__ __forceinline__ CellFluxes(const JobDev& J, const SysList& S, int k, size_t fW,
+                                        size_t gS) {
+    const size_t fE = fW + 1, gN = gS + J.nx;
+    constexpr int R1 = FRESH ? R : 1;
+    double X[R1][2][2], Y[R1][2][2];  // [node][variable 2, 3][face]
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const bool here = FRESH && r > 0;
+      const gdouble* qx = G(here ? J.FX[r - 1][0] : J.qx[S.src[r]]);
+      const gdouble* qy = G(here ? J.FY[r - 1][0] : J.qy[S.src[r]]);
+      q[0][r] = qy[gS];
+      q[1][r] = qx[fW];
+      q[2][r] = qx[fE];
+      q[3][r] = qy[gN];
+      if (!here) {
+        fu2[r] = G(J.FU2[S.src[r]])[k];
+        fu3[r] = G(J.FU3[S.src[r]])[k];
+      } else {
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+          X[r % R1][v][0] = G(J.FX[r - 1][v + 1])[fW];
+          X[r % R1][v][1] = G(J.FX[r - 1][v + 1])[fE];
+          Y[r % R1][v][0] = G(J.FY[r - 1][v + 1])[gS];
+          Y[r % R1][v][1] = G(J.FY[r - 1][v + 1])[gN];
+        }
+        fu2[r] = fu3[r] = 0.0;
+        if (J.bathy) {
+          fu2[r] = G(J.d2[r])[k];
+          fu3[r] = G(J.d3[r])[k];
+        } else if (J.wb) {
+          fu2[r] = 0.0 - G(J.SWB2)[k];
+          fu3[r] = 0.0 - G(J.SWB3)[k];
+        }
+      }
+    }
+    if (!FRESH) return;
+    const OverDx over(J);
+    Numerators seen{over.shared};
+    double dX[R1][2], dY[R1][2];
+#pragma unroll
+    for (int r = 1; r < R; ++r) {
+      for (int f = 0; f < 4; ++f) seen(q[f][r]);
+#pragma unroll
+      for (int v = 0; v < 2; ++v) {
+        dX[r % R1][v] = seen(X[r % R1][v][1] - X[r % R1][v][0]);
+        dY[r % R1][v] = seen(Y[r % R1][v][1] - Y[r % R1][v][0]);
+      }
+    }
+    auto form = [&](auto ox, auto oy) {
+#pragma unroll
+      for (int r = 1; r < R; ++r) {
+        q[0][r] = oy(q[0][r]);
+        q[1][r] = ox(q[1][r]);
+        q[2][r] = ox(q[2][r]);
+        q[3][r] = oy(q[3][r]);
+        fu2[r] = fu2[r] - ox(dX[r % R1][0]) - oy(dY[r % R1][0]);
+        fu3[r] = fu3[r] - ox(dX[r % R1][1]) - oy(dY[r % R1][1]);
+      }
+    };
+    // The signs of zero quotients reach nothing: the sources are not -0, and
+    // the mass fluxes are compared with 0 and taken by magnitude.
+    if (__all(seen.ok))
+      form([&](double a) { return div_by(a, over.dx, over.rdx); },
+           [&](double a) { return div_by(a, over.dy, over.rdy); });
+    else
+      form([&](double a) { return over.x(a); }, [&](double a) { return over.y(a); });
+  }
+};
 
 // ------------------------------------------------------------------------
 // Reductions
@@ -833,7 +917,7 @@ __device__ __forceinline__ const gdouble* system_rhs(const JobDev& J, const SysL
 // FIRST: the first sweep and its residual sums, for a launch per sweep; without
 // it only the matrix, for k_solve.  blockIdx.y picks the system where the grid
 // has that dimension (launch_assemble_matrix), else the block does them all.
-template <int R, bool FIRST>
+template <int R, bool FIRST, bool FRESH = false>
 __global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* blocks,
                                                   SysList S) {
   __shared__ double red[4];
@@ -857,14 +941,13 @@ __global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* b
     kW = j * nx + (i == 0 ? nx - 1 : i - 1);
     kE = j * nx + (i == nx - 1 ? 0 : i + 1);
     kN = (j == ny - 1 ? 0 : j + 1) * nx + i;
-    const size_t fW = (size_t)j * (nx + 1) + i, fE = fW + 1;
-    const size_t gS = (size_t)j * nx + i, gN = gS + nx;
+    const CellFluxes<R, FRESH> F(J, S, k, (size_t)j * (nx + 1) + i, (size_t)j * nx + i);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      sq[(0 * R + r) * 256 + tid] = G(J.qy[S.src[r]])[gS];
-      sq[(1 * R + r) * 256 + tid] = G(J.qx[S.src[r]])[fW];
-      sq[(2 * R + r) * 256 + tid] = -G(J.qx[S.src[r]])[fE];  // east and north slots:
-      sq[(3 * R + r) * 256 + tid] = -G(J.qy[S.src[r]])[gN];  // the flux oriented into the cell
+      sq[(0 * R + r) * 256 + tid] = F.q[0][r];
+      sq[(1 * R + r) * 256 + tid] = F.q[1][r];
+      sq[(2 * R + r) * 256 + tid] = -F.q[2][r];  // east and north slots: the flux
+      sq[(3 * R + r) * 256 + tid] = -F.q[3][r];  // oriented into the cell
     }
     const gdouble* rhs = system_rhs(J, S);
     if (FIRST) {
@@ -874,7 +957,7 @@ __global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* b
       bE = rhs[kE];
       bN = rhs[kN];
     }
-    momentum_cell<R>(J, S, s0, s1, k, dt);
+    momentum_cell<R>(J, S, s0, s1, k, dt, F.fu2, F.fu3);
   }
   // One system at a time, and within it one stencil slot at a time (S, W, E,
   // N: the CSR order), so that only one slot's divisions are live.  Each
@@ -1966,8 +2049,12 @@ void launch_assemble_matrix(const EngineArgs& E, const TileRef* cb, int ncb, con
                             hipStream_t s) {
   if (!ncb) return;
   const dim3 grid(ncb, ncb < 1024 ? S.count : 1);
-  if (S.nr == 2)
+  if (S.nr == 2 && S.fresh)
+    hipLaunchKernelGGL((k_assemble<2, false, true>), grid, dim3(256), 0, s, E, cb, S);
+  else if (S.nr == 2)
     hipLaunchKernelGGL((k_assemble<2, false>), grid, dim3(256), 0, s, E, cb, S);
+  else if (S.fresh)
+    hipLaunchKernelGGL((k_assemble<4, false, true>), grid, dim3(256), 0, s, E, cb, S);
   else
     hipLaunchKernelGGL((k_assemble<4, false>), grid, dim3(256), 0, s, E, cb, S);
 }
