@@ -139,12 +139,12 @@ struct DevVec {
 struct Tables {
   // k_fvtd's tiles per shape: x faces, y faces, sources; k_fvtd_source_update's
   // tiles; cell blocks; jobs
-  std::vector<TileRef> xt[kNumShapes], yt[kNumShapes], st[kNumShapes], ct, cb;
+  std::vector<TileRef> xt[kAllShapes], yt[kAllShapes], st[kAllShapes], ct, cb;
   std::vector<int> jl;
-  TileRef *dxt[kNumShapes] = {}, *dyt[kNumShapes] = {}, *dst[kNumShapes] = {};
+  TileRef *dxt[kAllShapes] = {}, *dyt[kAllShapes] = {}, *dst[kAllShapes] = {};
   TileRef *dct = nullptr, *dcb = nullptr;
   int* djl = nullptr;
-  int nxt[kNumShapes] = {}, nyt[kNumShapes] = {}, nst[kNumShapes] = {};
+  int nxt[kAllShapes] = {}, nyt[kAllShapes] = {}, nst[kAllShapes] = {};
   int nct = 0, ncb = 0, njobs = 0;
   // The Patankar solves: k_solve's blocks for launches of one and of kMaxSys
   // systems, cut into launches (first block, blocks); and the cell blocks and
@@ -315,14 +315,14 @@ void timed(swm_engine* e, int cat, F&& launch) {
 
 void add_sources(Tables& T, int id, const JobDev& d) {
   if (!d.bathy) return;
-  for (int sh = 0; sh < kNumShapes; ++sh) {
+  for (int sh = 0; sh < kAllShapes; ++sh) {
     const int nst = cdiv(d.nx, kShapes[sh].sw) * cdiv(d.ny, kShapes[sh].sh);
     for (int t = 0; t < nst; ++t) T.st[sh].push_back({id, t});
   }
 }
 
 void add_tiles(Tables& T, int id, const JobDev& d) {
-  for (int sh = 0; sh < kNumShapes; ++sh) {
+  for (int sh = 0; sh < kAllShapes; ++sh) {
     const FaceShape& F = kShapes[sh];
     const int nxt = cdiv(d.nx + 1, F.xw - 1) * cdiv(d.ny, F.xh);
     const int nyt = cdiv(d.nx, F.yw) * cdiv(d.ny + 1, F.yh - 1);
@@ -457,7 +457,7 @@ int upload_tables(swm_engine* e, Tables& T) {
     where.push_back({(void**)&dev, off});
     return (int)v.size();
   };
-  for (int sh = 0; sh < kNumShapes; ++sh) {
+  for (int sh = 0; sh < kAllShapes; ++sh) {
     T.nxt[sh] = put(T.dxt[sh], T.xt[sh]);
     T.nyt[sh] = put(T.dyt[sh], T.yt[sh]);
     T.nst[sh] = put(T.dst[sh], T.st[sh]);
@@ -486,7 +486,7 @@ int refresh(swm_engine* e) {
   for (size_t i = 0; i < nj; ++i) host[i] = e->jobs[i]->dev;
   if (nj) HIPCK(e, hipMemcpy(e->djobs.p, host.data(), nj * sizeof(JobDev), hipMemcpyHostToDevice));
   for (Tables& T : e->groups) {
-    for (int sh = 0; sh < kNumShapes; ++sh) {
+    for (int sh = 0; sh < kAllShapes; ++sh) {
       T.xt[sh].clear();
       T.yt[sh].clear();
       T.st[sh].clear();
@@ -536,16 +536,23 @@ EngineArgs eargs(swm_engine* e, const Tables& T) {
 // launch.  The device holds 262,144 at 4 waves per SIMD.
 constexpr long kFvtdTogether = 8L * 262144;
 
+// 16x16 face tiles of a launch up to which two lanes share a cell (split_faces):
+// about one per CU.
+constexpr int kSplitTiles = 256;
+
 // fluxes_left, where an assembly for k_solve follows: set when the update is
 // left to it (SysList::fresh).
 int fvtd_launch(swm_engine* e, Tables& T, const NodeList& L, int* fluxes_left = nullptr) {
   EngineArgs a = eargs(e, T);
   hipStream_t s = e->stream;
-  const int sh = e->cur_shape;
+  int sh = e->cur_shape;
+  if (e->tile_shape < 0 && !(e->prof.mask & 7u) &&
+      (T.nxt[0] + T.nyt[0]) * L.count <= kSplitTiles)
+    sh = kSplitShape;
   const TileRef *xt = T.dxt[sh], *yt = T.dyt[sh], *st = T.dst[sh];
   const int nxt = T.nxt[sh], nyt = T.nyt[sh], nst = T.nst[sh];
   const FaceShape& F = kShapes[sh];
-  const bool small = (long)(nxt + nyt) * L.count * F.xw * F.xh <= kFvtdTogether;
+  const bool small = (long)(nxt + nyt) * L.count * F.sw * F.sh <= kFvtdTogether;
   if (small && !(e->prof.mask & 7u)) {
     launch_fvtd(a, sh, xt, nxt, yt, nyt, st, nst, L, s);
     if (fluxes_left)
@@ -925,7 +932,7 @@ int step_body_graph(swm_engine* e, Tables& T, const StepPlan& P) {
   auto& c = *cp;
   bool same = c.exec && c.epoch == e->graph_epoch && c.device_dt == (int)P.device_dt &&
               c.track == (int)e->track_min && c.tables == (const void*)&T && c.group == group &&
-              c.shape == e->cur_shape && c.solve == (int)P.solve;
+              c.shape == e->cur_shape + kAllShapes * (e->tile_shape < 0) && c.solve == (int)P.solve;
   for (int i = 0; same && i < 5; ++i)
     same = c.sweeps[i] == P.sweeps[i] && c.limit[i] == P.limit[i];
   c.used = ++e->cap_clock;
@@ -951,7 +958,7 @@ int step_body_graph(swm_engine* e, Tables& T, const StepPlan& P) {
     c.track = e->track_min;
     c.tables = &T;
     c.group = group;
-    c.shape = e->cur_shape;
+    c.shape = e->cur_shape + kAllShapes * (e->tile_shape < 0);
     c.solve = P.solve;
     for (int i = 0; i < 5; ++i) {
       c.sweeps[i] = P.sweeps[i];

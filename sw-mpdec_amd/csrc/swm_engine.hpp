@@ -35,8 +35,12 @@ struct FaceShape {
   int xw, xh, yw, yh, sw, sh;
 };
 constexpr int kNumShapes = 2;
-constexpr FaceShape kShapes[kNumShapes] = {{16, 16, 16, 16, 16, 16},
-                                            {32, 16, 16, 32, 32, 16}};
+// The last shape is not for choosing: two lanes per cell on half tiles, for
+// launches that leave most of the device idle (kSplitTiles).
+constexpr int kAllShapes = kNumShapes + 1, kSplitShape = kNumShapes;
+constexpr FaceShape kShapes[kAllShapes] = {{16, 16, 16, 16, 16, 16},
+                                           {32, 16, 16, 32, 32, 16},
+                                           {16, 8, 8, 16, 16, 16}};
 constexpr int kCellBlock = 256;       // cells per block of the pointwise kernels
 constexpr int kSolveThreads = 512;    // threads of a k_solve block
 constexpr int kSolveWindow = 4;       // Jacobi sweeps between two exchanges of k_solve's blocks

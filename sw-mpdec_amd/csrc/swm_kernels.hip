@@ -88,6 +88,15 @@ __device__ __forceinline__ void cell_ij(int i0, int j0, int t, int nx, int& i, i
   }
 }
 
+// v of the lane that CTRL of the DPP encoding names; 0 where there is none, and
+// in the rows of 16 lanes left out of ROWS.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
 __device__ __forceinline__ int cdiv_d(int a, int b) { return (a + b - 1) / b; }
 
 // In the steps of a batch (E.gated) a job whose batch has stopped
@@ -150,8 +159,31 @@ struct FaceTile {
 };
 
 // Gauss sum of the Rusanov fluxes of one face (src/finitevolume.f90:546-640)
-// between WP of the cell below the face and wm of the one above it (value a
-// of 12 at wm[a * stride]).  The regular form holds for finite states with
+// with the reference's operations one by one, between WP of the cell below the
+// face and wm of the one above it (value a of 12 at wm[a * stride]).
+template <bool X>
+__device__ __forceinline__ void face_flux_general(const JobDev& J, const double WP[3][4],
+                                                  const double* wm, int stride, double& acc1,
+                                                  double& acc2, double& acc3) {
+  acc1 = acc2 = acc3 = 0.0;
+#pragma unroll 1
+  for (int g = 0; g < 4; ++g) {
+    double F1, F2, F3;
+    // the Gauss point's values by selects: WP stays in registers
+    double wp[3];
+#pragma unroll
+    for (int v = 0; v < 3; ++v)
+      wp[v] = g == 0 ? WP[v][0] : g == 1 ? WP[v][1] : g == 2 ? WP[v][2] : WP[v][3];
+    rusanov<X ? 1 : 0, X ? 0 : 1, X ? 0 : -1, X ? 1 : 0>(wp[0], wp[1], wp[2], wm[g * stride],
+                                                         wm[(4 + g) * stride],
+                                                         wm[(8 + g) * stride], J.g, F1, F2, F3);
+    acc1 = acc1 + J.wbnd[g] * F1;
+    acc2 = acc2 + J.wbnd[g] * F2;
+    acc3 = acc3 + J.wbnd[g] * F3;
+  }
+}
+
+// The same sum.  The regular form holds for finite states with
 // depths in range (irregular = 0); a state that is not finite shows in one of
 // its sums, and the face is then taken again with the reference's operations
 // one by one.
@@ -176,22 +208,7 @@ __device__ __forceinline__ void face_flux(const JobDev& J, const double WP[3][4]
     acc3 = X ? at : an;
     if ((int)is_finite(a1) & (int)is_finite(an) & (int)is_finite(at)) return;
   }
-  acc1 = acc2 = acc3 = 0.0;
-#pragma unroll 1
-  for (int g = 0; g < 4; ++g) {
-    double F1, F2, F3;
-    // the Gauss point's values by selects: WP stays in registers
-    double wp[3];
-#pragma unroll
-    for (int v = 0; v < 3; ++v)
-      wp[v] = g == 0 ? WP[v][0] : g == 1 ? WP[v][1] : g == 2 ? WP[v][2] : WP[v][3];
-    rusanov<X ? 1 : 0, X ? 0 : 1, X ? 0 : -1, X ? 1 : 0>(wp[0], wp[1], wp[2], wm[g * stride],
-                                                         wm[(4 + g) * stride],
-                                                         wm[(8 + g) * stride], J.g, F1, F2, F3);
-    acc1 = acc1 + J.wbnd[g] * F1;
-    acc2 = acc2 + J.wbnd[g] * F2;
-    acc3 = acc3 + J.wbnd[g] * F3;
-  }
+  face_flux_general<X>(J, WP, wm, stride, acc1, acc2, acc3);
 }
 
 template <int TW, int TH>
@@ -382,6 +399,186 @@ __device__ __forceinline__ void y_faces(double* smem, int& irregular, const JobD
 }
 
 // ------------------------------------------------------------------------
+// The faces of small grids, x (X) or y: two lanes per cell, one for the values
+// at its lower face (WM) and one for those at its upper face (WP), on half
+// tiles of 16 cells along the faces' normal (a) and 8 across (b).  Where a
+// launch has fewer tiles than the device has CUs the time is that of one wave
+// (a 16x16 tile: 1.3 us of loads, 1.9 of first sweeps, 4.7 of second sweeps,
+// 1.8 of limiter and fluxes); here a lane has three second sweeps instead of
+// six and two of the four Gauss points' fluxes, and idle CUs take the second
+// half of the tile.  The lanes of a cell are neighbours, and so are the two
+// lanes of a face (WP of cell a, WM of cell a + 1).
+// ------------------------------------------------------------------------
+constexpr int kSplitA = 16, kSplitB = 8;
+constexpr int kDppPair = 0xB1;     // quad_perm [1,0,3,2]: the cell's other lane
+constexpr int kDppNext = 0x130;    // wave_shl:1: the next lane
+
+// positivity_limit with wm in even lanes (side 0) and wp in odd ones.
+__device__ __forceinline__ double positivity_limit_pair(double vh, const double wbnd[4],
+                                                        double w[4], int side) {
+  double sum = wbnd[0] * w[0], mn = w[0];
+#pragma unroll
+  for (int g = 1; g < 4; ++g) {
+    sum = sum + wbnd[g] * w[g];
+    mn = min_n(mn, w[g]);
+  }
+  const double other = dpp<kDppPair, 0xf>(sum);
+  const double alpha = side ? other : sum, beta = side ? sum : other;
+  constexpr double c = 1. - 2. * kWLobatto;
+  const double csi = div_pos(vh - kWLobatto * alpha - kWLobatto * beta, c, 1. / c);
+  mn = min_n(min_n(mn, dpp<kDppPair, 0xf>(mn)), csi);
+  const double num = vh - kMinDepth;
+  double theta[4] = {1., 1., 1., 1.};
+  // the same numbers, and so the same branch, in both lanes of the cell
+  if (!((int)(fabs(num) >= fabs(vh - csi)) & (int)(fabs(num) >= fabs(vh - mn)))) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const double o = dpp<kDppPair, 0xf>(w[g]);
+      const double mmin = min_r(min_r(csi, side ? o : w[g]), side ? w[g] : o);
+      const double den = vh - mmin;
+      if (vh == mmin)
+        theta[g] = 1.;
+      else if ((int)(fabs(num) >= fabs(den)) & (int)(fabs(num) <= kHuge))
+        theta[g] = 1.;
+      else
+        theta[g] = min_r(1., fabs(num / den));
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < 4; ++g) w[g] = vh + theta[g] * (w[g] - vh);
+  return mn;
+}
+
+template <bool X>
+__device__ __forceinline__ void split_faces(double* smem, int& irregular, const JobDev& J,
+                                            int tile, int m, int slot, const NodeList& L) {
+  constexpr int TA = kSplitA, TB = kSplitB, NT = 2 * TA * TB;
+  constexpr int VA = TA + 4, VB = TB + 4, NV = VA * VB, NQ = VB * TA;
+  double* sV = smem;            // [3][VB][VA]
+  double* sQM = smem + 3 * NV;  // [3][VB][TA]
+  double* sQP = sQM + 3 * NQ;
+  const int nx = J.nx, ny = J.ny, na = X ? nx : ny, nb = X ? ny : nx;
+  const int nta = cdiv_d(na + 1, TA - 1);
+  const int tid = threadIdx.x, side = tid & 1, ca = (tid >> 1) % TA, cb = (tid >> 1) / TA;
+  const int a0 = (tile % nta) * (TA - 1), b0 = (tile / nta) * TB + 1;
+  const gdouble *h, *hu, *hv;
+  node_state(J, m, h, hu, hv);
+  if (tid == 0) irregular = !(J.g >= 0x1p-60 && J.g <= 0x1p60);
+
+  if (tid < NV) {
+    // x fastest
+    const int va = X ? tid % VA : tid / VB, vb = X ? tid / VA : tid % VB;
+    const int ia = wrap1(a0 - 2 + va, na), ib = wrap1(b0 - 2 + vb, nb);
+    const size_t k = X ? (size_t)ib * nx + ia : (size_t)ia * nx + ib;
+    double hh = h[k], u, v;
+    cons_to_prim(hh, hu[k], hv[k], u, v);
+    const int t = vb * VA + va;
+    sV[t] = hh;
+    sV[NV + t] = u;
+    sV[2 * NV + t] = v;
+  }
+  static_assert(NV <= NT, "one cell of the halo tile per thread");
+  __syncthreads();
+  for (int t = tid; t < 3 * NQ; t += NT) {
+    const int var = t / NQ, r = t % NQ;
+    const double* q = sV + var * NV + (r / TA) * VA + r % TA;
+    double wm, wp;
+    weno5_first(q[0], q[1], q[2], q[3], q[4], wm, wp);
+    sQM[t] = wm;
+    sQP[t] = wp;
+  }
+  __syncthreads();
+  double W[3][4];
+#pragma unroll
+  for (int var = 0; var < 3; ++var) {
+    const double* q = (side ? sQP : sQM) + var * NQ + cb * TA + ca;
+    weno5_second(q[0], q[TA], q[2 * TA], q[3 * TA], q[4 * TA], W[var]);
+  }
+  const int c = a0 + ca;
+  const double* cell = sV + (cb + 2) * VA + ca + 2;
+  if (J.recfix) {  // as in x_faces
+    const double* hrow = sV + (cb + 2) * VA;
+    const int lc = min(c + 1, na) - a0 + 2;
+    if (jameson_shock(hrow[lc - 1], hrow[lc], hrow[lc + 1])) {
+#pragma unroll
+      for (int var = 0; var < 3; ++var) {
+        const double* q = cell + var * NV;
+        double fm[4], fp[4];
+        reconstruction_fix(J.recfix, q[-1], q[0], q[1], X ? J.dx : J.dy, fm, fp);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) W[var][g] = side ? fp[g] : fm[g];
+      }
+    }
+  }
+  const double vh = cell[0];
+  double mn = vh;
+  if (c <= na) {
+    mn = positivity_limit_pair(vh, J.wbnd, W[0], side);
+  } else {  // the unlimited ghost: only its WM is used
+#pragma unroll
+    for (int g = 0; g < 4; ++g) mn = min_n(mn, W[0][g]);
+    if (side) mn = vh;
+  }
+  if (!depths_regular(vh, mn)) irregular = 1;
+  __syncthreads();
+  double* sW = smem;  // [12][NT]
+#pragma unroll
+  for (int a = 0; a < 12; ++a) sW[a * NT + tid] = W[a >> 2][a & 3];
+  __syncthreads();
+  // Gauss points 0, 1 of a face in its lower lane (WP), 2, 3 in its upper one
+  constexpr int N = X ? 1 : 2, T = X ? 2 : 1;  // normal and tangential velocity
+  const double* across = sW + (side ? min(tid + 1, NT - 1) : max(tid - 1, 0));
+  double P1[2], Pn[2], Pt[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int g = side ? q : 2 + q;
+    double own[3], far[3];
+#pragma unroll
+    for (int v = 0; v < 3; ++v) {
+      own[v] = side ? W[v][q] : W[v][2 + q];
+      far[v] = across[(4 * v + g) * NT];
+    }
+    double F1, Fn, Ft;
+    rusanov_regular(side ? own[0] : far[0], side ? own[N] : far[N], side ? own[T] : far[T],
+                    side ? far[0] : own[0], side ? far[N] : own[N], side ? far[T] : own[T], J.g,
+                    F1, Fn, Ft);
+    const double wg = side ? J.wbnd[q] : J.wbnd[2 + q];
+    P1[q] = wg * F1;
+    Pn[q] = wg * Fn;
+    Pt[q] = wg * Ft;
+  }
+  double acc1 = 0.0, accn = 0.0, acct = 0.0;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    acc1 = acc1 + P1[q];
+    accn = accn + Pn[q];
+    acct = acct + Pt[q];
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {  // the upper lane's points
+    acc1 = acc1 + dpp<kDppNext, 0xf>(P1[q]);
+    accn = accn + dpp<kDppNext, 0xf>(Pn[q]);
+    acct = acct + dpp<kDppNext, 0xf>(Pt[q]);
+  }
+  const int bb = b0 + cb;
+  if (!side || ca >= TA - 1 || c > na || bb > nb) return;
+  double acc2 = X ? accn : acct, acc3 = X ? acct : accn;
+  if (irregular | !((int)is_finite(acc1) & (int)is_finite(acc2) & (int)is_finite(acc3)))
+    face_flux_general<X>(J, W, sW + tid + 1, NT, acc1, acc2, acc3);
+  const size_t o = X ? (size_t)(bb - 1) * (nx + 1) + c : (size_t)c * nx + (bb - 1);
+  double* const* B = X ? J.FXWB : J.FYWB;
+  double* const* F = X ? J.FX[slot] : J.FY[slot];
+  if (J.wb && !L.wb_init) {  // less the well-balanced state's (src/finitevolume.f90:485-488)
+    acc1 = acc1 - G(B[0])[o];
+    acc2 = acc2 - G(B[1])[o];
+    acc3 = acc3 - G(B[2])[o];
+  }
+  G(F[0])[o] = acc1;
+  G(F[1])[o] = acc2;
+  G(F[2])[o] = acc3;
+}
+
+// ------------------------------------------------------------------------
 // Source term of a tile of TW x TH cells (1-based i = TW*bx + 1 + tx, j =
 // TH*by + 1 + ty).  SourceTerms (src/equation.f90:352-388): h point values at
 // the 4x4 Gauss points from a WENO5 second sweep along y (columns i-2..i+2)
@@ -459,10 +656,12 @@ struct FvtdTiles {
   int nxt, nyt, nst;
 };
 
-template <int XW, int XH, int YW, int YH, int SW, int SH>
-__global__ __launch_bounds__(XW * XH, 4) void k_fvtd(EngineArgs E, FvtdTiles T, NodeList L) {
-  static_assert(XW * XH == YW * YH && XW * XH == SW * SH, "one block size");
-  constexpr int LX = FaceTile<XW, XH>::LDS, LY = FaceTile<YW, YH>::LDS;
+template <int XW, int XH, int YW, int YH, int SW, int SH, bool SPLIT = false>
+__global__ __launch_bounds__(SW * SH, 4) void k_fvtd(EngineArgs E, FvtdTiles T, NodeList L) {
+  static_assert(XW * XH * (SPLIT ? 2 : 1) == SW * SH && YW * YH * (SPLIT ? 2 : 1) == SW * SH,
+                "one block size");
+  constexpr int LX = SPLIT ? 12 * SW * SH : FaceTile<XW, XH>::LDS;
+  constexpr int LY = SPLIT ? LX : FaceTile<YW, YH>::LDS;
   constexpr int LS = (SW + 4) * (SH + 4) + 4 * (SW + 4) * SH;
   __shared__ double smem[LX > LY ? (LX > LS ? LX : LS) : (LY > LS ? LY : LS)];
   __shared__ int irregular;  // a cell whose depths sqrt_regular may not take
@@ -500,10 +699,17 @@ __global__ __launch_bounds__(XW * XH, 4) void k_fvtd(EngineArgs E, FvtdTiles T, 
   const TileRef R = tile_of(E, x ? T.xt : T.yt, q - node * nt);
   const JobDev& J = E.jobs[R.job];
   if (skipped_stage(E, R.job)) return;
-  if (x)
+  if constexpr (SPLIT) {
+    static_assert(XW == kSplitA && XH == kSplitB && YH == kSplitA && YW == kSplitB, "the tiles");
+    if (x)
+      split_faces<true>(smem, irregular, J, R.tile, L.m[node], L.slot[node], L);
+    else
+      split_faces<false>(smem, irregular, J, R.tile, L.m[node], L.slot[node], L);
+  } else if (x) {
     x_faces<XW, XH>(smem, irregular, J, R.tile, L.m[node], L.slot[node], L);
-  else
+  } else {
     y_faces<YW, YH>(smem, irregular, J, R.tile, L.m[node], L.slot[node], L);
+  }
 }
 
 // Divisions by a job's dx and dy through one reciprocal each.
@@ -1176,15 +1382,6 @@ __device__ __forceinline__ double agent_load(const double* p) {
 }
 __device__ __forceinline__ void agent_store(double* p, double v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// v of lane (this - n) within rows of 16 lanes, or of the previous rows' last
-// lane (CTRL of the DPP encoding); 0 where there is none.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
-  return __hiloint2double(hi, lo);
 }
 
 // Sum over the wave in a fixed order, in every lane; six dependent steps
@@ -1982,7 +2179,7 @@ static inline unsigned cdiv(long a, long b) { return (unsigned)((a + b - 1) / b)
 
 void launch_fvtd(const EngineArgs& E, int shape, const TileRef* xt, int nxt, const TileRef* yt,
                  int nyt, const TileRef* st, int nst, const NodeList& L, hipStream_t s) {
-  static_assert(kNumShapes == 2 && kShapes[0].xw == 16 && kShapes[0].xh == 16 &&
+  static_assert(kNumShapes == 2 && kAllShapes == 3 && kShapes[0].xw == 16 && kShapes[0].xh == 16 &&
                     kShapes[0].yw == 16 && kShapes[0].yh == 16 && kShapes[0].sw == 16 &&
                     kShapes[0].sh == 16 && kShapes[1].xw == 32 && kShapes[1].xh == 16 &&
                     kShapes[1].yw == 16 && kShapes[1].yh == 32 && kShapes[1].sw == 32 &&
@@ -1991,7 +2188,10 @@ void launch_fvtd(const EngineArgs& E, int shape, const TileRef* xt, int nxt, con
   const FvtdTiles T = {xt, yt, st, nxt, nyt, nst};
   const unsigned groups = cdiv((long)(nxt + nyt) * L.count, 8) + cdiv(nst, 8) * L.count;
   if (!groups) return;
-  if (shape == 1)
+  if (shape == kSplitShape)
+    hipLaunchKernelGGL((k_fvtd<16, 8, 8, 16, 16, 16, true>), dim3(groups * 8), dim3(256), 0, s, E,
+                       T, L);
+  else if (shape == 1)
     hipLaunchKernelGGL((k_fvtd<32, 16, 16, 32, 32, 16>), dim3(groups * 8), dim3(512), 0, s, E, T,
                        L);
   else
