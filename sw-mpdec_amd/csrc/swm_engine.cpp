@@ -365,20 +365,19 @@ class SolveRight {
   int device_ = -1;
 };
 
-// Rows of the largest system that one k_solve block takes alone.  At 2048 rows
-// (4 per thread) its assembly is issue-bound at about 10 us and a sweep costs
-// about 1 us; tiles of 24x24 assemble in 5 us and pay 1.2 us a sweep with
-// their exchange, and at the 10 to 15 sweeps a solve needs the two break even.
+// Rows of the largest system that one k_solve block takes alone: 32^2 takes
+// 13.5 us a launch that way and 19.5 us in tiles, which pay an exchange every
+// fourth sweep; at 2048 rows (4 per thread) the sweeps have become as long.
 constexpr int kSolveAlone = 2048;
 
 // k_solve's blocks for the jobs of T.  A grid is taken when the blocks of one
 // system fit the device at once (blocks of a system wait for each other); the
 // blocks of several systems share a launch as long as all of them fit.  The
 // systems with several blocks take the tile size with the least launches times
-// launch time, kSolveUs (nine sweeps; 200 to 256 blocks): a larger tile makes
-// a sweep longer, a further launch repeats all of it.  Blocks without others
-// to wait for come last and are not counted.
-constexpr double kSolveUs[kSolveForms] = {24., 30., 50., 70.};
+// launch time, kSolveUs (257^2 at 2, 3, 5, 8 and 11 rows per thread, about nine
+// sweeps): a larger tile makes a sweep longer, a further launch repeats all of
+// it.  Blocks without others to wait for come last and are not counted.
+constexpr double kSolveUs[kSolveForms] = {19., 24., 28., 35., 47.};
 
 void solve_tables(swm_engine* e, Tables& T) {
   const int cap = std::min(e->solve_blocks_max, 256);

@@ -44,7 +44,7 @@ constexpr FaceShape kShapes[kAllShapes] = {{16, 16, 16, 16, 16, 16},
 constexpr int kCellBlock = 256;       // cells per block of the pointwise kernels
 constexpr int kSolveThreads = 512;    // threads of a k_solve block
 constexpr int kSolveWindow = 4;       // Jacobi sweeps between two exchanges of k_solve's blocks
-constexpr int kSolveForms = 4;        // k_solve's tile sizes (solve_tiles)
+constexpr int kSolveForms = 5;        // k_solve's tile sizes (solve_tiles)
 constexpr int kMaxSys = 3;            // Patankar systems solved together (nodes 2..4)
 constexpr int kSlots = 3;             // concurrent FVTD evaluations per job
 constexpr int kStates = 6;            // state / derivative slots of the explicit schemes
@@ -185,14 +185,15 @@ struct SolveRef {
 };
 
 // The tiles of a system in a form: ntx x nty tiles of at most tw x th cells,
-// the grid dealt out evenly.  With the window's halo the largest tile has
-// (tw + 8)(th + 8) = 1024, 2016, 4032 and 5184 rows: 2, 4, 8 and 11 per thread.
+// the grid dealt out evenly.  A block holds 64 columns and 8 kSolveRpt[form]
+// rows, less the window's halo.
+constexpr int kSolveRpt[kSolveForms] = {2, 3, 5, 8, 11};  // rows per thread
 struct SolveTiles {
   int tw, th, ntx, nty;
 };
 inline __host__ __device__ SolveTiles solve_tiles(int nx, int ny, int form) {
-  const int mw = form == 0 ? 24 : form == 1 ? 40 : 64;
-  const int mh = form == 0 ? 24 : form == 1 ? 34 : form == 2 ? 48 : 64;
+  const int mw = 64 - 2 * kSolveWindow;
+  const int mh = kSolveThreads / 64 * kSolveRpt[form] - 2 * kSolveWindow;
   SolveTiles t;
   t.ntx = (nx + mw - 1) / mw;
   t.nty = (ny + mh - 1) / mh;

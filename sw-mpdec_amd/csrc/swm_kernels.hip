@@ -19,6 +19,8 @@
 // L2, so the kernel boundary is the cheap way to publish partial sums.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "swm_engine.hpp"
 #include "swm_numerics.hpp"
 #include "swm_timestep.hpp"
@@ -1336,22 +1338,31 @@ __global__ __launch_bounds__(256) void k_decide(EngineArgs E, const int* jobs, S
 // systems fit the register files.
 //
 // A block of 512 threads owns a tile of a system and holds it with a halo of
-// kSolveWindow = 4 cells: the matrix rows in registers (up to 11 per thread),
-// the iterate in LDS.  It sweeps 4 times
-// without looking at the other blocks -- each sweep spoils one more ring of
-// the halo -- then the blocks exchange their outer 4 rings and the residual
+// kSolveWindow = 4 cells: a lane per column (64 with the halo) and a strip of
+// up to 11 rows per wave, matrix rows and iterate in registers.  It sweeps 4
+// times without looking at the other blocks -- each sweep spoils one more ring
+// of the halo -- then the blocks exchange their outer 4 rings and the residual
 // sums of the 4 sweeps, and the stop rule is applied to the sums in order.  A
-// solve that stopped inside the window takes the iterate of that sweep, which
-// is in LDS or at most two sweeps from the window's start.  The first window
-// needs no exchange before it: it starts from the right-hand side, known
-// everywhere.  So no sweep reads the matrix from memory, and no launch, host
-// prediction or empty sweep is paid per sweep.
+// solve that stopped inside the window sweeps again from the window's start to
+// that iterate.  The first window needs no exchange before it: it starts from
+// the right-hand side, known everywhere.  So no sweep reads the matrix from
+// memory, and no launch, host prediction or empty sweep is paid per sweep.
 //
-// Measured per correction (three systems): 32^2 190 -> 33 -> SOLVE32 us,
-// 257^2 135 -> 61 -> SOLVE257 us; the first figure with a launch per sweep and
-// one per stop decision, the second with row strips exchanged after every
-// sweep.  The exchange dominates there: 3.3 us for 64 blocks, against 0.6 us
-// for the sweep of a 40x40 tile.
+// Within a sweep a row's neighbours in the strip are the thread's own, those
+// to the west and east come by DPP moves; LDS carries only the strips' first
+// and last rows.  With the iterate in LDS a row took 5 reads and a write, and
+// with the full division (solve_row) 45 instructions in place of 19: 2.1 ->
+// 1.0 us a sweep of 11 rows per thread.  Small grids need one block (ALONE)
+// with any number of columns and keep the iterate in LDS.
+//
+// Measured per launch, three systems unless said: 257^2 31.4 -> 23.9 us,
+// 512^2 68 -> 53 us, one system of 1024^2 81 -> 64 us, 32^2 14.4 -> 13.5 us
+// (iterate in LDS and full division before); a launch per sweep and one per
+// stop decision took 190 us a correction at 32^2, 135 us at 257^2.  Of the
+// 64 us at 1024^2 (10 sweeps) 14 are the loads of the matrix (69 MB, 5 TB/s),
+// 15 the sweeps, 25 the three exchanges with their sums and halo loads.
+// Windows of 6 with halos of 6 lose as much in the tiles as they save in
+// exchanges (257^2: 27 us, 512^2: 60 us).
 //
 // The exchange goes through agent-scope atomic stores and loads, which bypass
 // the XCDs' separate L2s, so no cache is written back: a block drains its
@@ -1397,29 +1408,85 @@ __device__ __forceinline__ double wave_sum_dpp(double v) {
                           __builtin_amdgcn_readlane(__double2loint(v), 63));
 }
 
-constexpr int kSolveRows = 11 * kSolveThreads;  // rows of the largest tile with its halo
+constexpr int kSolveRows = kSolveRpt[kSolveForms - 1] * kSolveThreads;  // of the largest tile
 constexpr int kSolveWaves = kSolveThreads / 64;
+constexpr int kSolveAloneRows = 4 * kSolveThreads;  // most rows of a block without others
 static_assert(kSolveWaves == 8 && kSolveKinds <= 8, "the stop rule's lanes");
 
 struct SolveShared {
-  double x[3][kSolveRows];  // the iterate: the window's start and two buffers
-
+  union {
+    double x[3][kSolveAloneRows];  // ALONE: the iterate: the window's start and two buffers
+    struct {
+      double start[kSolveRows];            // the window's start, each thread's own rows
+      double edge[2][kSolveWaves][2][64];  // the strips' first and last rows, by parity
+    } t;
+  };
   double red[kSolveKinds][kSolveWaves];
   double tot[kSolveKinds][4];
   int lost;
+  // the round after which an iterate left the short form's range; ~0: a row is
+  // outside it from the start
+  unsigned irregular;
 };
+
+// Ranges in which a sweep needs none of the care for signed zeros, infinities
+// and rescaled divisions: with off-diagonal entries in [-2^40, 0], a diagonal
+// in [2^-8, 2^100], a right-hand side in [2^-200, 2^100] and an iterate in
+// [0, 2^200] at the start of the window, every product is <= 0, every numerator
+// in [2^-200, 2^392] and every quotient in [2^-300, 2^400] (a sweep lets the
+// iterate grow by less than 2^50).  There 0. + p, + 0.*x change nothing, and
+// the quotient has div_by's bits.
+__device__ __forceinline__ bool solve_row_regular(const double M[4], double D, double b) {
+  int ok = (int)(D >= 0x1p-8) & (int)(D <= 0x1p100) & (int)(b >= 0x1p-200) & (int)(b <= 0x1p100);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) ok &= (int)(M[q] >= -0x1p40) & (int)(M[q] <= 0.);
+  return ok;
+}
+
+// p, the same in every lane of the wave, in scalar registers.
+template <class T>
+__device__ __forceinline__ T* uniform(T* p) {
+  const unsigned long long v = (unsigned long long)p;
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
+  const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+  return (T*)((unsigned long long)hi << 32 | lo);
+}
+
+constexpr unsigned kSolveStartHi = (1023u + 200u) << 20;  // high word of 2^200; signs lie above
+
+// x_new of a row (src/jacobi_iteration.f90:72-80); R: recip_refined(D).
+template <bool SHORT>
+__device__ __forceinline__ double solve_row(const double M[4], double D, double R, double b,
+                                            double x, double yS, double yW, double yE,
+                                            double yN) {
+  if (SHORT) {
+    double p = M[0] * yS;
+    p = p + M[1] * yW;
+    p = p + M[2] * yE;
+    p = p + M[3] * yN;
+    return div_by(b - p, D, R);
+  }
+  double p = 0.;
+  p = p + M[0] * yS;
+  p = p + M[1] * yW;
+  p = p + 0. * x;
+  p = p + M[2] * yE;
+  p = p + M[3] * yN;
+  return (b - p) / D;
+}
+
 // ALONE: the whole grid in the block, no halo and no exchange.
 template <int RPT, bool ALONE>
 __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E, const SolveRef W,
                                             const SysList& S, int limit, int first_solve) {
   constexpr int NT = kSolveThreads, HALO = ALONE ? 0 : kSolveWindow;
   const JobDev& J = E.jobs[W.job];
-  const int tid = threadIdx.x, s = W.sys, m = S.m[s];
+  const int tid = threadIdx.x, lane = tid & 63, s = W.sys, m = S.m[s];
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nx = J.nx, ny = J.ny, n = J.n;
   JobStatus* st = E.status + W.job;
-  const gdouble* rhs = system_rhs(J, S);
-  // own cells [ox, ox + ow) x [oy, oy + oh); EW x EH with the halo
-  int nb = 1, ox = 0, oy = 0, ow = nx, oh = ny, EW = nx, EH = ny;
+  // own cells [ox, ox + ow) x [oy, oy + oh)
+  int nb = 1, ox = 0, oy = 0, ow = nx, oh = ny;
   unsigned round0 = 0;
   if (!ALONE) {
     const SolveTiles T = solve_tiles(nx, ny, W.form);
@@ -1428,89 +1495,127 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
     oy = (W.tile / T.ntx) * T.th;
     ow = min(T.tw, nx - ox);
     oh = min(T.th, ny - oy);
-    EW = T.tw + 2 * HALO;
-    EH = T.th + 2 * HALO;
     round0 = st->rounds[W.form][s];
   }
-  const int rows = EW * EH;
-  if (tid == 0) L.lost = 0;
+  if (tid == 0) {
+    L.lost = 0;
+    L.irregular = 0;
+  }
+  __syncthreads();
 
   // The thread's matrix rows, as k_assemble left them, and the start x = b.
-  // act: rows with all four neighbours in the tile; own: the block's own
-  // cells; outer: those that other blocks read.
-  double M[RPT][4], D[RPT], b[RPT];
-  int at[ALONE ? RPT : 1][4], gk[RPT];
-  unsigned act = 0, own = 0, outer = 0;
+  // ALONE: rows tid, tid + NT, ..  Else column `lane` of the tile, whose first
+  // own cell is HALO, in the wave's strip of RPT rows; what lies beyond the
+  // tile's halo are rows of the grid as well (lanes: rows x = 1 of their own),
+  // swept like the others and never looked at, so that no sweep asks.
+  double M[RPT][4], D[RPT], R[RPT], b[RPT], x[RPT];
+  int at[ALONE ? RPT : 1][4], row[RPT];  // row: the first cell of the grid's row
+  const int tx = lane - HALO, ty0 = wv * RPT - HALO;  // within the own cells
+  unsigned ci = tid;
+  const gdouble* Mp[5];
+#pragma unroll
+  for (int q = 0; q < 5; ++q) Mp[q] = uniform(G(J.M[s][q]));
+  const gdouble* rhs = uniform(system_rhs(J, S));
+  double* const buf0 = uniform(J.FX[s][0]);
+  double* const buf1 = uniform(J.FX[s][1]);
+  if (!ALONE) {
+    int c = (ox + tx) % nx, cj = (oy + ty0) % ny;
+    ci = c < 0 ? c + nx : c;
+    cj = cj < 0 ? cj + ny : cj;
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {
+      row[i] = cj * nx;
+      cj = cj + 1 == ny ? 0 : cj + 1;
+    }
+  }
+  const bool held_lane = lane < ow + 2 * HALO, own_lane = tx >= 0 && tx < ow;
+  auto held = [&](int i) { return ALONE ? i * NT + tid < n : held_lane; };
+  auto own_row = [&](int i) { return ty0 + i >= 0 && ty0 + i < oh; };
+  auto own = [&](int i) { return ALONE ? held(i) : own_lane && own_row(i); };
+  bool regular = true;
   double bsum = 0.;
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
-    const int l = i * NT + tid;
-    if (l < rows) {
-      const int ly = l / EW, lx = l - ly * EW;
-      int ci = lx, cj = ly;
-      if (ALONE) {
-        act |= 1u << i;
-        own |= 1u << i;
-        at[i][0] = (cj == 0 ? ny - 1 : cj - 1) * nx + ci;
-        at[i][1] = cj * nx + (ci == 0 ? nx - 1 : ci - 1);
-        at[i][2] = cj * nx + (ci == nx - 1 ? 0 : ci + 1);
-        at[i][3] = (cj == ny - 1 ? 0 : cj + 1) * nx + ci;
-      } else {
-        const int tx = lx - HALO, ty = ly - HALO;  // within the own cells
-        ci = (ox + tx) % nx;
-        cj = (oy + ty) % ny;
-        if (ci < 0) ci += nx;
-        if (cj < 0) cj += ny;
-        if (lx >= 1 && lx < EW - 1 && ly >= 1 && ly < EH - 1) act |= 1u << i;
-        if (tx >= 0 && tx < ow && ty >= 0 && ty < oh) {
-          own |= 1u << i;
-          if (tx < HALO || tx >= ow - HALO || ty < HALO || ty >= oh - HALO) outer |= 1u << i;
-        }
-      }
-      const int k = cj * nx + ci;
-      gk[i] = k;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) M[i][q] = G(J.M[s][q])[k];
-      D[i] = G(J.M[s][4])[k];
-      b[i] = rhs[k];
+    if (ALONE) {
+      const int l = i * NT + tid, cj = l / nx, c = l - cj * nx;
+      row[i] = i * NT;
+      at[ALONE ? i : 0][0] = (cj == 0 ? ny - 1 : cj - 1) * nx + c;
+      at[ALONE ? i : 0][1] = cj * nx + (c == 0 ? nx - 1 : c - 1);
+      at[ALONE ? i : 0][2] = cj * nx + (c == nx - 1 ? 0 : c + 1);
+      at[ALONE ? i : 0][3] = (cj == ny - 1 ? 0 : cj + 1) * nx + c;
     }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) M[i][q] = 0.;
+    D[i] = 1.;
+    b[i] = 1.;
+  }
+  if (held(0)) {
+#pragma unroll
+    for (int i = 0; i < RPT; ++i)
+      if (!ALONE || held(i)) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) M[i][q] = (Mp[q] + row[i])[ci];
+        D[i] = (Mp[4] + row[i])[ci];
+        b[i] = (rhs + row[i])[ci];
+      }
   }
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
-    const int l = i * NT + tid;
-    if (l < rows) L.x[0][l] = b[i];
-    if ((own >> i) & 1u) bsum += fabs(0.0 - b[i]);
+    R[i] = recip_refined(D[i]);
+    x[i] = b[i];
+    regular = regular & solve_row_regular(M[i], D[i], b[i]);
+    if (own(i)) bsum += fabs(0.0 - b[i]);
   }
 
-  // One sweep (src/jacobi_iteration.f90:72-80) of every row with its
-  // neighbours in the tile; returns the thread's part of the own cells'
-  // SUM(ABS(x_new - x_old)).
-  auto sweep = [&](const double* from, double* to) {
+  // One sweep of every row; returns the thread's part of the own cells'
+  // SUM(ABS(x_new - x_old)).  ALONE: from and to in LDS.  Else in the
+  // registers: the neighbours to the west and east are the next lanes', those
+  // beyond a strip's ends come from the edges of parity `par`, and the new ones
+  // go to the other parity unless it is the `last`.  The outermost row of the
+  // tile, or lane, takes what it finds, never less than 0: a sweep spoils it.
+  auto sweep = [&](auto shrt, const double* from, double* to, int par, bool last) {
+    constexpr bool SHORT = decltype(shrt)::value;
     double dsum = 0.;
-    constexpr int GR = RPT < 4 ? RPT : 4;  // rows with their loads in flight together
+    if (ALONE) {
 #pragma unroll
-    for (int i0 = 0; i0 < RPT; i0 += GR) {
-#pragma unroll
-      for (int i = i0; i < i0 + GR && i < RPT; ++i)
-        if ((act >> i) & 1u) {
+      for (int i = 0; i < RPT; ++i)
+        if (held(i)) {
           const int l = i * NT + tid;
           const int* a = at[ALONE ? i : 0];
-          const double yS = from[ALONE ? a[0] : l - EW], yW = from[ALONE ? a[1] : l - 1];
-          const double yE = from[ALONE ? a[2] : l + 1], yN = from[ALONE ? a[3] : l + EW];
-          const double x = from[l];
-          double p = 0.;
-          p = p + M[i][0] * yS;
-          p = p + M[i][1] * yW;
-          p = p + 0. * x;
-          p = p + M[i][2] * yE;
-          p = p + M[i][3] * yN;
-          const double xv = (b[i] - p) / D[i];
+          const double c = from[l];
+          const double xv = solve_row<SHORT>(M[i], D[i], R[i], b[i], c, from[a[0]], from[a[1]],
+                                             from[a[2]], from[a[3]]);
           to[l] = xv;
-          if ((own >> i) & 1u) dsum += fabs(xv - x);
+          dsum += fabs(xv - c);
         }
+      __syncthreads();
+      return dsum;
     }
-    __syncthreads();
-    return dsum;
+    double south = L.t.edge[par][wv ? wv - 1 : 0][1][lane];
+    const double north = L.t.edge[par][wv < kSolveWaves - 1 ? wv + 1 : wv][0][lane];
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {
+      const double c = x[i];
+      const double xv = solve_row<SHORT>(M[i], D[i], R[i], b[i], c, south, dpp<0x138, 0xf>(c),
+                                         dpp<0x130, 0xf>(c), i + 1 < RPT ? x[i + 1] : north);
+      if (SHORT)
+        dsum = fma(fabs(xv - c), own_row(i) ? 1. : 0., dsum);
+      else
+        dsum += own_row(i) ? fabs(xv - c) : 0.;
+      if (!SHORT) __builtin_amdgcn_sched_barrier(0);  // few registers are left at 11 rows
+      south = c;
+      x[i] = xv;
+    }
+    if (!last) {
+      L.t.edge[par ^ 1][wv][0][lane] = x[0];
+      L.t.edge[par ^ 1][wv][1][lane] = x[RPT - 1];
+      __syncthreads();
+    }
+    return own_lane ? dsum : 0.;
+  };
+  auto publish_edges = [&] {
+    L.t.edge[0][wv][0][lane] = x[0];
+    L.t.edge[0][wv][1][lane] = x[RPT - 1];
   };
 
   // certified_continue with the division by n taken to the other side: n tol
@@ -1525,25 +1630,51 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
     return sum + B <= tn_lo ? 0 : -1;
   };
 
+  if (ALONE) {
+#pragma unroll
+    for (int i = 0; i < RPT; ++i)
+      if (held(i)) L.x[0][i * NT + tid] = x[i];
+  } else {
+    publish_edges();
+  }
+  if (!regular) L.irregular = ~0u;
   __syncthreads();
-  double *p0 = L.x[0], *q0 = L.x[1], *q1 = L.x[2];
-  const double* result = nullptr;
+  regular = L.irregular != ~0u;
+  double *p0 = L.x[0], *q0 = L.x[1], *q1 = L.x[2];  // ALONE
   int k_sweeps = 0, end = kSolveConverged;
   bool zero = false;
   unsigned t = 0;
   for (;; ++t) {
     double sum[kSolveKinds];
-    sum[0] = sweep(p0, q0);
-    sum[1] = sweep(q0, q1);
-    sum[2] = sweep(q1, q0);
-    sum[3] = sweep(q0, q1);
-    static_assert(kSolveWindow == 4, "the sweeps above");
-    sum[kSolveWindow] = bsum;  // used in the first round only
-    double* buf = J.FX[s][t & 1];  // free between an FVTD's update and the next one's face kernels
     if (!ALONE) {
 #pragma unroll
+      for (int i = 0; i < RPT; ++i) L.t.start[i * NT + tid] = x[i];
+    }
+    static_assert(kSolveWindow == 4, "the sweeps of a window");
+    if (regular) {
+      constexpr std::true_type shrt;
+      sum[0] = sweep(shrt, p0, q0, 0, false);
+      sum[1] = sweep(shrt, q0, q1, 1, false);
+      sum[2] = sweep(shrt, q1, q0, 0, false);
+      sum[3] = sweep(shrt, q0, q1, 1, true);
+    } else {
+#pragma unroll 1
+      for (int k = 0; k < kSolveWindow; ++k) {
+        const double v = sweep(std::false_type(), k == 0 ? p0 : k & 1 ? q0 : q1, k & 1 ? q1 : q0,
+                               k & 1, k == kSolveWindow - 1);
+#pragma unroll
+        for (int q = 0; q < kSolveWindow; ++q)
+          if (q == k) sum[q] = v;
+      }
+    }
+    sum[kSolveWindow] = bsum;  // used in the first round only
+    double* buf = t & 1 ? buf1 : buf0;  // free between an FVTD's update and the next one's face kernels
+    if (!ALONE) {
+      const bool outer_lane = tx < HALO || tx >= ow - HALO;
+#pragma unroll
       for (int i = 0; i < RPT; ++i)
-        if ((outer >> i) & 1u) agent_store(buf + gk[i], q1[i * NT + tid]);
+        if (own(i) && (outer_lane || ty0 + i < HALO || ty0 + i >= oh - HALO))
+          agent_store(buf + row[i] + ci, x[i]);
     }
 #pragma unroll
     for (int q = 0; q < kSolveKinds; ++q) {
@@ -1592,12 +1723,10 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
       }
     }
     // the halo of the next window, on its way while the stop rule is applied
-    double halo[ALONE ? 1 : RPT];
     if (!ALONE) {
 #pragma unroll
       for (int i = 0; i < RPT; ++i)
-        if (i * NT + tid < rows && !((own >> i) & 1u))
-          halo[ALONE ? 0 : i] = agent_load(buf + gk[i]);
+        if (!own(i)) x[i] = held(i) && ty0 + i < oh + HALO ? agent_load(buf + row[i] + ci) : 1.;
     }
     // The stop rule (src/jacobi_iteration.f90:63-84), sweep by sweep: the same
     // numbers, and so the same decisions, in every block of the system.  Lane
@@ -1649,35 +1778,50 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
     if (stop) {
       // the iterate of the window's sweep j (counted from 1)
       if (end == kSolveOpen || zero) break;
-      if (j == 4) {
-        result = q1;
-      } else if (j == 3) {
-        result = q0;
-      } else {
-        sweep(p0, q0);
-        result = q0;
-        if (j == 2) {
-          sweep(q0, q1);
-          result = q1;
+      if (ALONE ? j <= 2 : j < kSolveWindow) {
+        if (!ALONE) {
+#pragma unroll
+          for (int i = 0; i < RPT; ++i) x[i] = L.t.start[i * NT + tid];
+          publish_edges();
+          __syncthreads();
         }
+#pragma unroll 1
+        for (int k = 0; k < j; ++k) {
+          const double *from = k ? q0 : p0;
+          double* to = k ? q1 : q0;
+          if (regular)
+            sweep(std::true_type(), from, to, k & 1, k == j - 1);
+          else
+            sweep(std::false_type(), from, to, k & 1, k == j - 1);
+        }
+      }
+      if (ALONE) {
+#pragma unroll
+        for (int i = 0; i < RPT; ++i)
+          if (held(i)) x[i] = (j & 1 ? q0 : q1)[i * NT + tid];
       }
       break;
     }
-    if (!ALONE) {
+    unsigned hi = 0;
 #pragma unroll
-      for (int i = 0; i < RPT; ++i)
-        if (i * NT + tid < rows && !((own >> i) & 1u)) q1[i * NT + tid] = halo[ALONE ? 0 : i];
+    for (int i = 0; i < RPT; ++i) {
+      if (ALONE && held(i)) x[i] = q1[i * NT + tid];
+      hi = max(hi, (unsigned)__double2hiint(x[i]));
     }
+    if (hi >= kSolveStartHi) L.irregular = t + 1;
+    if (!ALONE) publish_edges();
     __syncthreads();  // also: the sums have been read
+    regular = regular && L.irregular != t + 1;
     double* w = p0;
     p0 = q1;
     q1 = q0;
     q0 = w;
   }
   if (end != kSolveOpen) {
+    gdouble* to = uniform(G(J.hres[m]));
 #pragma unroll
     for (int i = 0; i < RPT; ++i)
-      if ((own >> i) & 1u) G(J.hres[m])[gk[i]] = zero ? 0. : result[i * NT + tid];
+      if (own(i)) (to + row[i])[ci] = zero ? 0. : x[i];
   }
   if (tid == 0) {
     if (!ALONE && L.lost) st->solve_lost = 1;  // keeps the step from being committed
@@ -1704,13 +1848,15 @@ __global__ __launch_bounds__(kSolveThreads) void k_solve(EngineArgs E, const Sol
   if (skipped_stage(E, W.job)) return;
   switch (W.form) {
     case 0:
-      return solve_block<2, false>(L, E, W, S, limit, first_solve);
+      return solve_block<kSolveRpt[0], false>(L, E, W, S, limit, first_solve);
     case 1:
-      return solve_block<4, false>(L, E, W, S, limit, first_solve);
+      return solve_block<kSolveRpt[1], false>(L, E, W, S, limit, first_solve);
     case 2:
-      return solve_block<8, false>(L, E, W, S, limit, first_solve);
+      return solve_block<kSolveRpt[2], false>(L, E, W, S, limit, first_solve);
     case 3:
-      return solve_block<11, false>(L, E, W, S, limit, first_solve);
+      return solve_block<kSolveRpt[3], false>(L, E, W, S, limit, first_solve);
+    case 4:
+      return solve_block<kSolveRpt[4], false>(L, E, W, S, limit, first_solve);
     case kSolveForms:
       return solve_block<1, true>(L, E, W, S, limit, first_solve);
     case kSolveForms + 1:

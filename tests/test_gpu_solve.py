@@ -27,12 +27,12 @@ def random_state(n, ny, seed, amp=0.3):
 
 # nx, ny, steps: 512, 1024 and 2048 cells are the most that one block takes at
 # 1, 2 and 4 rows per thread; from 2049 on the tiles of a system share a
-# solve: tiles of at most 24x24 cells (one of 24x24 and its neighbours one
-# wider; thinner than the 4 cells of halo; a grid thinner than its halo), of
-# 40x34 (both its edges), of 64x48 and of 64x64
+# solve: tiles of at most 56 x 8, 16, 32, 56 and 80 cells (full ones and one
+# cell more; thinner than the 4 cells of halo; a grid thinner than its halo)
 SIZES = [(3, 3, 3), (32, 16, 3), (27, 19, 3), (32, 32, 2), (41, 25, 2), (64, 32, 2), (3, 683, 2),
-         (683, 3, 2), (1500, 4, 2), (48, 48, 2), (49, 73, 2), (101, 67, 2), (192, 193, 1),
-         (240, 238, 1), (241, 239, 1), (419, 418, 1), (517, 513, 1)]
+         (683, 3, 2), (1500, 4, 2), (48, 48, 2), (49, 73, 2), (56, 40, 2), (57, 41, 2),
+         (101, 67, 2), (112, 80, 2), (192, 193, 1), (240, 238, 1), (241, 239, 1), (419, 418, 1),
+         (517, 513, 1)]
 
 
 @pytest.mark.parametrize("size", SIZES, ids=lambda s: f"{s[0]}x{s[1]}")
@@ -48,7 +48,26 @@ def test_solve_matches_oracle(size):
         it = it[0] if isinstance(it, tuple) else it
         assert dt == dts[k]
         assert list(sweeps[k]) == list(it)[:13]
+    assert s.execution_stats()["redone_steps"] == 0
     assert same_bits(s.download(), o.get_U()), describe_diff(s.download(), o.get_U())
+
+
+@pytest.mark.parametrize("low", [0.0, 1e-65])
+@pytest.mark.parametrize("n", [20, 44, 90, 300])
+def test_rows_out_of_the_short_form_range(n, low):
+    """Depths of zero and below 2^-200 around a dam: their blocks take the full
+    form of the sweep, the others the short one.  (The momenta there are NaN.)"""
+    p = P.dam_break(n, 1, dry=low)
+    s = swm.Solver.from_problem(p)
+    o = Oracle(p)
+    dts, sweeps, _ = s.run_steps(1)
+    it = o.step(dts[0])
+    it = it[0] if isinstance(it, tuple) else it
+    assert list(sweeps[0]) == list(it)[:13]
+    assert s.execution_stats()["redone_steps"] == 0
+    U, V = s.download(), o.get_U()
+    assert same_bits(U[..., 0], V[..., 0])
+    assert (np.isnan(U) == np.isnan(V)).all()
 
 
 @pytest.mark.parametrize("scheme", [6, 7])
