@@ -1122,6 +1122,19 @@ __device__ __forceinline__ const gdouble* system_rhs(const JobDev& J, const SysL
   return G(S.hp_view ? J.hres[2] : J.h);
 }
 
+// Cell blocks per block of the assembly with the first sweep, on large grids:
+// the block's look-ups and its four sums over the block are shared by 1024
+// cells, and k_decide, which reads all partial sums with one block at 14 bytes
+// a nanosecond, has a quarter of them (2048^2: 410 + 34 -> 358 + 13 us; 1500^2:
+// 226 + 23 -> 203 + 11).  k_sweep stays at a block per 256 cells: it is bound
+// by its loads and lost as much (78 -> 93 us) as its decision gained.  Below
+// 4096 cell blocks the device would be left idle, and the tables of several
+// jobs name cell blocks one by one.
+constexpr int kSumBlocks = 4, kSumBlocksFrom = 4096;
+__host__ __device__ inline int sum_blocks(const EngineArgs& E, int nblk) {
+  return E.single >= 0 && nblk >= kSumBlocksFrom ? kSumBlocks : 1;
+}
+
 // FIRST: the first sweep and its residual sums, for a launch per sweep; without
 // it only the matrix, for k_solve.  blockIdx.y picks the system where the grid
 // has that dimension (launch_assemble_matrix), else the block does them all.
@@ -1135,78 +1148,91 @@ __global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* b
   if (skipped_stage(E, T.job)) return;
   const int nx = J.nx, ny = J.ny, n = J.n;
   const int tid = threadIdx.x;
-  const int k = T.tile * kCellBlock + tid;
-  const bool in = k < n;
   const double dt = E.status[T.job].dt;
   const int s0 = gridDim.y > 1 ? blockIdx.y : 0, s1 = gridDim.y > 1 ? s0 + 1 : S.count;
-  int kS = 0, kW = 0, kE = 0, kN = 0;  // neighbours
-  double b = 0., bS = 0., bW = 0., bE = 0., bN = 0.;
-  if (in) {
-    const int k0 = T.tile * kCellBlock;
-    int i, j;
-    cell_ij(k0 % nx, k0 / nx, tid, nx, i, j);
-    kS = (j == 0 ? ny - 1 : j - 1) * nx + i;
-    kW = j * nx + (i == 0 ? nx - 1 : i - 1);
-    kE = j * nx + (i == nx - 1 ? 0 : i + 1);
-    kN = (j == ny - 1 ? 0 : j + 1) * nx + i;
-    const CellFluxes<R, FRESH> F(J, S, k, (size_t)j * (nx + 1) + i, (size_t)j * nx + i);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      sq[(0 * R + r) * 256 + tid] = F.q[0][r];
-      sq[(1 * R + r) * 256 + tid] = F.q[1][r];
-      sq[(2 * R + r) * 256 + tid] = -F.q[2][r];  // east and north slots: the flux
-      sq[(3 * R + r) * 256 + tid] = -F.q[3][r];  // oriented into the cell
-    }
-    const gdouble* rhs = system_rhs(J, S);
-    if (FIRST) {
-      b = rhs[k];
-      bS = rhs[kS];
-      bW = rhs[kW];
-      bE = rhs[kE];
-      bN = rhs[kN];
-    }
-    momentum_cell<R>(J, S, s0, s1, k, dt, F.fu2, F.fu3);
-  }
-  // One system at a time, and within it one stencil slot at a time (S, W, E,
-  // N: the CSR order), so that only one slot's divisions are live.  Each
-  // thread reads back only its own column of sq, so no barrier is needed.
+  const int per = FIRST ? sum_blocks(E, J.nblk) : 1;
+  double dsum[kMaxSys] = {}, bsum = 0.;
 #pragma unroll 1
-  for (int s = s0; s < s1; ++s) {
-    double d = 0.;
+  for (int g = 0; g < per; ++g) {
+    const int tile = T.tile * per + g, k = tile * kCellBlock + tid;
+    const bool in = k < n;
+    int kS = 0, kW = 0, kE = 0, kN = 0;  // neighbours
+    double b = 0., bS = 0., bW = 0., bE = 0., bN = 0.;
     if (in) {
-      const int m = S.m[s];
-      const gdouble* hp = system_hp(J, S, m);
-      const double hK = hp[k], hS = hp[kS], hW = hp[kW], hE = hp[kE], hN = hp[kN];
-      const PdDepth pK = pd_depth(hK);
-      const int pos = THETA_POS[S.theta][m];
-      double c[R];
+      const int k0 = tile * kCellBlock;
+      int i, j;
+      cell_ij(k0 % nx, k0 / nx, tid, nx, i, j);
+      kS = (j == 0 ? ny - 1 : j - 1) * nx + i;
+      kW = j * nx + (i == 0 ? nx - 1 : i - 1);
+      kE = j * nx + (i == nx - 1 ? 0 : i + 1);
+      kN = (j == ny - 1 ? 0 : j + 1) * nx + i;
+      const CellFluxes<R, FRESH> F(J, S, k, (size_t)j * (nx + 1) + i, (size_t)j * nx + i);
 #pragma unroll
-      for (int r = 0; r < R; ++r) c[r] = dt * THETA[S.theta][m][r];
-      // sol = (rhs - prod)/diag; rows of a wave with no depth below
-      // MIN_DEPTH take the branch without the dry-depth selects
-      double D = 1.;
-      const bool dry = pK.dry | (hS < kMinDepth) | (hW < kMinDepth) | (hE < kMinDepth) |
-                       (hN < kMinDepth);
-      auto put = [&](int sl, double v) { G(J.M[s][sl])[k] = v; };
-      const double p = __any(dry)
-                           ? patankar_row<R, false, 256>(put, sq + tid, pos, c, pK, hS, hW, hE, hN,
-                                                         bS, bW, bE, bN, b, D)
-                           : patankar_row<R, true, 256>(put, sq + tid, pos, c, pK, hS, hW, hE, hN,
-                                                        bS, bW, bE, bN, b, D);
-      G(J.M[s][4])[k] = D;
-      if (FIRST) {
-        double x1 = (b - p) / D;
-        G(J.xj[m][1])[k] = x1;
-        d = fabs(x1 - b);
+      for (int r = 0; r < R; ++r) {
+        sq[(0 * R + r) * 256 + tid] = F.q[0][r];
+        sq[(1 * R + r) * 256 + tid] = F.q[1][r];
+        sq[(2 * R + r) * 256 + tid] = -F.q[2][r];  // east and north slots: the flux
+        sq[(3 * R + r) * 256 + tid] = -F.q[3][r];  // oriented into the cell
       }
+      const gdouble* rhs = system_rhs(J, S);
+      if (FIRST) {
+        b = rhs[k];
+        bS = rhs[kS];
+        bW = rhs[kW];
+        bE = rhs[kE];
+        bN = rhs[kN];
+      }
+      momentum_cell<R>(J, S, s0, s1, k, dt, F.fu2, F.fu3);
     }
-    if (!FIRST) continue;
-    double t = block_sum_all(d, red);
-    if (tid == 0) J.part[(size_t)s * J.nblk + T.tile] = t;
+    // One system at a time, and within it one stencil slot at a time (S, W, E,
+    // N: the CSR order), so that only one slot's divisions are live.  Each
+    // thread reads back only its own column of sq, so no barrier is needed.
+#pragma unroll 1
+    for (int s = s0; s < s1; ++s) {
+      double d = 0.;
+      if (in) {
+        const int m = S.m[s];
+        const gdouble* hp = system_hp(J, S, m);
+        const double hK = hp[k], hS = hp[kS], hW = hp[kW], hE = hp[kE], hN = hp[kN];
+        const PdDepth pK = pd_depth(hK);
+        const int pos = THETA_POS[S.theta][m];
+        double c[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) c[r] = dt * THETA[S.theta][m][r];
+        // sol = (rhs - prod)/diag; rows of a wave with no depth below
+        // MIN_DEPTH take the branch without the dry-depth selects
+        double D = 1.;
+        const bool dry = pK.dry | (hS < kMinDepth) | (hW < kMinDepth) | (hE < kMinDepth) |
+                         (hN < kMinDepth);
+        auto put = [&](int sl, double v) { G(J.M[s][sl])[k] = v; };
+        const double p = __any(dry)
+                             ? patankar_row<R, false, 256>(put, sq + tid, pos, c, pK, hS, hW, hE, hN,
+                                                           bS, bW, bE, bN, b, D)
+                             : patankar_row<R, true, 256>(put, sq + tid, pos, c, pK, hS, hW, hE, hN,
+                                                          bS, bW, bE, bN, b, D);
+        G(J.M[s][4])[k] = D;
+        if (FIRST) {
+          double x1 = (b - p) / D;
+          G(J.xj[m][1])[k] = x1;
+          d = fabs(x1 - b);
+        }
+      }
+      if (!FIRST) continue;
+#pragma unroll
+      for (int q = 0; q < kMaxSys; ++q) dsum[q] += q == s ? d : 0.;
+    }
+    if (FIRST && in) bsum += fabs(0.0 - b);
   }
   if (!FIRST) return;
-  double t = block_sum_all(in ? fabs(0.0 - b) : 0., red);
-  if (tid == 0) J.part[(size_t)kMaxSys * J.nblk + T.tile] = t;
+  const size_t nsum = cdiv_d(J.nblk, per);
+#pragma unroll
+  for (int s = 0; s < kMaxSys; ++s)
+    if (s < S.count) {
+      const double t = block_sum_all(dsum[s], red);
+      if (tid == 0) J.part[s * nsum + T.tile] = t;
+    }
+  const double t = block_sum_all(bsum, red);
+  if (tid == 0) J.part[kMaxSys * nsum + T.tile] = t;
 }
 
 // One Jacobi sweep of every still-active system (src/jacobi_iteration.f90:72-80).
@@ -1266,7 +1292,7 @@ __global__ __launch_bounds__(256) void k_decide(EngineArgs E, const int* jobs, S
   const JobDev& J = E.jobs[job];
   JobStatus* st = E.status + job;
   if (skipped(E, job)) return;
-  const int n = J.n, nb = J.nblk;
+  const int n = J.n, nb = FIRST ? cdiv_d(J.nblk, sum_blocks(E, J.nblk)) : J.nblk;
   double tot[kMaxSys + 1] = {0., 0., 0., 0.};
   int act[kMaxSys] = {0, 0, 0}, cur[kMaxSys] = {0, 0, 0};
   for (int s = 0; s < S.count; ++s) {
@@ -2365,10 +2391,11 @@ void launch_keep_state(const EngineArgs& E, const TileRef* cb, int ncb, int m, h
 void launch_assemble(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl, int njobs,
                      const SysList& S, hipStream_t s) {
   if (!ncb) return;
+  const dim3 grid(cdiv(ncb, sum_blocks(E, ncb)));  // one job: ncb is its nblk
   if (S.nr == 2)
-    hipLaunchKernelGGL((k_assemble<2, true>), dim3(ncb), dim3(256), 0, s, E, cb, S);
+    hipLaunchKernelGGL((k_assemble<2, true>), grid, dim3(256), 0, s, E, cb, S);
   else
-    hipLaunchKernelGGL((k_assemble<4, true>), dim3(ncb), dim3(256), 0, s, E, cb, S);
+    hipLaunchKernelGGL((k_assemble<4, true>), grid, dim3(256), 0, s, E, cb, S);
   hipLaunchKernelGGL(k_decide<true>, dim3(njobs), dim3(256), 0, s, E, jl, S);
 }
 

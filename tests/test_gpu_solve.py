@@ -101,6 +101,19 @@ def test_several_launches_match_plain_solvers():
         assert same_bits(eng.fetch(j), s.download())
 
 
+@pytest.mark.parametrize("size", [(1027, 1023), (1023, 1024)], ids=lambda s: f"{s[0]}x{s[1]}")
+def test_grouped_residual_sums(size):
+    """The last grid with a residual sum per 256 cells and the first, ragged,
+    with one per 1024: sweeps launched one by one, against the solve in one
+    launch."""
+    p = random_state(*size, 7)
+    a, b = swm.Solver.from_problem(p), swm.Solver.from_problem(p)
+    b.set_execution(0, -2)
+    ra, rb = a.run_steps(1), b.run_steps(1)
+    assert ra[0] == rb[0] and (ra[1] == rb[1]).all()
+    assert same_bits(a.download(), b.download())
+
+
 @pytest.mark.parametrize("size", [(32, 32), (80, 80)], ids=lambda s: f"{s[0]}x{s[1]}")
 def test_open_decision_is_taken_by_the_sequential_sum(size):
     """A uniform depth 1 at rest with the tolerance 1: the initial residual is
