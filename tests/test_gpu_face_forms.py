@@ -44,7 +44,8 @@ def state(kind, n, ny, seed):
     return P.Problem(n, U, kind=kind, ny=ny)
 
 
-@pytest.mark.parametrize("shape", [0, 1])
+# shape -1: the launch's own choice, two lanes per cell at these sizes
+@pytest.mark.parametrize("shape", [0, 1, -1])
 @pytest.mark.parametrize("size", [(17, 31), (33, 32), (48, 15)])
 @pytest.mark.parametrize("kind", sorted(KINDS))
 def test_fvtd_matches_oracle(kind, size, shape):
@@ -56,3 +57,15 @@ def test_fvtd_matches_oracle(kind, size, shape):
     for k in FVTD_KEYS:
         a, b = fvtd_view(got, k), fvtd_view(ref, k)
         assert same_bits(a, b), f"{kind} {size} {k}: {describe_diff(a, b)}"
+
+
+@pytest.mark.parametrize("recfix", [1, 2])
+@pytest.mark.parametrize("size", [(3, 5), (15, 17), (31, 48)])
+def test_two_lanes_per_cell_with_the_shock_fix(size, recfix):
+    p = state("dry", *size, seed=11)
+    ref = Oracle(p, recfix=recfix).fvtd()
+    s = swm.Solver.from_problem(p, recfix=recfix)
+    got = s.fvtd()
+    for k in FVTD_KEYS:
+        a, b = fvtd_view(got, k), fvtd_view(ref, k)
+        assert same_bits(a, b), f"{size} fix {recfix} {k}: {describe_diff(a, b)}"
