@@ -29,8 +29,9 @@ constexpr int kTile = 16;             // k_fvtd_source_update tiles: 16x16 cells
 
 // Tile shapes of k_fvtd: an x-face tile takes xw x xh threads and produces
 // xw-1 faces per row; a y-face tile yw x yh threads and yh-1 faces per column;
-// a source tile sw x sh threads and cells.  Wider tiles recompute fewer halo sweeps; narrower ones waste
-// fewer threads on small grids.  The engine's autotuner picks one.
+// a source tile sw x sh threads and cells.  Wider tiles recompute fewer halo
+// sweeps; narrower ones waste fewer threads on small grids.  The engine's
+// autotuner picks one.
 struct FaceShape {
   int xw, xh, yw, yh, sw, sh;
 };

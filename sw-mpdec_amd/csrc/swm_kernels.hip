@@ -3,20 +3,26 @@
 // build, and the explicit schemes of the build without it -- over all active
 // jobs of an engine.
 //
-// One FVTimeDerivative (src/finitevolume.f90:402-440) is two launches, each
-// covering every job and up to three DeC nodes:
+// One FVTimeDerivative (src/finitevolume.f90:402-440) covers every job and up
+// to three DeC nodes:
 //   k_fvtd         x faces: halo tile -> ConsToPrim -> WENO5 first sweep along
 //                  x (shared through LDS) -> second sweep along y at the 4 Gauss
 //                  points -> positivity limiter on h -> Rusanov -> Gauss sum;
 //                  y faces: the same; source term (h-only WENO5 point values
-//                  times -g db)
-//   k_fvtd_update  UpdateTimeDerivative: Ut(2:3) and face mass fluxes / dx
-// The Patankar assembly fuses the first Jacobi sweep and carries the DeC
-// momentum update of the same nodes (disjoint arrays).  Every Jacobi sweep
-// writes per-block sums of |x_new - x_old|; a one-block-per-job kernel takes
-// the stop decision of src/jacobi_iteration.f90:71 on the device.  No grid-wide
-// fences are used: on a multi-XCD device an agent-scope fence writes back the
-// L2, so the kernel boundary is the cheap way to publish partial sums.
+//                  times -g db): one launch where the device would be left
+//                  idle, launches of their own on large grids
+//   the update     UpdateTimeDerivative: Ut(2:3) and face mass fluxes / dx, in
+//                  k_fvtd_update, with the sources in k_fvtd_source_update, or
+//                  inside the assembly that reads them
+// The Patankar assembly carries the DeC momentum update of the same nodes
+// (disjoint arrays).  k_solve runs the Jacobi iteration of the grids whose
+// systems fit the register files, stop decisions included (swm_engine.cpp,
+// solve_tables).  Larger grids get a launch per sweep: the first inside the
+// assembly, each with per-block sums of |x_new - x_old|, and a one-block-per-job
+// kernel takes the stop decision of src/jacobi_iteration.f90:71 on the device.
+// Outside k_solve no grid-wide waits are used: on a multi-XCD device an
+// agent-scope fence writes back the L2, so the kernel boundary is the cheap way
+// to publish partial sums.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -643,7 +649,8 @@ __device__ __forceinline__ void source_tile(double* smem, const JobDev& J, int t
 // launches, the sources: x-face, y-face and source tiles of every job in one
 // launch, the three kinds being independent of each other.  On grids that do
 // not fill the device they then run side by side (32^2: 11.8 us for 11.3 + 10.6
-// one after the other; 128^2 lake: 20.9 us with the sources).  Launches that
+// one after the other, 7.9 with two lanes per cell; 128^2 lake: 22 us with the
+// sources).  Launches that
 // fill it several times over gain nothing from that, and their sources run
 // better with the update (k_fvtd_source_update).
 //
@@ -1122,6 +1129,19 @@ __device__ __forceinline__ const gdouble* system_rhs(const JobDev& J, const SysL
   return G(S.hp_view ? J.hres[2] : J.h);
 }
 
+// Block b's place among k_assemble's n, for every XCD to work on one run of
+// them (blocks are dealt round-robin to the 8 XCDs, each with an L2 of its
+// own): the fluxes and depths of a cell's row neighbours are then read by the
+// same XCD, a few blocks earlier or later (257^2 17.9 -> 15.7 us, 1024^2 80 ->
+// 75.5, 2048^2 363 -> 351; k_sweep, with one stencil value per system, gained
+// nothing).  Launched with xcd_blocks(n) blocks, those with places >= n to
+// spare; few blocks are taken as they come.
+constexpr int kXcdFrom = 64;
+__device__ __forceinline__ int xcd_chunk(int b, int n) {
+  return n < kXcdFrom ? b : (b & 7) * ((n + 7) / 8) + (b >> 3);
+}
+inline int xcd_blocks(int n) { return n < kXcdFrom ? n : (n + 7) / 8 * 8; }
+
 // Cell blocks per block of the assembly with the first sweep, on large grids:
 // the block's look-ups and its four sums over the block are shared by 1024
 // cells, and k_decide, which reads all partial sums with one block at 14 bytes
@@ -1139,11 +1159,13 @@ __host__ __device__ inline int sum_blocks(const EngineArgs& E, int nblk) {
 // it only the matrix, for k_solve.  blockIdx.y picks the system where the grid
 // has that dimension (launch_assemble_matrix), else the block does them all.
 template <int R, bool FIRST, bool FRESH = false>
-__global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* blocks,
+__global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* blocks, int nblocks,
                                                   SysList S) {
   __shared__ double red[4];
   __shared__ double sq[4 * R * 256];  // [slot*R + node][thread]: face mass fluxes
-  const TileRef T = tile_of(E, blocks, blockIdx.x);
+  const int place = xcd_chunk(blockIdx.x, nblocks);
+  if (place >= nblocks) return;
+  const TileRef T = tile_of(E, blocks, place);
   const JobDev& J = E.jobs[T.job];
   if (skipped_stage(E, T.job)) return;
   const int nx = J.nx, ny = J.ny, n = J.n;
@@ -1982,7 +2004,8 @@ __device__ __forceinline__ bool solves_open(const JobStatus* st, int nsolve) {
 // U^{n+1} = Ua(MSteps) (src/timediscretization.f90:564,662,762), node
 // mf = MSteps - 1 here, of the accepted steps.  TimeStep's partial maxima of
 // the next step (next_dt) come from the values on their way, for a pass over
-// the state less (2048^2: 35 + 35 -> COMMIT2048 us).
+// the state less; small grids save a launch, 2048^2 breaks even (35 + 35 us
+// apart, 71 here).
 __global__ __launch_bounds__(256) void k_commit(EngineArgs E, const TileRef* blocks, int mf,
                                                 int nsolve, int next_dt) {
   const TileRef T = tile_of(E, blocks, blockIdx.x);
@@ -2391,11 +2414,12 @@ void launch_keep_state(const EngineArgs& E, const TileRef* cb, int ncb, int m, h
 void launch_assemble(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl, int njobs,
                      const SysList& S, hipStream_t s) {
   if (!ncb) return;
-  const dim3 grid(cdiv(ncb, sum_blocks(E, ncb)));  // one job: ncb is its nblk
+  const int nb = cdiv(ncb, sum_blocks(E, ncb));  // one job: ncb is its nblk
+  const dim3 grid(xcd_blocks(nb));
   if (S.nr == 2)
-    hipLaunchKernelGGL((k_assemble<2, true>), grid, dim3(256), 0, s, E, cb, S);
+    hipLaunchKernelGGL((k_assemble<2, true>), grid, dim3(256), 0, s, E, cb, nb, S);
   else
-    hipLaunchKernelGGL((k_assemble<4, true>), grid, dim3(256), 0, s, E, cb, S);
+    hipLaunchKernelGGL((k_assemble<4, true>), grid, dim3(256), 0, s, E, cb, nb, S);
   hipLaunchKernelGGL(k_decide<true>, dim3(njobs), dim3(256), 0, s, E, jl, S);
 }
 
@@ -2416,20 +2440,20 @@ void launch_sweep(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl
 }
 
 // A block of k_assemble holds 33 KB of LDS, so 1024 run at once; below that
-// the systems of a cell get blocks of their own (32^2: 12 -> ASM32 us), from
+// the systems of a cell get blocks of their own (32^2: 12 -> 6 us), from
 // there on one block shares the face fluxes between them.
 void launch_assemble_matrix(const EngineArgs& E, const TileRef* cb, int ncb, const SysList& S,
                             hipStream_t s) {
   if (!ncb) return;
-  const dim3 grid(ncb, ncb < 1024 ? S.count : 1);
+  const dim3 grid(xcd_blocks(ncb), ncb < 1024 ? S.count : 1);
   if (S.nr == 2 && S.fresh)
-    hipLaunchKernelGGL((k_assemble<2, false, true>), grid, dim3(256), 0, s, E, cb, S);
+    hipLaunchKernelGGL((k_assemble<2, false, true>), grid, dim3(256), 0, s, E, cb, ncb, S);
   else if (S.nr == 2)
-    hipLaunchKernelGGL((k_assemble<2, false>), grid, dim3(256), 0, s, E, cb, S);
+    hipLaunchKernelGGL((k_assemble<2, false>), grid, dim3(256), 0, s, E, cb, ncb, S);
   else if (S.fresh)
-    hipLaunchKernelGGL((k_assemble<4, false, true>), grid, dim3(256), 0, s, E, cb, S);
+    hipLaunchKernelGGL((k_assemble<4, false, true>), grid, dim3(256), 0, s, E, cb, ncb, S);
   else
-    hipLaunchKernelGGL((k_assemble<4, false>), grid, dim3(256), 0, s, E, cb, S);
+    hipLaunchKernelGGL((k_assemble<4, false>), grid, dim3(256), 0, s, E, cb, ncb, S);
 }
 
 void launch_solve(const EngineArgs& E, const SolveRef* refs, int first, int nblk, int form, int nb,
