@@ -541,7 +541,8 @@ constexpr int kSplitTiles = 256;
 
 // fluxes_left, where an assembly for k_solve follows: set when the update is
 // left to it (SysList::fresh).
-int fvtd_launch(swm_engine* e, Tables& T, const NodeList& L, int* fluxes_left = nullptr) {
+int fvtd_launch(swm_engine* e, Tables& T, const NodeList& L, int* fluxes_left = nullptr,
+                bool always_left = false) {
   EngineArgs a = eargs(e, T);
   hipStream_t s = e->stream;
   int sh = e->cur_shape;
@@ -561,7 +562,10 @@ int fvtd_launch(swm_engine* e, Tables& T, const NodeList& L, int* fluxes_left = 
   } else {  // also while events tell the kinds apart
     timed(e, 0, [&] { launch_fvtd(a, sh, xt, nxt, nullptr, 0, nullptr, 0, L, s); });
     timed(e, 1, [&] { launch_fvtd(a, sh, nullptr, 0, yt, nyt, nullptr, 0, L, s); });
-    timed(e, 2, [&] { launch_fvtd_source_update(a, T.dct, T.nct, L, s); });
+    if (fluxes_left && always_left && nst == 0 && !(e->prof.mask & 7u))
+      *fluxes_left = 1;
+    else
+      timed(e, 2, [&] { launch_fvtd_source_update(a, T.dct, T.nct, L, s); });
   }
   LAUNCHCK(e);
   return SWM_OK;
@@ -662,6 +666,9 @@ constexpr double kBRK65[6] = {0.077777777777777778, 0., 0.35555555555555556,
 int explicit_body(swm_engine* e, Tables& T, const SchemeDef& D) {
   EngineArgs a = eargs(e, T);
   hipStream_t s = e->stream;
+  // the scratch slot whose fluxes a derivative slot still is, or -1
+  int left[kStates];
+  std::fill(left, left + kStates, -1);
   // FVTimeDerivative of state slots into derivative slots, Ut(1:3)
   auto fvtd = [&](std::initializer_list<std::pair<int, int>> in_out) {
     NodeList L{};
@@ -672,10 +679,27 @@ int explicit_body(swm_engine* e, Tables& T, const SchemeDef& D) {
       L.slot[L.count] = L.count;
       ++L.count;
     }
-    return fvtd_launch(e, T, L);
+    int fluxes = 0;
+    const int rc = fvtd_launch(e, T, L, &fluxes, true);
+    for (int i = 0; i < L.count; ++i) left[L.out[i]] = fluxes ? L.slot[i] : -1;
+    return rc;
   };
-  auto comb = [&](const CombOp& op) {
+  // store: mask of the derivative slots that a later combination reads again
+  auto comb = [&](CombOp op, unsigned store = 0) {
+    op.nfresh = 0;
+    for (int t = 0; t < op.nterm; ++t) {
+      op.fresh[t] = -1;
+      if (!op.deriv[t] || left[op.src[t]] < 0) continue;
+      for (int q = 0; q < op.nfresh; ++q)
+        if (op.fsrc[q] == op.src[t]) op.fresh[t] = q;
+      if (op.fresh[t] >= 0) continue;
+      op.fresh[t] = op.nfresh;
+      op.fslot[op.nfresh] = left[op.src[t]];
+      op.fsrc[op.nfresh] = op.src[t];
+      op.fstore[op.nfresh++] = (store >> op.src[t]) & 1u;
+    }
     timed(e, 3, [&] { launch_combine(a, T.dcb, T.ncb, op, s); });
+    std::fill(left, left + kStates, -1);
   };
   // the writer's state: the input of the step's last FVTD, before a stage
   // combination overwrites its slot
@@ -701,7 +725,8 @@ int explicit_body(swm_engine* e, Tables& T, const SchemeDef& D) {
                    {{X, 0, 0.62010185138540}, {X, 2, 0.37989814861460}, {F, 0, 0.25189177424738}}));
       if ((rc = fvtd({{3, 0}}))) return rc;
       comb(comb_op(0, 4, 0,
-                   {{X, 0, 0.17807995410773}, {X, 3, 0.82192004589227}, {F, 0, 0.54497475021237}}));
+                   {{X, 0, 0.17807995410773}, {X, 3, 0.82192004589227}, {F, 0, 0.54497475021237}}),
+           1u);
       // K5 = Ut of stage 4 stays in derivative slot 0; stage 5's goes to 1
       if ((rc = fvtd({{4, 1}}))) return rc;
       keep(4);
@@ -720,7 +745,7 @@ int explicit_body(swm_engine* e, Tables& T, const SchemeDef& D) {
           op.c[0][op.nterm] = kARK65[st][j];
           ++op.nterm;
         }
-        comb(op);
+        comb(op, 1u << (st - 1));
         if ((rc = fvtd({{1, st}}))) return rc;
       }
       keep(1);
@@ -751,7 +776,7 @@ int explicit_body(swm_engine* e, Tables& T, const SchemeDef& D) {
           op.src[r] = src[r];
         }
         op.nterm = 4;
-        comb(op);
+        comb(op, kk == 1 ? 1u : 0u);
         if (kk != 5) {
           if ((rc = fvtd({{1, 1}, {2, 2}, {3, 3}}))) return rc;
           if (kk == 4) keep(3);

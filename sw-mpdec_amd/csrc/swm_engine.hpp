@@ -271,6 +271,10 @@ struct CombOp {
   int out[kMaxOut];
   int deriv[kMaxTerms];
   int src[kMaxTerms];
+  // the derivatives that are still fluxes: scratch slot, derivative slot, and
+  // whether to store them there; fresh: a term's index among them, or -1
+  int nfresh, fslot[kSlots], fsrc[kSlots], fstore[kSlots];
+  int fresh[kMaxTerms];
   double c[kMaxOut][kMaxTerms];
 };
 

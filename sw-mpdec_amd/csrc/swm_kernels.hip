@@ -1129,7 +1129,7 @@ __device__ __forceinline__ const gdouble* system_rhs(const JobDev& J, const SysL
   return G(S.hp_view ? J.hres[2] : J.h);
 }
 
-// Block b's place among k_assemble's n, for every XCD to work on one run of
+// Block b's place among n (k_assemble's), for every XCD to work on one run of
 // them (blocks are dealt round-robin to the 8 XCDs, each with an L2 of its
 // own): the fluxes and depths of a cell's row neighbours are then read by the
 // same XCD, a few blocks earlier or later (257^2 17.9 -> 15.7 us, 1024^2 80 ->
@@ -2208,21 +2208,95 @@ __device__ __forceinline__ const gdouble* deriv_var(const JobDev& J, int v, int 
 // Every source value is loaded once per variable (fully unrolled over
 // kMaxTerms, guarded by nterm, so the values stay in registers) and serves
 // each of the op.nout outputs, which differ only in their weights.
-__global__ __launch_bounds__(256) void k_combine(EngineArgs E, const TileRef* blocks, CombOp op) {
-  const TileRef T = tile_of(E, blocks, blockIdx.x);
+//
+// FRESH: op.nfresh derivatives are still the fluxes of the FVTD before, in
+// their scratch slots, with the sources in d2, d3; they are taken from there
+// (update_cell's arithmetic) and stored only where a later stage reads them
+// again.  That spares the update's launch and its pass over memory: per stage
+// 64^2 7.7 -> 5.8 us (RK65), 300x417 11.0 -> 8.3 (SSPRK4), 1000x700 55 -> 38
+// (DeC5, three nodes), 1500x1400 87 -> 68 (RK65).  Bound by latency on small
+// grids, by memory on large ones, where the blocks in runs per XCD share the
+// rows' y fluxes (1000x700: 45 -> 38).
+template <bool FRESH>
+__global__ __launch_bounds__(256) void k_combine(EngineArgs E, const TileRef* blocks, int nblocks,
+                                                 CombOp op) {
+  const int place = FRESH ? xcd_chunk(blockIdx.x, nblocks) : blockIdx.x;
+  if (FRESH && place >= nblocks) return;
+  const TileRef T = tile_of(E, blocks, place);
   const JobDev& J = E.jobs[T.job];
   if (skipped_stage(E, T.job)) return;
-  const int k = T.tile * kCellBlock + threadIdx.x;
+  const int k0 = T.tile * kCellBlock, k = k0 + threadIdx.x;
   if (k >= J.n) return;
   const double dt = E.status[T.job].dt;
+  // The loads of a phase before any use or store: a chain of them, pointers from
+  // the job's descriptor first, is most of what small grids wait for.
+  double base[3], x[3][kMaxTerms];
 #pragma unroll
-  for (int v = 0; v < 3; ++v) {
-    double x[kMaxTerms];
+  for (int t = 0; t < kMaxTerms; ++t)
+    if (t < op.nterm && !(FRESH && op.fresh[t] >= 0)) {
+#pragma unroll
+      for (int v = 0; v < 3; ++v)
+        x[v][t] = op.deriv[t] ? deriv_var(J, v, op.src[t])[k] : state_var(J, v, op.src[t])[k];
+    }
+#pragma unroll
+  for (int v = 0; v < 3; ++v) base[v] = op.mode == 0 ? 0. : state_var(J, v, op.base)[k];
+  if (FRESH) {
+    int ci, cj;
+    cell_ij(k0 % J.nx, k0 / J.nx, threadIdx.x, J.nx, ci, cj);
+    const size_t fw = (size_t)cj * (J.nx + 1) + ci, fe = fw + 1;  // x faces
+    const size_t gs = k, gn = gs + J.nx;                          // y faces
+    const OverDx over(J);
+    double ut[kSlots][3];
+#pragma unroll
+    for (int q = 0; q < kSlots; ++q)
+      if (q < op.nfresh) {
+        const int sl = op.fslot[q], to = op.fsrc[q];
+        double a[3], b[3], qa[3], qb[3], S[3] = {0., 0., 0.};
+        Numerators num{over.shared};
+#pragma unroll
+        for (int v = 0; v < 3; ++v) {
+          const double fxe = G(J.FX[sl][v])[fe], fxw = G(J.FX[sl][v])[fw];
+          const double fyn = G(J.FY[sl][v])[gn], fys = G(J.FY[sl][v])[gs];
+          if (v > 0 && J.bathy)
+            S[v] = deriv_var(J, v, to)[k];
+          else if (v > 0 && J.wb)
+            S[v] = S[v] - G(v == 1 ? J.SWB2 : J.SWB3)[k];
+          a[v] = fxe - fxw;
+          b[v] = fyn - fys;
+        }
+#pragma unroll
+        for (int v = 0; v < 3; ++v) {
+          qa[v] = div_by(num(a[v]), over.dx, over.rdx);
+          qb[v] = div_by(num(b[v]), over.dy, over.rdy);
+        }
+        if (!num.ok) {
+#pragma unroll
+          for (int v = 0; v < 3; ++v) {
+            qa[v] = over.x(a[v]);
+            qb[v] = over.y(b[v]);
+          }
+        }
+        // the source is never -0, so the sign of a zero quotient has no effect
+#pragma unroll
+        for (int v = 0; v < 3; ++v) ut[q][v] = S[v] - qa[v] - qb[v];
+        if (op.fstore[q]) {
+          G(J.d1[to])[k] = ut[q][0];
+          G(J.d2[to])[k] = ut[q][1];
+          G(J.d3[to])[k] = ut[q][2];
+        }
+        // a derivative at a time: the loads of all three take 152 registers
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
     for (int t = 0; t < kMaxTerms; ++t)
-      if (t < op.nterm)
-        x[t] = op.deriv[t] ? deriv_var(J, v, op.src[t])[k] : state_var(J, v, op.src[t])[k];
-    const double base = op.mode == 0 ? 0. : state_var(J, v, op.base)[k];
+#pragma unroll
+      for (int v = 0; v < 3; ++v)
+#pragma unroll
+        for (int q = 0; q < kSlots; ++q)
+          if (t < op.nterm && op.fresh[t] == q) x[v][t] = ut[q][v];
+  }
+#pragma unroll
+  for (int v = 0; v < 3; ++v) {
 #pragma unroll
     for (int o = 0; o < kMaxOut; ++o) {
       if (o >= op.nout) break;
@@ -2232,7 +2306,7 @@ __global__ __launch_bounds__(256) void k_combine(EngineArgs E, const TileRef* bl
 #pragma unroll
         for (int t = 0; t < kMaxTerms; ++t)
           if (t < op.nterm) {
-            const double term = op.deriv[t] ? (c[t] * x[t]) * dt : c[t] * x[t];
+            const double term = op.deriv[t] ? (c[t] * x[v][t]) * dt : c[t] * x[v][t];
             acc = t == 0 ? term : acc + term;
           }
       } else if (op.mode == 1) {
@@ -2240,15 +2314,15 @@ __global__ __launch_bounds__(256) void k_combine(EngineArgs E, const TileRef* bl
 #pragma unroll
         for (int t = 0; t < kMaxTerms; ++t)
           if (t < op.nterm) {
-            const double term = c[t] * x[t];
+            const double term = c[t] * x[v][t];
             sum = t == 0 ? term : sum + term;
           }
-        acc = base + sum * dt;
+        acc = base[v] + sum * dt;
       } else {
-        acc = base;
+        acc = base[v];
 #pragma unroll
         for (int t = 0; t < kMaxTerms; ++t)
-          if (t < op.nterm) acc = acc + (dt * c[t]) * x[t];
+          if (t < op.nterm) acc = acc + (dt * c[t]) * x[v][t];
       }
       const int out = op.out[o];
       G(v == 0 ? J.sh[out] : v == 1 ? J.shu[out] : J.shv[out])[k] = acc;
@@ -2429,7 +2503,11 @@ void launch_hp_view(const EngineArgs& E, const TileRef* cb, int ncb, int from_un
 
 void launch_combine(const EngineArgs& E, const TileRef* cb, int ncb, const CombOp& op,
                     hipStream_t s) {
-  if (ncb) hipLaunchKernelGGL(k_combine, dim3(ncb), dim3(256), 0, s, E, cb, op);
+  if (!ncb) return;
+  if (op.nfresh)
+    hipLaunchKernelGGL(k_combine<true>, dim3(xcd_blocks(ncb)), dim3(256), 0, s, E, cb, ncb, op);
+  else
+    hipLaunchKernelGGL(k_combine<false>, dim3(ncb), dim3(256), 0, s, E, cb, ncb, op);
 }
 
 void launch_sweep(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl, int njobs,
