@@ -539,10 +539,11 @@ constexpr long kFvtdTogether = 8L * 262144;
 // about one per CU.
 constexpr int kSplitTiles = 256;
 
-// fluxes_left, where an assembly for k_solve follows: set when the update is
-// left to it (SysList::fresh).
+// fluxes_left: set when the update is left to what follows (SysList::fresh,
+// CombOp::fresh).  Small launches leave it with small_left, large ones where no
+// job has bathymetry (with sources the update runs with them).
 int fvtd_launch(swm_engine* e, Tables& T, const NodeList& L, int* fluxes_left = nullptr,
-                bool always_left = false) {
+                bool small_left = false) {
   EngineArgs a = eargs(e, T);
   hipStream_t s = e->stream;
   int sh = e->cur_shape;
@@ -555,14 +556,14 @@ int fvtd_launch(swm_engine* e, Tables& T, const NodeList& L, int* fluxes_left = 
   const bool small = (long)(nxt + nyt) * L.count * F.sw * F.sh <= kFvtdTogether;
   if (small && !(e->prof.mask & 7u)) {
     launch_fvtd(a, sh, xt, nxt, yt, nyt, st, nst, L, s);
-    if (fluxes_left)
+    if (fluxes_left && small_left)
       *fluxes_left = 1;
     else
       launch_fvtd_update(a, T.dcb, T.ncb, L, s);
   } else {  // also while events tell the kinds apart
     timed(e, 0, [&] { launch_fvtd(a, sh, xt, nxt, nullptr, 0, nullptr, 0, L, s); });
     timed(e, 1, [&] { launch_fvtd(a, sh, nullptr, 0, yt, nyt, nullptr, 0, L, s); });
-    if (fluxes_left && always_left && nst == 0 && !(e->prof.mask & 7u))
+    if (fluxes_left && nst == 0 && !(e->prof.mask & 7u))
       *fluxes_left = 1;
     else
       timed(e, 2, [&] { launch_fvtd_source_update(a, T.dct, T.nct, L, s); });
@@ -892,7 +893,7 @@ int step_body(swm_engine* e, Tables& T, const StepPlan& P) {
         L.slot[k] = k;
       }
       S.fresh = 0;
-      rc = fvtd_launch(e, T, L, P.solve && T.ncbw == 0 ? &S.fresh : nullptr);
+      rc = fvtd_launch(e, T, L, &S.fresh, P.solve && T.ncbw == 0);
       if (rc) return rc;
       if (e->keep_count && kk == D.kcorr - 1)
         launch_keep_state(a, T.dcb, T.ncb, D.msteps - 1, s);

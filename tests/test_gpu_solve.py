@@ -114,6 +114,27 @@ def test_grouped_residual_sums(size):
     assert same_bits(a.download(), b.download())
 
 
+@pytest.mark.parametrize("scheme,wb", [(5, False), (5, True), (7, False)])
+@pytest.mark.parametrize("size", [(1000, 900), (1100, 1030)], ids=lambda s: f"{s[0]}x{s[1]}")
+def test_assembly_of_large_grids_from_the_fluxes(size, scheme, wb):
+    """Without bathymetry the assembly takes the fluxes as they are, before the
+    one-launch solve and before launches per sweep; recording events keeps the
+    update before it."""
+    p = random_state(*size, 9)
+    if wb:
+        p.wellbalanced, p.Uwb = True, random_state(*size, 10, 0.01).U0
+    out = []
+    for events in (False, True):
+        s = swm.Solver.from_problem(p)
+        s.set_timescheme(scheme)
+        s.set_hp_association(swm.HP_BY_NODE)
+        s.profile(events)
+        dts, sweeps, _ = s.run_steps(2)
+        out.append((s.download(), dts, sweeps))
+    assert (out[0][1] == out[1][1]).all() and (out[0][2] == out[1][2]).all()
+    assert same_bits(out[0][0], out[1][0])
+
+
 @pytest.mark.parametrize("size", [(32, 32), (80, 80)], ids=lambda s: f"{s[0]}x{s[1]}")
 def test_open_decision_is_taken_by_the_sequential_sum(size):
     """A uniform depth 1 at rest with the tolerance 1: the initial residual is
