@@ -541,9 +541,10 @@ constexpr int kSplitTiles = 256;
 
 // fluxes_left: set when the update is left to what follows (SysList::fresh,
 // CombOp::fresh).  Small launches leave it with small_left, large ones where no
-// job has bathymetry (with sources the update runs with them).
-int fvtd_launch(swm_engine* e, Tables& T, const NodeList& L, int* fluxes_left = nullptr,
-                bool small_left = false) {
+// job has bathymetry (with sources the update runs with them).  source0: the
+// slot that takes the first node's sources then, in place of its own.
+int fvtd_launch(swm_engine* e, Tables& T, NodeList L, int* fluxes_left = nullptr,
+                bool small_left = false, int source0 = -1) {
   EngineArgs a = eargs(e, T);
   hipStream_t s = e->stream;
   int sh = e->cur_shape;
@@ -555,8 +556,10 @@ int fvtd_launch(swm_engine* e, Tables& T, const NodeList& L, int* fluxes_left = 
   const FaceShape& F = kShapes[sh];
   const bool small = (long)(nxt + nyt) * L.count * F.sw * F.sh <= kFvtdTogether;
   if (small && !(e->prof.mask & 7u)) {
+    const bool leave = fluxes_left && small_left;
+    if (leave && source0 >= 0) L.out[0] = source0;
     launch_fvtd(a, sh, xt, nxt, yt, nyt, st, nst, L, s);
-    if (fluxes_left && small_left)
+    if (leave)
       *fluxes_left = 1;
     else
       launch_fvtd_update(a, T.dcb, T.ncb, L, s);
@@ -805,13 +808,15 @@ int step_body(swm_engine* e, Tables& T, const StepPlan& P) {
   L0.m[0] = 0;
   L0.out[0] = 0;
   L0.slot[0] = 0;
-  int rc = fvtd_launch(e, T, L0);
+  int left0 = 0;
+  int rc = fvtd_launch(e, T, L0, &left0, P.solve && T.ncbw == 0, kNode0Source);
   if (rc) return rc;
   // the writer's state: the input of the step's last FVTD (U^n when the
   // scheme has a single correction)
   if (e->keep_count && D.kcorr == 1) launch_keep_state(a, T.dcb, T.ncb, 0, s);
   SysList S{};
   for (int r = 0; r < 4; ++r) S.src[r] = 0;
+  S.fresh = left0 ? 2 : 0;
   S.hp_is_un = 1;
   S.track_min = e->track_min ? 1 : 0;
   S.nr = D.msteps;

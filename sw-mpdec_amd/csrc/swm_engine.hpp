@@ -278,6 +278,8 @@ struct CombOp {
   double c[kMaxOut][kMaxTerms];
 };
 
+constexpr int kNode0Source = 1;
+
 // Patankar/Jacobi launch parameters (the same for every job of a step).
 struct SysList {
   int count;
@@ -289,7 +291,9 @@ struct SysList {
   int theta;            // THETA block: 0 mPDeC5, 1 the two-node schemes
   int hp_view;          // 1: denominators from hres[3], rhs from hres[2] (k_hp_view)
   int fresh;            // 1: nodes 1.. have their fluxes in slots 0.. and their sources in
-                        // d2, d3, and the assembly takes Ut and the mass fluxes from those
+                        // d2, d3, and the assembly takes Ut and the mass fluxes from those;
+                        // 2: so has node 0 (sources in slot kNode0Source), which stands for
+                        // all, and they are kept
 };
 
 // The time schemes, by the reference's timescheme number: the modified-

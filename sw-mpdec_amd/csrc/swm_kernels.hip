@@ -878,25 +878,29 @@ __device__ __forceinline__ void momentum_cell(const JobDev& J, const SysList& S,
 
 // What the assembly and the momentum update of a cell take from the FVTDs: the
 // mass fluxes / dx of its south, west, east and north faces at the R DeC nodes
-// and Ut(2:3).  Node 0's are kept by k_fvtd_update for all corrections.  With
-// FRESH the other nodes' are formed here from the face fluxes and the source
+// and Ut(2:3).  Node 0's are kept for all corrections, by the update or, FRESH =
+// 2, by the first correction's assembly, for which all nodes are node 0 (`keep`;
+// at_w, at_s: the cell has the first x or y face of its row or column).  With
+// FRESH = 1 the other nodes' are formed here from the face fluxes and the source
 // (as update_cell does), for a launch less per correction and, on large grids,
 // a pass over memory (update + assembly without bathymetry: 900x800 98 -> 68 us,
-// 1024^2 119 -> 99, 1500^2 331 -> 245, 2048^2 590 -> 448, three nodes); all
-// loads go out before the first quotient.
-template <int R, bool FRESH>
+// 1024^2 119 -> 99, 1500^2 331 -> 245, 2048^2 590 -> 448, three nodes; node 0:
+// 32^2 11.3 -> 6.2, 257^2 17.6 -> 13.0, 1024^2 92 -> 78); all loads go out
+// before the first quotient.
+template <int R, int FRESH>
 struct CellFluxes {
   double q[4][R], fu2[R], fu3[R];
   __device__ __forceinline__ CellFluxes(const JobDev& J, const SysList& S, int k, size_t fW,
-                                        size_t gS) {
+                                        size_t gS, bool keep, bool at_w, bool at_s) {
     const size_t fE = fW + 1, gN = gS + J.nx;
-    constexpr int R1 = FRESH ? R : 1;
+    constexpr int R0 = FRESH == 2 ? 0 : 1;         // the nodes formed here
+    constexpr int RL = FRESH == 2 ? 1 : R, R1 = FRESH ? RL : 1;
     double X[R1][2][2], Y[R1][2][2];  // [node][variable 2, 3][face]
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const bool here = FRESH && r > 0;
-      const gdouble* qx = G(here ? J.FX[r - 1][0] : J.qx[S.src[r]]);
-      const gdouble* qy = G(here ? J.FY[r - 1][0] : J.qy[S.src[r]]);
+    for (int r = 0; r < RL; ++r) {
+      const bool here = FRESH && r >= R0;
+      const gdouble* qx = G(here ? J.FX[r - R0][0] : J.qx[S.src[r]]);
+      const gdouble* qy = G(here ? J.FY[r - R0][0] : J.qy[S.src[r]]);
       q[0][r] = qy[gS];
       q[1][r] = qx[fW];
       q[2][r] = qx[fE];
@@ -907,15 +911,15 @@ struct CellFluxes {
       } else {
 #pragma unroll
         for (int v = 0; v < 2; ++v) {
-          X[r % R1][v][0] = G(J.FX[r - 1][v + 1])[fW];
-          X[r % R1][v][1] = G(J.FX[r - 1][v + 1])[fE];
-          Y[r % R1][v][0] = G(J.FY[r - 1][v + 1])[gS];
-          Y[r % R1][v][1] = G(J.FY[r - 1][v + 1])[gN];
+          X[r % R1][v][0] = G(J.FX[r - R0][v + 1])[fW];
+          X[r % R1][v][1] = G(J.FX[r - R0][v + 1])[fE];
+          Y[r % R1][v][0] = G(J.FY[r - R0][v + 1])[gS];
+          Y[r % R1][v][1] = G(J.FY[r - R0][v + 1])[gN];
         }
         fu2[r] = fu3[r] = 0.0;
-        if (J.bathy) {
-          fu2[r] = G(J.d2[r])[k];
-          fu3[r] = G(J.d3[r])[k];
+        if (J.bathy) {  // node 0's sources are in slot 1: other blocks may still read
+          fu2[r] = G(J.d2[FRESH == 2 ? kNode0Source : r])[k];  // them when FU2 is written
+          fu3[r] = G(J.d3[FRESH == 2 ? kNode0Source : r])[k];
         } else if (J.wb) {
           fu2[r] = 0.0 - G(J.SWB2)[k];
           fu3[r] = 0.0 - G(J.SWB3)[k];
@@ -927,7 +931,7 @@ struct CellFluxes {
     Numerators seen{over.shared};
     double dX[R1][2], dY[R1][2];
 #pragma unroll
-    for (int r = 1; r < R; ++r) {
+    for (int r = R0; r < RL; ++r) {
       for (int f = 0; f < 4; ++f) seen(q[f][r]);
 #pragma unroll
       for (int v = 0; v < 2; ++v) {
@@ -937,7 +941,7 @@ struct CellFluxes {
     }
     auto form = [&](auto ox, auto oy) {
 #pragma unroll
-      for (int r = 1; r < R; ++r) {
+      for (int r = R0; r < RL; ++r) {
         q[0][r] = oy(q[0][r]);
         q[1][r] = ox(q[1][r]);
         q[2][r] = ox(q[2][r]);
@@ -953,6 +957,22 @@ struct CellFluxes {
            [&](double a) { return div_by(a, over.dy, over.rdy); });
     else
       form([&](double a) { return over.x(a); }, [&](double a) { return over.y(a); });
+    if (FRESH != 2) return;
+    if (keep) {
+      G(J.FU2[0])[k] = fu2[0];
+      G(J.FU3[0])[k] = fu3[0];
+      G(J.qx[0])[fE] = q[2][0];
+      G(J.qy[0])[gN] = q[3][0];
+      if (at_w) G(J.qx[0])[fW] = q[1][0];
+      if (at_s) G(J.qy[0])[gS] = q[0][0];
+    }
+#pragma unroll
+    for (int r = 1; r < R; ++r) {
+#pragma unroll
+      for (int f = 0; f < 4; ++f) q[f][r] = q[f][0];
+      fu2[r] = fu2[0];
+      fu3[r] = fu3[0];
+    }
   }
 };
 
@@ -1160,7 +1180,7 @@ __host__ __device__ inline int sum_blocks(const EngineArgs& E, int nblk) {
 // FIRST: the first sweep and its residual sums, for a launch per sweep; without
 // it only the matrix, for k_solve.  blockIdx.y picks the system where the grid
 // has that dimension (launch_assemble_matrix), else the block does them all.
-template <int R, bool FIRST, bool FRESH = false>
+template <int R, bool FIRST, int FRESH = 0>
 __global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* blocks, int nblocks,
                                                   SysList S) {
   __shared__ double red[4];
@@ -1190,7 +1210,8 @@ __global__ __launch_bounds__(256) void k_assemble(EngineArgs E, const TileRef* b
       kW = j * nx + (i == 0 ? nx - 1 : i - 1);
       kE = j * nx + (i == nx - 1 ? 0 : i + 1);
       kN = (j == ny - 1 ? 0 : j + 1) * nx + i;
-      const CellFluxes<R, FRESH> F(J, S, k, (size_t)j * (nx + 1) + i, (size_t)j * nx + i);
+      const CellFluxes<R, FRESH> F(J, S, k, (size_t)j * (nx + 1) + i, (size_t)j * nx + i,
+                                     s0 == 0, i == 0, j == 0);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         sq[(0 * R + r) * 256 + tid] = F.q[0][r];
@@ -2487,19 +2508,23 @@ void launch_keep_state(const EngineArgs& E, const TileRef* cb, int ncb, int m, h
   if (ncb) hipLaunchKernelGGL(k_keep_state, dim3(ncb), dim3(256), 0, s, E, cb, m);
 }
 
+template <bool FIRST>
+void assemble(dim3 grid, const EngineArgs& E, const TileRef* cb, int nb, const SysList& S,
+              hipStream_t s) {
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, E, cb, nb, S); };
+  if (S.nr == 2)
+    S.fresh == 2 ? go(k_assemble<2, FIRST, 2>)
+                 : S.fresh ? go(k_assemble<2, FIRST, 1>) : go(k_assemble<2, FIRST>);
+  else
+    S.fresh == 2 ? go(k_assemble<4, FIRST, 2>)
+                 : S.fresh ? go(k_assemble<4, FIRST, 1>) : go(k_assemble<4, FIRST>);
+}
+
 void launch_assemble(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl, int njobs,
                      const SysList& S, hipStream_t s) {
   if (!ncb) return;
   const int nb = cdiv(ncb, sum_blocks(E, ncb));  // one job: ncb is its nblk
-  const dim3 grid(xcd_blocks(nb));
-  if (S.nr == 2 && S.fresh)
-    hipLaunchKernelGGL((k_assemble<2, true, true>), grid, dim3(256), 0, s, E, cb, nb, S);
-  else if (S.nr == 2)
-    hipLaunchKernelGGL((k_assemble<2, true>), grid, dim3(256), 0, s, E, cb, nb, S);
-  else if (S.fresh)
-    hipLaunchKernelGGL((k_assemble<4, true, true>), grid, dim3(256), 0, s, E, cb, nb, S);
-  else
-    hipLaunchKernelGGL((k_assemble<4, true>), grid, dim3(256), 0, s, E, cb, nb, S);
+  assemble<true>(dim3(xcd_blocks(nb)), E, cb, nb, S, s);
   hipLaunchKernelGGL(k_decide<true>, dim3(njobs), dim3(256), 0, s, E, jl, S);
 }
 
@@ -2529,15 +2554,7 @@ void launch_sweep(const EngineArgs& E, const TileRef* cb, int ncb, const int* jl
 void launch_assemble_matrix(const EngineArgs& E, const TileRef* cb, int ncb, const SysList& S,
                             hipStream_t s) {
   if (!ncb) return;
-  const dim3 grid(xcd_blocks(ncb), ncb < 1024 ? S.count : 1);
-  if (S.nr == 2 && S.fresh)
-    hipLaunchKernelGGL((k_assemble<2, false, true>), grid, dim3(256), 0, s, E, cb, ncb, S);
-  else if (S.nr == 2)
-    hipLaunchKernelGGL((k_assemble<2, false>), grid, dim3(256), 0, s, E, cb, ncb, S);
-  else if (S.fresh)
-    hipLaunchKernelGGL((k_assemble<4, false, true>), grid, dim3(256), 0, s, E, cb, ncb, S);
-  else
-    hipLaunchKernelGGL((k_assemble<4, false>), grid, dim3(256), 0, s, E, cb, ncb, S);
+  assemble<false>(dim3(xcd_blocks(ncb), ncb < 1024 ? S.count : 1), E, cb, ncb, S, s);
 }
 
 void launch_solve(const EngineArgs& E, const SolveRef* refs, int first, int nblk, int form, int nb,
