@@ -313,19 +313,35 @@ void timed(swm_engine* e, int cat, F&& launch) {
     e->prof.used = 2 * e->prof.cats.size();
 }
 
+// 16x16 face tiles of a launch up to which two lanes share a cell (split_faces):
+// about one per CU.
+constexpr int kSplitTiles = 256;
+
+int x_tiles(const JobDev& d, int sh) {
+  return cdiv(d.nx + 1, kShapes[sh].xw - 1) * cdiv(d.ny, kShapes[sh].xh);
+}
+int y_tiles(const JobDev& d, int sh) {
+  return cdiv(d.nx, kShapes[sh].yw) * cdiv(d.ny + 1, kShapes[sh].yh - 1);
+}
+// The shapes a grid can get: a large one, and any job set with it, never the
+// split one, which has most tiles (2048^2: half a millisecond of tables).
+int shapes_of(const JobDev& d) {
+  return x_tiles(d, 0) + y_tiles(d, 0) > kSplitTiles ? kNumShapes : kAllShapes;
+}
+
 void add_sources(Tables& T, int id, const JobDev& d) {
   if (!d.bathy) return;
-  for (int sh = 0; sh < kAllShapes; ++sh) {
+  for (int sh = 0; sh < shapes_of(d); ++sh) {
     const int nst = cdiv(d.nx, kShapes[sh].sw) * cdiv(d.ny, kShapes[sh].sh);
     for (int t = 0; t < nst; ++t) T.st[sh].push_back({id, t});
   }
 }
 
 void add_tiles(Tables& T, int id, const JobDev& d) {
-  for (int sh = 0; sh < kAllShapes; ++sh) {
-    const FaceShape& F = kShapes[sh];
-    const int nxt = cdiv(d.nx + 1, F.xw - 1) * cdiv(d.ny, F.xh);
-    const int nyt = cdiv(d.nx, F.yw) * cdiv(d.ny + 1, F.yh - 1);
+  for (int sh = 0; sh < shapes_of(d); ++sh) {
+    const int nxt = x_tiles(d, sh), nyt = y_tiles(d, sh);
+    T.xt[sh].reserve(T.xt[sh].size() + nxt);
+    T.yt[sh].reserve(T.yt[sh].size() + nyt);
     for (int t = 0; t < nxt; ++t) T.xt[sh].push_back({id, t});
     for (int t = 0; t < nyt; ++t) T.yt[sh].push_back({id, t});
   }
@@ -456,6 +472,10 @@ int upload_tables(swm_engine* e, Tables& T) {
     where.push_back({(void**)&dev, off});
     return (int)v.size();
   };
+  size_t total = 0;
+  for (int sh = 0; sh < kAllShapes; ++sh)
+    total += T.xt[sh].size() + T.yt[sh].size() + T.st[sh].size();
+  host.reserve((total + T.ct.size() + 3 * T.cb.size()) * sizeof(TileRef));
   for (int sh = 0; sh < kAllShapes; ++sh) {
     T.nxt[sh] = put(T.dxt[sh], T.xt[sh]);
     T.nyt[sh] = put(T.dyt[sh], T.yt[sh]);
@@ -534,10 +554,6 @@ EngineArgs eargs(swm_engine* e, const Tables& T) {
 // Threads of face tiles up to which the three kinds of k_fvtd's tiles share a
 // launch.  The device holds 262,144 at 4 waves per SIMD.
 constexpr long kFvtdTogether = 8L * 262144;
-
-// 16x16 face tiles of a launch up to which two lanes share a cell (split_faces):
-// about one per CU.
-constexpr int kSplitTiles = 256;
 
 // fluxes_left: set when the update is left to what follows (SysList::fresh,
 // CombOp::fresh).  Small launches leave it with small_left, large ones where no
