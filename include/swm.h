@@ -311,6 +311,7 @@ int swm_stage_min_h(swm_solver_t *h, double *hmin);
 int swm_set_execution(swm_solver_t *h, int use_graph, int margin);
 int swm_execution_stats(const swm_solver_t *h, long long stats[6]);
 int swm_status_reads(const swm_solver_t *h, long long *n);
+int swm_solve_stats(const swm_solver_t *h, long long stats[3]);
 int swm_set_tile_shape(swm_solver_t *h, int shape);
 int swm_tile_shape(const swm_solver_t *h, int dims[4]);
 
@@ -434,6 +435,15 @@ int swm_engine_execution_stats(const swm_engine_t *e, long long stats[6]);
  * the reference): one per batch of steps of the device time loop, plus one
  * per Jacobi check while a step runs in polling mode. */
 int swm_engine_status_reads(const swm_engine_t *e, long long *n);
+/* The Patankar solves in one launch (no counterpart in the reference; results
+ * are bitwise the same without them).  Their blocks wait for each other, each
+ * wait for about 25 ms at most; where one runs out, because other work keeps
+ * blocks off the device, the step is run again with a launch per sweep, and the
+ * next batches (16 the first time, twice as many each time, 4096 at most) go
+ * without such solves before they are tried again.
+ * stats: speculative steps launched with them, waits that ran out, batches
+ * left without them. */
+int swm_engine_solve_stats(const swm_engine_t *e, long long stats[3]);
 /* Tile shape of the face kernels (no counterpart in the reference; results
  * are bitwise the same with every shape): 0 = 16x16 threads for both face
  * directions, 1 = 32x16 for x faces and 16x32 for y faces (fewer redundant
@@ -478,6 +488,11 @@ int swm_debug_sync_cost(int nblk, int rounds, double us_per_round[3]);
  * :999-1136) on n five-point stencils q[5i..5i+4]: first[2i..2i+1] = (wm, wp),
  * second[4i..4i+3] = the 4 Gauss-point values. */
 int swm_debug_weno5(int n, const double *q, double *first, double *second);
+
+/* Test override of the polls after which a block of such a solve gives up
+ * waiting (0: every wait runs out at once, so every step that takes them is run
+ * again; < 0: the default, which no value exceeds). */
+int swm_debug_solve_polls(swm_solver_t *h, int polls);
 
 #ifdef __cplusplus
 }

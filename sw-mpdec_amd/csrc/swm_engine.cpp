@@ -184,6 +184,7 @@ struct Job {
   int hp_assoc = SWM_HP_AS_REFERENCE;     // depth view of the two-node schemes
   Tables own;          // tables covering this job alone
   int own_bathy = 0;   // dev.bathy as the tables have it
+  bool slots_clear = false;    // k_solve's slots and rounds agree (clear_slots)
   double* vout_buf = nullptr;  // the writer's state (dev.vout), when kept
   bool vout_valid = false;     // vout holds the state of the last step
 };
@@ -228,7 +229,12 @@ struct swm_engine {
   bool track_min = false;        // fold every stage depth into JobStatus::hmin
   int device = -1;
   int solve_blocks_max = 0;      // blocks of k_solve the device holds at once
-  bool solve_lost = false;       // a wait inside k_solve ran out: not used any more
+  int solve_polls = kSolvePolls;  // of a slot in k_solve's waits
+  // A wait inside k_solve ran out: batches left until k_solve is used again
+  // (solve_rest), and how often that was
+  int solve_rest = 0;
+  long long solve_losses = 0;
+  long long solve_steps = 0;     // speculative steps with k_solve
   // Step execution (results are identical either way; only speed differs):
   // speculative steps launch each correction's predicted sweeps without host
   // reads and check once at the end; they may be replayed from a captured
@@ -1108,6 +1114,23 @@ void consume_batch(swm_engine* e, Tables& T, const SchemeDef* sc,
   }
 }
 
+// Slots and rounds of a job's k_solve from the start: no slot holds the tag a
+// first round expects.  Wanted before the first solve and after a wait that ran
+// out, when a block may have published rounds that others never saw.
+int clear_slots(swm_engine* e, Job& J) {
+  const size_t n = solve_slot(J.dev.nx, J.dev.ny, kSolveForms, 0, 0, 0);
+  HIPCK(e, hipMemsetAsync(J.dev.slots, 0, n * sizeof(*J.dev.slots), e->stream));
+  HIPCK(e, hipMemsetAsync(&J.dev.status->rounds, 0, sizeof(JobStatus::rounds), e->stream));
+  J.slots_clear = true;
+  return SWM_OK;
+}
+
+// Batches without k_solve after the n-th wait that ran out: what kept blocks off
+// the device (another process, say) may pass or stay, and while it stays each
+// try costs the 25 ms of the wait and a step run twice.  Doubling from 16 to 4096
+// batches keeps that below 1% of the time.
+int solve_rest(long long losses) { return 16 << std::min<long long>(losses - 1, 8); }
+
 // The device time loop's clipping and stop test (src/timediscretization.f90:
 // 58-59, 83-94) for a plain solve.
 struct LoopArgs {
@@ -1135,7 +1158,11 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
   // every grid and no sweep limit is set) or every job swept by a launch per
   // sweep has a prediction for the scheme.
   bool spec = e->margin != -2 && !is_explicit(*sc);  // nothing to predict without solves
-  P.solve = spec && !e->solve_lost && !e->track_min && !T.sv[0].empty();
+  P.solve = spec && !e->track_min && !T.sv[0].empty();
+  if (P.solve && T.solve_waits && e->solve_rest > 0) {
+    --e->solve_rest;
+    P.solve = false;
+  }
   SolveRight right;
   if (P.solve && T.solve_waits) P.solve = right.take(e->device);
   const bool open_limit = P.solve && e->margin < 0;  // k_solve runs to the stop rule
@@ -1150,12 +1177,19 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
   if (host_dt || (!spec && !is_explicit(*sc)) || tune) steps = 1;
   BatchArgs B{};
   B.max_steps = steps;
+  B.polls = e->solve_polls;
   if (loop) {
     B.loop = 1;
     B.t = loop->t;
     B.t_an = loop->t_an;
     B.t_end = loop->t_end;
   }
+  if (P.solve && T.solve_waits)
+    for (int id : T.jl)
+      if (!e->jobs[id]->slots_clear) {
+        int rc = clear_slots(e, *e->jobs[id]);
+        if (rc) return rc;
+      }
   e->gated = 1;
   struct Ungate {
     swm_engine* e;
@@ -1231,11 +1265,15 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
     }
     if (rc) return rc;
     e->spec_steps += steps;
-    bool overrun = false;
+    if (P.solve) e->solve_steps += steps;
+    bool overrun = false, lost = false;
     for (int q = 0; q < T.njobs; ++q) {
       overrun = overrun || e->hstatus[T.jl[q]].halt == kHaltOverrun;
-      e->solve_lost = e->solve_lost || e->hstatus[T.jl[q]].solve_lost;
+      if (!e->hstatus[T.jl[q]].solve_lost) continue;
+      e->jobs[T.jl[q]]->slots_clear = false;
+      lost = true;
     }
+    if (lost) e->solve_rest = solve_rest(++e->solve_losses);
     if (tune && !overrun) {
       const bool captured = e->graph_captures != captures0;
       if (captured && e->tune_skips < 2) {
@@ -1524,6 +1562,7 @@ int alloc_job(swm_engine* e, int nx, int ny, double dx, double dy, double g, dou
   for (int i = 0; i < 13; ++i) J.pred[i] = 4;
   J.have_pred = false;
   J.pred_sc = nullptr;
+  J.slots_clear = false;
   J.log = nullptr;
   J.scheme = &kSchemes[0];
   J.hp_assoc = SWM_HP_AS_REFERENCE;
@@ -1534,8 +1573,6 @@ int alloc_job(swm_engine* e, int nx, int ny, double dx, double dy, double g, dou
   int rc = upload_tables(e, J.own);
   if (rc) return rc;
   HIPCK(e, hipMemsetAsync(e->dstatus.p + id, 0, sizeof(JobStatus), e->stream));
-  // no slot holds the tag a first round expects
-  HIPCK(e, hipMemsetAsync(D.slots, 0, nslots * sizeof(*D.slots), e->stream));
   // the step-count stop of the device time loop (-1: none)
   launch_set_steps_left(e->dstatus.p + id, nsteps > 0 ? nsteps : -1, e->stream);
   LAUNCHCK(e);
@@ -2067,6 +2104,14 @@ int swm_engine_execution_stats(const swm_engine_t* e, long long out[6]) {
 int swm_engine_status_reads(const swm_engine_t* e, long long* n) {
   if (!e || !n) return SWM_E_ARG;
   *n = e->status_reads;
+  return SWM_OK;
+}
+
+int swm_engine_solve_stats(const swm_engine_t* e, long long out[3]) {
+  if (!e || !out) return SWM_E_ARG;
+  out[0] = e->solve_steps;
+  out[1] = e->solve_losses;
+  out[2] = e->solve_rest;
   return SWM_OK;
 }
 
@@ -2623,6 +2668,17 @@ int swm_execution_stats(const swm_solver_t* s, long long stats[6]) {
 int swm_status_reads(const swm_solver_t* s, long long* n) {
   if (!s) return SWM_E_ARG;
   return swm_engine_status_reads(s->e, n);
+}
+
+int swm_solve_stats(const swm_solver_t* s, long long stats[3]) {
+  if (!s) return SWM_E_ARG;
+  return swm_engine_solve_stats(s->e, stats);
+}
+
+int swm_debug_solve_polls(swm_solver_t* s, int polls) {
+  if (!s) return SWM_E_ARG;
+  s->e->solve_polls = polls < 0 ? kSolvePolls : std::min(polls, kSolvePolls);
+  return SWM_OK;
 }
 
 int swm_set_jacobi_limits(swm_solver_t* s, int max_iter, double tol) {

@@ -46,6 +46,7 @@ constexpr int kCellBlock = 256;       // cells per block of the pointwise kernel
 constexpr int kSolveThreads = 512;    // threads of a k_solve block
 constexpr int kSolveWindow = 4;       // Jacobi sweeps between two exchanges of k_solve's blocks
 constexpr int kSolveForms = 5;        // k_solve's tile sizes (solve_tiles)
+constexpr int kSolvePolls = 1 << 15;  // polls of a slot in k_solve's waits, about 25 ms
 constexpr int kMaxSys = 3;            // Patankar systems solved together (nodes 2..4)
 constexpr int kSlots = 3;             // concurrent FVTD evaluations per job
 constexpr int kStates = 6;            // state / derivative slots of the explicit schemes
@@ -124,9 +125,11 @@ struct JobStatus {
   double t, t_an, t_end;
   StepRec rec[kMaxBatch];
   // k_solve: rounds done so far by form and system, the base of the tags its
-  // blocks exchange; and 1 once a wait on another block ran out
+  // blocks exchange; polls of a slot before a wait is given up; and 1 once a wait
+  // ran out, until the next batch begins: polls is 0 then, and the batch's later
+  // solves give up their first exchange at once
   unsigned rounds[kSolveForms][kMaxSys];
-  int solve_lost;
+  int polls, solve_lost;
 };
 
 struct JobDev {
@@ -240,6 +243,7 @@ struct EngineArgs {
 // k_batch_begin's settings for every job of a batch (redo = 1: only jobs
 // halted by an overrun run, the others are masked).
 struct BatchArgs {
+  int polls;  // JobStatus::polls
   int max_steps;
   int redo;
   int loop;

@@ -1455,10 +1455,11 @@ __global__ __launch_bounds__(256) void k_decide(EngineArgs E, const int* jobs, S
 // the same: when it runs out (another process on the device, say), or a stop
 // decision lies inside the certified window, the solve ends as kSolveOpen, the
 // step is not committed and the host runs it again with the launches of one
-// sweep each.
+// sweep each.  After a wait that ran out the tags of the blocks no longer agree:
+// the job's solves that are on the stream already give up their first exchange
+// at once (JobStatus::polls; looked at before the sweeps it cost 1 us a launch),
+// and the host clears slots and rounds before the next one (engine_batch).
 // ------------------------------------------------------------------------
-constexpr int kSolvePolls = 1 << 15;  // about 25 ms
-
 __device__ __forceinline__ double agent_load(const double* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1559,6 +1560,7 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
   // own cells [ox, ox + ow) x [oy, oy + oh)
   int nb = 1, ox = 0, oy = 0, ow = nx, oh = ny;
   unsigned round0 = 0;
+  int most = 0;  // polls
   if (!ALONE) {
     const SolveTiles T = solve_tiles(nx, ny, W.form);
     nb = T.ntx * T.nty;
@@ -1567,6 +1569,7 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
     ow = min(T.tw, nx - ox);
     oh = min(T.th, ny - oy);
     round0 = st->rounds[W.form][s];
+    most = st->polls;
   }
   if (tid == 0) {
     L.lost = 0;
@@ -1770,7 +1773,7 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
       const int nk = half == 0 && t == 0 ? 3 : 2;
       unsigned long long v[3] = {tag, tag, tag};
       if (blk < nb) {
-        int polls = 0;
+        int polls = most;
         bool missing;
         do {
           missing = false;
@@ -1780,8 +1783,8 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
                                      __HIP_MEMORY_SCOPE_AGENT);
             missing |= (unsigned)(v[q] & 0xffu) != tag;
           }
-        } while (missing && ++polls < kSolvePolls);
-        if (missing) L.lost = 1;
+        } while (missing && --polls > 0);
+        if (missing || most <= 0) L.lost = 1;
       }
       for (int q = 0; q < nk; ++q) {
         const double w = wave_sum_dpp(__longlong_as_double((long long)(v[q] & ~0xffull)));
@@ -1895,7 +1898,10 @@ __device__ __forceinline__ void solve_block(SolveShared& L, const EngineArgs& E,
       if (own(i)) (to + row[i])[ci] = zero ? 0. : x[i];
   }
   if (tid == 0) {
-    if (!ALONE && L.lost) st->solve_lost = 1;  // keeps the step from being committed
+    if (!ALONE && L.lost) {
+      st->solve_lost = 1;  // keeps the step from being committed
+      st->polls = 0;
+    }
     if (W.tile == 0) {
       st->ended[first_solve + s] = end;
       st->iters[first_solve + s] = k_sweeps;
@@ -2071,6 +2077,7 @@ __global__ void k_batch_begin(EngineArgs E, const int* jobs, BatchArgs B) {
   }
   st->halt = kHaltNone;
   st->solve_lost = 0;
+  st->polls = B.polls;
   st->batch_done = 0;
   st->batch_max = B.max_steps;
   if (B.redo) return;  // the redone step keeps the loop's t

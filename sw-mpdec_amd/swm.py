@@ -18,6 +18,7 @@ PKG = Path(__file__).resolve().parent
 LIB_PATH = Path(os.environ.get("SWM_LIBRARY") or PKG / "lib" / "libswm.so")
 
 _dp = ctypes.POINTER(ctypes.c_double)
+SOLVE_STATS = ("steps", "lost", "resting")
 EXEC_STATS = ("speculative_steps", "redone_steps", "graph_launches", "graph_captures", "graph",
               "margin")
 _ip = ctypes.POINTER(ctypes.c_int)
@@ -138,6 +139,8 @@ def lib():
     L.swm_tile_shape.argtypes = [vp, ctypes.POINTER(ctypes.c_int)]
     L.swm_execution_stats.argtypes = [vp, ctypes.POINTER(ctypes.c_longlong)]
     L.swm_status_reads.argtypes = [vp, ctypes.POINTER(ctypes.c_longlong)]
+    L.swm_solve_stats.argtypes = [vp, ctypes.POINTER(ctypes.c_longlong)]
+    L.swm_debug_solve_polls.argtypes = [vp, ctypes.c_int]
     L.swm_stage_min_h.argtypes = [vp, _dp]
     L.swm_debug_weno5.argtypes = [ctypes.c_int, _dp, _dp, _dp]
     L.swm_profile_enable.argtypes = [vp, ctypes.c_int]
@@ -397,6 +400,18 @@ class Solver:
         self._check(lib().swm_status_reads(self._h, ctypes.byref(n)), "swm_status_reads")
         return n.value
 
+    def solve_stats(self):
+        """The one-launch Patankar solves: steps launched with them, waits that
+        ran out, batches left without them."""
+        out = (ctypes.c_longlong * 3)()
+        self._check(lib().swm_solve_stats(self._h, out), "swm_solve_stats")
+        return dict(zip(SOLVE_STATS, list(out)))
+
+    def debug_solve_polls(self, polls=-1):
+        """Polls after which a block of such a solve gives up waiting (0: at
+        once; -1: the default)."""
+        self._check(lib().swm_debug_solve_polls(self._h, int(polls)), "swm_debug_solve_polls")
+
     def set_tile_shape(self, shape=-1):
         """Face-kernel tile shape: 0 (16x16), 1 (32x16 / 16x32), -1 autotuned."""
         self._check(lib().swm_set_tile_shape(self._h, int(shape)), "swm_set_tile_shape")
@@ -554,6 +569,7 @@ def _engine_lib():
     L.swm_engine_tile_shape.argtypes = [vp, ctypes.POINTER(ctypes.c_int)]
     L.swm_engine_execution_stats.argtypes = [vp, ctypes.POINTER(ctypes.c_longlong)]
     L.swm_engine_status_reads.argtypes = [vp, ctypes.POINTER(ctypes.c_longlong)]
+    L.swm_engine_solve_stats.argtypes = [vp, ctypes.POINTER(ctypes.c_longlong)]
     L.swm_engine_stage_min_h.argtypes = [vp, ctypes.c_int, _dp]
     L._engine_bound = True
     return L
@@ -770,6 +786,11 @@ class Engine:
         self._check(_engine_lib().swm_engine_status_reads(self._e, ctypes.byref(n)),
                     "swm_engine_status_reads")
         return n.value
+
+    def solve_stats(self):
+        out = (ctypes.c_longlong * 3)()
+        self._check(_engine_lib().swm_engine_solve_stats(self._e, out), "swm_engine_solve_stats")
+        return dict(zip(SOLVE_STATS, list(out)))
 
     def set_tile_shape(self, shape=-1):
         self._check(_engine_lib().swm_engine_set_tile_shape(self._e, int(shape)),
