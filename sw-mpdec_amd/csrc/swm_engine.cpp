@@ -263,7 +263,7 @@ struct swm_engine {
   Captured caps[2 * kGroups];    // captured steps by table set in use, with and without k_solve
   long long cap_clock = 0;
   Profiler prof;
-  std::shared_ptr<HostRing> ring;  // transfers of states
+  std::shared_ptr<HostRing> ring;  // downloads of states
   std::string err;
 };
 
@@ -1364,7 +1364,7 @@ int upload_state(swm_engine* e, Job& J, const double* U, int ghosts, double* h, 
   size_t cnt = 3 * (size_t)(nx + 2 * ghosts) * (ny + 2 * ghosts);
   Staging tmp;
   HIPCK(e, tmp.get(J, cnt));
-  hipError_t er = e->ring->to_device(tmp.p, U, cnt * sizeof(double), e->stream);
+  hipError_t er = hipMemcpyAsync(tmp.p, U, cnt * sizeof(double), hipMemcpyHostToDevice, e->stream);
   if (er == hipSuccess) {
     launch_aos_to_soa(nx, ny, ghosts, tmp.p, h, hu, hv, e->stream);
     er = hipGetLastError();

@@ -1,13 +1,19 @@
-// swm_transfer.hpp -- copies between the caller's pageable arrays and the
-// device for the boundary's large arrays.
+// swm_transfer.hpp -- copies of states from the device to the caller's arrays.
 //
-// A copy from or to pageable memory goes through the runtime: into fresh pages
-// it brought 1 MB down in 0.62 ms, 25 MB in 6.0 and 100 MB in 23.9 ms, one
-// thread taking the page faults and moving the bytes.  Here a few threads move
-// chunks between the array and a pinned ring, each chunk's transfer overlapping
-// the others' host copies: 0.24, 1.6 and 5 ms.  Upwards
-// the runtime pins larger arrays in place at 27 GB/s, as fast as the ring;
-// below that it takes 0.37 ms for 1 MB and 0.72 for 2, the ring 0.06 and 0.10.
+// A copy to pageable memory goes through the runtime, one thread taking the page
+// faults and moving the bytes.  Here a few threads move chunks between the array
+// and a pinned ring, each chunk's transfer overlapping the others' host copies.
+// Downloads by the runtime and by the ring, in us, with the layout kernel (fresh:
+// into an array whose pages are not there yet):
+//     bytes      fresh          used before    pinned
+//     0.39 MB     39 / 45         38 / 45        29 / 45
+//     0.96 MB    203 / 196        64 / 71        40 / 71
+//     1.6 MB     365 / 278       106 / 99        51 / 104
+//     6.3 MB     949 / 462       368 / 337      140 / 364
+//     101 MB    9503 / 4610     5803 / 4570    1823 / 4679
+// so the ring takes pageable arrays from 1.5 MB on, and the runtime pinned ones,
+// smaller ones and all uploads (fresh arrays of 0.39 MB 34 / 37, 1.6 MB 94 / 116,
+// 101 MB 3536 / 4798).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -47,25 +53,13 @@ class HostRing {
     if (ring_) (void)hipHostFree(ring_);
   }
 
-  // host[0..bytes) to the device, ordered on the stream (the caller
-  // synchronizes before host may change), and back, complete on return.  A
-  // transfer that finds the ring in use by another thread's leaves it to the
-  // runtime.
-  hipError_t to_device(void* dev, const void* host, size_t bytes, hipStream_t s) {
-    if (bytes <= kRingUp && use_.try_lock()) {
-      std::lock_guard<std::mutex> g(use_, std::adopt_lock);
-      if (prepare() == hipSuccess)
-        return copy(static_cast<char*>(dev), const_cast<char*>(static_cast<const char*>(host)),
-                    bytes, s, true);
-    }
-    return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
-  }
+  // The device's bytes to host, complete on return.  A transfer that finds the
+  // ring in use by another thread's leaves it to the runtime.
   hipError_t to_host(void* host, const void* dev, size_t bytes, hipStream_t s) {
-    if (use_.try_lock()) {
+    if (bytes >= kRingFrom && pageable(host) && use_.try_lock()) {
       std::lock_guard<std::mutex> g(use_, std::adopt_lock);
       if (prepare() == hipSuccess)
-        return copy(const_cast<char*>(static_cast<const char*>(dev)), static_cast<char*>(host),
-                    bytes, s, false);
+        return copy(static_cast<const char*>(dev), static_cast<char*>(host), bytes, s);
     }
     const hipError_t er = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
     return er == hipSuccess ? hipStreamSynchronize(s) : er;
@@ -74,9 +68,17 @@ class HostRing {
  private:
   HostRing() = default;
   static constexpr size_t kChunk = size_t(1) << 19;
-  static constexpr size_t kRingUp = size_t(4) << 20;
+  static constexpr size_t kRingFrom = 3 * kChunk;
   static constexpr int kThreads = 8;
   static constexpr int kSlots = 2 * kThreads;  // two per thread: one moves while one is copied
+
+  // Memory the runtime does not know.
+  static bool pageable(const void* p) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return true;
+  }
 
   hipError_t prepare() {
     hipError_t er = hipSuccess;
@@ -89,72 +91,61 @@ class HostRing {
     return er;
   }
 
-  // Slot i once its last transfer, of this call or an earlier one, is done.
-  hipError_t slot(int i, char*& p) {
-    p = ring_ + (size_t)i * kChunk;
-    return hipEventSynchronize(done_[i]);
-  }
-
-  hipError_t copy(char* dev, char* host, size_t bytes, hipStream_t s, bool up) {
-    if (bytes == 0) return hipSuccess;
+  // Two chunks of every thread are on their way at a time.  The first ones start
+  // before the threads do.  All are awaited, so the next call finds every slot free.
+  hipError_t copy(const char* dev, char* host, size_t bytes, hipStream_t s) {
     const size_t chunks = (bytes + kChunk - 1) / kChunk;
     // a thread costs about 20 us to start: one per 2 chunks
     const int nt = (int)std::min<size_t>(kThreads, (chunks + 1) / 2);
-    std::vector<hipError_t> err(nt, hipSuccess);
-    auto work = [&](int w) {
-      if (w > 0) (void)hipSetDevice(device_);
-      err[w] = up ? up_part(dev, host, bytes, chunks, nt, w, s)
-                  : down_part(dev, host, bytes, chunks, nt, w, s);
-    };
-    std::vector<std::thread> threads;
-    for (int w = 1; w < nt; ++w) {
-      try {
-        threads.emplace_back(work, w);
-      } catch (...) {  // no thread to be had: this one does its part
-        work(w);
+    hipError_t err[kThreads] = {};
+    for (size_t c = 0; c < std::min<size_t>(chunks, 2 * nt) && err[0] == hipSuccess; ++c)
+      err[0] = start(dev, bytes, c, nt, s);
+    if (err[0] == hipSuccess) {
+      auto work = [&](int w) {
+        if (w > 0) (void)hipSetDevice(device_);
+        err[w] = part(dev, host, bytes, chunks, nt, w, s);
+      };
+      std::thread threads[kThreads];
+      for (int w = 1; w < nt; ++w) {
+        try {
+          threads[w] = std::thread(work, w);
+        } catch (...) {  // no thread to be had: this one does its part
+          work(w);
+        }
       }
+      work(0);
+      for (int w = 1; w < nt; ++w)
+        if (threads[w].joinable()) threads[w].join();
     }
-    work(0);
-    for (std::thread& t : threads) t.join();
     for (hipError_t e : err)
-      if (e != hipSuccess) return e;
+      if (e != hipSuccess) {
+        (void)hipStreamSynchronize(s);
+        return e;
+      }
     return hipSuccess;
   }
 
   static size_t length(size_t bytes, size_t c) { return std::min(kChunk, bytes - c * kChunk); }
 
-  hipError_t up_part(char* dev, const char* host, size_t bytes, size_t chunks, int nt, int w,
-                     hipStream_t s) {
-    int turn = 0;
-    for (size_t c = w; c < chunks; c += nt, turn ^= 1) {
-      char* p;
-      hipError_t er = slot(2 * w + turn, p);
-      if (er != hipSuccess) return er;
-      std::memcpy(p, host + c * kChunk, length(bytes, c));
-      er = hipMemcpyAsync(dev + c * kChunk, p, length(bytes, c), hipMemcpyHostToDevice, s);
-      if (er == hipSuccess) er = hipEventRecord(done_[2 * w + turn], s);
-      if (er != hipSuccess) return er;
-    }
-    return hipSuccess;
+  // Chunk c is thread c % nt's, by turns in its two slots.
+  static int slot(size_t c, int nt) { return 2 * (int)(c % nt) + (int)(c / nt % 2); }
+
+  hipError_t start(const char* dev, size_t bytes, size_t c, int nt, hipStream_t s) {
+    const int i = slot(c, nt);
+    const hipError_t er = hipMemcpyAsync(ring_ + i * kChunk, dev + c * kChunk, length(bytes, c),
+                                         hipMemcpyDeviceToHost, s);
+    return er == hipSuccess ? hipEventRecord(done_[i], s) : er;
   }
 
-  hipError_t down_part(const char* dev, char* host, size_t bytes, size_t chunks, int nt, int w,
-                       hipStream_t s) {
-    auto start = [&](size_t c, int turn) {
-      char* p;
-      hipError_t er = slot(2 * w + turn, p);
-      if (er == hipSuccess)
-        er = hipMemcpyAsync(p, dev + c * kChunk, length(bytes, c), hipMemcpyDeviceToHost, s);
-      return er == hipSuccess ? hipEventRecord(done_[2 * w + turn], s) : er;
-    };
-    int turn = 0;
-    hipError_t er = (size_t)w < chunks ? start(w, 0) : hipSuccess;
-    for (size_t c = w; c < chunks && er == hipSuccess; c += nt, turn ^= 1) {
-      if (c + nt < chunks) er = start(c + nt, turn ^ 1);
+  hipError_t part(const char* dev, char* host, size_t bytes, size_t chunks, int nt, int w,
+                  hipStream_t s) {
+    hipError_t er = hipSuccess;
+    for (size_t c = w; c < chunks && er == hipSuccess; c += nt) {
+      const int i = slot(c, nt);
+      er = hipEventSynchronize(done_[i]);
       if (er != hipSuccess) break;
-      er = hipEventSynchronize(done_[2 * w + turn]);
-      if (er == hipSuccess)
-        std::memcpy(host + c * kChunk, ring_ + (size_t)(2 * w + turn) * kChunk, length(bytes, c));
+      std::memcpy(host + c * kChunk, ring_ + i * kChunk, length(bytes, c));
+      if (c + 2 * nt < chunks) er = start(dev, bytes, c + 2 * nt, nt, s);
     }
     return er;
   }
