@@ -1364,7 +1364,7 @@ int upload_state(swm_engine* e, Job& J, const double* U, int ghosts, double* h, 
   size_t cnt = 3 * (size_t)(nx + 2 * ghosts) * (ny + 2 * ghosts);
   Staging tmp;
   HIPCK(e, tmp.get(J, cnt));
-  hipError_t er = hipMemcpyAsync(tmp.p, U, cnt * sizeof(double), hipMemcpyHostToDevice, e->stream);
+  hipError_t er = e->ring->to_device(tmp.p, U, cnt * sizeof(double), e->stream);
   if (er == hipSuccess) {
     launch_aos_to_soa(nx, ny, ghosts, tmp.p, h, hu, hv, e->stream);
     er = hipGetLastError();

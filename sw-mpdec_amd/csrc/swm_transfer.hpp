@@ -1,19 +1,25 @@
-// swm_transfer.hpp -- copies of states from the device to the caller's arrays.
+// swm_transfer.hpp -- copies of states between the caller's arrays and the device.
 //
-// A copy to pageable memory goes through the runtime, one thread taking the page
-// faults and moving the bytes.  Here a few threads move chunks between the array
-// and a pinned ring, each chunk's transfer overlapping the others' host copies.
-// Downloads by the runtime and by the ring, in us, with the layout kernel (fresh:
-// into an array whose pages are not there yet):
-//     bytes      fresh          used before    pinned
-//     0.39 MB     39 / 45         38 / 45        29 / 45
-//     0.96 MB    203 / 196        64 / 71        40 / 71
-//     1.6 MB     365 / 278       106 / 99        51 / 104
-//     6.3 MB     949 / 462       368 / 337      140 / 364
-//     101 MB    9503 / 4610     5803 / 4570    1823 / 4679
-// so the ring takes pageable arrays from 1.5 MB on, and the runtime pinned ones,
-// smaller ones and all uploads (fresh arrays of 0.39 MB 34 / 37, 1.6 MB 94 / 116,
-// 101 MB 3536 / 4798).
+// A copy of pageable memory goes through the runtime, one thread taking the page
+// faults and moving the bytes, by way of a buffer of 16 MB per stream.  Here a few
+// threads move chunks between the array and a pinned ring of 8 MB, each chunk's way
+// over the bus, by a small kernel, overlapping the others' host copies.  By the
+// runtime and by the ring, in us, with the layout kernel; down: into an array whose
+// pages are not there yet; (new): the first transfer of a new solver, the ring's
+// pinning with it:
+//     bytes      down            up             down (new), after a step   up (new)
+//     3.8 MB      275 / 142      176 / 159        600 / 170                 180 / 160
+//     6.3 MB      426 / 200      244 / 221        980 / 210                 240 / 220
+//     25 MB      1525 / 618      754 / 692       3690 / 640          820-6100 / 700-1800
+//     101 MB    10283 / 3307    4031 / 2508     15700 / 2980        3900-9000 / 2500-3900
+// A first transfer of 2.2 MB takes 380 by the runtime and as much by the ring, which
+// has 0.3 ms of pinning then; so the ring takes pageable arrays from 3 MB on, and the
+// runtime smaller ones and pinned ones (6.3 MB down 140, 101 MB 1823).
+//
+// The chunks go by a kernel because the runtime's copies are not even: after a new
+// solver's first step some hundred of them take 0.1 ms more each than later ones
+// (25 MB down by chunks of 512 KB 5.4 ms, then 1.2), and the first pass over a new
+// stream's buffer takes 0.3 ms a MB wherever its pages were not used before.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -26,6 +32,9 @@
 #include <vector>
 
 namespace swm {
+
+// n doubles from device memory to the pinned ring or (up) back (swm_kernels.hip).
+void launch_ring_copy(const double* from, double* to, size_t n, bool up, hipStream_t s);
 
 class HostRing {
  public:
@@ -53,23 +62,22 @@ class HostRing {
     if (ring_) (void)hipHostFree(ring_);
   }
 
-  // The device's bytes to host, complete on return.  A transfer that finds the
-  // ring in use by another thread's leaves it to the runtime.
+  // The device's bytes (a multiple of 8) to host and back, complete on return.  A
+  // transfer that finds the ring in use by another thread's leaves it to the runtime.
   hipError_t to_host(void* host, const void* dev, size_t bytes, hipStream_t s) {
-    if (bytes >= kRingFrom && pageable(host) && use_.try_lock()) {
-      std::lock_guard<std::mutex> g(use_, std::adopt_lock);
-      if (prepare() == hipSuccess)
-        return copy(static_cast<const char*>(dev), static_cast<char*>(host), bytes, s);
-    }
-    const hipError_t er = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
-    return er == hipSuccess ? hipStreamSynchronize(s) : er;
+    char* d = const_cast<char*>(static_cast<const char*>(dev));
+    return transfer(d, static_cast<char*>(host), bytes, s, false);
+  }
+  hipError_t to_device(void* dev, const void* host, size_t bytes, hipStream_t s) {
+    char* h = const_cast<char*>(static_cast<const char*>(host));
+    return transfer(static_cast<char*>(dev), h, bytes, s, true);
   }
 
  private:
   HostRing() = default;
-  static constexpr size_t kChunk = size_t(1) << 19;
+  static constexpr size_t kChunk = size_t(1) << 20;
   static constexpr size_t kRingFrom = 3 * kChunk;
-  static constexpr int kThreads = 8;
+  static constexpr int kThreads = 4;
   static constexpr int kSlots = 2 * kThreads;  // two per thread: one moves while one is copied
 
   // Memory the runtime does not know.
@@ -85,25 +93,37 @@ class HostRing {
     for (int i = 0; i < kSlots && er == hipSuccess; ++i)
       if (!done_[i]) er = hipEventCreateWithFlags(&done_[i], hipEventDisableTiming);
     if (er == hipSuccess && !ring_) {
-      er = hipHostMalloc((void**)&ring_, kSlots * kChunk, hipHostMallocDefault);
+      er = hipHostMalloc((void**)&ring_, kSlots * kChunk, hipHostMallocCoherent);
       if (er != hipSuccess) ring_ = nullptr;
     }
     return er;
   }
 
-  // Two chunks of every thread are on their way at a time.  The first ones start
-  // before the threads do.  All are awaited, so the next call finds every slot free.
-  hipError_t copy(const char* dev, char* host, size_t bytes, hipStream_t s) {
+  hipError_t transfer(char* dev, char* host, size_t bytes, hipStream_t s, bool up) {
+    if (bytes >= kRingFrom && pageable(host) && use_.try_lock()) {
+      std::lock_guard<std::mutex> g(use_, std::adopt_lock);
+      if (prepare() == hipSuccess) return copy(dev, host, bytes, s, up);
+    }
+    const hipError_t er = up ? hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s)
+                             : hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
+    return er == hipSuccess ? hipStreamSynchronize(s) : er;
+  }
+
+  // Two chunks of every thread are on their way at a time; the first ones down
+  // start before the threads do.  All are awaited, so the next call finds every
+  // slot free.
+  hipError_t copy(char* dev, char* host, size_t bytes, hipStream_t s, bool up) {
     const size_t chunks = (bytes + kChunk - 1) / kChunk;
     // a thread costs about 20 us to start: one per 2 chunks
     const int nt = (int)std::min<size_t>(kThreads, (chunks + 1) / 2);
     hipError_t err[kThreads] = {};
-    for (size_t c = 0; c < std::min<size_t>(chunks, 2 * nt) && err[0] == hipSuccess; ++c)
-      err[0] = start(dev, bytes, c, nt, s);
+    for (size_t c = 0; !up && c < std::min<size_t>(chunks, 2 * nt) && err[0] == hipSuccess; ++c)
+      err[0] = start(dev, bytes, c, nt, s, false);
     if (err[0] == hipSuccess) {
       auto work = [&](int w) {
         if (w > 0) (void)hipSetDevice(device_);
-        err[w] = part(dev, host, bytes, chunks, nt, w, s);
+        err[w] = up ? part_up(dev, host, bytes, chunks, nt, w, s)
+                    : part_down(dev, host, bytes, chunks, nt, w, s);
       };
       std::thread threads[kThreads];
       for (int w = 1; w < nt; ++w) {
@@ -117,12 +137,13 @@ class HostRing {
       for (int w = 1; w < nt; ++w)
         if (threads[w].joinable()) threads[w].join();
     }
+    hipError_t first = up ? hipStreamSynchronize(s) : hipSuccess;
     for (hipError_t e : err)
       if (e != hipSuccess) {
         (void)hipStreamSynchronize(s);
         return e;
       }
-    return hipSuccess;
+    return first;
   }
 
   static size_t length(size_t bytes, size_t c) { return std::min(kChunk, bytes - c * kChunk); }
@@ -130,22 +151,37 @@ class HostRing {
   // Chunk c is thread c % nt's, by turns in its two slots.
   static int slot(size_t c, int nt) { return 2 * (int)(c % nt) + (int)(c / nt % 2); }
 
-  hipError_t start(const char* dev, size_t bytes, size_t c, int nt, hipStream_t s) {
+  hipError_t start(char* dev, size_t bytes, size_t c, int nt, hipStream_t s, bool up) {
     const int i = slot(c, nt);
-    const hipError_t er = hipMemcpyAsync(ring_ + i * kChunk, dev + c * kChunk, length(bytes, c),
-                                         hipMemcpyDeviceToHost, s);
+    double* d = reinterpret_cast<double*>(dev + c * kChunk);
+    double* r = reinterpret_cast<double*>(ring_ + i * kChunk);
+    launch_ring_copy(up ? r : d, up ? d : r, length(bytes, c) / sizeof(double), up, s);
+    const hipError_t er = hipGetLastError();
     return er == hipSuccess ? hipEventRecord(done_[i], s) : er;
   }
 
-  hipError_t part(const char* dev, char* host, size_t bytes, size_t chunks, int nt, int w,
-                  hipStream_t s) {
+  hipError_t part_down(char* dev, char* host, size_t bytes, size_t chunks, int nt, int w,
+                       hipStream_t s) {
     hipError_t er = hipSuccess;
     for (size_t c = w; c < chunks && er == hipSuccess; c += nt) {
       const int i = slot(c, nt);
       er = hipEventSynchronize(done_[i]);
       if (er != hipSuccess) break;
       std::memcpy(host + c * kChunk, ring_ + i * kChunk, length(bytes, c));
-      if (c + 2 * nt < chunks) er = start(dev, bytes, c + 2 * nt, nt, s);
+      if (c + 2 * nt < chunks) er = start(dev, bytes, c + 2 * nt, nt, s, false);
+    }
+    return er;
+  }
+
+  hipError_t part_up(char* dev, const char* host, size_t bytes, size_t chunks, int nt, int w,
+                     hipStream_t s) {
+    hipError_t er = hipSuccess;
+    for (size_t c = w; c < chunks && er == hipSuccess; c += nt) {
+      const int i = slot(c, nt);
+      if (c >= (size_t)(2 * nt)) er = hipEventSynchronize(done_[i]);
+      if (er != hipSuccess) break;
+      std::memcpy(ring_ + i * kChunk, host + c * kChunk, length(bytes, c));
+      er = start(dev, bytes, c, nt, s, true);
     }
     return er;
   }
