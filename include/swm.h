@@ -419,16 +419,21 @@ int swm_engine_fetch_output_primitive(swm_engine_t *e, int job_id, double *V);
 int swm_engine_release(swm_engine_t *e, int job_id);
 int swm_engine_set_jacobi_limits(swm_engine_t *e, int max_iter, double tol);
 /* Step execution (no counterpart in the reference; results are bitwise the
- * same in every mode).  Once every job has run a step, a step launches each
- * correction's predicted Jacobi sweeps (last step's counts + margin) without
- * reading back, replayed from a captured HIP graph when use_graph is 1, and
- * checks once before committing; a step whose solves needed more sweeps is
- * redone with read-backs.  -1 lets the built-in autotuner time the
- * candidates (face-kernel tile shape, then graph 0/1 x margin 1/2) on the
- * first speculative steps and keep the fastest; margin = -2 turns
- * speculation off (every step reads back).
- * stats: speculative steps, redone steps, graph launches, graph captures,
- * graph and margin in use. */
+ * same in every mode).  Grids up to about 1.1M cells have each Patankar solve in
+ * one launch that runs to its stop rule, and step without read-backs from the
+ * first step on, replayed from a captured HIP graph when use_graph is 1.
+ * Larger ones, and any while stage minima are tracked or while the one-launch
+ * solves rest (swm_engine_solve_stats), have a launch per sweep: once every such
+ * job has run a step, a step launches each correction's predicted sweeps (last
+ * step's counts + margin) without reading back, replayed when use_graph is 1,
+ * and checks once before committing; a step whose solves needed more sweeps is
+ * redone with read-backs.  For job sets with such grids -1 lets the built-in
+ * autotuner time the candidates (face-kernel tile shape, then graph 0/1 x margin
+ * 1/2) on the first speculative steps and keep the fastest.  A margin >= 0 limits
+ * the one-launch solves to the predicted sweeps as well; margin = -2 turns
+ * speculation, and with it those solves, off (every step reads back).
+ * stats: speculative steps, redone steps, graph launches, graph captures, and
+ * the graph and margin in use where there is a launch per sweep. */
 int swm_engine_set_execution(swm_engine_t *e, int use_graph, int margin);
 int swm_engine_execution_stats(const swm_engine_t *e, long long stats[6]);
 /* Times the host has waited for the device status so far (no counterpart in
@@ -447,10 +452,12 @@ int swm_engine_solve_stats(const swm_engine_t *e, long long stats[3]);
 /* Tile shape of the face kernels (no counterpart in the reference; results
  * are bitwise the same with every shape): 0 = 16x16 threads for both face
  * directions, 1 = 32x16 for x faces and 16x32 for y faces (fewer redundant
- * halo sweeps, more idle threads on small grids), -1 = chosen by the
- * autotuner (the default).  swm_engine_tile_shape returns the shape in use
- * (the tuned one once tuning has finished, 0 before) and, if dims is not
- * NULL, its x-kernel and y-kernel thread extents. */
+ * halo sweeps, more idle threads on small grids), -1 = chosen by the library
+ * (the default): by the autotuner for job sets with a launch per sweep, else 0;
+ * launches of at most 256 tiles of shape 0 then take half tiles with two lanes
+ * per cell instead.  swm_engine_tile_shape returns the shape in use (the tuned
+ * one once tuning has finished, 0 before; the half tiles are not reported) and,
+ * if dims is not NULL, its x-kernel and y-kernel thread extents. */
 int swm_engine_set_tile_shape(swm_engine_t *e, int shape);
 int swm_engine_tile_shape(const swm_engine_t *e, int dims[4]);
 

@@ -398,7 +398,10 @@ constexpr int kSolveAlone = 2048;
 // systems with several blocks take the tile size with the least launches times
 // launch time, kSolveUs (257^2 at 2, 3, 5, 8 and 11 rows per thread, about nine
 // sweeps): a larger tile makes a sweep longer, a further launch repeats all of
-// it.  Blocks without others to wait for come last and are not counted.
+// it.  Of the five sizes it takes the fastest, or one within 1% of it, on 49^2 to
+// 860^2 (a step of 230^2 in tiles of 2 to 11 rows per thread: 472, 344, 347, 376,
+// 434 us, it takes 3; 400^2: 712, 769, 711, 653, 712, it takes 8).  Blocks without
+// others to wait for come last and are not counted.
 constexpr double kSolveUs[kSolveForms] = {19., 24., 28., 35., 47.};
 
 void solve_tables(swm_engine* e, Tables& T) {
@@ -1038,6 +1041,16 @@ int step_body_graph(swm_engine* e, Tables& T, const StepPlan& P) {
 // that candidates timed while jobs join and leave compare fairly.
 // Explicit settings (swm_engine_set_execution, swm_engine_set_tile_shape)
 // override their dimension.
+//
+// Job sets whose grids k_solve takes are not timed (with margin -1: a set margin
+// limits its sweeps and is tuned as before).  There is no margin to choose; replay
+// gains nothing (16 steps without it and with it: 32^2 2.36 / 2.38 ms, 257^2 6.28 /
+// 6.36, 1024^2 54.7 / 54.8; 64 grids of 32^2 to 38^2 8.4 / 8.4) and capturing costs a
+// new solver's first step 0.08 to 0.15 ms, so they go without it; and the shapes
+// differ by 4% at most (16 steps of 257^2, 400^2, 512^2 and 1024^2 in 16x16 / 32x16
+// tiles: without bathymetry 6.34 / 6.39, 10.41 / 10.31, 15.4 / 15.1 and 55.1 / 55.0
+// ms, with it 6.62 / 6.86, 11.8 / 11.9, 17.5 / 18.1 and 68.4 / 67.3; 32^2 2.67 /
+// 3.15), so they keep the 16x16 tiles.
 struct TuneCand {
   int graph, margin, shape;
 };
@@ -1221,7 +1234,7 @@ int engine_batch(swm_engine* e, Tables& T, const SchemeDef* sc, int hp_assoc,
   if (spec) {
     int graph, margin;
     if (all_solved) {
-      graph = e->use_graph != 0;
+      graph = e->use_graph > 0;
       margin = 0;
     } else {
       tune_choice(e, graph, margin);

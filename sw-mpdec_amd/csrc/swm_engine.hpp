@@ -31,7 +31,8 @@ constexpr int kTile = 16;             // k_fvtd_source_update tiles: 16x16 cells
 // xw-1 faces per row; a y-face tile yw x yh threads and yh-1 faces per column;
 // a source tile sw x sh threads and cells.  Wider tiles recompute fewer halo
 // sweeps; narrower ones waste fewer threads on small grids.  The engine's
-// autotuner picks one.
+// autotuner picks one for job sets with a launch per sweep; the others, and the
+// explicit schemes before such a set has tuned, take the first.
 struct FaceShape {
   int xw, xh, yw, yh, sw, sh;
 };

@@ -172,8 +172,10 @@ __device__ __forceinline__ void weno5_den_exact(double qm2, double qm1, double q
 // The range in which a reconstruction takes the shared reciprocals: the three
 // (eps + beta)^2 in [2^-240, 2^240).  Then the products of recip3 and recip4
 // lie in 2^+-976, the alphas in [2^-244, 2^240], their sums in
-// [2^-244, 2^242] and the weights above 2^-486; and every q is finite and
-// below 2^100, since an Inf or NaN q would make one of the three Inf or NaN.
+// [2^-244, 2^242] and the weights above 2^-486; and every q is finite, since an
+// Inf or NaN q would make one of the three Inf or NaN, and below 2^512, where
+// the squares overflow (mostly far below: a q of 2^100 needs neighbours equal to
+// it, the betas being differences), so that the candidates are finite too.
 // They are squares, so their high words compare as unsigned integers (a NaN
 // of either sign is above the range): two three-operand min/max and two
 // compares instead of six FP64 compares.

@@ -385,8 +385,8 @@ class Solver:
 
     def set_execution(self, use_graph=-1, margin=-1):
         """Step execution mode (results are identical in every mode): use_graph
-        0/1, margin >= 0 extra speculative sweeps; -1 = autotuned; margin -2 =
-        no speculation."""
+        0/1, margin >= 0 extra speculative sweeps; -1 = the library's choice;
+        margin -2 = no speculation."""
         self._check(lib().swm_set_execution(self._h, use_graph, margin), "swm_set_execution")
 
     def execution_stats(self):
@@ -413,7 +413,8 @@ class Solver:
         self._check(lib().swm_debug_solve_polls(self._h, int(polls)), "swm_debug_solve_polls")
 
     def set_tile_shape(self, shape=-1):
-        """Face-kernel tile shape: 0 (16x16), 1 (32x16 / 16x32), -1 autotuned."""
+        """Face-kernel tile shape: 0 (16x16), 1 (32x16 / 16x32), -1 the library's
+        choice."""
         self._check(lib().swm_set_tile_shape(self._h, int(shape)), "swm_set_tile_shape")
 
     def tile_shape(self):

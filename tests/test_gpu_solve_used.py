@@ -37,6 +37,7 @@ def test_used_from_the_first_step(size):
     st = s.execution_stats()
     assert s.solve_stats() == {"steps": 3, "lost": 0, "resting": 0}
     assert st["speculative_steps"] == 3 and st["redone_steps"] == 0
+    assert st["graph_captures"] == 0  # replay gains nothing: only where it is asked for
     t = swm.Solver.from_problem(p)
     t.set_execution(0, -2)
     t.run_steps(3)
