@@ -62,7 +62,8 @@ class HostRing {
     if (ring_) (void)hipHostFree(ring_);
   }
 
-  // The device's bytes (a multiple of 8) to host and back, complete on return.  A
+  // The device's bytes (a multiple of 8) to host, complete on return, and back,
+  // ordered on the stream (the caller synchronizes before host may change).  A
   // transfer that finds the ring in use by another thread's leaves it to the runtime.
   hipError_t to_host(void* host, const void* dev, size_t bytes, hipStream_t s) {
     char* d = const_cast<char*>(static_cast<const char*>(dev));
@@ -104,8 +105,8 @@ class HostRing {
       std::lock_guard<std::mutex> g(use_, std::adopt_lock);
       if (prepare() == hipSuccess) return copy(dev, host, bytes, s, up);
     }
-    const hipError_t er = up ? hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s)
-                             : hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
+    if (up) return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
+    const hipError_t er = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
     return er == hipSuccess ? hipStreamSynchronize(s) : er;
   }
 
@@ -137,13 +138,13 @@ class HostRing {
       for (int w = 1; w < nt; ++w)
         if (threads[w].joinable()) threads[w].join();
     }
-    hipError_t first = up ? hipStreamSynchronize(s) : hipSuccess;
     for (hipError_t e : err)
       if (e != hipSuccess) {
         (void)hipStreamSynchronize(s);
         return e;
       }
-    return first;
+    // on the way up the last kernels may still run, out of the ring
+    return up ? hipStreamSynchronize(s) : hipSuccess;
   }
 
   static size_t length(size_t bytes, size_t c) { return std::min(kChunk, bytes - c * kChunk); }
